@@ -45,6 +45,16 @@ struct iu8_tile {
   // the share). The int32 sum does not depend on the order; tiles that start at different depths do
   // not all ask the same memory channels for the same K at the same time.
   int rot = 0;
+  int tab = 0;  // the tile's entry in the caller's tables (iu8_tabs)
+};
+
+// A caller that has a workgroup's tiles resolved up front may hand their row maps and scales over in LDS as well: entry
+// `tab` of a tile is BM rows of A (gathered and clamped), BM activation scales and BN weight scales. The K loop then
+// never waits for an ordinary load: those return in order behind the load stream, so one of them at a tile's end or at
+// the crossing into the next drains everything the stream has in flight.
+struct iu8_tabs {
+  const int *row;
+  const float *am, *ws;
 };
 
 // Dense tile order of a persistent launch of G workgroups over gx x gy tiles. The hardware deals
@@ -105,11 +115,11 @@ constexpr int iu8_pf32_lds_bytes() {
 // a fragment), turns them into codes by the law's own routine (iu8_code4_rcp: the bytes of the
 // producer kernel) one step later and writes the fragment into its stage; the weights keep their
 // LDS-DMA stream. One conversion a workgroup and step, whatever the columns of the tile.
-template <bool W8, int WMW, int WNW, int TM, int TN, bool ACC, int STMAX, bool DEEP = false, bool SPARSE = false, bool ARM = false, bool EXT_LDS = false, bool AQ = false, class TileAt>
+template <bool W8, int WMW, int WNW, int TM, int TN, bool ACC, int STMAX, bool DEEP = false, bool SPARSE = false, bool ARM = false, bool EXT_LDS = false, bool AQ = false, bool TAB = false, class TileAt>
 __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const float *__restrict__ as,
                                              void *__restrict__ Cv, int N, int K, TileAt tile_at,
                                              int *__restrict__ P = nullptr, int *__restrict__ cnt = nullptr,
-                                             iu8_u8 *ext_lds = nullptr) {
+                                             iu8_u8 *ext_lds = nullptr, iu8_tabs tabs = {}) {
   // tile_at(r, t): fills the workgroup's r-th tile, false when it has none
   constexpr int NWAVE = WMW * WNW;
   constexpr int BMT = WMW * TM * 2, BNT = WNW * TN * 2;  // 16-row tiles a workgroup, both ways
@@ -182,7 +192,7 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
       // rows past the edge: the last one of the padded 16-row tile (the int8 operand is padded to whole tiles); the
       // fused-quant form reads the caller's bf16 rows and their scales, which hold exactly `rows` rows: the last live one
       const int mrow = t.mbase + (f >> 1) * 16 + (lane & 15);
-      const int ar = iu8_arow(t.R, AQ ? min(mrow, t.R.rows - 1) : mrow);
+      const int ar = TAB ? tabs.row[t.tab * BM + mrow - t.mbase] : iu8_arow(t.R, AQ ? min(mrow, t.R.rows - 1) : mrow);
       if constexpr (AQ) {  // bf16 rows: 2 bytes an element
         oa[p] = (unsigned)(((size_t)ar * K + (f & 1) * 64 + (lane >> 4) * 16) * 2);
         os[p] = as[ar];
@@ -200,7 +210,7 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) iu8_u8 *)smem;
   // (with fewer K steps a tile than the stream runs ahead, it would be more than one tile ahead of the MFMAs and
   // two sets would not do: such a launch fetches the scales in the epilogue)
-  const bool stashed = iu8_pf32_stashes<SPARSE, WMW, WNW, TM, TN>() && steps >= NST + (DEEP ? 1 : 0);  // the stream's lead in steps (the deep form fetches a step ahead of its MFMAs), and one to spare
+  const bool stashed = !TAB && iu8_pf32_stashes<SPARSE, WMW, WNW, TM, TN>() && steps >= NST + (DEEP ? 1 : 0);  // the stream's lead in steps (the deep form fetches a step ahead of its MFMAs), and one to spare
   // Rows in place: both tables come by LDS-DMA like the operands (a dword a lane, 64 consecutive entries a
   // wave-load), so nothing waits for them at the crossing. Gathered rows: the row's scale hangs on its
   // row_tok entry, an ordinary dependent load -- the crossing of such a tile waits for that entry anyway,
@@ -652,13 +662,13 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const int m = C.mbase + (wm * TM + i) * 32 + r32;
-        const float am = as[iu8_arow(C.R, min(m, M - 1))];
+        const float am = TAB ? tabs.am[C.tab * BM + m - C.mbase] : as[iu8_arow(C.R, min(m, M - 1))];
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             const int n = ncol0 + j * 32 + g * 8 + nq;
-            const float4 w4 = *(const float4 *)(C.ws + min(n, N - 4));
+            const float4 w4 = TAB ? *(const float4 *)&tabs.ws[C.tab * BN + n - C.nt0 * 16] : *(const float4 *)(C.ws + min(n, N - 4));
             const float u = W8 ? 1.f : 0.0625f;  // exact: a power of two
             const unsigned lo = iu8_bf16_pack(iu8_epi(acc[i][j][g * 4], am, w4.x * u), iu8_epi(acc[i][j][g * 4 + 1], am, w4.y * u));
             const unsigned hi = iu8_bf16_pack(iu8_epi(acc[i][j][g * 4 + 2], am, w4.z * u), iu8_epi(acc[i][j][g * 4 + 3], am, w4.w * u));
@@ -677,7 +687,9 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
       float am[TM];
 #pragma unroll
       for (int i = 0; i < TM; ++i)
-        am[i] = stashed ? s_am[r & 1][(wm * TM + i) * 32 + r32] : as[iu8_arow(C.R, min(C.mbase + (wm * TM + i) * 32 + r32, M - 1))];
+        am[i] = TAB       ? tabs.am[C.tab * BM + (wm * TM + i) * 32 + r32]
+                : stashed ? s_am[r & 1][(wm * TM + i) * 32 + r32]
+                          : as[iu8_arow(C.R, min(C.mbase + (wm * TM + i) * 32 + r32, M - 1))];
       // a column block's weight scales are read once, for all the wave's row blocks
 #pragma unroll
       for (int jb = 0; jb < TN / CB; ++jb) {
@@ -686,7 +698,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
         for (int jj = 0; jj < CB; ++jj)
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            const float4 w4 = stashed ? *(const float4 *)&s_wsu[r & 1][wn * TN * 32 + jb * (CB * 32) + jj * 32 + g * 8 + nq]
+            const float4 w4 = TAB       ? *(const float4 *)&tabs.ws[C.tab * BN + wn * TN * 32 + jb * (CB * 32) + jj * 32 + g * 8 + nq]
+                              : stashed ? *(const float4 *)&s_wsu[r & 1][wn * TN * 32 + jb * (CB * 32) + jj * 32 + g * 8 + nq]
                                       : *(const float4 *)(C.ws + min(ncol0 + jb * (CB * 32) + jj * 32 + g * 8 + nq, N - 4));
             const float u = W8 ? 1.f : 0.0625f;  // exact: a power of two
             wsu[jj][g] = float4{w4.x * u, w4.y * u, w4.z * u, w4.w * u};

@@ -733,10 +733,16 @@ MOE_GROUPED_DEC(moe_iu8_grouped_w4_decpb_g1, true, 4, 8, 8, 2, 0, 1, 5)
 // An expert's last tile is often nearly empty. On the tile cell such a tile still moves whole stages
 // of mostly dead rows behind a barrier a step: measured, some 70 % of a full tile's time for a
 // twentieth of its work. The two-cell form (LIGHT) runs the light tiles on a second cell in the same
-// LDS, 64 rows x 256 columns (2 x 4 waves, the deep form of iu8_pf32.h), whose small stages keep five
-// steps of loads in flight and move no dead rows; its K steps start at a depth that differs from
-// item to item (iu8_tile::rot), which spreads the weight streams of the light items over the memory
-// channels (512 tokens, gate+up: 187 -> 160 us). Light tiles together are bound by the memory rate,
+// LDS, 64 rows x 256 columns, whose small stages keep four steps of loads in flight and move no dead
+// rows; its K steps start at a depth that differs from item to item (iu8_tile::rot), which spreads
+// the weight streams of the light items over the memory channels (512 tokens, gate+up: 187 -> 160 us).
+// The light cell's eight waves stand side by side, each 64 rows x 32 columns: a W4 operand is unpacked
+// once and serves both row blocks (on 2 x 4 waves every weight fragment was read from LDS and unpacked
+// twice, and an item of mostly few rows is bound by that issue work once its weights arrive), and rows,
+// activation scales and weight scales of the light items come from tables in LDS (iu8_tabs), filled
+// beside the item table: no ordinary load stands between two items and drains the stream (a layer at
+// 120 / 300 / 1,000 / 2,000 tokens: 269 / 277 / 337 / 493 us on 2 x 4 waves in the deep form, 259 / 266 /
+// 335 / 482 on 8 waves side by side, 252 / 261 / 329 / 479 with the tables). Light tiles together are bound by the memory rate,
 // the heavy ones by the matrix pipes, so a workgroup runs its light items between two parts of its
 // heavy ones, after (workgroup / 8) mod (rounds + 1) rounds, the light walk dealt from the last
 // workgroup down: at any time a slice of every XCD's CUs streams light tiles under the others'
@@ -750,7 +756,7 @@ MOE_GROUPED_DEC(moe_iu8_grouped_w4_decpb_g1, true, 4, 8, 8, 2, 0, 1, 5)
 // light tile (1,536 to 2,048 tokens) lost 2 to 4 % to the two-cell kernel's heavier item switch.
 #define MOE_ORDER_CAP 4096  // tiles the ordering holds in LDS; beyond, table order on the big cell
 #define MOE_LIGHT_ROWS 64
-#define MOE_LIGHT_ST 6
+#define MOE_LIGHT_ST 5
 #define MOE_HEAVY_ROUNDS 8  // rounds of items a workgroup resolves at a time: the item table in LDS
 #define MOE_LIGHT_ROUNDS 8
 struct moe_item {
@@ -871,20 +877,23 @@ static __device__ __forceinline__ void moe_grouped_pf_two(
   constexpr int BN = WNW * TN * 32;
   static_assert(BN == 256 && WMW * WNW == 8, "both cells are 8 waves and 256 columns wide");
   constexpr int LB = iu8_pf32_lds_bytes<false, WMW, WNW, TM, TN, ST, true>();
-  constexpr int LL = iu8_pf32_lds_bytes<false, 2, 4, 1, 2, MOE_LIGHT_ST>();
+  constexpr int LL = iu8_pf32_lds_bytes<false, 1, 8, 2, 1, MOE_LIGHT_ST>();
   __shared__ __attribute__((aligned(1024))) iu8_u8 lds[LB > LL ? LB : LL];
   __shared__ unsigned short s_order[MOE_ORDER_CAP];
   /* the walk's numbers and this workgroup's resolved items live in LDS */
   __shared__ int s_par[4];
   __shared__ moe_item s_item[MOE_HEAVY_ROUNDS + MOE_LIGHT_ROUNDS];
+  __shared__ int s_row[MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS];
+  __shared__ float s_am[MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS];
+  __shared__ __attribute__((aligned(16))) float s_ws[MOE_LIGHT_ROUNDS * BN];
   auto par = [&](int i) { return __builtin_amdgcn_readfirstlane(((volatile int *)s_par)[i]); };
-  auto item = [&](int q, iu8_tile &t) {
+  auto item = [&](int q, iu8_tile &t, int tab = 0) {
     const volatile int *p32 = (const volatile int *)&s_item[q];
     auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(p32[i]); };
     if (u(1) < 0) return false;
     const unsigned long long wp = (unsigned)u(4) | ((unsigned long long)(unsigned)u(5) << 32);
     const unsigned long long sp = (unsigned)u(6) | ((unsigned long long)(unsigned)u(7) << 32);
-    t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, u(0), u(1)}, 0, u(2), (const unsigned char *)wp, (const float *)sp, 0, u(3)};
+    t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, u(0), u(1)}, 0, u(2), (const unsigned char *)wp, (const float *)sp, 0, u(3), tab};
     return true;
   };
   const int nt = meta[0];
@@ -919,12 +928,30 @@ static __device__ __forceinline__ void moe_grouped_pf_two(
         s_item[q] = it;
       }
       __syncthreads();
+      /* the light items' tables: rows of A, their scales, the columns' scales */
+      static_assert(MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS == WMW * WNW * 64 && MOE_LIGHT_ROUNDS * BN == WMW * WNW * 64 * 4, "a thread an entry");
+      if (lrounds > 0) {
+        const int ri = threadIdx.x / MOE_LIGHT_ROWS, m = threadIdx.x % MOE_LIGHT_ROWS;
+        const int ci = threadIdx.x / (BN / 4), col = threadIdx.x % (BN / 4) * 4;
+        if (ri < lrounds && s_item[rounds + ri].rows > 0) {
+          const moe_item &it = s_item[rounds + ri];
+          const int ar = iu8_arow(iu8_rows{GATHER ? row_tok : nullptr, it.row0, it.rows}, m);
+          s_row[threadIdx.x] = ar;
+          s_am[threadIdx.x] = as[GATHER ? ar : min(ar, it.row0 + it.rows - 1)];
+        }
+        if (ci < lrounds && s_item[rounds + ci].rows > 0) {
+          const moe_item &it = s_item[rounds + ci];
+          *(float4 *)&s_ws[threadIdx.x * 4] = *(const float4 *)(it.ws + min(it.nt0 * 16 + col, n - 4));
+        }
+        __syncthreads();
+      }
     }
     for (int part = 0; part < 2; ++part) {
       if (part == 1) {
         if (par(1) == 0) break;
-        iu8_pf32_run<false, 2, 4, 1, 2, false, MOE_LIGHT_ST, true, false, GATHER == 2, true>(
-            a, as, c, n, k, [&](int r, iu8_tile &t) { return r < par(1) && item(par(0) + r, t); }, nullptr, nullptr, lds);
+        iu8_pf32_run<false, 1, 8, 2, 1, false, MOE_LIGHT_ST, false, true, GATHER == 2, true, false, true>(
+            a, as, c, n, k, [&](int r, iu8_tile &t) { return r < par(1) && item(par(0) + r, t, r); }, nullptr, nullptr, lds,
+            iu8_tabs{s_row, s_am, s_ws});
         __syncthreads();
       }
       iu8_pf32_run<false, WMW, WNW, TM, TN, false, ST, false, true, GATHER == 2, true>(

@@ -325,6 +325,24 @@ def test_grouped_tile_kernels_on_a_tiny_grid(ctx):
         assert torch.equal(layer.gu[:rows][live], want[:rows][live])
 
 
+@pytest.mark.parametrize("counts", [(1, 16, 17, 32, 33, 63, 64, 65), (2, 15, 31, 34, 47, 48, 49, 66)])
+def test_light_tiles_at_their_edges(ctx, counts):
+    """Experts of exactly the rows at which a light tile changes shape (a row, a 16-row block, a 32-row
+    MFMA block and one to either side, the heavy limit), on a K shorter and one longer than the load
+    stream's lead and a last column block that is half empty: same bytes as the oracle."""
+    say(f"light tiles of {counts} rows")
+    T, E, k, H, I = max(counts), 128, 8, 640, 384
+    case = synth.moe_case(T=T, E=E, topk=k, H=H, I=I, seed=sum(counts), experts=4)
+    lg = np.zeros((T, E), np.float32)
+    for s, c in enumerate(counts):
+        lg[:c, s] = 8.0 - 0.5 * s       # the first c tokens' route s
+        lg[c:, 8 + s] = 8.0 - 0.5 * s   # the others': a second set of experts
+    case["logits"] = synth.f32_to_bf16_bits(lg)
+    layer = run_layer(ctx, case, tile_blocks=8, fused_back=False)
+    check_layer(layer, case)
+    assert sorted(layer.buf["expert_cnt"].tolist())[-16:] == sorted(list(counts) + [T - c for c in counts])
+
+
 def test_moe_router_ties_and_skew(ctx):
     say("moe router: ties and one hot expert")
     case = synth.moe_case(T=40, E=128, topk=8, H=512, I=256, seed=5, experts=4)
