@@ -176,17 +176,19 @@ static __device__ __forceinline__ float iu8_wave_max_nonneg(float v) {
 // memory and its completion (vmcnt) means it is visible there, such a load comes from there. So a
 // producer stores its partials this way, waits for their completion, meets its workgroup and bumps a
 // device-scope atomic counter; the consumer that finds the counter full loads the partials this way.
-// The order is the hardware's in-order completion count, not a language-level fence: these helpers
-// are asm for that reason.
+// The order is the hardware's in-order completion count, not a language-level fence: the store and its
+// wait are asm for that reason; the loads stand behind the counter's value, a branch and a barrier.
 static __device__ __forceinline__ void iu8_store_through(int *p, iu8_v4i v) {
   // the wait states behind it: a store of more than 8 bytes reads its data registers for two more
   // cycles, and the compiler's hazard recognizer does not look inside an asm statement
   asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
 }
 static __device__ __forceinline__ iu8_v4i iu8_load_through(const int *p) {
-  iu8_v4i v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" : "=v"(v) : "v"(p) : "memory");
-  return v;
+  // two relaxed system-scope loads: both scope bits, no fence, and the compiler counts them, so many can be in flight
+  const unsigned long long *q = (const unsigned long long *)p;
+  const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  const unsigned long long hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  return iu8_v4i{(int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32)};
 }
 static __device__ __forceinline__ void iu8_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // one lane, after the workgroup met behind its completed stores: count the arrival

@@ -83,6 +83,14 @@ template <bool SPARSE, int WMW, int WNW, int TM, int TN>
 constexpr bool iu8_pf32_stashes() {
   return SPARSE && WMW * TM * 32 * WNW * TN * 32 >= 128 * 256;
 }
+// A loaded value is taken here, on every path. What the epilogue loads and uses only under a test (rows or columns of the
+// tile that exist) otherwise stays an open load to the compiler when control returns to the K loop, which then re-uses
+// those registers: it puts an `s_waitcnt vmcnt(0)` in front of the re-use, inside the loop, and every K step waits for all
+// of the load stream -- the stages ahead of the MFMAs are then worth one. (Taken in the deep form and the
+// small-tile epilogue alone: the cells of large wave tiles, whose steps are long, measured 0-4 % slower with it.)
+static __device__ __forceinline__ void iu8_taken(float &v) { asm volatile("" : "+v"(v)); }
+static __device__ __forceinline__ void iu8_taken(float4 &v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+
 // LDS bytes of a cell (what iu8_pf32_run declares, or expects from its caller): its stages and, where the
 // cell stashes them (STASH: iu8_pf32_stashes), two sets of a tile's epilogue scales (BM + BN floats each)
 // behind them.
@@ -599,7 +607,14 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
     const int ncol0 = (C.nt0 + wn * TN * 2) * 16;  // first column of the wave tile
     if (Z > 1) {
       // ---- a share of K: the partial goes out straight through memory, the last share to arrive at
-      // the tile's counter sums all of them in share order (exact in int32) and runs the epilogue
+      // the tile's counter adds the others' to its own registers (exact in int32, so in any order) and
+      // runs the epilogue. A share's partials lie quad-major, [N / 4][M][4 columns]: a wave's store and
+      // load of one accumulator quad are two runs of 512 bytes, at the same addresses in every share, and
+      // the reader asks for three shares of a block before it adds the first. (Row-major, read back one
+      // quad at a time by an element loop, the last arriver's loads were some 23 memory round trips in a
+      // row: 5120 x 17408 at 45 / 64 / 128 / 180 rows 25.2 / 28.9 / 31.0 / 35.3 us,
+      // now 18.5 / 19.3 / 22.8 / 28.5, the wave layout included.)
+      auto part = [&](int zq, int m, int n) { return P + (((size_t)zq * (N >> 2) + (n >> 2)) * M + m) * 4; };
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const int m = C.mbase + (wm * TM + i) * 32 + r32;
@@ -611,7 +626,7 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
             if (m >= M || n >= N) continue;
             const iu8_v4i v = share_empty ? iu8_v4i{0, 0, 0, 0}
                                           : iu8_v4i{acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
-            iu8_store_through(&P[((size_t)z * M + C.R.row0 + m) * N + n], v);
+            iu8_store_through(part(z, m, n), v);
           }
       }
       iu8_stores_done();
@@ -620,23 +635,52 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
       wait_vm(std::integral_constant<int, 63>{}, true);
       __builtin_amdgcn_s_barrier();
       if (s_last) {
-              if (tid == 0) __hip_atomic_store(&cnt[C.id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        constexpr int BM = WMW * TM * 32, BN = WNW * TN * 32;
-        const int nb = C.nt0 * 16, rows = min(BM, M - C.mbase), cols4 = min(BN, N - nb) >> 2;
-        for (int idx = tid; idx < rows * cols4; idx += NWAVE * 64) {
-          const int r = idx / cols4, m = C.mbase + r, n = nb + (idx - r * cols4) * 4;
-          iu8_v4i sum = iu8_v4i{0, 0, 0, 0};
-          for (int q = 0; q < Z; ++q) sum += iu8_load_through(&P[((size_t)q * M + C.R.row0 + m) * N + n]);
-          const size_t crow = (size_t)(C.R.row0 + m) * N;
-          if constexpr (ACC) {
-            *(iu8_v4i *)((int *)Cv + crow + n) = sum;
-          } else {
-            const float am = as[iu8_arow(C.R, m)];
-            const float4 w4 = *(const float4 *)(C.ws + n);
-            const float u = W8 ? 1.f : 0.0625f;
-            const unsigned lo = iu8_bf16_pack(iu8_epi(sum[0], am, w4.x * u), iu8_epi(sum[1], am, w4.y * u));
-            const unsigned hi = iu8_bf16_pack(iu8_epi(sum[2], am, w4.z * u), iu8_epi(sum[3], am, w4.w * u));
-            *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{lo, hi};
+        if (tid == 0) __hip_atomic_store(&cnt[C.id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        constexpr int SH = 3;  // shares asked for at a time
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int m = C.mbase + (wm * TM + i) * 32 + r32;
+          const float am = as[iu8_arow(C.R, min(m, M - 1))];
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            iu8_v4i sum[4];
+            float4 w4[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) w4[g] = *(const float4 *)(C.ws + min(ncol0 + j * 32 + g * 8 + nq, N - 4));
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+              sum[g] = share_empty ? iu8_v4i{0, 0, 0, 0}
+                                   : iu8_v4i{acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
+            for (int q0 = 1; q0 < Z; q0 += SH) {
+              iu8_v4i v[SH][4];
+#pragma unroll
+              for (int u = 0; u < SH; ++u)
+                if (q0 + u < Z) {
+                  const int zq = z + q0 + u < Z ? z + q0 + u : z + q0 + u - Z;
+#pragma unroll
+                  for (int g = 0; g < 4; ++g) v[u][g] = iu8_load_through(part(zq, min(m, M - 1), min(ncol0 + j * 32 + g * 8 + nq, N - 4)));
+                }
+#pragma unroll
+              for (int u = 0; u < SH; ++u)
+                if (q0 + u < Z) {
+#pragma unroll
+                  for (int g = 0; g < 4; ++g) sum[g] += v[u][g];
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const int n = ncol0 + j * 32 + g * 8 + nq;
+              if (m >= M || n >= N) continue;
+              const size_t at = (size_t)(C.R.row0 + m) * N + n;
+              if constexpr (ACC) {
+                *(iu8_v4i *)((int *)Cv + at) = sum[g];
+              } else {
+                const float u = W8 ? 1.f : 0.0625f;
+                const unsigned lo = iu8_bf16_pack(iu8_epi(sum[g][0], am, w4[g].x * u), iu8_epi(sum[g][1], am, w4[g].y * u));
+                const unsigned hi = iu8_bf16_pack(iu8_epi(sum[g][2], am, w4[g].z * u), iu8_epi(sum[g][3], am, w4[g].w * u));
+                *(iu8_v2u *)((unsigned short *)Cv + at) = iu8_v2u{lo, hi};
+              }
+            }
           }
         }
       }
@@ -662,13 +706,15 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const int m = C.mbase + (wm * TM + i) * 32 + r32;
-        const float am = TAB ? tabs.am[C.tab * BM + m - C.mbase] : as[iu8_arow(C.R, min(m, M - 1))];
+        float am = TAB ? tabs.am[C.tab * BM + m - C.mbase] : as[iu8_arow(C.R, min(m, M - 1))];
+        iu8_taken(am);
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             const int n = ncol0 + j * 32 + g * 8 + nq;
-            const float4 w4 = TAB ? *(const float4 *)&tabs.ws[C.tab * BN + n - C.nt0 * 16] : *(const float4 *)(C.ws + min(n, N - 4));
+            float4 w4 = TAB ? *(const float4 *)&tabs.ws[C.tab * BN + n - C.nt0 * 16] : *(const float4 *)(C.ws + min(n, N - 4));
+            iu8_taken(w4);
             const float u = W8 ? 1.f : 0.0625f;  // exact: a power of two
             const unsigned lo = iu8_bf16_pack(iu8_epi(acc[i][j][g * 4], am, w4.x * u), iu8_epi(acc[i][j][g * 4 + 1], am, w4.y * u));
             const unsigned hi = iu8_bf16_pack(iu8_epi(acc[i][j][g * 4 + 2], am, w4.z * u), iu8_epi(acc[i][j][g * 4 + 3], am, w4.w * u));
@@ -690,6 +736,10 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
         am[i] = TAB       ? tabs.am[C.tab * BM + (wm * TM + i) * 32 + r32]
                 : stashed ? s_am[r & 1][(wm * TM + i) * 32 + r32]
                           : as[iu8_arow(C.R, min(C.mbase + (wm * TM + i) * 32 + r32, M - 1))];
+      if constexpr (DEEP) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) iu8_taken(am[i]);
+      }
       // a column block's weight scales are read once, for all the wave's row blocks
 #pragma unroll
       for (int jb = 0; jb < TN / CB; ++jb) {
@@ -704,6 +754,12 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
             const float u = W8 ? 1.f : 0.0625f;  // exact: a power of two
             wsu[jj][g] = float4{w4.x * u, w4.y * u, w4.z * u, w4.w * u};
           }
+        if constexpr (DEEP) {
+#pragma unroll
+          for (int jj = 0; jj < CB; ++jj)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) iu8_taken(wsu[jj][g]);
+        }
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
           if (C.mbase + (wm * TM + i) * 32 >= M) continue;  // a row block past the tile's rows (the whole wave)

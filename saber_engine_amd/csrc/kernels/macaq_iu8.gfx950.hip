@@ -128,7 +128,7 @@ IU8_PF32K(macaq_iu8_pf_w4_t128x128_ks, false, 4, 2, 1, 2, 3, 1, false)
 IU8_PF32K(macaq_iu8_pf_w8_t128x128_ks, true, 4, 2, 1, 2, 3, 1, false)
 IU8_PF32K(macaq_iu8_pf_w4_t256x160_ks, false, 8, 1, 1, 5, 3, 1, false)
 IU8_PF32K(macaq_iu8_pf_w8_t256x160_ks, true, 8, 1, 1, 5, 3, 1, false)
-IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 2, 2, 1, 2, 5, 2, true)
+IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 1, 4, 2, 1, 5, 2, true)
 #undef IU8_PF32K
 #define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP)
 #include "iu8_variants.def"
