@@ -278,15 +278,20 @@ static bool int_arg(const saber_iu8_desc &d, const char *name, int64_t *v) {
 // tiling and one staging form), M and K.
 int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_desc *out, int order) {
   static const char PREFIX[] = "macaq_iu8_dec_w4_";
-  // a half the law gave the staged persistent form is paired as its streamed form: the pair kernels are that geometry
+  // a half the law gave the staged persistent form, or 17 to 48 rows at another block width, is paired as its streamed
+  // form: the pair kernels are that geometry
+  auto other_form = [](const saber_iu8_desc &h) {
+    return !strncmp(h.kernel, "macaq_iu8_dec_w4_tm1_s80", 24) || !strcmp(h.kernel, "macaq_iu8_dec_w4_tm2_n1") ||
+           !strcmp(h.kernel, "macaq_iu8_dec_w4_tm3_n2");
+  };
   for (const saber_iu8_desc *h : {&first, &second})
-    if (!strncmp(h->kernel, "macaq_iu8_dec_w4_tm1_s80", 24)) {
+    if (other_form(*h)) {
       saber_iu8_desc s[2];
       const saber_iu8_desc *in[2] = {&first, &second};
       for (int i = 0; i < 2; ++i) {
         int64_t hm = 0, hn = 0, hk = 0;
         s[i] = *in[i];
-        if (!strncmp(in[i]->kernel, "macaq_iu8_dec_w4_tm1_s80", 24)) {
+        if (other_form(*in[i])) {
           if (!int_arg(*in[i], "m", &hm) || !int_arg(*in[i], "n", &hn) || !int_arg(*in[i], "k", &hk))
             return fail(SABER_IU8_E_RULE, "macaq iu8 pair: a half without its m, n, k");
           if (int rc = describe(dec_stream_name("w4", (uint32_t)hm, (uint32_t)hk), (uint32_t)hm, (uint32_t)hn, (uint32_t)hk, 1, &s[i])) return rc;
@@ -342,17 +347,21 @@ int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_de
 
 int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) {
   if (wkind != SABER_IU8_W4 && wkind != SABER_IU8_W8) return fail(SABER_IU8_E_ARG, "unknown weight kind");
-  const char *tag = wkind == SABER_IU8_W8 ? "w8" : "w4";
-  if (int rc = check_shape(wkind == SABER_IU8_W8 ? "gemm_i8a8" : "gemm_i4a8", m, n, k)) return rc;
+  const bool w8 = wkind == SABER_IU8_W8;
+  const char *tag = w8 ? "w8" : "w4";
+  if (int rc = check_shape(w8 ? "gemm_i8a8" : "gemm_i4a8", m, n, k)) return rc;
   // The decode band ends where the tile GEMM's small cells overtake the streaming form (speed data of
-  // this card: 17..32 rows stream unless the output is very wide, 33..48 unless it is wide, from 49
-  // rows the tiles win on every shape measured).
+  // this card: 17..32 rows stream unless the output is very wide, 33..64 unless it is wide; from 49 rows a short K
+  // goes to the tiles as well: 8192 x 1024 at 50 / 64 rows 7.4 / 7.6 us streamed, 5.2 / 5.1 on 64 x 64, 5120 x 5120 within
+  // a tenth either way, 5120 x 6144 12.2 / 12.5 against 14.1; 4096 x 1024 5.5 against 5.1, 4096 x 4096 8.2 against 10.4).
   // A deep, narrow linear leaves the band at 33 rows already: where the tile law shares K over workgroups
   // (pf_split), its 64 x 128 cell overtakes the three-tile streaming form (5120 x 17408 at 33 / 40 / 48 rows:
   // 23.7 / 23.9 / 25.8 us on four shares against 28.2 / 28.3 / 31.3; up to 32 rows streaming wins, 18.0 against 22.4).
   const PfVariant *split_cell = nullptr;
   const uint32_t tile_ks = pf_split(wkind == SABER_IU8_W8, m, n, k, &split_cell);
-  const bool stream = m <= 16 || (m <= 32 && n <= 16384) || (m <= 48 && n <= 8192 && tile_ks == 0);
+  const bool narrow = n <= 16 * CU_COUNT, two_wide = !narrow && n <= 32 * CU_COUNT;  // a 16- / 32-column block a CU
+  const bool stream = m <= 16 || (m <= 32 && n <= 16384) || (m <= 48 && n <= 8192 && tile_ks == 0) ||
+                      (tile_ks == 0 && ((narrow && k >= 2048) || (two_wide && k >= 6144)));
   if (m <= DECODE_MAX_M && stream) {
     // Up to 16 rows of K <= 5120: the persistent form that stages the 16-row tile once a workgroup (`_s80`) where
     // it measured faster than the streamed one, which re-reads the tile from L2 once a 32-column block. W4, 9-16
@@ -373,13 +382,39 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
     // and on 16384 x 8192 (12.4 -> 12.8) the streamed form stays
     if (m >= 2 && m <= 4 && k >= 16384 && wkind == SABER_IU8_W4 && staged80_holds(m, k))
       return describe_s80(false, true, m, n, k, 1, out);
-    const std::string name = dec_stream_name(tag, m, k);
+    // 17 to 64 rows: the block width that gives every CU one column block (iu8_variants.def has the timings). 33 to 48
+    // rows keep `tm3` at a short K (8192 x 1024 at 40 rows 6.1 us against 6.2 on `_n2`).
+    std::string name = dec_stream_name(tag, m, k);
+    if (m > 16 && m <= 32 && narrow) name += "_n1";
+    else if (m > 32 && two_wide && k >= 4096) name += "_n2";
+    else if (m > 48) name += "_k16";
     const DecVariant *v = dec_variant(name);
     if (!v) return fail(SABER_IU8_E_RULE, name + ": no such variant");
     const uint32_t nblk = (n + v->block_n() - 1) / v->block_n();
     return describe_dec(*v, m, n, k, decode_split(m, n, k, nblk, v->kw), out);
   }
   if (tile_ks) return describe_pf(*split_cell, m, n, k, tile_ks, out);
+  // One row tile, past the streaming band: a tile's chain of K steps is what the launch takes, so the cell is the
+  // narrowest that needs one round of the 256 CUs (the estimate of pf_cell is fitted to 65 rows and more and took 64 x 64
+  // up to 32,768 columns: two rounds). W4, us on 64 x 64 / 64 x 128 at 17 / 45 / 64 rows: 20480 x 5120 18.6 / 20.6 / 22.5 ->
+  // 15.0 / 16.3 / 17.2, 28672 x 5120 20.3 / 22.4 / 24.4 -> 16.8 / 18.0-20.6 / 18.6-19.3, 24576 x 2048 at 20 / 50 rows
+  // 10.3 / 11.4 -> 8.8 / 9.2; at 32768 columns 23.4 / 23.6 / 25.3 -> 19.6 / 23.7 / 24.8; up to 16,384 columns 64 x 64 is one
+  // round (16384 x 5120 13.5 against 15.6-16.7) and pf_cell's pick. 160 columns wide up to 40,960 columns (40960 x 5120 at 17 /
+  // 33 / 64 rows 29.6 / 32.5 / 33.5 -> 24.8 / 28.9 / 30.2, W8 52.9 / - / 57.0 -> 42.0 / - / 41.6). Int8 weights up to
+  // 32,768 columns stay with the estimate (64 x 64 and 64 x 128 within 10 % of each other).
+  if (m <= 64 && n > 32 * 2 * CU_COUNT && n <= 160 * CU_COUNT) {
+    const char *cell = n > 128 * CU_COUNT ? (!w8 && m <= 32 ? "t32x160_s" : "t64x160_s") : w8 ? nullptr : "t64x128_s";
+    if (cell) return describe_pf(*pf_variant(fmt("macaq_iu8_pf_%s_%s", tag, cell)), m, n, k, 0, out);
+  }
+  // Int8 weights: 128 x 160 where it is one round and 128 x 128 is two; us against the estimate's pick -- 5120 x 17408 at
+  // 777 / 1,000 rows 121 / 122 -> 91 / 96, 5120 x 5120 42.4 / 40.6 -> 30.6 / 33.0, 10240 x 5120 at 400 / 512 rows 41 / 42 ->
+  // 33 / 35, 6144 x 5120 at 700 rows 39.5 -> 35.7, 20480 x 5120 at 130 / 200 rows 37.7 / 45.1 -> 36.1 / 37.5. One round of
+  // both (5120 columns at 700 rows, 25.8 against 32.6) and two of both (8192 x 8192 at 777, 67 against 90) stay as they
+  // were, and so do 1,024 rows and more.
+  if (w8 && m > 64 && m < 1024) {
+    auto tiles = [&](uint32_t bn) { return (uint64_t)((n + bn - 1) / bn) * ((m + 127) / 128); };
+    if (tiles(160) <= CU_COUNT && tiles(128) > CU_COUNT) return describe_pf(*pf_variant("macaq_iu8_pf_w8_t128x160"), m, n, k, 0, out);
+  }
   return describe_pf(*pf_cell(wkind == SABER_IU8_W8, m, n, k), m, n, k, 0, out);
 }
 

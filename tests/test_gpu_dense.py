@@ -412,3 +412,31 @@ def test_sixteen_row_tile_staged_once_a_workgroup(ctx, M, N, K, grid, w8):
             with pytest.raises(iu8.IU8Error) as e:
                 ctx.launch(bad, bufs)
             assert e.value.code == iu8.E_RULE, field
+
+
+BAND = [  # rows, N, K, the law's W4 / W8 kernel past "macaq_iu8_": both sides of every line the law draws at 17 to 64 rows
+    (17, 16, 128, "dec_{}_tm2_n1", "dec_{}_tm2_n1"), (32, 4096, 640, "dec_{}_tm2_n1", "dec_{}_tm2_n1"),
+    (31, 4112, 256, "dec_{}_tm2", "dec_{}_tm2"), (33, 4112, 4096, "dec_{}_tm3_n2", "dec_{}_tm3_n2"),
+    (48, 8192, 4224, "dec_{}_tm3_n2", "dec_{}_tm3_n2"), (40, 4112, 3968, "dec_{}_tm3", "dec_{}_tm3"),
+    (49, 48, 2048, "dec_{}_tm4_k16", "dec_{}_tm4_k16"), (64, 4096, 2176, "dec_{}_tm4_k16", "dec_{}_tm4_k16"),
+    (64, 4096, 1920, "pf_{}_t64x64_s", None), (50, 4112, 6144, "dec_{}_tm4_n2", "dec_{}_tm4_n2"), (64, 8176, 6272, "dec_{}_tm4_n2", "dec_{}_tm4_n2"),
+    (17, 16400, 256, "pf_{}_t64x128_s", None), (64, 32768, 640, "pf_{}_t64x128_s", None),
+    (17, 32784, 128, "pf_{}_t32x160_s", "pf_{}_t64x160_s"), (32, 40960, 1664, "pf_{}_t32x160_s", "pf_{}_t64x160_s"),
+    (33, 32784, 256, "pf_{}_t64x160_s", "pf_{}_t64x160_s"), (64, 40960, 896, "pf_{}_t64x160_s", "pf_{}_t64x160_s"),
+    (65, 40960, 128, None, "pf_{}_t128x160"), (896, 5136, 384, None, "pf_{}_t128x160"), (1023, 5120, 640, None, "pf_{}_t128x160")]
+
+
+@pytest.mark.parametrize("shape", BAND, ids=lambda b: "x".join(map(str, b[:3])))
+def test_band_of_17_to_64_rows_and_its_cells(ctx, shape):
+    """One column block a CU: the streaming cells by block width, the one-round tiles, and the 128 x 160 tile of int8
+    weights. The law picks what the table says and the bytes are the oracle's."""
+    M, N, K = shape[:3]
+    for tag, w8, want in (("w4", False, shape[3]), ("w8", True, shape[4])):
+        if want is None:
+            continue
+        print(f"band {shape} {tag}", flush=True)
+        case = synth.dense_case(M, N, K, w8=w8, seed=M + N)
+        run = DenseRun(ctx, case, want_acc=False)
+        assert run.desc.kernel.decode() == "macaq_iu8_" + want.format(tag) and run.desc.ks == 1
+        r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+        np.testing.assert_array_equal(run.C, r["C"])
