@@ -962,8 +962,8 @@ int saber_iu8_moe_silu_mul_quant(saber_iu8_ctx *ctx, const void *gu, void *q, fl
                                  const saber_iu8_moe_tables *t, void *stream) {
   if (!t) return fail(SABER_IU8_E_ARG, "moe_silu_mul_quant: null tables");
   saber_iu8_desc d;
-  // From a few thousand rows the table form (memory-bound) overtakes the computed one (bound by the
-  // exp and divide of every element); below, copying the table into LDS costs more than it saves.
+  // From a few thousand rows the table form overtakes the computed one (4,096 rows of 1,536: 11.6 against 14.0 us,
+  // 33,792: 67.9 against 68.5); below, copying the table into LDS costs more than it saves.
   if (t->silu_lut && rows_cap >= 4096 && n % 16 == 0 && n <= 4096) {
     const uint32_t tiles = (rows_cap + 15) / 16;
     const uint32_t grid[3] = {tiles < CU_COUNT ? tiles : CU_COUNT, 1, 1};

@@ -59,11 +59,39 @@ static __device__ __forceinline__ unsigned iu8_bf16_pack(float lo, float hi) {
   const iu8_v2bf r = __builtin_convertvector(iu8_v2f{lo, hi}, iu8_v2bf);
   return *(const unsigned *)&r;
 }
-// bf16(silu(x)) as the producer kernels compute it (macaq_i8q: i8q_silu_bf16; the law
+// bf16(silu(x)) as the producer kernels compute it (the law
 // crates/saber-kernels/hip/mxfp4_hadi8.hip:118-146): x / (1 + expf(-x)), IEEE divide, one bf16 rounding.
 static __device__ __forceinline__ float iu8_silu_bf16(float x) {
 #pragma clang fp contract(off)
   return iu8_bf16_f32((unsigned short)iu8_bf16_bits(x / (1.f + expf(-x))));
+}
+
+// The same bytes without the library exponential and the IEEE divide (some 50 VALU operations an element, which is
+// what bound the row producers): x * rcp(1 + exp2(-x log2 e)) on the hardware's own exp2 and reciprocal, about 10. A
+// gate is one of 65,536 bf16 values, so the difference is a table, and it was read in full on the card: the two
+// round to the same bf16 everywhere but at 5.9375, where this form lands on the tie itself, and at -87.5, -88 and -88.5,
+// whose reciprocal is subnormal (up to 55 units in the last place of f32 apart elsewhere, no tie between them). So
+// four gates whose results come within two units of a tie, or one of which is under -87, take the law's own routine;
+// tests/test_gpu_dense.py::test_silu_producers_on_every_gate_value compares every input. NaN, infinities and zeros come out the same.
+//
+// Four gates (two packed pairs) -> the packed bf16 products bf16(bf16(silu(g)) * u).
+static __device__ __forceinline__ void iu8_silu_mul4(unsigned g0, unsigned g1, unsigned u0, unsigned u1, unsigned &p0, unsigned &p1) {
+#pragma clang fp contract(off)
+  const float x[4] = {__uint_as_float(g0 << 16), __uint_as_float(g0 & 0xFFFF0000u), __uint_as_float(g1 << 16), __uint_as_float(g1 & 0xFFFF0000u)};
+  float r[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = x[i] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x[i] * -1.44269504088896340736f));
+  unsigned t0 = iu8_bf16_pack(r[0], r[1]), t1 = iu8_bf16_pack(r[2], r[3]);
+  auto off = [&](int i) { return (unsigned short)(__float_as_uint(r[i]) + 0x8002u); };  // 0..4: within two units of a tie
+  const unsigned short a = off(0) < off(1) ? off(0) : off(1), b = off(2) < off(3) ? off(2) : off(3);
+  const bool law = (a < b ? a : b) <= 4 || fminf(fminf(x[0], x[1]), fminf(x[2], x[3])) < -87.f;
+  if (__builtin_expect(law, 0)) {
+    asm volatile("");  // stays a branch (iu8_code4_rcp has the reason)
+    t0 = iu8_bf16_pack(iu8_silu_bf16(x[0]), iu8_silu_bf16(x[1]));
+    t1 = iu8_bf16_pack(iu8_silu_bf16(x[2]), iu8_silu_bf16(x[3]));
+  }
+  p0 = iu8_bf16_pack(__uint_as_float(t0 << 16) * __uint_as_float(u0 << 16), __uint_as_float(t0 & 0xFFFF0000u) * __uint_as_float(u0 & 0xFFFF0000u));
+  p1 = iu8_bf16_pack(__uint_as_float(t1 << 16) * __uint_as_float(u1 << 16), __uint_as_float(t1 & 0xFFFF0000u) * __uint_as_float(u1 & 0xFFFF0000u));
 }
 
 template <bool W8>

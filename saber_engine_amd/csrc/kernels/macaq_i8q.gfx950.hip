@@ -94,11 +94,11 @@ static __device__ __forceinline__ void i8q_pk_load(unsigned (&g)[8], const unsig
 #pragma unroll
   for (int w = 0; w < 4; ++w) g[w] = lo[w], g[4 + w] = hi[w];
 }
-template <int I8Q_MAXG, bool RM, bool SCALE_ONLY>
+template <int I8Q_MAXG, bool RM, bool SCALE_ONLY, int T = I8Q_T>
 static __device__ __forceinline__ void i8q_tail_pk(const unsigned (&pk)[I8Q_MAXG][8], int G, iu8_u8 *__restrict__ q,
                                                    float *__restrict__ scale, int row, int K) {
   const int tid = threadIdx.x;
-  const float amax = i8q_block_max(iu8_pk_amax(pk));
+  const float amax = i8q_block_max<T>(iu8_pk_amax(pk));
   const float sc = fmaxf(__fdiv_rn(amax, 127.f), 1e-30f);
   const float rcp = __fdiv_rn(1.f, sc);
   if (tid == 0) scale[row] = sc;
@@ -106,7 +106,7 @@ static __device__ __forceinline__ void i8q_tail_pk(const unsigned (&pk)[I8Q_MAXG
   iu8_u8 *qrow = q + (size_t)(row >> 4) * (K >> 6) * 1024 + (row & 15) * 16;
 #pragma unroll
   for (int i = 0; i < I8Q_MAXG; ++i) {
-    const int g = tid + i * I8Q_T;
+    const int g = tid + i * T;
     if (g >= G) continue;
     const iu8_v4u d = iu8_pk_codes(pk[i], sc, rcp);
     if constexpr (RM) *(iu8_v4u *)(q + (size_t)row * K + g * 16) = d;
@@ -200,11 +200,20 @@ I8Q_QUANT_ROWS(macaq_i8_quant_rows_t256_g2, 2)
 I8Q_QUANT_ROWS(macaq_i8_quant_rows_t256_g1, 1)
 #undef I8Q_QUANT_ROWS
 
-static __device__ __forceinline__ float i8q_silu_bf16(float x) {
-#pragma clang fp contract(off)
-  return iu8_bf16_f32((unsigned short)iu8_bf16_bits(x / (1.f + expf(-x))));
+// a group's 16 products from its gates and ups
+static __device__ __forceinline__ void i8q_silu_mul16(const unsigned short *gate, const unsigned short *up, unsigned (&p)[8]) {
+  const iu8_v4u g0 = *(const iu8_v4u *)gate, g1 = *(const iu8_v4u *)(gate + 8), u0 = *(const iu8_v4u *)up, u1 = *(const iu8_v4u *)(up + 8);
+  iu8_silu_mul4(g0[0], g0[1], u0[0], u0[1], p[0], p[1]);
+  iu8_silu_mul4(g0[2], g0[3], u0[2], u0[3], p[2], p[3]);
+  iu8_silu_mul4(g1[0], g1[1], u1[0], u1[1], p[4], p[5]);
+  iu8_silu_mul4(g1[2], g1[3], u1[2], u1[3], p[6], p[7]);
 }
 
+// The products stay packed as bf16 pairs (8 registers a group): 40 registers in the 1024-thread form, two workgroups a
+// CU. us before (exp and divide of the law, products as floats) and now, rows of 17,408: 5 rows 8.0 -> 6.9, 200 11.2 -> 9.9,
+// 777 26.1 -> 22.0, 2,048 48.0 -> 41.3, 8,192 164.6 -> 137.8 (5.2 TB/s: bound by memory). Requesting a group ahead of the
+// one in work measured 2-5 % slower (the registers it takes).
+//
 // `row_tok` / `meta` are optional (may be null): with them the kernel runs on the expert-major
 // rows of a routed layer and skips pad rows (row_tok < 0) and rows past meta[1]
 // (signature crates/saber-kernels/src/abi.rs:344-351).
@@ -217,23 +226,15 @@ static __device__ __forceinline__ void i8q_silu_body(const unsigned short *__res
   if (meta != nullptr && row >= meta[1]) return;
   if (row_tok != nullptr && row_tok[row] < 0) return;
   const unsigned short *gr = gu + (size_t)row * 2 * n;
-  float v[I8Q_MAXG][16];
+  unsigned pk[I8Q_MAXG][8];  // the products, packed: the codes are made from them behind the row's maximum
 #pragma unroll
   for (int i = 0; i < I8Q_MAXG; ++i) {
     const int g = threadIdx.x + i * T;
-    if (g >= G) continue;
-    union { iu8_v4u u[2]; unsigned short h[16]; } vg, vu;
-    vg.u[0] = *(const iu8_v4u *)(gr + g * 16);
-    vg.u[1] = *(const iu8_v4u *)(gr + g * 16 + 8);
-    vu.u[0] = *(const iu8_v4u *)(gr + n + g * 16);
-    vu.u[1] = *(const iu8_v4u *)(gr + n + g * 16 + 8);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float t = i8q_silu_bf16(iu8_bf16_f32(vg.h[j]));
-      v[i][j] = iu8_bf16_f32((unsigned short)iu8_bf16_bits(t * iu8_bf16_f32(vu.h[j])));
-    }
+    for (int w = 0; w < 8; ++w) pk[i][w] = 0;
+    if (g < G) i8q_silu_mul16(gr + g * 16, gr + n + g * 16, pk[i]);
   }
-  i8q_tail<I8Q_MAXG, false, false, T>(v, G, q, scale, row, n);
+  i8q_tail_pk<I8Q_MAXG, false, false, T>(pk, G, q, scale, row, n);
 }
 #define I8Q_SILU(name, MAXG)                                                                                     \
   extern "C" __global__ __launch_bounds__(I8Q_T) void name(                                                      \
@@ -329,31 +330,32 @@ extern "C" __global__ __launch_bounds__(256) void macaq_i8_silu_mul_quant_w64(
   if (meta != nullptr && row >= meta[1]) return;
   if (row_tok != nullptr && row_tok[row] < 0) return;
   const unsigned short *gr = gu + (size_t)row * 2 * n;
-  float v[I8Q_WG][16];
+  unsigned pk[I8Q_WG][8];
 #pragma unroll
   for (int i = 0; i < I8Q_WG; ++i) {
     const int g = lane + i * 64;
-    if (g >= G) continue;
-    union { iu8_v4u u[2]; unsigned short h[16]; } vg, vu;
-    vg.u[0] = *(const iu8_v4u *)(gr + g * 16);
-    vg.u[1] = *(const iu8_v4u *)(gr + g * 16 + 8);
-    vu.u[0] = *(const iu8_v4u *)(gr + n + g * 16);
-    vu.u[1] = *(const iu8_v4u *)(gr + n + g * 16 + 8);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float t = i8q_silu_bf16(iu8_bf16_f32(vg.h[j]));
-      v[i][j] = iu8_bf16_f32((unsigned short)iu8_bf16_bits(t * iu8_bf16_f32(vu.h[j])));
-    }
+    for (int w = 0; w < 8; ++w) pk[i][w] = 0;
+    if (g < G) i8q_silu_mul16(gr + g * 16, gr + n + g * 16, pk[i]);
   }
-  i8q_tail_w64(v, G, q, scale, row, n);
+  const float amax = iu8_wave_max_nonneg(iu8_pk_amax(pk));
+  const float sc = fmaxf(__fdiv_rn(amax, 127.f), 1e-30f);
+  const float rcp = __fdiv_rn(1.f, sc);
+  if (lane == 0) scale[row] = sc;
+  iu8_u8 *qrow = q + (size_t)(row >> 4) * (n >> 6) * 1024 + (row & 15) * 16;
+#pragma unroll
+  for (int i = 0; i < I8Q_WG; ++i) {
+    const int g = lane + i * 64;
+    if (g < G) *(iu8_v4u *)(qrow + (size_t)(g >> 2) * 1024 + (g & 3) * 256) = iu8_pk_codes(pk[i], sc, rcp);
+  }
 }
 
 // The same op for many rows, with the bf16 silu read from a table: `lut` holds the silu of every
 // bf16 bit pattern as macaq_silu_bf16_table wrote it (128 KiB), each workgroup copies it into LDS
 // once and its 16 waves then walk the rows, a wave a row, the 16 rows of an A tile on one workgroup
-// (tile = blockIdx.x + r * gridDim.x) so that the tile's 256-byte runs fill in one L2. The computed
-// form spends about 60 VALU operations an element on exp and the IEEE divide and is bound by them;
-// this one is bound by memory. Same bytes: the table is that form's own output.
+// (tile = blockIdx.x + r * gridDim.x) so that the tile's 256-byte runs fill in one L2. Against the computed
+// form, us at 4,096 / 8,192 / 16,384 / 33,792 rows of 1,536: 11.6 / 18.9 / 32.6 / 67.9 here, 14.0 / 22.2 / 36.8 / 68.5
+// there (16.4 / 26.4 / 43.7 / 83.1 before its SiLU left the library exponential). Same bytes: the table is that form's own output.
 extern "C" __global__ __launch_bounds__(1024) void macaq_i8_silu_mul_quant_lut_w64(
     const unsigned short *__restrict__ gu, unsigned char *__restrict__ q, float *__restrict__ scale, int n,
     const int *__restrict__ row_tok, const int *__restrict__ meta, const unsigned short *__restrict__ lut) {
@@ -392,5 +394,5 @@ extern "C" __global__ __launch_bounds__(1024) void macaq_i8_silu_mul_quant_lut_w
 
 extern "C" __global__ __launch_bounds__(256) void macaq_silu_bf16_table(unsigned short *__restrict__ out) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
-  out[i] = (unsigned short)iu8_bf16_bits(i8q_silu_bf16(iu8_bf16_f32((unsigned short)i)));
+  out[i] = (unsigned short)iu8_bf16_bits(iu8_silu_bf16(iu8_bf16_f32((unsigned short)i)));
 }

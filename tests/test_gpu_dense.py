@@ -368,6 +368,27 @@ def test_row_producers_every_form_that_holds_the_row(ctx, M, K):
             np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, K), wq, err_msg=name)
 
 
+def test_silu_producers_on_every_gate_value(ctx):
+    """Every bf16 gate, one a row with an up of 1 (the other gates zero): the row's scale is the product's magnitude and
+    the code its sign, so a SiLU that rounds another way anywhere shows. Every form that holds the row."""
+    M, K = 65536, 64
+    gu = np.zeros((M, 2 * K), dtype=np.uint16)
+    gu[:, K:] = 0x3F80
+    gu[np.arange(M), np.arange(M) * 7 % K] = np.arange(M, dtype=np.uint16)
+    want_q, want_s, _ = ref.silu_mul_quant(gu)
+    src = dev_bf16_bits(gu)
+    for name, block in _row_forms("macaq_i8_silu_mul_quant", K) + [("macaq_i8_silu_mul_quant_w64", 256)]:
+        say(f"every gate value: {name}")
+        d = iu8.resolve_silu_mul_quant(M, K)
+        d.kernel, d.block[0], d.grid[0] = name.encode(), block, M // 4 if name.endswith("_w64") else M
+        q = torch.full((iu8.a_bytes(M, K),), 0x55, dtype=torch.uint8, device="cuda")
+        s = torch.zeros(M, dtype=torch.float32, device="cuda")
+        ctx.launch(d, {"gu": src.data_ptr(), "q": q.data_ptr(), "scale": s.data_ptr()})
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), want_s.view(np.uint32), err_msg=name)
+        np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, K), want_q, err_msg=name)
+
+
 @pytest.mark.parametrize("w8", [False, True])
 @pytest.mark.parametrize("M,N,K,grid", [(16, 5120, 5120, 0), (9, 96, 5120, 0), (13, 34816, 5120, 0), (11, 7184, 640, 0), (5, 4112, 128, 0),
                                         (1, 256, 5120, 0), (16, 2048, 3072, 8), (12, 2064, 384, 9),
