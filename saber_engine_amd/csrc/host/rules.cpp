@@ -426,6 +426,8 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
 // the partials cost ks*M*N*4 bytes each way and the last arriver sums alone -- so the rule is this
 // narrow. The launch then needs the `decode_partial` / `decode_counter` workspaces the descriptor lists.
 uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant **cell) {
+  // (timings of this comment from before the cell stood on four waves side by side and the reduction read in batches, which
+  // took 5120 x 17408 at 45 / 64 / 128 / 180 rows from 25.2 / 28.9 / 31.0 / 35.3 to 18.5 / 19.3 / 22.8 / 28.5 us)
   // measured at 33..192 rows; above, the partials (ks * M * N * 4 bytes each way) grow with M (at 256 rows the unsplit
   // cell is level or ahead: 5120 x 17408 43.9 against 43.9-58.6 us). Up to 128 tiles, i.e. two shares at least:
   // 81-128 tiles on two shares against the law's unsplit pick, us -- 5120 x 17408 at 129 / 160 / 192 rows 33.7 / 34.1 /
@@ -675,7 +677,7 @@ int resolve_gate_up_act(uint32_t m, uint32_t hidden, uint32_t inter, saber_iu8_d
 // Rows wider than 4,096 whose count leaves the card part idle go 16 waves a row (`base`_t1024): measured on this
 // card, graph replay, 256-thread form / 1024-thread form in us -- the quantiser at 1 / 16 / 256 rows of 5,120:
 // 2.57/2.34, 2.98/2.74, 3.41/3.20; of 17,408: 3.90/2.91, 5.09/3.92, 6.72/5.49; at 512 rows 3.98/4.52 and 7.92/7.09, at
-// 1,024 4.84/6.32 and 13.3/14.3. The activation (exp and an IEEE divide an element) at 1 / 16 / 512 rows of 5,120:
+// 1,024 4.84/6.32 and 13.3/14.3. The activation (timed with the library exp and an IEEE divide an element, its four-a-time form is 13-16 % faster) at 1 / 16 / 512 rows of 5,120:
 // 6.36/4.64, 6.75/5.02, 8.22/7.13; of 17,408: 13.6/7.50, 14.3/8.06, 18.8/14.9, and 47.0/42.4 at 2,048 rows (5,120
 // there: 17.5/22.1). Rows of 4,096: the two forms are within 3 % (a thread of either owns one group).
 static std::string row_form(const char *base, uint32_t rows, uint32_t width, bool silu = false) {
