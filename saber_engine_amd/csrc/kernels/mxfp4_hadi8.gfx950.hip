@@ -41,6 +41,10 @@ static __device__ __forceinline__ void had_quant_body(const unsigned short *__re
   had_tail<T>(sv, NV, q, scale, row, K);
 }
 
+// Bound by the VALU (transform, codes, activation) and by a row's latency for few rows: the activation is the hardware's exp2
+// and reciprocal where they give the law's bf16 (iu8_silu_mul4), and the row's pieces leave in one batch of loads instead of
+// one a group. us before / now: rows of 17,408 at 1 / 45 / 200 rows (t1024) 8.70 / 9.41 / 10.85 -> 6.62 / 7.37 / 9.26, at 777 /
+// 2,048 / 6,144 (t512) 27.6 / 57.2 / 154.0 -> 23.6 / 44.1 / 118.9; 2,048 rows of 5,120 (t256) 19.7 -> 16.5, of 2,048 9.9 -> 8.2.
 template <int T>
 static __device__ __forceinline__ void had_silu_body(const unsigned short *__restrict__ gu, iu8_u8 *__restrict__ q,
                                                      float *__restrict__ scale, int N,
@@ -48,19 +52,24 @@ static __device__ __forceinline__ void had_silu_body(const unsigned short *__res
 #pragma clang fp contract(off)
   const int row = had_row(), tid = threadIdx.x, NV = N >> 3;
   gu += (size_t)row * 2 * N;
+  // all of the row's pieces are requested before the first is used
+  iu8_v4u rg[HAD_MAXG], ru[HAD_MAXG];
+#pragma unroll
+  for (int i = 0; i < HAD_MAXG; ++i) {
+    const int g = tid + i * T;
+    rg[i] = ru[i] = iu8_v4u{0u, 0u, 0u, 0u};
+    if (g < NV) rg[i] = *(const iu8_v4u *)(gu + (unsigned)(g * 8)), ru[i] = *(const iu8_v4u *)(gu + N + (unsigned)(g * 8));
+  }
   float sv[HAD_MAXG][8];
 #pragma unroll
   for (int i = 0; i < HAD_MAXG; ++i) {
     const int g = tid + i * T;
     if (g >= NV) continue;
-    float vg[8], vu[8];
-    had_load8(gu + g * 8, vg);
-    had_load8(gu + N + g * 8, vu);
+    unsigned p[4];
+    iu8_silu_mul4(rg[i][0], rg[i][1], ru[i][0], ru[i][1], p[0], p[1]);
+    iu8_silu_mul4(rg[i][2], rg[i][3], ru[i][2], ru[i][3], p[2], p[3]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float t = iu8_bf16_f32((unsigned short)iu8_bf16_bits(vg[j] / (1.f + expf(-vg[j]))));
-      sv[i][j] = iu8_bf16_f32((unsigned short)iu8_bf16_bits(t * vu[j]));
-    }
+    for (int w = 0; w < 4; ++w) sv[i][2 * w] = __uint_as_float(p[w] << 16), sv[i][2 * w + 1] = __uint_as_float(p[w] & 0xFFFF0000u);
     had32(sv[i], had_t + 8 * g, tid);
   }
   had_tail<T>(sv, NV, q, scale, row, N);
@@ -220,8 +229,9 @@ HAD_SMQ(silu_mul_quant_hadi8_t1024, 1024)  // 16 waves a row: few long rows (no 
 
 // silu_mul_quant with the bf16 silu read from a table: `lut` holds bf16(silu(x)) of every bf16 bit pattern x as
 // macaq_silu_bf16_table (code object `macaq_i8q`) wrote it, i.e. this file's own expression
-// vg / (1 + expf(-vg)) rounded to bf16, so the bytes are those of the computed form, which spends about 30 of
-// its 55 VALU operations an element on the exp and the divide and is bound by them. A workgroup copies the
+// vg / (1 + expf(-vg)) rounded to bf16, so the bytes are those of the computed form. Rows of 17,408, us on the computed
+// form / here: 1 / 200 rows 6.62 / 9.26, 5.92 / 8.82; 777 / 2,048 / 6,144 rows 23.6 / 44.1 / 118.9, 21.2 / 42.9 / 116.7; rows of
+// 5,120 within 6 % either way; rows of 2,048 up to 512 rows 0.35-0.5 us in favour of the computed form. A workgroup copies the
 // table's middle -- magnitudes from 2^-17 up to 2^15, both signs: 2 x 4,096 entries, 16 KiB -- into LDS beside
 // its row's loads; a gate outside (one in some hundred thousand of unit-scale rows) is computed as before.
 // The kernel is the computed form otherwise (a workgroup a row, the same lane map). No counterpart among
