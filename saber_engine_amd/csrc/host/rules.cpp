@@ -279,7 +279,7 @@ static bool int_arg(const saber_iu8_desc &d, const char *name, int64_t *v) {
 int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_desc *out, int order) {
   static const char PREFIX[] = "macaq_iu8_dec_w4_";
   // a half the law gave the staged persistent form, or 17 to 48 rows at another block width, is paired as its streamed
-  // form: the pair kernels are that geometry
+  // form, which is the pair kernels' geometry, on the split count it was given
   auto other_form = [](const saber_iu8_desc &h) {
     return !strncmp(h.kernel, "macaq_iu8_dec_w4_tm1_s80", 24) || !strcmp(h.kernel, "macaq_iu8_dec_w4_tm2_n1") ||
            !strcmp(h.kernel, "macaq_iu8_dec_w4_tm3_n2");
@@ -294,7 +294,7 @@ int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_de
         if (other_form(*in[i])) {
           if (!int_arg(*in[i], "m", &hm) || !int_arg(*in[i], "n", &hn) || !int_arg(*in[i], "k", &hk))
             return fail(SABER_IU8_E_RULE, "macaq iu8 pair: a half without its m, n, k");
-          if (int rc = describe(dec_stream_name("w4", (uint32_t)hm, (uint32_t)hk), (uint32_t)hm, (uint32_t)hn, (uint32_t)hk, 1, &s[i])) return rc;
+          if (int rc = describe(dec_stream_name("w4", (uint32_t)hm, (uint32_t)hk), (uint32_t)hm, (uint32_t)hn, (uint32_t)hk, in[i]->ks, &s[i])) return rc;
         }
       }
       return pair(s[0], s[1], out, order);

@@ -162,6 +162,18 @@ def test_pair_lays_two_decode_grids_end_to_end():
         assert e.value.code == iu8.E_RULE and "pair" in str(e.value)
 
 
+def test_pair_keeps_the_split_of_a_half_at_another_block_width():
+    """A `_tm2_n1` / `_tm3_n2` half is paired in the streamed form of the pair kernels with the split count it was given:
+    the descriptor is the one its `tm2` / `tm3` twin gives, grid and workspaces with it."""
+    for m, wide, twin in ((32, "macaq_iu8_dec_w4_tm2_n1", "macaq_iu8_dec_w4_tm2"), (40, "macaq_iu8_dec_w4_tm3_n2", "macaq_iu8_dec_w4_tm3")):
+        for ks_a, ks_b in ((1, 1), (3, 1), (1, 2), (3, 2)):
+            for name_b in (wide, twin):
+                d = iu8.pair(iu8.describe(wide, m, 4112, 4096, ks=ks_a), iu8.describe(name_b, m, 96, 4096, ks=ks_b))
+                want = iu8.pair(iu8.describe(twin, m, 4112, 4096, ks=ks_a), iu8.describe(twin, m, 96, 4096, ks=ks_b))
+                assert bytes(d) == bytes(want), (wide, name_b, ks_a, ks_b)
+                assert d.arg("ks").ival == ks_a and d.arg("ks_b").ival == ks_b and d.n_workspaces == 2 * ((ks_a > 1) + (ks_b > 1))
+
+
 def test_pair_variants_share_their_decode_twin_geometry():
     text = open(os.path.join(iu8.PKG, "csrc", "kernels", "iu8_variants.def")).read()
     dec = {m[0]: m[1:] for m in re.findall(r"^IU8_DEC_VARIANT\((\w+), (\d+), (\w+), (\d+), (\d+), (\d+), (\d+), (\d+), (\w+)\)", text, flags=re.M)}
