@@ -409,11 +409,23 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // Int8 weights: 128 x 160 where it is one round and 128 x 128 is two; us against the estimate's pick -- 5120 x 17408 at
   // 777 / 1,000 rows 121 / 122 -> 91 / 96, 5120 x 5120 42.4 / 40.6 -> 30.6 / 33.0, 10240 x 5120 at 400 / 512 rows 41 / 42 ->
   // 33 / 35, 6144 x 5120 at 700 rows 39.5 -> 35.7, 20480 x 5120 at 130 / 200 rows 37.7 / 45.1 -> 36.1 / 37.5. One round of
-  // both (5120 columns at 700 rows, 25.8 against 32.6) and two of both (8192 x 8192 at 777, 67 against 90) stay as they
-  // were, and so do 1,024 rows and more.
+  // both (5120 columns at 700 rows, 25.8 against 32.6) and two of both (8192 x 8192 at 777, 67 against 90) are the
+  // estimate's. Where the estimate has a 64-row cell (the rows' last block of 128 is at most half live), from K = 5,120:
+  // 18432 x 1024 / 2048 / 4096 / 5120 at 129 rows 12.0 / 18.7 / 28.8 / 36.3 there, 11.6 / 17.0 / 27.7 / 32.6 here, but
+  // 7168 x 1024 / 2048 / 4096 / 5120 at 513 rows 12.0 / 16.7 / 29.1 / 37.8 against 13.6 / 20.1 / 30.1 / 39.6 and every
+  // such launch of K <= 256 4-24 % slower here; of 466 timed at K = 5,120 and 6,144 eight are 3-5 % slower, the rest up to 40 %
+  // faster. Where it has a larger cell: a tile count that is not whole eighths leaves the order by XCD (iu8_dense_tile_at),
+  // which costs what the round saves at K of 512 to 2,048 (1024 deep, 5760 columns at 784 rows 13.3 -> 15.2, 5632 columns,
+  // 216 tiles, at 720 rows 13.5 -> 11.0); one row block never lost. 1,024 rows and more stay with the
+  // estimate, whose table does not hold this cell: not for its speed at 1,024 rows themselves, where it is as many tiles as
+  // at 1,000 (5120 x 5120 / 17408 32.6 / 99 us, 128 x 256 41.2 / 118); from 1,025 rows of 5,120 columns it is two rounds
+  // (55.4 / 174 against 42.4 / 124).
   if (w8 && m > 64 && m < 1024) {
     auto tiles = [&](uint32_t bn) { return (uint64_t)((n + bn - 1) / bn) * ((m + 127) / 128); };
-    if (tiles(160) <= CU_COUNT && tiles(128) > CU_COUNT) return describe_pf(*pf_variant("macaq_iu8_pf_w8_t128x160"), m, n, k, 0, out);
+    const PfVariant *est = pf_cell(w8, m, n, k);
+    const bool pays = est->block_m() == 64 ? k >= 5120 : m <= 128 || k < 512 || k >= 3072 || tiles(160) % 8 == 0;
+    if (pays && tiles(160) <= CU_COUNT && tiles(128) > CU_COUNT) return describe_pf(*pf_variant("macaq_iu8_pf_w8_t128x160"), m, n, k, 0, out);
+    return describe_pf(*est, m, n, k, 0, out);
   }
   return describe_pf(*pf_cell(wkind == SABER_IU8_W8, m, n, k), m, n, k, 0, out);
 }

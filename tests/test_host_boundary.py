@@ -402,6 +402,20 @@ def test_prefill_launch_is_persistent_and_covers_the_output():
             assert d.n_workspaces == 0 and d.ks == 1
 
 
+def test_int8_128x160_cell_only_where_it_measured_faster():
+    """The 128 x 160 cell of int8 weights against the estimate's pick: not where a 64-row cell wastes less of a half live
+    last row block on a short K, and not on a tile count that leaves the order by XCD at a K of 512 to 2,944."""
+    mine = "macaq_iu8_pf_w8_t128x160"
+    for m, n, k, takes in ((513, 7168, 128, False), (513, 7168, 2048, False), (385, 9216, 4096, False), (272, 12288, 1024, False),
+                           (513, 7168, 4992, False), (513, 7168, 5120, True), (385, 8208, 5120, True), (129, 16400, 8192, True),
+                           (784, 5760, 384, True), (784, 5760, 512, False), (784, 5760, 2944, False), (784, 5760, 3072, True),
+                           (720, 5632, 1024, True), (777, 5120, 1024, True), (1000, 5120, 512, True), (200, 18432, 1024, True),
+                           (200, 17408, 1024, False), (65, 32784, 1024, True), (128, 40960, 2048, True), (100, 34816, 512, True)):
+        assert (iu8.resolve(iu8.W8, m, n, k).kernel.decode() == mine) == takes, (m, n, k)
+        if not takes:   # what the estimate gives, not another of the law's rules
+            assert iu8.resolve(iu8.W8, m, n, k).kernel.decode().startswith(("macaq_iu8_pf_w8_t64x", "macaq_iu8_pf_w8_t256x160")), (m, n, k)
+
+
 def test_prefill_cells_of_the_benchmark_shapes():
     # speed data of this card: the cell that was fastest in the sustained sweep of each shape, weights cold (every cell on
     # the four 27B-class shapes x 14 row counts; the law's tables are fitted to those timings, one a weight kind)
