@@ -5,6 +5,7 @@ import sys
 import numpy as np
 import torch
 
+from oracle import ref
 from saber_engine_amd import iu8
 
 
@@ -80,3 +81,16 @@ def assert_dense_matches(run, ref, w8):
     if run.acc is not None:
         np.testing.assert_array_equal(run.acc, ref["S"] if w8 else ref["S"] * 16)
     np.testing.assert_array_equal(run.C, ref["C"])
+
+
+def every_gate_rows(K):
+    """[gate | up] rows of K elements that hold every bf16 gate, one a row, among zeros. The gate's up is 1, and 2^100 (exact:
+    a power of two) where the SiLU is below 2^-60 in magnitude, subnormal ones included: no row whose SiLU is a number other
+    than zero then reaches the floor of the scale, so its scale is the SiLU's magnitude and a bf16 unit changes it."""
+    M = 65536
+    silu = (ref.silu_bf16_table().astype(np.uint32) << 16).view(np.float32)
+    gu = np.zeros((M, 2 * K), dtype=np.uint16)
+    at = np.arange(M) * 7 % K
+    gu[np.arange(M), at] = np.arange(M, dtype=np.uint16)
+    gu[np.arange(M), K + at] = np.where(np.abs(silu) < 2.0 ** -60, 0x7180, 0x3F80)
+    return gu, np.isfinite(silu) & (silu != 0)

@@ -6,7 +6,7 @@ import torch
 
 from oracle import ref
 from saber_engine_amd import iu8, synth
-from tests.gpu_util import DenseRun, assert_dense_matches, dev_bf16_bits, dev_f32, dev_u8, host_u16, say
+from tests.gpu_util import DenseRun, assert_dense_matches, dev_bf16_bits, dev_f32, dev_u8, every_gate_rows, host_u16, say
 
 pytestmark = pytest.mark.gpu
 
@@ -369,13 +369,12 @@ def test_row_producers_every_form_that_holds_the_row(ctx, M, K):
 
 
 def test_silu_producers_on_every_gate_value(ctx):
-    """Every bf16 gate, one a row with an up of 1 (the other gates zero): the row's scale is the product's magnitude and
-    the code its sign, so a SiLU that rounds another way anywhere shows. Every form that holds the row."""
+    """Every bf16 gate, one a row (the other gates zero), its up chosen so that the row's scale is the product's magnitude
+    and the code its sign (every_gate_rows): a SiLU that rounds another way anywhere shows. Every form that holds the row."""
     M, K = 65536, 64
-    gu = np.zeros((M, 2 * K), dtype=np.uint16)
-    gu[:, K:] = 0x3F80
-    gu[np.arange(M), np.arange(M) * 7 % K] = np.arange(M, dtype=np.uint16)
+    gu, numbers = every_gate_rows(K)
     want_q, want_s, _ = ref.silu_mul_quant(gu)
+    assert (want_s[numbers] > 1e-29).all() and (np.abs(want_q[numbers]).max(axis=1) == 127).all()
     src = dev_bf16_bits(gu)
     for name, block in _row_forms("macaq_i8_silu_mul_quant", K) + [("macaq_i8_silu_mul_quant_w64", 256)]:
         say(f"every gate value: {name}")

@@ -6,7 +6,7 @@ import torch
 
 from oracle import ref
 from saber_engine_amd import iu8, synth
-from tests.gpu_util import dev_bf16_bits, dev_f32, host_u16, say
+from tests.gpu_util import dev_bf16_bits, dev_f32, every_gate_rows, host_u16, say
 
 pytestmark = pytest.mark.gpu
 
@@ -44,6 +44,28 @@ def test_silu_mul_quant_had(ctx, M, N):
     wq, wsc = ref.silu_mul_quant_had(gu, t)
     np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32))
     np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, N), wq)
+
+
+def test_silu_mul_quant_had_on_every_gate_value(ctx):
+    """Every bf16 gate, one a row, its up chosen so that the row's scale shows the product's last bit (every_gate_rows): the
+    computed form in each workgroup size and the table form against the oracle."""
+    M, N = 65536, 64
+    gu, numbers = every_gate_rows(N)
+    t = np.random.default_rng(64).choice([-1.0, 1.0], size=N).astype(np.float32)
+    wq, wsc = ref.silu_mul_quant_had(gu, t)
+    assert (wsc[numbers] > 1e-29).all()
+    gd, td = dev_bf16_bits(gu), dev_f32(t)
+    lut = torch.zeros(65536, dtype=torch.int16, device="cuda")
+    ctx.silu_table(lut.data_ptr())
+    for T, name in ((256, "silu_mul_quant_hadi8_t256_tiled1"), (512, "silu_mul_quant_hadi8_t512_tiled1"), (1024, "silu_mul_quant_hadi8_t1024"),
+                    (256, "silu_mul_quant_hadi8_lut_t256")):
+        say(f"had, every gate value: {name}")
+        q, s = outs(M, N)
+        d = iu8.describe_raw(name, (M, 1, 1), T, plugin="mxfp4_hadi8", n=N)
+        ctx.launch(d, dict(gu=gd.data_ptr(), q=q.data_ptr(), scale=s.data_ptr(), had_t=td.data_ptr(), **({"lut": lut.data_ptr()} if "lut" in name else {})))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32), err_msg=name)
+        np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, N), wq, err_msg=name)
 
 
 @pytest.mark.parametrize("M,N", [(2, 2048), (130, 6144), (33, 10240), (70, 10304), (523, 17408), (19, 20480), (77, 64), (40, 1536)])
