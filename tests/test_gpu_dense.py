@@ -434,7 +434,9 @@ def test_sixteen_row_tile_staged_once_a_workgroup(ctx, M, N, K, grid, w8):
             assert e.value.code == iu8.E_RULE, field
 
 
-BAND = [  # rows, N, K, the law's W4 / W8 kernel past "macaq_iu8_": both sides of every line the law draws at 17 to 64 rows
+# rows, N, K, the law's W4 / W8 kernel past "macaq_iu8_": each cell of 17 to 64 rows, and 128 x 160, at the edges of its range
+# (both sides of the law's lines: tests/test_host_boundary.py::test_lines_of_the_launch_law_at_17_to_64_rows)
+BAND = [
     (17, 16, 128, "dec_{}_tm2_n1", "dec_{}_tm2_n1"), (32, 4096, 640, "dec_{}_tm2_n1", "dec_{}_tm2_n1"),
     (31, 4112, 256, "dec_{}_tm2", "dec_{}_tm2"), (33, 4112, 4096, "dec_{}_tm3_n2", "dec_{}_tm3_n2"),
     (48, 8192, 4224, "dec_{}_tm3_n2", "dec_{}_tm3_n2"), (40, 4112, 3968, "dec_{}_tm3", "dec_{}_tm3"),

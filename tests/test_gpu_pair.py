@@ -47,8 +47,8 @@ def test_pair_matches_the_oracle_and_two_launches(ctx, M, K, n0, n1):
 
 
 def test_pair_of_named_cells_past_the_streaming_band(ctx):
-    """From 49 rows the launch law hands a linear to the tile GEMM, which does not pair (refused by name);
-    the four-tile streaming cell still pairs when it is named."""
+    """From 49 rows the launch law gives a linear the tile GEMM or a four-tile streaming cell at another block width, neither
+    of which has a pair kernel (refused by name); the four-tile cell `tm4` still pairs when it is named."""
     say("pair of named tm4 cells, M=64")
     M, K, n0, n1 = 64, 512, 80, 48
     rng = np.random.default_rng(64)

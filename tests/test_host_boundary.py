@@ -402,6 +402,37 @@ def test_prefill_launch_is_persistent_and_covers_the_output():
             assert d.n_workspaces == 0 and d.ks == 1
 
 
+def test_lines_of_the_launch_law_at_17_to_64_rows():
+    """Either side of each line that `resolve` draws in rows, columns and K at 17 to 64 rows and for the 128 x 160 cell of
+    int8 weights (the bytes of the cells named here: tests/test_gpu_dense.py)."""
+    def picks(m, n, k):
+        return tuple(iu8.resolve(wk, m, n, k).kernel.decode()[len("macaq_iu8_"):].replace(f"_{tag}_", "_") for wk, tag in ((iu8.W4, "w4"), (iu8.W8, "w8")))
+
+    for (m, n, k), want in {
+            # 17-32 rows: a 16-column block a CU, 32-column blocks, tiles
+            (16, 4096, 6144): "dec_tm1_a0", (17, 4096, 128): "dec_tm2_n1", (32, 4096, 128): "dec_tm2_n1", (32, 4112, 128): "dec_tm2",
+            (32, 16384, 5120): "dec_tm2", (32, 16400, 5120): ("pf_t64x128_s", "pf_t64x64_s"),
+            # 33-48: 32-column blocks from K = 4,096, up to 8,192 columns
+            (33, 4096, 6144): "dec_tm3", (33, 4112, 4096): "dec_tm3_n2", (33, 8192, 3968): "dec_tm3", (48, 8192, 4096): "dec_tm3_n2",
+            (48, 8208, 4096): "pf_t64x64_s",
+            # 49-64: streamed from K = 2,048 (up to 4,096 columns) and 6,144 (up to 8,192)
+            (49, 4096, 1920): "pf_t64x64_s", (49, 4096, 2048): "dec_tm4_k16", (64, 4096, 2048): "dec_tm4_k16", (64, 4096, 6144): "dec_tm4_k16",
+            (64, 4112, 6016): "pf_t64x64_s", (64, 4112, 6144): "dec_tm4_n2", (49, 8192, 6016): "pf_t64x64_s", (49, 8192, 6144): "dec_tm4_n2",
+            (64, 8192, 6144): "dec_tm4_n2", (64, 8208, 6144): "pf_t64x64_s", (65, 4096, 2048): "pf_t64x64_s", (65, 8192, 6144): "pf_t64x64_s",
+            # one row tile past the band: 64, 128 and 160 columns a CU
+            (64, 16384, 640): "pf_t64x64_s", (64, 16400, 640): ("pf_t64x128_s", "pf_t64x64_s"), (32, 32768, 640): ("pf_t64x128_s", "pf_t64x64_s"),
+            (32, 32784, 640): ("pf_t32x160_s", "pf_t64x160_s"), (33, 32784, 640): "pf_t64x160_s", (32, 40960, 640): ("pf_t32x160_s", "pf_t64x160_s"),
+            (64, 40960, 640): "pf_t64x160_s", (17, 40976, 640): ("pf_t64x128_s", "pf_t64x64_s"), (64, 40976, 640): ("pf_t64x128_s", "pf_t64x64_s"),
+            # K shared over workgroups leaves the streaming band to int8 weights
+            (33, 4096, 16384): ("pf_t64x128_s_ks", "dec_tm3"), (33, 4096, 16256): "dec_tm3", (48, 8192, 16384): ("pf_t64x128_s_ks", "dec_tm3_n2")}.items():
+        assert picks(m, n, k) == ((want, want) if isinstance(want, str) else want), (m, n, k)
+    # 128 x 160: one round where 128 x 128 is two, 65 to 1,023 rows
+    for m, n, takes in ((64, 40960, False), (65, 40960, True), (65, 40976, False), (65, 32784, True), (65, 32768, False), (128, 40960, True),
+                        (129, 40960, False), (129, 20480, True), (129, 20496, False), (129, 16400, True), (129, 16384, False),
+                        (1023, 5120, True), (1023, 5136, False), (1023, 4112, True), (1023, 4096, False), (1024, 5120, False)):
+        assert (picks(m, n, 5120)[1] == "pf_t128x160") == takes, (m, n)
+
+
 def test_int8_128x160_cell_only_where_it_measured_faster():
     """The 128 x 160 cell of int8 weights against the estimate's pick: not where a 64-row cell wastes less of a half live
     last row block on a short K, and not on a tile count that leaves the order by XCD at a K of 512 to 2,944."""
