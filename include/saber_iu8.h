@@ -273,10 +273,10 @@ int saber_iu8_silu_mul_quant_had(saber_iu8_ctx *ctx, const void *gu_bf16, void *
 /* saber_iu8_silu_mul_quant_had with a table of the bf16 silu at hand (`silu_lut`: u16 [65536] on the device
  * as saber_iu8_silu_table wrote it, a 128 KiB persistent workspace of the caller, filled once): for rows of
  * SABER_IU8_SILU_LUT_MIN_WIDTH elements and more the launch reads bf16(silu(gate)) from the table's middle,
- * which every workgroup copies into LDS (kernels silu_mul_quant_hadi8_lut_t{256,512}; the computed form
- * spends more than half of its arithmetic on the exp and the divide and is bound by it); narrower rows, or a
- * null table, are saber_iu8_silu_mul_quant_had. Same bytes either way: the table is the computed form's own
- * output. No counterpart among the reference's operators: its producer computes
+ * which every workgroup copies into LDS (kernels silu_mul_quant_hadi8_lut_t{256,512}: 5-11 % ahead of the computed
+ * form on up to 2,048 rows of 17,408, 2-10 % on any width from 2,048 rows on; 2-20 % behind it on up to 512 rows of
+ * 2,048 to 4,096); narrower rows, or a null table, are saber_iu8_silu_mul_quant_had. Same bytes either way: the
+ * table is the computed form's own output. No counterpart among the reference's operators: its producer computes
  * (crates/saber-kernels/hip/mxfp4_hadi8.hip:117-146). */
 #define SABER_IU8_SILU_LUT_MIN_WIDTH 2048u
 int saber_iu8_silu_mul_quant_had_lut(saber_iu8_ctx *ctx, const void *gu_bf16, void *q, float *scale, uint32_t m, uint32_t n,

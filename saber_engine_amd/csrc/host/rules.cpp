@@ -354,9 +354,10 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // this card: 17..32 rows stream unless the output is very wide, 33..64 unless it is wide; from 49 rows a short K
   // goes to the tiles as well: 8192 x 1024 at 50 / 64 rows 7.4 / 7.6 us streamed, 5.2 / 5.1 on 64 x 64, 5120 x 5120 within
   // a tenth either way, 5120 x 6144 12.2 / 12.5 against 14.1; 4096 x 1024 5.5 against 5.1, 4096 x 4096 8.2 against 10.4).
-  // A deep, narrow linear leaves the band at 33 rows already: where the tile law shares K over workgroups
-  // (pf_split), its 64 x 128 cell overtakes the three-tile streaming form (5120 x 17408 at 33 / 40 / 48 rows:
-  // 23.7 / 23.9 / 25.8 us on four shares against 28.2 / 28.3 / 31.3; up to 32 rows streaming wins, 18.0 against 22.4).
+  // A deep, narrow linear of int4 weights leaves the band at 33 rows already: where the tile law shares K over workgroups
+  // (pf_split), its 64 x 128 cell overtakes the streaming form (5120 x 17408 at 33 / 45 rows on four shares 18.6 / 18.9 us,
+  // 21.0 / 22.5 on `tm3_n2`; up to 32 rows streaming wins, 15.5 against 17.5 at 17. A narrower one would stay: 3072 x 16384 at
+  // 33 / 45 rows 17.3 / 17.7 shared, 13.7 / 15.0 on `tm3`).
   const PfVariant *split_cell = nullptr;
   const uint32_t tile_ks = pf_split(wkind == SABER_IU8_W8, m, n, k, &split_cell);
   const bool narrow = n <= 16 * CU_COUNT, two_wide = !narrow && n <= 32 * CU_COUNT;  // a 16- / 32-column block a CU
@@ -400,8 +401,10 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // 15.0 / 16.3 / 17.2, 28672 x 5120 20.3 / 22.4 / 24.4 -> 16.8 / 18.0-20.6 / 18.6-19.3, 24576 x 2048 at 20 / 50 rows
   // 10.3 / 11.4 -> 8.8 / 9.2; at 32768 columns 23.4 / 23.6 / 25.3 -> 19.6 / 23.7 / 24.8; up to 16,384 columns 64 x 64 is one
   // round (16384 x 5120 13.5 against 15.6-16.7) and pf_cell's pick. 160 columns wide up to 40,960 columns (40960 x 5120 at 17 /
-  // 33 / 64 rows 29.6 / 32.5 / 33.5 -> 24.8 / 28.9 / 30.2, W8 52.9 / - / 57.0 -> 42.0 / - / 41.6). Int8 weights up to
-  // 32,768 columns stay with the estimate (64 x 64 and 64 x 128 within 10 % of each other).
+  // 33 / 64 rows 29.6 / 32.5 / 33.5 -> 24.8 / 28.9 / 30.2, W8 52.9 / - / 57.0 -> 42.0 / - / 41.6). There is no line in K: a K of
+  // 512 and less, which no decoder linear this wide has, is 3-23 % slower on the 160-column cells (32784 x 256 at 33 rows W4
+  // / W8 +17 / +12 %, level from 640; 36864 columns W4 +8 %, W8 faster). Int8 weights up to 32,768 columns stay with the estimate
+  // (64 x 64 and 64 x 128 within 10 % of each other).
   if (m <= 64 && n > 32 * 2 * CU_COUNT && n <= 160 * CU_COUNT) {
     const char *cell = n > 128 * CU_COUNT ? (!w8 && m <= 32 ? "t32x160_s" : "t64x160_s") : w8 ? nullptr : "t64x128_s";
     if (cell) return describe_pf(*pf_variant(fmt("macaq_iu8_pf_%s_%s", tag, cell)), m, n, k, 0, out);
@@ -432,21 +435,18 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
 
 // K shares of a tile launch (0: none). A deep, narrow linear at a few dozen rows gives the unsplit
 // law so few tiles that half to two thirds of the CUs idle through hundreds of K steps; there, 2-4 workgroups
-// a tile of the 64x128 cell, each on a share of K, measured 9-19 % faster although the partials
-// travel through memory (5120 x 17408: M=64 34.1 -> 28.6 us, M=128 33.6 -> 30.7 us). On every other
-// shape timed (K <= 6144 at any M, more than 128 tiles at any K, 256 rows and more) the unsplit cell won --
-// the partials cost ks*M*N*4 bytes each way and the last arriver sums alone -- so the rule is this
-// narrow. The launch then needs the `decode_partial` / `decode_counter` workspaces the descriptor lists.
+// a tile of the 64x128 cell, each on a share of K, are faster although the partials travel through memory (ks * M * N * 4
+// bytes each way, and the last share to arrive sums the others). The launch then needs the `decode_partial` /
+// `decode_counter` workspaces the descriptor lists.
 uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant **cell) {
-  // (timings of this comment from before the cell stood on four waves side by side and the reduction read in batches, which
-  // took 5120 x 17408 at 45 / 64 / 128 / 180 rows from 25.2 / 28.9 / 31.0 / 35.3 to 18.5 / 19.3 / 22.8 / 28.5 us)
-  // measured at 33..192 rows; above, the partials (ks * M * N * 4 bytes each way) grow with M (at 256 rows the unsplit
-  // cell is level or ahead: 5120 x 17408 43.9 against 43.9-58.6 us). Up to 128 tiles, i.e. two shares at least:
-  // 81-128 tiles on two shares against the law's unsplit pick, us -- 5120 x 17408 at 129 / 160 / 192 rows 33.7 / 34.1 /
-  // 35.3 against 35.4 / 36.7 / 36.5, 5120 x 20480 38.2 / 38.8 / 38.4 against 40.4 / 42.1 / 42.5, 4096 x 16384 31.0 / 31.4 /
-  // 32.0 against 32.3 / 33.4 / 33.6; 8192 x 16384 at 96 / 128 rows 33.0 / 34.6 against 36.4 / 37.9, 12288 x 16384 at
-  // 49 / 64 rows 33.3 / 34.6 against 35.8 / 35.5; 72 tiles on three shares (3072 x 16384 at 129-192 rows) 28.1-28.7
-  // against 31.7-32.0.
+  // us, the law's shares against the fastest unsplit cell: 5120 x 17408 at 64 / 128 / 160 / 192 rows 19.4 / 22.4 / 28.8 / 29.3
+  // against 24.6 / 33.5 / 33.5 / 33.8, at 200 / 256 rows three shares 37.4 / 38.1 against 35.4 / 39.6; 8192 x 16384 at 96 / 128 rows
+  // 27.7 / 28.7 against 32.4 / 33.1, and past 128 tiles, at 160 rows, 49.9 against 35.2; 3072 x 16384 at 160 / 192 rows 21.1 / 21.1
+  // against 31. The lines in K and rows were drawn with a slower reduction and are narrower than these timings would have
+  // them: K = 12,288 is not shared (5120 columns at 96 / 128 / 192 rows 18.0 / 18.3 / 22.1 on shares, 24.6 / 24.8 / 25.2 as it
+  // is), nor 96 tiles at 200-256 rows (3072 x 16384 25.7 against 31.5), nor 2-4 tiles of K = 5,120 (96 columns at 96-256
+  // rows 10.0 against 11.6); six shares of 40 tiles are 2-3 % ahead of four at 33-64 rows, eight behind. (A `_ks`
+  // workgroup takes 81,924 bytes of LDS: one a CU, not the two of `occ`.)
   if (w8 || k < 16384 || m > 192) return 0;
   const PfVariant *v = pf_variant("macaq_iu8_pf_w4_t64x128_s");
   if (!v || !signature_for(std::string(v->name) + "_ks")) return 0;
@@ -470,9 +470,12 @@ uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant *
 // cold (successive launches walk copies that exceed the memory-side cache; with warm weights the 64 x 64
 // cell overtakes the 64 x 128 one at 256 rows, which no layer of a model sees), and checked on shapes the fit had
 // not seen -- the served 27B graph's own 16384 x 5120, 14336 x 5120, 5120 x 6144 and 96 x 5120 at eight row counts,
-// which moved three small-cell rates and took the side-by-side term off the 64-row cells. W4: 850 timings, the
-// pick is within 0.6 % of the fastest measured cell on all 88 shape x M points; W8, output-side shapes: every
-// pick the fastest. The reference keeps its band tables the same way
+// which moved three small-cell rates and took the side-by-side term off the 64-row cells. The W4 64 x 128 cell has
+// since moved to four waves side by side and is 12-16 % faster than its constants here say; with it the pick is within
+// 0.6 % of the fastest cell on 105 of 111 points (eight shapes, 65 to 8,192 rows) and within 3 % on 108; off are 300 rows
+// of 7168 x 5120 (23.5 us on 128 x 128, 20.5 on 64 x 128) and of 34816 x 5120 (76.6 on 256 x 320, 69.9). W8, output-side shapes
+// from 2,048 rows: every pick the fastest; at 1,025 to 1,280 rows up to 7 % off (256 x 160, 128 x 128 two a CU). The
+// reference keeps its band tables the same way
 // (crates/saber-kernels/src/macaq_iu8.rs:150-212). One table for both kinds had sent the int8-weight
 // O and down projections at 2,048 rows to the 128 x 320 cell, 17-22 % behind the 256 x 160 cell there.
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
@@ -689,9 +692,10 @@ int resolve_gate_up_act(uint32_t m, uint32_t hidden, uint32_t inter, saber_iu8_d
 // Rows wider than 4,096 whose count leaves the card part idle go 16 waves a row (`base`_t1024): measured on this
 // card, graph replay, 256-thread form / 1024-thread form in us -- the quantiser at 1 / 16 / 256 rows of 5,120:
 // 2.57/2.34, 2.98/2.74, 3.41/3.20; of 17,408: 3.90/2.91, 5.09/3.92, 6.72/5.49; at 512 rows 3.98/4.52 and 7.92/7.09, at
-// 1,024 4.84/6.32 and 13.3/14.3. The activation (timed with the library exp and an IEEE divide an element, its four-a-time form is 13-16 % faster) at 1 / 16 / 512 rows of 5,120:
-// 6.36/4.64, 6.75/5.02, 8.22/7.13; of 17,408: 13.6/7.50, 14.3/8.06, 18.8/14.9, and 47.0/42.4 at 2,048 rows (5,120
-// there: 17.5/22.1). Rows of 4,096: the two forms are within 3 % (a thread of either owns one group).
+// 1,024 4.84/6.32 and 13.3/14.3. The activation at 1 / 16 / 256 / 300 / 512 rows of 5,120: 4.16/3.64, 4.47/3.92, 5.34/4.86,
+// 5.66/5.72, 5.85/6.24 (the two cross at about 300 rows, the line lies at 512; of 8,192 at 512: 6.99/7.10); of 17,408 at 1 / 16 /
+// 512 / 2,048: 7.92/5.55, 8.35/6.02, 14.0/12.4, 35.9/32.6 (5,120 there: 13.5/16.7); of 12,288 at 2,048 / 4,096 rows 25.8/24.6 and
+// 42.4/43.3. Rows of 4,096: the two forms are within 4 % up to 256 rows (a thread of either owns one group).
 static std::string row_form(const char *base, uint32_t rows, uint32_t width, bool silu = false) {
   if (width <= 2048 && rows % 4 == 0 && rows >= 64) return std::string(base) + "_w64";  // up to two groups a lane
   if (width > T1024_WIDTH_OVER &&
