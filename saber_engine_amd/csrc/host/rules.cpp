@@ -354,6 +354,9 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // this card: 17..32 rows stream unless the output is very wide, 33..64 unless it is wide; from 49 rows a short K
   // goes to the tiles as well: 8192 x 1024 at 50 / 64 rows 7.4 / 7.6 us streamed, 5.2 / 5.1 on 64 x 64, 5120 x 5120 within
   // a tenth either way, 5120 x 6144 12.2 / 12.5 against 14.1; 4096 x 1024 5.5 against 5.1, 4096 x 4096 8.2 against 10.4).
+  // All of it with weights that come from memory, as in a model's pass: at 64 rows streamed / on 64 x 64, int4 4096 x 2048 7.1 / 7.0,
+  // 2048 x 3072 7.0 / 8.7, int8 6.3 / 7.2, 7.1 / 9.4; on weights still in the memory-side cache 7.7 / 6.9, 7.6 / 8.7, 6.9 / 5.9,
+  // 7.7 / 7.1 (there int8 of up to 3,072 columns would stay on the tiles to K of some 5,000).
   // A deep, narrow linear of int4 weights leaves the band at 33 rows already: where the tile law shares K over workgroups
   // (pf_split), its 64 x 128 cell overtakes the streaming form (5120 x 17408 at 33 / 45 rows on four shares 18.6 / 18.9 us,
   // 21.0 / 22.5 on `tm3_n2`; up to 32 rows streaming wins, 15.5 against 17.5 at 17. A narrower one would stay: 3072 x 16384 at
@@ -403,7 +406,8 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // round (16384 x 5120 13.5 against 15.6-16.7) and pf_cell's pick. 160 columns wide up to 40,960 columns (40960 x 5120 at 17 /
   // 33 / 64 rows 29.6 / 32.5 / 33.5 -> 24.8 / 28.9 / 30.2, W8 52.9 / - / 57.0 -> 42.0 / - / 41.6). There is no line in K: a K of
   // 512 and less, which no decoder linear this wide has, is 3-23 % slower on the 160-column cells (32784 x 256 at 33 rows W4
-  // / W8 +17 / +12 %, level from 640; 36864 columns W4 +8 %, W8 faster). Int8 weights up to 32,768 columns stay with the estimate
+  // / W8 +17 / +12 %; W4 level from 1,024 there and from 640 at 34,816 columns and more, W8 from 384; 36864 columns W4 +8 %, W8
+  // faster). Int8 weights up to 32,768 columns stay with the estimate
   // (64 x 64 and 64 x 128 within 10 % of each other).
   if (m <= 64 && n > 32 * 2 * CU_COUNT && n <= 160 * CU_COUNT) {
     const char *cell = n > 128 * CU_COUNT ? (!w8 && m <= 32 ? "t32x160_s" : "t64x160_s") : w8 ? nullptr : "t64x128_s";
