@@ -462,3 +462,15 @@ def test_band_of_17_to_64_rows_and_its_cells(ctx, shape):
         assert run.desc.kernel.decode() == "macaq_iu8_" + want.format(tag) and run.desc.ks == 1
         r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
         np.testing.assert_array_equal(run.C, r["C"])
+
+
+@pytest.mark.parametrize("kernel,ks", [("macaq_iu8_dec_w4_tm1_a0", 1), ("macaq_iu8_dec_w8_tm1_a0", 3), ("macaq_iu8_dec_w4_tm2", 2),
+                                       ("macaq_iu8_dec_w4_tm3_n2", 3), ("macaq_iu8_dec_w8_tm4_n2", 5), ("macaq_iu8_dec_w4_tm4_k16", 1)])
+def test_streamed_cells_spread_their_sums_over_the_waves(ctx, kernel, ks):
+    """Every wave sums and stores its share of a block's 16 x 16 tiles: a block with one live tile, row tiles without a
+    live row, k-waves without a step, shares of K added by the last to arrive. Exact against the oracle."""
+    tm = int(kernel.split("_tm")[1][0])
+    for M, N, K in [(tm * 16, 16, 128 * ks), (tm * 16 - 15, 48, 128 * (ks + 8)), (1, 80, 128 * 17), (tm * 16 - 1, 272, 2560)]:
+        case = synth.dense_case(M, N, K, w8="_w8_" in kernel, seed=M + N + K)
+        run = DenseRun(ctx, case, kernel=kernel, ks=ks, want_acc=False)
+        assert_dense_matches(run, ref.linear(case["X"], case["W"], case["ws"], "_w8_" in kernel), "_w8_" in kernel)
