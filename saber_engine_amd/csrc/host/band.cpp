@@ -262,7 +262,11 @@ std::string band_toml() {
       put(o, "regime", std::string("decode"));
       putb(o, "w8", v->w8 != 0);
       put(o, "rows_max", (uint64_t)v->tm * 16);
-      put(o, "block_n", v->block_n());
+      put(o, "block_n", v->block_n(1, 1));
+      if (v->block_n(1, 2) != v->block_n(1, 1)) {  // past one round of the own blocks, and for a split of K
+        put(o, "block_n_wide", v->block_n(1, 2));
+        put(o, "wide_from_n", 32 * 256 + 16);
+      }
       put(o, "threads", v->threads());
       put(o, "grid", std::string("[ceil(n / block_n), 1, ks]"));
       put(o, "kernarg", std::string("dec"));
@@ -276,6 +280,14 @@ std::string band_toml() {
       put(o, "threads", 1024);
       put(o, "grid", std::string("[blocks = ceil(n / 32); blocks <= cu_count ? blocks : ceil(blocks / min(8, ceil(blocks / cu_count))), 1, 1] persistent"));
       put(o, "kernarg", std::string("dec"));
+    } else if (const WideVariant *v = wide_variant(name)) {
+      put(o, "regime", std::string("wide"));
+      putb(o, "w8", v->w8 != 0);
+      put(o, "rows_max", v->block_m());
+      put(o, "block_n", v->block_n());
+      put(o, "threads", v->threads());
+      put(o, "grid", std::string("[ceil(n / block_n), 1, 1]"));
+      put(o, "kernarg", std::string("pf"));
     } else if (const PfVariant *v = pf_variant(ks_form ? name.substr(0, name.size() - 3) : name)) {
       put(o, "regime", std::string("prefill"));
       putb(o, "w8", v->w8 != 0);

@@ -18,6 +18,10 @@ static const PfVariant PF_VARIANTS[] = {
 #define IU8_PF_TAP(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) {#name, W8, WMW, WNW, TM, TN, ACC, OCC},
 #include "../kernels/iu8_variants.def"
 };
+static const WideVariant WIDE_VARIANTS[] = {
+#define IU8_WIDE_VARIANT(name, TM, W8, NT, KW, D) {#name, TM, W8, NT, KW},
+#include "../kernels/iu8_variants.def"
+};
 static const DecVariant PAIR_VARIANTS[] = {
 #define IU8_PAIR_VARIANT(name, TM, NT, KW, WPB, D, ALDS, BFIRST) {#name, TM, false, NT, KW, WPB, D, ALDS, false},
 #include "../kernels/iu8_variants.def"
@@ -30,6 +34,11 @@ const DecVariant *dec_variant(const std::string &name) {
 }
 const DecVariant *pair_variant(const std::string &name) {
   for (const DecVariant &v : PAIR_VARIANTS)
+    if (name == v.name) return &v;
+  return nullptr;
+}
+const WideVariant *wide_variant(const std::string &name) {
+  for (const WideVariant &v : WIDE_VARIANTS)
     if (name == v.name) return &v;
   return nullptr;
 }
@@ -99,12 +108,6 @@ static int check_shape(const char *op, uint32_t m, uint32_t n, uint32_t k) {
   return 0;
 }
 
-// The grid-level split of a decode GEMM. The k-waves of a workgroup already split K through LDS, and
-// a split across workgroups adds 1.5-2 us of hand-over (partials through memory, a device-scope
-// counter) to launches whose fixed cost dominates: measured on the 27B-class shapes it never wins
-// by more than the noise, so the law does not split; `describe` still takes an explicit count.
-uint32_t decode_split(uint32_t, uint32_t, uint32_t, uint32_t, uint32_t) { return 1; }
-
 static int describe_dec(const DecVariant &v, uint32_t m, uint32_t n, uint32_t k, uint32_t ks, saber_iu8_desc *d) {
   const char *op = v.w8 ? "gemm_i8a8" : "gemm_i4a8";
   if (int rc = check_shape(op, m, n, k)) return rc;
@@ -114,7 +117,7 @@ static int describe_dec(const DecVariant &v, uint32_t m, uint32_t n, uint32_t k,
   copy_name(d->op, sizeof d->op, op);
   copy_name(d->plugin, sizeof d->plugin, "macaq_iu8");
   copy_name(d->kernel, sizeof d->kernel, v.name);
-  const uint32_t nblk = (n + v.block_n() - 1) / v.block_n();
+  const uint32_t bn = v.block_n(n, ks), nblk = (n + bn - 1) / bn;
   d->grid[0] = nblk, d->grid[1] = 1, d->grid[2] = ks;
   d->block[0] = v.threads(), d->block[1] = 1, d->block[2] = 1;
   d->n_launches = 1;
@@ -175,6 +178,25 @@ static int describe_pf(const PfVariant &v, uint32_t m, uint32_t n, uint32_t k, u
   return 0;
 }
 
+static int describe_wide(const WideVariant &v, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *d) {
+  const char *op = v.w8 ? "gemm_i8a8" : "gemm_i4a8";
+  if (int rc = check_shape(op, m, n, k)) return rc;
+  if (m > (uint32_t)v.block_m()) return fail(SABER_IU8_E_RULE, fmt("%s: %s holds %d rows, M=%u", op, v.name, v.block_m(), m));
+  memset(d, 0, sizeof *d);
+  copy_name(d->op, sizeof d->op, op);
+  copy_name(d->plugin, sizeof d->plugin, "macaq_iu8");
+  copy_name(d->kernel, sizeof d->kernel, v.name);
+  d->grid[0] = (n + v.block_n() - 1) / v.block_n(), d->grid[1] = 1, d->grid[2] = 1;
+  d->block[0] = v.threads(), d->block[1] = 1, d->block[2] = 1;
+  d->n_launches = 1;
+  d->ks = 1;
+  if (int rc = fill_slots(v.name, d)) return rc;
+  set_i32(d, "m", m);
+  set_i32(d, "n", n);
+  set_i32(d, "k", k);
+  return 0;
+}
+
 static uint64_t staged_bytes(uint32_t m, uint32_t k);
 // The streaming decode cell of M rows: tm 16-row tiles; one tile's live rows staged in LDS when they fit the 20 KiB
 // form, else streamed from L2 beside the weights.
@@ -225,6 +247,10 @@ int describe(const std::string &kernel, uint32_t m, uint32_t n, uint32_t k, uint
   if (kernel == "macaq_iu8_dec_w4_tm1_s80" || kernel == "macaq_iu8_dec_w8_tm1_s80") return describe_s80(kernel[15] == '8', false, m, n, k, ks, out);
   if (kernel == "macaq_iu8_dec_w4_tm1_s80r" || kernel == "macaq_iu8_dec_w8_tm1_s80r") return describe_s80(kernel[15] == '8', true, m, n, k, ks, out);
   if (const DecVariant *v = dec_variant(kernel)) return describe_dec(*v, m, n, k, ks, out);
+  if (const WideVariant *v = wide_variant(kernel)) {
+    if (ks != 1) return fail(SABER_IU8_E_RULE, kernel + ": the wide streamed cell does not split K");
+    return describe_wide(*v, m, n, k, out);
+  }
   if (const PfVariant *v = pf_variant(kernel)) {
     if (ks != 1) return fail(SABER_IU8_E_RULE, kernel + ": the prefill tile does not split K (its `_ks` form does)");
     return describe_pf(*v, m, n, k, 0, out);
@@ -316,7 +342,9 @@ int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_de
   const std::string name = std::string("macaq_iu8f_") + form + "_w4_" + k0.substr(sizeof PREFIX - 1);
   const DecVariant *pv = pair_variant(name);
   if (!pv) return fail(SABER_IU8_E_RULE, name + ": the fused object carries no such pair");
-  const uint32_t nb0 = first.grid[0], nb1 = second.grid[0], ks0 = first.ks, ks1 = second.ks;
+  const uint32_t ks0 = first.ks, ks1 = second.ks;
+  auto blocks = [&](int64_t n, uint32_t ks) { return (uint32_t)((n + pv->block_n((uint32_t)n, ks) - 1) / pv->block_n((uint32_t)n, ks)); };
+  const uint32_t nb0 = blocks(n0, ks0), nb1 = blocks(n1, ks1);
   memset(out, 0, sizeof *out);
   copy_name(out->op, sizeof out->op, "gemm_i4a8_pair");
   copy_name(out->plugin, sizeof out->plugin, "macaq_iu8f");
@@ -338,11 +366,70 @@ int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_de
     } else {
       for (uint32_t i = 0; i < half[h]->n_workspaces; ++i) {
         const saber_iu8_workspace &w = half[h]->workspaces[i];
-        add_ws(out, (std::string(w.name) + sfx).c_str(), w.kind, w.bytes, w.zero_once);
+        add_ws(out, (std::string(w.name) + sfx).c_str(), w.kind, strcmp(w.name, "decode_counter") ? w.bytes : (uint64_t)(h ? nb1 : nb0) * 4, w.zero_once);
       }
     }
   }
   return 0;
+}
+
+// 33 to 64 rows on the streaming cells' 64-column blocks (iu8_stream_law.h) from three quarters of the CUs, where the 64 x 64
+// tile had them. us before / here, W4: 16384 x 5120 at 45 / 64 rows 14.8 / 15.4 -> 11.8 / 13.3, 14336 x 5120 13.8 / 14.7 -> 11.5 / 12.9, x
+// 2048 at 40 rows 1.12, x 3072 at 56 rows 1.03 times faster (x 1024 / 2048 0.95 / 1.06); W8 14336 x 4096 at 40 rows 1.08, x 5120 1.06 (x
+// 3072 1.02, at 56 rows 0.99).
+static bool stream_wide_blocks(bool w8, uint32_t m, uint32_t n, uint32_t k) {
+  if (m <= 32 || n <= (CU_COUNT * 3 / 4 - 1) * 64 || n > 64 * CU_COUNT) return false;
+  return m <= 48 ? k >= (w8 ? 4096u : 2048u) : !w8 && k >= 3072;
+}
+
+// K shares of a streaming launch of 9 to 48 rows. A deep linear of 3,000 to 5,440 columns has too few 64-column blocks for the
+// CUs and, on narrower ones, reads its rows once a block: three or four workgroups a block, each on a share of K, divide
+// the rows' bytes as well (the partials, shares * M * N * 4 bytes each way, cost some 2 us). us unsplit / here, N = 5120, W4: 16 rows of
+// K = 10240 / 12288 / 17408 9.0 / 10.0 / 13.7 -> 8.6 / 9.5 / 11.2 (8192: 7.5 -> 8.0), 32 rows of 8192 / 12288 / 17408 9.1 / 12.5 / 17.4 -> 8.4 /
+// 10.3 / 12.7, 48 rows of 8192 / 12288 10.6 / 14.8 -> 9.6 / 11.5 (6144 level); W8 16 / 32 / 48 rows of 12288 14.7 / 17.8 / 20.2 -> 14.2 / 15.2 /
+// 16.4. 4096 columns on four shares, 16 / 32 rows of 16384 12.2 / 13.2 -> 11.3 / 11.9, 20 rows of 10240 level. Up to eight rows it is
+// level at best. The static workspace holds it (3.9 MB), and a caller that binds no workspaces gets the launch in one piece.
+static uint32_t stream_split(uint32_t m, uint32_t n, uint32_t k) {
+  const uint32_t blocks = (n + 16 * IU8_STREAM_WIDE_NT - 1) / (16 * IU8_STREAM_WIDE_NT);
+  const uint32_t z = blocks ? std::min(4u, CU_COUNT / blocks) : 0;
+  if (m <= 8 || m > 48 || z < 3 || blocks * 4 < CU_COUNT * 3 / 4) return 1;
+  return k >= (m <= 16 ? 10240u : n <= 4096 ? 12288u : 8192u) ? z : 1;
+}
+
+// The wide streamed cells: blocks of 64, 96 or 144 columns that give three quarters of the CUs and more one block each, from
+// the K at which they measured faster than the tile the law had (a short K is all pipeline fill and hand-over in LDS, which
+// grow with the block). Before / here in us, K = 5,120 unless it says so -- W4 34816 columns at 24 / 40 / 56 / 72 / 88 rows, ratio 1.18 /
+// 1.12 / 1.07 / 1.32 / 1.26; 24576 columns 1.22 / 1.15 / 1.07 / 1.15 / 1.10; 16384 at 72 / 88 rows 1.24 / 1.07; W8 20480 columns 1.37 /
+// 1.41 / 1.37 / 1.17 / 1.11, 28672 at 24 / 40 / 56 rows 1.15 / 1.15 / 1.12, 34816 1.07 / 1.03 / 1.03, 14336 at 72 / 88 rows 1.29 / 1.21. One step
+// of K below each line: W4 24576 x 1024 at 40 rows 0.93, x 2048 at 56 / 88 rows 0.96 / 0.96; 34816 x 1024 at 40 / 56 / 88 rows 0.96 / 0.86 /
+// 0.98; 28672 x 5120 at 40 rows 0.94 (no line there); W8 24576 x 1024 at 72 rows 0.90, 28672 x 2048 at 40 / 56 rows 0.94 / 0.91, 34816 x
+// 3072 at 40 rows 1.01. (fifteen widths x six K x five row counts of each kind, weights from memory.)
+static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
+  if (m <= 16 || m > 96) return nullptr;
+  struct Line {
+    uint32_t nt, n_over, n_max;  // columns (n_over, n_max]
+    uint32_t k4[5], k8[5];       // least K at 17-32, 33-48, 49-64, 65-80, 81-96 rows, int4 / int8 weights; 0: not taken
+  };
+  constexpr uint32_t BUSY = CU_COUNT * 3 / 4 - 1;
+  static const Line LINES[] = {
+      {4, BUSY * 64, 64 * CU_COUNT, {0, 0, 0, 8192, 8192}, {0, 0, 0, 2048, 3072}},
+      {6, BUSY * 96, 96 * CU_COUNT, {1024, 2048, 4096, 3072, 5120}, {1024, 1024, 2048, 3072, 4096}},
+      {9, BUSY * 144, 128 * CU_COUNT, {4096, 0, 0, 0, 0}, {1024, 3072, 4096, 0, 0}},
+      {9, 128 * CU_COUNT, 144 * CU_COUNT, {1024, 2048, 4096, 2048, 2048}, {1024, 5120, 8192, 0, 0}},
+  };
+  const uint32_t tm = (m + 15) / 16;
+  for (const Line &l : LINES) {
+    if (n <= l.n_over || n > l.n_max) continue;
+    const uint32_t k_min = (w8 ? l.k8 : l.k4)[tm - 2];
+    return k_min && k >= k_min ? wide_variant(fmt("macaq_iu8_pf_%s_t%ux%u_w", w8 ? "w8" : "w4", tm * 16, l.nt * 16)) : nullptr;
+  }
+  return nullptr;
+}
+
+int unsplit_stream(saber_iu8_desc *d) {
+  int64_t m = 0, n = 0, k = 0;
+  if (d->ks <= 1 || !dec_variant(d->kernel) || !int_arg(*d, "m", &m) || !int_arg(*d, "n", &n) || !int_arg(*d, "k", &k)) return 0;
+  return describe(std::string(d->kernel), (uint32_t)m, (uint32_t)n, (uint32_t)k, 1, d);
 }
 
 int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) {
@@ -365,6 +452,7 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   const uint32_t tile_ks = pf_split(wkind == SABER_IU8_W8, m, n, k, &split_cell);
   const bool narrow = n <= 16 * CU_COUNT, two_wide = !narrow && n <= 32 * CU_COUNT;  // a 16- / 32-column block a CU
   const bool stream = m <= 16 || (m <= 32 && n <= 16384) || (m <= 48 && n <= 8192 && tile_ks == 0) ||
+                      (tile_ks == 0 && m <= 64 && stream_wide_blocks(w8, m, n, k)) ||
                       (tile_ks == 0 && ((narrow && k >= 2048) || (two_wide && k >= 6144)));
   if (m <= DECODE_MAX_M && stream) {
     // Up to 16 rows of K <= 5120: the persistent form that stages the 16-row tile once a workgroup (`_s80`) where
@@ -391,12 +479,12 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
     std::string name = dec_stream_name(tag, m, k);
     if (m > 16 && m <= 32 && narrow) name += "_n1";
     else if (m > 32 && two_wide && k >= 4096) name += "_n2";
-    else if (m > 48) name += "_k16";
+    else if (m > 48 && narrow) name += "_k16";
     const DecVariant *v = dec_variant(name);
     if (!v) return fail(SABER_IU8_E_RULE, name + ": no such variant");
-    const uint32_t nblk = (n + v->block_n() - 1) / v->block_n();
-    return describe_dec(*v, m, n, k, decode_split(m, n, k, nblk, v->kw), out);
+    return describe_dec(*v, m, n, k, stream_split(m, n, k), out);
   }
+  if (const WideVariant *v = stream_wide_cell(w8, m, n, k)) return describe_wide(*v, m, n, k, out);
   if (tile_ks) return describe_pf(*split_cell, m, n, k, tile_ks, out);
   // One row tile, past the streaming band: a tile's chain of K steps is what the launch takes, so the cell is the
   // narrowest that needs one round of the 256 CUs (the estimate of pf_cell is fitted to 65 rows and more and took 64 x 64

@@ -1,19 +1,31 @@
 // The gfx950 launch law of the iu8 path: which kernel, grid, block, split and workspaces a
 // GEMM of m x n x k runs. The counterpart of crates/saber-kernels/src/macaq_iu8.rs
-// (cell :286-358, decode_split :267-279, describe :429-489); the tables are this object's own
+// (cell :286-358, the decode split :267-279, describe :429-489); the tables are this object's own
 // speed data (256 CUs in 8 XCDs instead of the reference's 64-CU card).
 #pragma once
+#include <algorithm>
 #include <string>
 
 #include "../../../include/saber_iu8.h"
+#include "../kernels/iu8_stream_law.h"
 
 namespace iu8 {
 
 struct DecVariant {
   const char *name;
   int tm, w8, nt, kw, wpb, depth, alds, acc;
-  int block_n() const { return wpb / kw * nt * 16; }
+  // columns a workgroup: a streamed symbol (no staged rows) holds 64-column blocks as well (iu8_stream_law.h)
+  int block_n(uint32_t n, uint32_t ks) const {
+    return alds == 0 && iu8_stream_wide(kw, (int)std::min<uint32_t>(n, 0x7FFFFFFF), (int)ks) ? IU8_STREAM_WIDE_NT * 16 : wpb / kw * nt * 16;
+  }
   int threads() const { return wpb * 64; }
+};
+struct WideVariant {  // the streamed cell on the prefill kernarg list: one block of block_n columns a workgroup
+  const char *name;
+  int tm, w8, nt, kw;
+  int block_m() const { return tm * 16; }
+  int block_n() const { return nt * 16; }
+  int threads() const { return kw * 64; }
 };
 struct PfVariant {
   const char *name;
@@ -25,6 +37,7 @@ struct PfVariant {
 
 const DecVariant *dec_variant(const std::string &name);
 const PfVariant *pf_variant(const std::string &name);
+const WideVariant *wide_variant(const std::string &name);
 // The prefill cell (tile shape) the launch law picks for a shape.
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k);
 uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant **cell);
@@ -45,10 +58,9 @@ constexpr uint32_t T1024_QUANT_ROWS = 256, T1024_QUANT_ROWS_WIDE = 512;
 constexpr uint32_t T1024_SILU_ROWS = 512;
 constexpr uint32_t T1024_WIDE = 12288;
 
-// Grid-level split of a decode GEMM whose grid has `nblk` column blocks.
-uint32_t decode_split(uint32_t m, uint32_t n, uint32_t k, uint32_t nblk, uint32_t kw);
-
 int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out);
+// The launch of a caller that binds no workspaces: `d` itself, or its streamed cell with K in one piece.
+int unsplit_stream(saber_iu8_desc *d);
 int describe(const std::string &kernel, uint32_t m, uint32_t n, uint32_t k, uint32_t ks, saber_iu8_desc *out);
 // Two W4 decode descriptors of one M, K and kernel -> the one-dispatch pair (macaq_iu8.rs:632-704).
 // order: -1 the law's block order, 0 problem 0 first (`pair`), 1 the second problem first (`pairb`).

@@ -548,6 +548,8 @@ int saber_iu8_gemm(saber_iu8_ctx *ctx, int wkind, const void *a, const float *as
                    void *c, uint32_t m, uint32_t n, uint32_t k, void *partial, void *counter, void *stream) {
   saber_iu8_desc d;
   if (int rc = resolve(wkind, m, n, k, &d)) return rc;
+  if (!partial && !counter)  // a streamed launch in one piece needs neither
+    if (int rc = unsplit_stream(&d)) return rc;
   return launch_gemm(ctx, d, a, as, w, ws, c, partial, counter, stream);
 }
 
@@ -559,6 +561,7 @@ int saber_iu8_gemm_static(saber_iu8_ctx *ctx, int wkind, const void *a, const fl
   if (!ctx) return fail(SABER_IU8_E_ARG, "gemm_static: null context");
   saber_iu8_desc d;
   if (int rc = resolve(wkind, m, n, k, &d)) return rc;
+  if (int rc = unsplit_stream(&d)) return rc;  // the array is one a GPU: what can do without it does, so that such calls may overlap
   void *partial = nullptr, *counter = nullptr;
   for (uint32_t i = 0; i < d.n_workspaces; ++i) {
     const saber_iu8_workspace &wsp = d.workspaces[i];
@@ -589,6 +592,8 @@ int saber_iu8_gemm_pair(saber_iu8_ctx *ctx, const void *a, const float *as, cons
   saber_iu8_desc d0, d1, d;
   if (int rc = resolve(SABER_IU8_W4, m, n, k, &d0)) return rc;
   if (int rc = resolve(SABER_IU8_W4, m, n_b, k, &d1)) return rc;
+  if (int rc = unsplit_stream(&d0)) return rc;
+  if (int rc = unsplit_stream(&d1)) return rc;
   if (int rc = pair(d0, d1, &d)) return rc;
   if (d.n_workspaces) return fail(SABER_IU8_E_RULE, "gemm_pair: a half splits K; bind its workspaces through saber_iu8_pair + saber_iu8_launch");
   const saber_iu8_binding b[] = {{"a", (void *)a},     {"as", (void *)as},     {"w", (void *)w}, {"ws", (void *)ws}, {"c", c},

@@ -4,14 +4,19 @@
 #pragma once
 #include "iu8_gemm.h"
 #include "iu8_pf32.h"
+#include "iu8_stream.h"
 
 #define IU8_DEC(name, TM, W8, NT, KW, WPB, D, ALDS, ACC)                                                         \
   extern "C" __global__ __launch_bounds__(WPB * 64) void name(                                                    \
       const unsigned char *__restrict__ a, const unsigned char *__restrict__ w, const float *__restrict__ as,     \
       const float *__restrict__ ws, int *__restrict__ decode_partial, int *__restrict__ decode_counter,           \
       unsigned short *__restrict__ c, int m, int n, int k) {                                                       \
-    iu8_dec_body<TM, W8, NT, KW, WPB, D, ALDS, ACC>(a, w, as, ws, decode_partial, decode_counter, c,          \
-                                                    iu8_rows{nullptr, 0, m}, n, k);     \
+    if constexpr (ALDS == 0) {                                                                                      \
+      iu8_stream_cells<TM, W8, NT, KW, D, ACC>(a, w, as, ws, decode_partial, decode_counter, c, m, n, k);           \
+    } else {                                                                                                       \
+      iu8_dec_body<TM, W8, NT, KW, WPB, D, ALDS, ACC>(a, w, as, ws, decode_partial, decode_counter, c,              \
+                                                      iu8_rows{nullptr, 0, m}, n, k);                               \
+    }                                                                                                              \
   }
 
 // Persistent launch: gridDim.x workgroups (one or OCC a CU) walk the tiles of the m x n output.

@@ -63,25 +63,11 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
   constexpr int WSTEP = W8 ? 2048 : 1024;  // bytes of one 16-row weight tile per 128-deep K step
   constexpr int WV = W8 ? 2 : 1;           // 16-byte loads a lane per step per tile
   constexpr int BN = WN * NT * 16;         // columns a workgroup
-  // The k-waves' partials are summed and stored by all waves, a 16 x 16 tile at a time (the streamed dense forms), or by the
-  // first k-wave of each column group (OWN), which holds the sum in the registers it accumulated in. With the spread tail
-  // the compiler puts the unpack of the staged form's whole ring, and the wait for it, in front of the cases of its last
-  // steps (5120 x 5120 at one row 4.8 -> 5.2 us, 94 registers instead of 64), and the grouped launches, eight waves a
-  // SIMD on weights of hundreds of experts, lost a quarter (the routed layer at 16 tokens 139 -> 175 us).
-  constexpr bool OWN = ALDS > 0 || !EXACT;
-  static_assert(KW > 1, "several k-waves");
-  constexpr int RED = (OWN ? KW - 1 : KW) * WN * TM * NT * 1024;
-  constexpr int ITEMS = WN * TM * NT;                      // 16 x 16 output tiles of the workgroup: item (wn, i, j)
-  constexpr int NI = (ITEMS + WPB - 1) / WPB;              // ... a wave sums and stores
-  // the epilogue's scales are requested in front of everything else and wait in registers: asked for behind the last
-  // K step they are one or two memory latencies on the launch (the grouped launches have no registers to spare)
-  constexpr bool PRE = !OWN && !ACC;
-  static_assert(!PRE || BN <= NTHR, "a thread a column");
+  constexpr int RED = (KW > 1 ? KW - 1 : 1) * WN * TM * NT * 1024;
   constexpr int ABYTES = ALDS * 1024;
   // one LDS block: the staged activation rows, re-used for the k-waves' partials at the end
   __shared__ __attribute__((aligned(16))) iu8_u8 s_mem[ABYTES > RED ? ABYTES : RED];
   __shared__ int s_last;
-  __shared__ float s_sc[PRE ? BN + TM * 16 : 1];
   int *s_red = (int *)s_mem;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -104,8 +90,6 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
     // (EXACT: a k-wave past a short K issues the first ring all the same, on the share's last step, and drops it)
     wp[j] = W + ((size_t)ntj * steps + (EXACT && ALDS > 0 ? min(s_lo + wk, steps - 1) : s_lo + wk)) * WSTEP + lane * 16;
   }
-
-  float pre_ws = 0.f, pre_as = 0.f;
 
   iu8_v4i acc[TM][NT];
 #pragma unroll
@@ -160,8 +144,6 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
       }
     }
   }
-
-  if constexpr (PRE) pre_ws = ws[min(B.bx * BN + tid, N - 1)], pre_as = as[iu8_arow(R, min(tid, M - 1))];
 
   // ---- the weight ring
   iu8_v4u ring[D][NT][WV];
@@ -386,211 +368,111 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
     }
   }
 
-  if constexpr (OWN) {
-    // ---- the k-waves' partials meet in LDS (exact int32 adds)
-    if constexpr (KW > 1) {
-      if (wk > 0) {
+  // ---- the k-waves' partials meet in LDS (exact int32 adds)
+  if constexpr (KW > 1) {
+    if (wk > 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          *(iu8_v4i *)&s_red[((((wk - 1) * WN + wn) * TM + i) * NT + j) * 256 + lane * 4] = acc[i][j];
+    }
+    __syncthreads();
+    if (wk == 0) {
+#pragma unroll
+      for (int q = 0; q < KW - 1; ++q)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            *(iu8_v4i *)&s_red[((((wk - 1) * WN + wn) * TM + i) * NT + j) * 256 + lane * 4] = acc[i][j];
-      }
-      __syncthreads();
-      if (wk == 0) {
-#pragma unroll
-        for (int q = 0; q < KW - 1; ++q)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-              acc[i][j] += *(const iu8_v4i *)&s_red[(((q * WN + wn) * TM + i) * NT + j) * 256 + lane * 4];
-      }
+            acc[i][j] += *(const iu8_v4i *)&s_red[(((q * WN + wn) * TM + i) * NT + j) * 256 + lane * 4];
     }
-
-    const int nq = lg * 4;
-    if constexpr (PAIR) {
-#pragma clang fp contract(off)
-      const int half = N >> 1;
-      if (wk != 0 || ml >= M) return;
-      const float am = as[iu8_arow(R, ml)];
-#pragma unroll
-      for (int jj = 0; jj < NP; ++jj) {
-        const int tp = (B.bx * WN + wn) * NP + jj;  // this wave's jj-th tile of p
-        if (tp >= (ntiles >> 1)) continue;
-        const int n = tp * 16 + nq;
-        unsigned h[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float g = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[0][jj][r], am, iu8_wsu<W8>(ws, n + r))));
-          const float u = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[0][NP + jj][r], am, iu8_wsu<W8>(ws, half + n + r))));
-          h[r] = iu8_bf16_bits(iu8_silu_bf16(g) * u);
-        }
-        *(iu8_v2u *)((unsigned short *)Cv + (size_t)(R.row0 + ml) * half + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-      }
-      return;
-    }
-    if (Z == 1) {
-      if (wk != 0) return;
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        if (nt0 + j >= ntiles) continue;
-        const int n = (nt0 + j) * 16 + nq;
-        float wsu[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wsu[r] = iu8_wsu<W8>(ws, n + r);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int m = i * 16 + ml;
-          if (m >= M) continue;
-          const size_t crow = (size_t)(R.row0 + m) * N;
-          if constexpr (ACC) {
-            *(iu8_v4i *)((int *)Cv + crow + n) = acc[i][j];
-          } else {
-            const float am = AQ ? s_rsc[m] : as[iu8_arow(R, m)];
-            unsigned h[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(acc[i][j][r], am, wsu[r]));
-            *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-          }
-        }
-      }
-      return;
-    }
-
-    // ---- grid-level split: partials to `decode_partial`, the last-arriving workgroup of this
-    // column block sums them and runs the epilogue; the counter is left at zero.
-    if (wk == 0) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        if (nt0 + j >= ntiles) continue;
-        const int n = (nt0 + j) * 16 + nq;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int m = i * 16 + ml;
-          if (m < M) iu8_store_through(&P[((size_t)z * M + m) * N + n], acc[i][j]);
-        }
-      }
-      iu8_stores_done();
-    }
-    __syncthreads();
-    if (tid == 0) s_last = (iu8_arrive(&cnt[B.bx]) == Z - 1);
-    __syncthreads();
-    if (!s_last) return;
-    if (tid == 0) __hip_atomic_store(&cnt[B.bx], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int nb = B.bx * BN, nw4 = min(BN, N - nb) >> 2;
-    for (int idx = tid; idx < nw4 * M; idx += NTHR) {
-      const int m = idx / nw4, n = nb + (idx % nw4) * 4;
-      iu8_v4i sum = iu8_v4i{0, 0, 0, 0};
-      for (int q = 0; q < Z; ++q) sum += iu8_load_through(&P[((size_t)q * M + m) * N + n]);
-      const size_t crow = (size_t)(R.row0 + m) * N;
-      if constexpr (ACC) {
-        *(iu8_v4i *)((int *)Cv + crow + n) = sum;
-      } else {
-        const float am = as[iu8_arow(R, m)];
-        unsigned h[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(sum[r], am, iu8_wsu<W8>(ws, n + r)));
-        *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-      }
-    }
-    return;
-  } else {
-  // ---- the k-waves' partials meet in LDS (exact int32 adds), and every wave sums and stores its share of the
-  // workgroup's 16 x 16 tiles: with wave 0 of each column group doing all of it behind scales asked for only here, the end
-  // of a launch was a chain of memory latencies. us before / now, weights from memory: W4 45 rows 5120 x 6144 10.6 / 9.0,
-  // 64 rows 12.5 / 10.2, 20 rows 5120 x 5120 7.7 / 6.4, 32 rows 16384 x 5120 13.0 / 12.2, 16 rows 5120 x 17408 13.6 / 13.4 and
-  // 5120 x 6144 6.6 / 6.3, 5 rows 5120 x 5120 5.9 / 5.1, 16 rows 96 x 5120 4.6 / 3.4; W8 64 rows 5120 x 17408 33.6 / 31.3.
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-      *(iu8_v4i *)&s_red[(((wk * WN + wn) * TM + i) * NT + j) * 256 + lane * 4] = acc[i][j];
-  if constexpr (PRE) {
-    if (tid < BN) s_sc[tid] = iu8_wsu<W8>(&pre_ws, 0);
-    if (tid < TM * 16) s_sc[BN + tid] = pre_as;
   }
-  __syncthreads();
-  auto summed = [&](int item) {
-    iu8_v4i v = iu8_v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < KW; ++q) v += *(const iu8_v4i *)&s_red[(q * ITEMS + item) * 256 + lane * 4];
-    return v;
-  };
 
   const int nq = lg * 4;
-  // this wave's items: the tile's row and first column, its sums
-  struct at_t {
-    int m, n, col;  // col: of the workgroup's columns
-    bool live;
-  };
-  auto at = [&](int u) {
-    const int item = wave + u * WPB;
-    const int w = item / (TM * NT), i = (item / NT) % TM, j = item % NT, col = (w * NT + j) * 16 + nq;
-    return at_t{i * 16 + ml, B.bx * BN + col, col, item < ITEMS && i * 16 + ml < M && B.bx * BN + col < N};
-  };
-  iu8_v4i sum[NI];
+  if constexpr (PAIR) {
+#pragma clang fp contract(off)
+    const int half = N >> 1;
+    if (wk != 0 || ml >= M) return;
+    const float am = as[iu8_arow(R, ml)];
 #pragma unroll
-  for (int u = 0; u < NI; ++u) {
-    sum[u] = wave + u * WPB < ITEMS ? summed(wave + u * WPB) : iu8_v4i{0, 0, 0, 0};
-  }
-  auto store = [&](int u) {
-    const at_t t = at(u);
-    if (!t.live) return;
-    const size_t crow = (size_t)(R.row0 + t.m) * N;
-    if constexpr (ACC) {
-      *(iu8_v4i *)((int *)Cv + crow + t.n) = sum[u];
-    } else {
-      const float am = PRE ? s_sc[BN + t.m] : as[iu8_arow(R, t.m)];
+    for (int jj = 0; jj < NP; ++jj) {
+      const int tp = (B.bx * WN + wn) * NP + jj;  // this wave's jj-th tile of p
+      if (tp >= (ntiles >> 1)) continue;
+      const int n = tp * 16 + nq;
       unsigned h[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(sum[u][r], am, PRE ? s_sc[t.col + r] : iu8_wsu<W8>(ws, t.n + r)));
-      *(iu8_v2u *)((unsigned short *)Cv + crow + t.n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+      for (int r = 0; r < 4; ++r) {
+        const float g = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[0][jj][r], am, iu8_wsu<W8>(ws, n + r))));
+        const float u = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[0][NP + jj][r], am, iu8_wsu<W8>(ws, half + n + r))));
+        h[r] = iu8_bf16_bits(iu8_silu_bf16(g) * u);
+      }
+      *(iu8_v2u *)((unsigned short *)Cv + (size_t)(R.row0 + ml) * half + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
     }
-  };
+    return;
+  }
   if (Z == 1) {
+    if (wk != 0) return;
 #pragma unroll
-    for (int u = 0; u < NI; ++u) store(u);
+    for (int j = 0; j < NT; ++j) {
+      if (nt0 + j >= ntiles) continue;
+      const int n = (nt0 + j) * 16 + nq;
+      float wsu[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) wsu[r] = iu8_wsu<W8>(ws, n + r);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = i * 16 + ml;
+        if (m >= M) continue;
+        const size_t crow = (size_t)(R.row0 + m) * N;
+        if constexpr (ACC) {
+          *(iu8_v4i *)((int *)Cv + crow + n) = acc[i][j];
+        } else {
+          const float am = AQ ? s_rsc[m] : as[iu8_arow(R, m)];
+          unsigned h[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(acc[i][j][r], am, wsu[r]));
+          *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+        }
+      }
+    }
     return;
   }
 
-  // ---- grid-level split: partials to `decode_partial`, quad-major ([N / 4][M][4 columns] a share: a wave's store and load
-  // of a tile are four runs of 256 bytes), the last-arriving workgroup of this column block adds the others' to its own
-  // and runs the epilogue; the counter is left at zero.
-  auto part = [&](int q, const at_t &t) { return &P[(((size_t)q * (N >> 2) + (t.n >> 2)) * M + t.m) * 4]; };
+  // ---- grid-level split: partials to `decode_partial`, the last-arriving workgroup of this
+  // column block sums them and runs the epilogue; the counter is left at zero.
+  if (wk == 0) {
 #pragma unroll
-  for (int u = 0; u < NI; ++u) {
-    const at_t t = at(u);
-    if (t.live) iu8_store_through(part(z, t), sum[u]);
+    for (int j = 0; j < NT; ++j) {
+      if (nt0 + j >= ntiles) continue;
+      const int n = (nt0 + j) * 16 + nq;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = i * 16 + ml;
+        if (m < M) iu8_store_through(&P[((size_t)z * M + m) * N + n], acc[i][j]);
+      }
+    }
+    iu8_stores_done();
   }
-  iu8_stores_done();
   __syncthreads();
   if (tid == 0) s_last = (iu8_arrive(&cnt[B.bx]) == Z - 1);
   __syncthreads();
   if (!s_last) return;
   if (tid == 0) __hip_atomic_store(&cnt[B.bx], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  constexpr int SH = 3;  // shares asked for at a time
-  for (int q0 = 1; q0 < Z; q0 += SH) {
-    iu8_v4i v[SH][NI];
+  const int nb = B.bx * BN, nw4 = min(BN, N - nb) >> 2;
+  for (int idx = tid; idx < nw4 * M; idx += NTHR) {
+    const int m = idx / nw4, n = nb + (idx % nw4) * 4;
+    iu8_v4i sum = iu8_v4i{0, 0, 0, 0};
+    for (int q = 0; q < Z; ++q) sum += iu8_load_through(&P[((size_t)q * M + m) * N + n]);
+    const size_t crow = (size_t)(R.row0 + m) * N;
+    if constexpr (ACC) {
+      *(iu8_v4i *)((int *)Cv + crow + n) = sum;
+    } else {
+      const float am = as[iu8_arow(R, m)];
+      unsigned h[4];
 #pragma unroll
-    for (int s = 0; s < SH; ++s)
-      if (q0 + s < Z) {
-        const int q = z + q0 + s < Z ? z + q0 + s : z + q0 + s - Z;
-#pragma unroll
-        for (int u = 0; u < NI; ++u) {
-          at_t t = at(u);
-          t.m = min(t.m, M - 1), t.n = min(t.n, N - 4);  // (a tile that does not exist: some entry, dropped)
-          v[s][u] = iu8_load_through(part(q, t));
-        }
-      }
-#pragma unroll
-    for (int s = 0; s < SH; ++s)
-      if (q0 + s < Z) {
-#pragma unroll
-        for (int u = 0; u < NI; ++u) sum[u] += v[s][u];
-      }
-  }
-#pragma unroll
-  for (int u = 0; u < NI; ++u) store(u);
+      for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(sum[r], am, iu8_wsu<W8>(ws, n + r)));
+      *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    }
   }
 }

@@ -14,10 +14,11 @@
 //           workgroup's activation rows are staged once in LDS (only the live rows, behind the
 //           first ring of weight loads); lanes of dead rows read row 0, which is harmless: a
 //           row of A only reaches its own row of C, and dead rows are never stored. The k-waves'
-//           partials are reduced through LDS (exact int32). An optional grid-level split
+//           partials are reduced through LDS (exact int32). More rows are streamed from L2 beside
+//           the weights (iu8_stream.h, up to 96 rows on wide outputs). A grid-level split of K
 //           (gridDim.z) goes through the `decode_partial` / `decode_counter` workspaces with the
 //           last-arriving workgroup summing (partials handed over straight through memory, no
-//           cache flush); the launch law does not use it by default.
+//           cache flush); the launch law takes it for 9 to 48 rows of a deep, narrow linear.
 //   prefill (M > 64)   MFMA-bound tile GEMM on v_mfma_i32_32x32x32_i8 (iu8_pf32.h): persistent
 //           workgroups of 8 waves (two a SIMD) walk an XCD-aware tile order; the fragments of a
 //           128-deep K step go from HBM/L2 into one of three LDS stages by LDS-DMA loads, two steps
@@ -130,6 +131,14 @@ IU8_PF32K(macaq_iu8_pf_w4_t256x160_ks, false, 8, 1, 1, 5, 3, 1, false)
 IU8_PF32K(macaq_iu8_pf_w8_t256x160_ks, true, 8, 1, 1, 5, 3, 1, false)
 IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 1, 4, 2, 1, 5, 2, true)
 #undef IU8_PF32K
+#define IU8_WIDE_VARIANT(name, TM, W8, NT, KW, D)                                                                     \
+  extern "C" __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4, KW / 4))) void name(  \
+      const unsigned char *__restrict__ a, const unsigned char *__restrict__ w, const float *__restrict__ as,     \
+      const float *__restrict__ ws, unsigned short *__restrict__ c, int m, int n, int k) {                         \
+    __shared__ __attribute__((aligned(16))) unsigned char lds[iu8_stream_geo<TM, NT, KW, 144>::BYTES];             \
+    iu8_stream_body<TM, W8, NT, KW, D, false, 144, W8 ? NT == 4 : NT == 9 && TM >= 3>(                             \
+        lds, a, w, as, ws, nullptr, nullptr, c, m, n, k, iu8_blk{(int)blockIdx.x, 0, 1});                          \
+  }
 #define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP)
 #include "iu8_variants.def"
 

@@ -12,6 +12,7 @@
 // problem's workgroups in front of problem 0's (the reference's ba-first order,
 // crates/saber-kernels/src/macaq_iu8.rs:549-553): the same bytes, the small half not in the tail.
 #include "iu8_gemm.h"
+#include "iu8_stream.h"
 #include "iu8_chain.h"
 
 #define IU8F_PAIR(name, TM, NT, KW, WPB, D, ALDS, BFIRST)                                                                \
@@ -24,10 +25,14 @@
     const int b0 = nb * ks, b1 = nb_b * ks_b, bx = (int)blockIdx.x;                                                 \
     const bool p1 = BFIRST ? bx < b1 : bx >= b0;                                                                    \
     const int bl = BFIRST ? (p1 ? bx : bx - b1) : (p1 ? bx - b0 : bx), nbp = p1 ? nb_b : nb;                        \
-    iu8_dec_body<TM, false, NT, KW, WPB, D, ALDS, false>(                                                           \
-        a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial,                                \
-        p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, iu8_rows{nullptr, 0, m}, p1 ? n_b : n, k,             \
-        iu8_blk{bl % nbp, bl / nbp, p1 ? ks_b : ks});                                                               \
+    const iu8_blk blk{bl % nbp, bl / nbp, p1 ? ks_b : ks};                                                          \
+    if constexpr (ALDS == 0)                                                                                        \
+      iu8_stream_cells<TM, false, NT, KW, D, false>(a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial, \
+                                                   p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, m, p1 ? n_b : n, k, blk); \
+    else                                                                                                            \
+      iu8_dec_body<TM, false, NT, KW, WPB, D, ALDS, false>(                                                         \
+          a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial,                              \
+          p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, iu8_rows{nullptr, 0, m}, p1 ? n_b : n, k, blk);     \
   }
 #define IU8_PAIR_VARIANT(name, TM, NT, KW, WPB, D, ALDS, BFIRST) IU8F_PAIR(name, TM, NT, KW, WPB, D, ALDS, BFIRST)
 #include "iu8_variants.def"

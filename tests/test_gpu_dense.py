@@ -1,5 +1,8 @@
 """GPU parity of the dense W4A8-iu8 linear: quant codes, int32 accumulators and bf16 outputs of the
 HIP path, called through the C ABI, against the CPU oracle on the same seeded inputs."""
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -474,3 +477,38 @@ def test_streamed_cells_spread_their_sums_over_the_waves(ctx, kernel, ks):
         case = synth.dense_case(M, N, K, w8="_w8_" in kernel, seed=M + N + K)
         run = DenseRun(ctx, case, kernel=kernel, ks=ks, want_acc=False)
         assert_dense_matches(run, ref.linear(case["X"], case["W"], case["ws"], "_w8_" in kernel), "_w8_" in kernel)
+
+
+WIDE = re.findall(r"^IU8_WIDE_VARIANT\((macaq_iu8_pf_w\d_t(\d+)x(\d+)_w),", open(os.path.join(iu8.PKG, "csrc", "kernels", "iu8_variants.def")).read(), flags=re.M)
+
+
+@pytest.mark.parametrize("kernel,rows,cols", WIDE, ids=lambda v: str(v))
+def test_wide_streamed_cells(ctx, kernel, rows, cols):
+    """Every wide streamed cell by name: full and one-row last row tile, a last block of one and of all but one column tile,
+    fewer K steps than k-waves, an odd count."""
+    w8, rows, cols = "_w8_" in kernel, int(rows), int(cols)
+    for M, N, K in [(rows, cols + 16, 128), (rows - 15, 2 * cols - 16, 128 * 7), (3, 16, 128 * 9), (rows - 1, 3 * cols, 128 * 21)]:
+        case = synth.dense_case(M, N, K, w8=w8, seed=M + N + K)
+        run = DenseRun(ctx, case, kernel=kernel, want_acc=False)
+        assert_dense_matches(run, ref.linear(case["X"], case["W"], case["ws"], w8), w8)
+
+
+@pytest.mark.parametrize("M,N,K,w8", [(16, 5120, 10240, False), (9, 3024, 12288, True), (31, 5424, 8192, False), (48, 4096, 12288, True),
+                                      (20, 8208, 384, False), (33, 12240, 2048, False), (50, 12256, 3072, False), (32, 16384, 256, True)])
+def test_streamed_blocks_of_64_columns(ctx, M, N, K, w8):
+    """The streamed symbols' 64-column blocks as the law launches them: past one round of their own blocks, and with K on
+    three or four workgroups -- where the call without workspaces runs in one piece and gives the same bytes."""
+    case = synth.dense_case(M, N, K, w8=w8, seed=M + N + K)
+    run = DenseRun(ctx, case, want_acc=False)
+    r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+    np.testing.assert_array_equal(run.C, r["C"])
+    assert "_dec_" in run.desc.kernel.decode() and (run.desc.ks > 1) == (N < 6000)
+    if run.desc.ks > 1:
+        assert not run.counter.cpu().numpy().any()
+        d, c = run.dev, torch.zeros((M, N), dtype=torch.int16, device="cuda")
+        codes, s = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"])
+        for call in (ctx.gemm, ctx.gemm_static):
+            c.zero_()
+            call(iu8.W8 if w8 else iu8.W4, codes.data_ptr(), s.data_ptr(), d["wf"].data_ptr(), d["ws"].data_ptr(), c.data_ptr(), M, N, K)
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(host_u16(c), r["C"])

@@ -748,3 +748,41 @@ def test_repack_refuses_ragged_shapes():
         iu8.repack_w4(np.zeros((24, 64), np.uint8))
     with pytest.raises(iu8.IU8Error):
         iu8.repack_w8(np.zeros((16, 192), np.int8))
+
+
+def test_lines_of_the_streamed_cells_past_one_round():
+    """Either side of the lines in rows, columns and K: 64-column blocks of the streamed symbols, the wide streamed cells,
+    shares of K on deep linears. A launch without workspaces and a pair stay in one piece."""
+    def law(w8, m, n, k):
+        d = iu8.resolve(iu8.W8 if w8 else iu8.W4, m, n, k)
+        return d.kernel.decode()[len("macaq_iu8_"):], d.grid[0], d.ks
+
+    for (w8, m, n, k), want in {
+            (0, 32, 8192, 1024): ("dec_w4_tm2", 256, 1), (0, 32, 8208, 1024): ("dec_w4_tm2", 129, 1), (1, 17, 16384, 128): ("dec_w8_tm2", 256, 1),
+            (0, 33, 12224, 5120): ("pf_w4_t64x64_s", 191, 1), (0, 33, 12240, 5120): ("dec_w4_tm3", 192, 1), (0, 48, 16384, 2048): ("dec_w4_tm3", 256, 1),
+            (0, 48, 16384, 1920): ("pf_w4_t64x64_s", 256, 1), (1, 48, 16384, 4096): ("dec_w8_tm3", 256, 1), (1, 48, 16384, 3968): ("pf_w8_t64x64_s", 256, 1),
+            (0, 64, 16384, 3072): ("dec_w4_tm4", 256, 1), (0, 64, 16384, 2944): ("pf_w4_t64x64_s", 256, 1),
+            (0, 32, 18336, 1024): ("pf_w4_t64x128_s", 144, 1), (0, 32, 18352, 1024): ("pf_w4_t32x96_w", 192, 1), (0, 48, 24576, 2048): ("pf_w4_t48x96_w", 256, 1),
+            (0, 49, 24576, 3968): ("pf_w4_t64x128_s", 192, 1), (0, 49, 24576, 4096): ("pf_w4_t64x96_w", 256, 1), (0, 80, 20480, 3072): ("pf_w4_t80x96_w", 214, 1),
+            (0, 96, 20480, 5120): ("pf_w4_t96x96_w", 214, 1), (1, 64, 24576, 2048): ("pf_w8_t64x96_w", 256, 1), (1, 96, 24576, 4096): ("pf_w8_t96x96_w", 256, 1),
+            (0, 32, 32768, 4096): ("pf_w4_t32x144_w", 228, 1), (0, 33, 32768, 5120): ("pf_w4_t64x128_s", 256, 1), (1, 33, 32768, 3072): ("pf_w8_t48x144_w", 228, 1),
+            (0, 45, 34816, 5120): ("pf_w4_t48x144_w", 242, 1), (0, 64, 36864, 4096): ("pf_w4_t64x144_w", 256, 1), (0, 64, 36880, 5120): ("pf_w4_t64x160_s", 231, 1),
+            (0, 96, 34816, 2048): ("pf_w4_t96x144_w", 242, 1), (1, 72, 14336, 2048): ("pf_w8_t80x64_w", 224, 1), (0, 72, 14336, 8192): ("pf_w4_t80x64_w", 224, 1),
+            (0, 8, 5120, 17408): ("dec_w4_tm1_a0", 160, 1), (0, 9, 5120, 10240): ("dec_w4_tm1_a0", 80, 3), (0, 16, 5120, 10112): ("dec_w4_tm1_a0", 160, 1),
+            (0, 17, 5120, 8192): ("dec_w4_tm2", 80, 3), (1, 48, 5440, 8192): ("dec_w8_tm3_n2", 85, 3), (1, 48, 5456, 8192): ("dec_w8_tm3_n2", 171, 1),
+            (1, 49, 5120, 8192): ("dec_w8_tm4_n2", 160, 1), (0, 48, 4096, 12288): ("dec_w4_tm3", 64, 4), (0, 48, 4096, 12160): ("dec_w4_tm3", 256, 1),
+            (0, 16, 3024, 12288): ("dec_w4_tm1_a0", 48, 4), (0, 16, 3008, 12288): ("dec_w4_tm1_a0", 94, 1)}.items():
+        assert law(w8, m, n, k) == want, (w8, m, n, k, law(w8, m, n, k))
+    d = iu8.resolve(iu8.W4, 16, 5120, 17408)
+    assert iu8.gemm_workspace(iu8.W4, 16, 5120, 17408) == (3 * 16 * 5120 * 4, 80 * 4) and d.grid[2] == 3
+    p = iu8.pair(d, iu8.describe("macaq_iu8_dec_w4_tm1_a0", 16, 9600, 17408, ks=1))
+    assert (p.arg("nb").ival, p.arg("ks").ival, p.arg("nb_b").ival, p.arg("ks_b").ival) == (80, 3, 150, 1) and p.grid[0] == 80 * 3 + 150
+    assert p.workspace("decode_counter").bytes == 80 * 4
+    for name, m, ok in (("macaq_iu8_pf_w4_t48x144_w", 48, True), ("macaq_iu8_pf_w4_t48x144_w", 49, False)):
+        if ok:
+            assert iu8.describe(name, m, 160, 128).grid[0] == 2
+        else:
+            with pytest.raises(iu8.IU8Error):
+                iu8.describe(name, m, 160, 128)
+    with pytest.raises(iu8.IU8Error):
+        iu8.describe("macaq_iu8_pf_w4_t48x144_w", 48, 160, 256, ks=2)
