@@ -102,7 +102,7 @@ static __device__ __forceinline__ void had_add_rms_body(const unsigned short *__
       ssq = __builtin_fmaf(v, v, ssq);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = iu8_bf16_bits(sv[i][2 * j]) | (iu8_bf16_bits(sv[i][2 * j + 1]) << 16);
+    for (int j = 0; j < 4; ++j) o[j] = iu8_bf16_pack(sv[i][2 * j], sv[i][2 * j + 1]);
     *(iu8_v4u *)(res_out + g * 8) = iu8_v4u{o[0], o[1], o[2], o[3]};
   }
   // the reference's trees (32 lanes, then the T/32 partials), so the sum's bits are its own
@@ -125,8 +125,8 @@ static __device__ __forceinline__ void had_add_rms_body(const unsigned short *__
     float vw[8];
     had_load8(w + g * 8, vw);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      sv[i][j] = iu8_bf16_f32((unsigned short)iu8_bf16_bits((sv[i][j] * inv) * (vw[j] + 1.f)));
+    for (int j = 0; j < 8; ++j) sv[i][j] = (sv[i][j] * inv) * (vw[j] + 1.f);
+    had_bf16_round(sv[i]);
     had32(sv[i], had_t + 8 * g, tid);
   }
   had_tail<T>(sv, NV, q, scale, row, K);
@@ -134,10 +134,11 @@ static __device__ __forceinline__ void had_add_rms_body(const unsigned short *__
 
 // add_rms for few rows of up to 8,192 elements, 16 waves a row, with the sum of squares in the 256-thread form's order
 // (which is part of its law: thread t of 256 runs one fma chain over its groups t, t + 256, t + 512, t + 768 in turn, then
-// the 32-lane and 8-partial trees). Here thread tid owns group tid, and the chain of "thread" t = tid % 256 is handed
-// from slice tid / 256 to the next through LDS -- four short turns -- while everything else (the loads, y + res and its
-// store, the weights, the transform, the codes) runs on four times the threads. Same bits as
-// add_rms_quant_hadi8_t256_tiled1.
+// the 32-lane and 8-partial trees). Here thread tid owns group tid and puts y + res in LDS, from where the first 256 threads
+// run the chains; everything else (the loads, y + res and its store, the weights, the transform, the codes) runs on four
+// times the threads. Same bits as add_rms_quant_hadi8_t256_tiled1. (The chain was handed from slice to slice of 256 threads in
+// four turns, six barriers in all: 5,120 wide at 1 / 16 / 200 rows 4.56 / 4.92 / 5.87 us, here 3.96 / 4.28 / 5.19; the t256 form,
+// which has the one-addition lane stages and the paired roundings as well, at 777 / 2,048 rows 10.9 / 21.0 -> 9.8 / 19.1.)
 static __device__ __forceinline__ void had_add_rms_v256_body(const unsigned short *__restrict__ y,
                                                              const unsigned short *__restrict__ res,
                                                              const unsigned short *__restrict__ w, iu8_u8 *__restrict__ q,
@@ -145,58 +146,56 @@ static __device__ __forceinline__ void had_add_rms_v256_body(const unsigned shor
                                                              int K, float eps, const float *__restrict__ had_t) {
 #pragma clang fp contract(off)
   constexpr int T = 1024, V = 256;
-  __shared__ float s_chain[V];
+  __shared__ __attribute__((aligned(16))) float s_v[T * 8];
   __shared__ float s_sum[V / 32];
-  const int row = had_row(), tid = threadIdx.x, NV = K >> 3, g = tid, t = tid & (V - 1), slice = tid >> 8;
+  const int row = had_row(), tid = threadIdx.x, NV = K >> 3, g = tid;
   const bool live = g < NV;
   y += (size_t)row * K, res += (size_t)row * K, res_out += (size_t)row * K;
-  float sv[HAD_MAXG][8];
-  float vw[8];
-  if (live) {
+  float sv[1][8], vw[8];
+  iu8_v4f t_lo = {0.f, 0.f, 0.f, 0.f}, t_hi = t_lo;
+  if (live) {  // everything the row needs is requested before the first of it is used
     float vy[8], vr[8];
-    had_load8(y + g * 8, vy);
-    had_load8(res + g * 8, vr);
+    const iu8_v4u ry = *(const iu8_v4u *)(y + g * 8), rr = *(const iu8_v4u *)(res + g * 8);
     had_load8(w + g * 8, vw);
+    t_lo = *(const iu8_v4f *)(had_t + 8 * g), t_hi = *(const iu8_v4f *)(had_t + 8 * g + 4);
+    had_unpack8(ry, vy), had_unpack8(rr, vr);
     unsigned o[4];
 #pragma unroll
     for (int j = 0; j < 8; ++j) sv[0][j] = vy[j] + vr[j];
+    // element-pair-major: a wave's 8-byte pieces lie side by side
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = iu8_bf16_bits(sv[0][2 * j]) | (iu8_bf16_bits(sv[0][2 * j + 1]) << 16);
+    for (int j = 0; j < 4; ++j) {
+      *(iu8_v2f *)&s_v[(j * T + g) * 2] = iu8_v2f{sv[0][2 * j], sv[0][2 * j + 1]};
+      o[j] = iu8_bf16_pack(sv[0][2 * j], sv[0][2 * j + 1]);
+    }
     *(iu8_v4u *)(res_out + g * 8) = iu8_v4u{o[0], o[1], o[2], o[3]};
   }
-  for (int turn = 0; turn < T / V; ++turn) {
-    if (slice == turn) {
-      float ssq = turn ? s_chain[t] : 0.f;
-      if (live) {
+  __syncthreads();
+  if (tid < V) {  // thread t's chain over the groups t, t + 256, t + 512, t + 768
+    float ssq = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ssq = __builtin_fmaf(sv[0][j], sv[0][j], ssq);
+    for (int i = 0; i < T / V; ++i)
+      if (tid + i * V < NV) {
+        iu8_v2f p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = *(const iu8_v2f *)&s_v[(j * T + tid + i * V) * 2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ssq = __builtin_fmaf(p[j].x, p[j].x, ssq), ssq = __builtin_fmaf(p[j].y, p[j].y, ssq);
       }
-      s_chain[t] = ssq;
-    }
-    __syncthreads();
-  }
-  if (tid < V) {
-    float ssq = s_chain[tid];
-#pragma unroll
-    for (int o = 16; o; o >>= 1) ssq = ssq + __shfl_down(ssq, o, 32);
+    ssq = had_sum32(ssq);
     if ((tid & 31) == 0) s_sum[tid >> 5] = ssq;
   }
   __syncthreads();
-  if (tid < V / 32) {
-    float v = s_sum[tid];
-#pragma unroll
-    for (int o = V / 64; o; o >>= 1) v = v + __shfl_down(v, o, 32);
-    if (tid == 0) s_sum[0] = v;
-  }
-  __syncthreads();
-  const float inv = __fdiv_rn(1.f, __builtin_sqrtf(__fdiv_rn(s_sum[0], (float)K) + eps));
+  // the tree over the 8 partials (4, 2, 1 apart), by every thread
+  const float ms = ((s_sum[0] + s_sum[4]) + (s_sum[2] + s_sum[6])) + ((s_sum[1] + s_sum[5]) + (s_sum[3] + s_sum[7]));
+  const float inv = __fdiv_rn(1.f, __builtin_sqrtf(__fdiv_rn(ms, (float)K) + eps));
   if (live) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      sv[0][j] = iu8_bf16_f32((unsigned short)iu8_bf16_bits((sv[0][j] * inv) * (vw[j] + 1.f)));
-    had32(sv[0], had_t + 8 * g, tid);
+    for (int j = 0; j < 8; ++j) sv[0][j] = (sv[0][j] * inv) * (vw[j] + 1.f);
+    had_bf16_round(sv[0]);
+    had32(sv[0], t_lo, t_hi, tid);
   }
-  had_tail<T>(sv, NV, q, scale, row, K);
+  had_tail<T, 1>(sv, NV, q, scale, row, K);
 }
 extern "C" __global__ __launch_bounds__(1024) void add_rms_quant_hadi8_t1024(
     const unsigned short *__restrict__ y, const unsigned short *__restrict__ res, const unsigned short *__restrict__ w,
@@ -230,7 +229,7 @@ HAD_SMQ(silu_mul_quant_hadi8_t1024, 1024)  // 16 waves a row: few long rows (no 
 // silu_mul_quant with the bf16 silu read from a table: `lut` holds bf16(silu(x)) of every bf16 bit pattern x as
 // macaq_silu_bf16_table (code object `macaq_i8q`) wrote it, i.e. this file's own expression
 // vg / (1 + expf(-vg)) rounded to bf16, so the bytes are those of the computed form. Rows of 17,408, us on the computed
-// form / here: 1 / 200 rows 6.62 / 9.26, 5.92 / 8.82; 777 / 2,048 / 6,144 rows 23.6 / 44.1 / 118.9, 21.2 / 42.9 / 116.7; rows of
+// form / here: 1 / 200 rows 6.51 / 9.12, 6.09 / 9.00; 777 / 2,048 rows 23.8 / 41.9, 22.5 / 41.3 (a branch and an address an element: 23.3 / 43.1); rows of
 // 5,120 within 6 % either way; rows of 2,048 up to 512 rows 0.35-0.5 us in favour of the computed form. A workgroup copies the
 // table's middle -- magnitudes from 2^-17 up to 2^15, both signs: 2 x 4,096 entries, 16 KiB -- into LDS beside
 // its row's loads; a gate outside (one in some hundred thousand of unit-scale rows) is computed as before.
@@ -257,21 +256,26 @@ static __device__ __forceinline__ void had_silu_lut_body(const unsigned short *_
   tb.request(lut, tid);
   tb.commit(s_lut, tid);
   __syncthreads();
-  auto silu = [&](unsigned b) {  // bf16 pattern (low 16 bits) -> bf16(silu) as f32
-    unsigned at;
-    if (__builtin_expect(had_lut_index(b, at), 1)) return iu8_bf16_f32(s_lut[at]);
-    const float x = iu8_bf16_f32((unsigned short)b);
-    return iu8_bf16_f32((unsigned short)iu8_bf16_bits(x / (1.f + expf(-x))));
-  };
   float sv[HAD_MAXG][8];
 #pragma unroll
   for (int i = 0; i < HAD_MAXG; ++i) {
     const int g = tid + i * T;
     if (g >= NV) continue;
+    unsigned t[4];
+    bool far;
+    had_lut8(s_lut, rg[i], t, far);
+    if (__builtin_expect(far, 0)) {
+      asm volatile("");  // stays a branch (iu8_code4_rcp has the reason)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        if (!had_lut_inside(rg[i][w])) t[w] = (t[w] & 0xFFFF0000u) | (__float_as_uint(iu8_silu_bf16(__uint_as_float(rg[i][w] << 16))) >> 16);
+        if (!had_lut_inside(rg[i][w] >> 16)) t[w] = (t[w] & 0xFFFFu) | __float_as_uint(iu8_silu_bf16(__uint_as_float(rg[i][w] & 0xFFFF0000u)));
+      }
+    }
 #pragma unroll
     for (int w = 0; w < 4; ++w) {  // two products a v_cvt_pk_bf16_f32
-      const float t0 = silu(rg[i][w] & 0xFFFFu), t1 = silu(rg[i][w] >> 16);
-      const unsigned p2 = iu8_bf16_pack(t0 * __uint_as_float(ru[i][w] << 16), t1 * __uint_as_float(ru[i][w] & 0xFFFF0000u));
+      const unsigned p2 = iu8_bf16_pack(__uint_as_float(t[w] << 16) * __uint_as_float(ru[i][w] << 16),
+                                        __uint_as_float(t[w] & 0xFFFF0000u) * __uint_as_float(ru[i][w] & 0xFFFF0000u));
       sv[i][2 * w] = __uint_as_float(p2 << 16);
       sv[i][2 * w + 1] = __uint_as_float(p2 & 0xFFFF0000u);
     }
@@ -315,6 +319,7 @@ static __device__ __forceinline__ void had_gdn_norm_body(const unsigned short *_
 #pragma unroll
   for (int i = 0; i < HAD_MAXG; ++i) {
     // whole heads (16 lanes) are live or not together: NV is a multiple of 16, T a multiple of 16
+    if (i * T >= NV) continue;
     const int g = tid + i * T;
     const bool on = g < NV;
     const int gl = on ? g : 0;
@@ -324,18 +329,47 @@ static __device__ __forceinline__ void had_gdn_norm_body(const unsigned short *_
     ssq = __builtin_fmaf(sv[i][0], sv[i][0], ssq);
 #pragma unroll
     for (int j = 2; j < 8; ++j) ssq = __builtin_fmaf(sv[i][j], sv[i][j], ssq);
-#pragma unroll
-    for (int o = 8; o; o >>= 1) ssq = ssq + __shfl_xor(ssq, o, 16);
+    ssq = had_head_sum(ssq);
     if (!on) continue;
     const float inv = __fdiv_rn(1.f, __builtin_sqrtf(ssq * (1.f / 128.f) + eps));
     had_load8(z + g * 8, vz);
     had_load8(w + (g & 15) * 8, vw);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      sv[i][j] = iu8_bf16_f32((unsigned short)iu8_bf16_bits(((sv[i][j] * inv) * vw[j]) * had_silu_f32(vz[j])));
+    for (int j = 0; j < 8; ++j) sv[i][j] = ((sv[i][j] * inv) * vw[j]) * had_silu_f32(vz[j]);
+    had_bf16_round(sv[i]);
     had32(sv[i], had_t + 8 * g, tid);
   }
   had_tail<T>(sv, NV, q, scale, row, N);
+}
+
+// The same for rows of at most 8 T elements: one group a thread, everything requested before the first of it is used.
+// Few rows are bound by one CU's arithmetic (a quarter of it the gate's exponential and
+// divide) and the row's latencies: 6,144 wide at 1 / 16 / 45 / 200 rows 5.54 / 5.86 / 6.02 / 6.77 us in the loop of five groups, here
+// 4.24 / 4.53 / 4.69 / 5.66; the loop, which now stops at the row's end, at 777 / 2,048 rows 14.0 / 25.4 -> 13.1 / 24.6.
+template <int T>
+static __device__ __forceinline__ void had_gdn_norm_one(const unsigned short *__restrict__ x, const unsigned short *__restrict__ z,
+                                                        long zs, const unsigned short *__restrict__ w, iu8_u8 *__restrict__ q,
+                                                        float *__restrict__ scale, int N, float eps, const float *__restrict__ had_t) {
+#pragma clang fp contract(off)
+  const int row = had_row(), tid = threadIdx.x, NV = N >> 3, g = min(tid, NV - 1);  // whole heads past the row's end repeat its last group
+  const iu8_v4u rx = *(const iu8_v4u *)(x + (size_t)row * N + g * 8), rz = *(const iu8_v4u *)(z + (size_t)row * zs + g * 8);
+  const iu8_v4u rw = *(const iu8_v4u *)(w + (g & 15) * 8);
+  const iu8_v4f t_lo = *(const iu8_v4f *)(had_t + 8 * g), t_hi = *(const iu8_v4f *)(had_t + 8 * g + 4);
+  float sv[1][8], vz[8], vw[8];
+  had_unpack8(rx, sv[0]), had_unpack8(rz, vz), had_unpack8(rw, vw);
+  float ssq = sv[0][1] * sv[0][1];
+  ssq = __builtin_fmaf(sv[0][0], sv[0][0], ssq);
+#pragma unroll
+  for (int j = 2; j < 8; ++j) ssq = __builtin_fmaf(sv[0][j], sv[0][j], ssq);
+  ssq = had_head_sum(ssq);
+  if (tid < NV) {
+    const float inv = __fdiv_rn(1.f, __builtin_sqrtf(ssq * (1.f / 128.f) + eps));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sv[0][j] = ((sv[0][j] * inv) * vw[j]) * had_silu_f32(vz[j]);
+    had_bf16_round(sv[0]);
+    had32(sv[0], t_lo, t_hi, tid);
+  }
+  had_tail<T, 1>(sv, NV, q, scale, row, N);
 }
 
 extern "C" __global__ __launch_bounds__(256) void gdn_norm_quant_hadi8_t256_tiled1(
@@ -349,5 +383,6 @@ extern "C" __global__ __launch_bounds__(1024) void gdn_norm_quant_hadi8_t1024(
     const unsigned short *__restrict__ x, const unsigned short *__restrict__ z, long zs,
     const unsigned short *__restrict__ w, unsigned char *__restrict__ q, float *__restrict__ scale, int N, float eps,
     const float *__restrict__ had_t) {
-  had_gdn_norm_body<1024>(x, z, zs, w, q, scale, N, eps, had_t);
+  if (N <= 8 * 1024) had_gdn_norm_one<1024>(x, z, zs, w, q, scale, N, eps, had_t);
+  else had_gdn_norm_body<1024>(x, z, zs, w, q, scale, N, eps, had_t);
 }

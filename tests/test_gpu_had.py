@@ -341,3 +341,34 @@ def test_had_refusals(ctx):
         with pytest.raises(iu8.IU8Error) as e:
             ctx.attn_gate_quant_had(*args)
         assert e.value.code == iu8.E_RULE
+
+
+@pytest.mark.parametrize("W", [4096, 8064, 8192, 8320])
+def test_few_row_norm_producers_at_the_one_group_edge(ctx, W):
+    """The 16-wave norms on both sides of one 8-element group a thread (8,192): rows that end inside the last wave, fill it
+    and pass it, with a row of infinities and NaN, against the oracle."""
+    M = 3
+    rng = np.random.default_rng(W)
+    t = rng.choice([-1.0, 1.0], size=W).astype(np.float32)
+    X = synth.activations(rng, M, W)
+    X[1, 5], X[1, W - 1] = 0x7F80, 0x7FC0
+    z = synth.f32_to_bf16_bits((rng.standard_normal((M, W)) * 3).astype(np.float32))
+    w = synth.f32_to_bf16_bits((1 + rng.standard_normal(128) * 0.1).astype(np.float32))
+    td, xd, zd, wd = dev_f32(t), dev_bf16_bits(X), dev_bf16_bits(z), dev_bf16_bits(w)
+    q, s = outs(M, W)
+    ctx.gdn_norm_quant_had(xd.data_ptr(), zd.data_ptr(), W, wd.data_ptr(), q.data_ptr(), s.data_ptr(), M, W, 1e-6, td.data_ptr())
+    torch.cuda.synchronize()
+    wq, wsc = ref.gdn_norm_quant_had(X, z, w, t, 1e-6, silu_tab=device_silu_f32_table(ctx))
+    np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32))
+    np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, W), wq)
+    res = synth.f32_to_bf16_bits((rng.standard_normal((M, W)) * 4).astype(np.float32))
+    wn = synth.f32_to_bf16_bits((rng.standard_normal(W) * 0.1).astype(np.float32))
+    rd, wnd, ro = dev_bf16_bits(res), dev_bf16_bits(wn), torch.zeros((M, W), dtype=torch.int16, device="cuda")
+    X[1, 5], X[1, W - 1] = 0, 0
+    xd = dev_bf16_bits(X)
+    ctx.add_rms_quant_had(xd.data_ptr(), rd.data_ptr(), wnd.data_ptr(), q.data_ptr(), s.data_ptr(), ro.data_ptr(), M, W, 1e-6, td.data_ptr())
+    torch.cuda.synchronize()
+    wq, wsc, wro = ref.add_rms_quant_had(X, res, wn, t, 1e-6, 256)
+    np.testing.assert_array_equal(host_u16(ro), wro)
+    np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32))
+    np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, W), wq)
