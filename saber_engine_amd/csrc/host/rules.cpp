@@ -3,6 +3,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "../kernels/iu8_pf_law.h"
 #include "abi.h"
 #include "util.h"
 
@@ -596,6 +597,11 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
     const uint64_t q = tiles / grid, rem = tiles - q * grid;
     if (!strcmp(c.tile, "tn4_lbk64") && q >= 1 && rem > 0 && 2 * rem <= grid)
       cu_tiles = (double)q + (double)((4 * rem + grid - 1) / grid) * 0.25 * (c.tops_per_cu / quarter_rate);
+    // ... and a few rows past the last whole 256 as thin tiles (int4 weights: the estimate of the int8 cells is drawn without)
+    if (!strcmp(c.tile, "tn4_lbk64") && !w8 && tiles < (1u << 20) && k < (1u << 30)) {
+      const iu8_pf_plan plan = iu8_pf_plan256((int)m, (int)((n + 255) / 256), (int)grid, (int)k);
+      if (plan.thin) cu_tiles = std::min(cu_tiles, plan.cost * 0.0108);  // (a margin: level picks stay as they were)
+    }
     const double tile_bytes = bm * k + bn * k * (w8 ? 1.0 : 0.5);
     const double t_mfma = cu_tiles * bm * bn * k * 2.0 / (c.tops_per_cu * 1e6);
     const double t_cu = cu_tiles * tile_bytes / (law.cu_gbps * 1e3);

@@ -421,3 +421,23 @@ def test_config4_moe_prefill_shape(ctx):
     layer = run_layer(ctx, case)
     assert layer.tb == 16 and layer.gather == 2
     check_layer(layer, case, taps=False)
+
+
+@pytest.mark.parametrize("M,N,grid", [(257, 1008, 5), (288, 1296, 8), (384, 784, 6), (777, 1008, 6), (600, 3296, 8), (641, 2304, 11)])
+@pytest.mark.parametrize("tag,w8", [("w4", False), ("w8", True)])
+def test_rows_past_the_last_whole_256_run_as_thin_tiles(ctx, M, N, grid, tag, w8):
+    """The 256 x 256 cell's thin tiles (1, 32, 128, 9, 88 and 129 -> whole rows past the last whole 256; a ragged last column block;
+    on the workgroups with a whole tile less, three and one each, on all of them, and behind quarter tiles): the oracle's bytes."""
+    K = 1024
+    say(f"256x256 cell, thin tiles: {M} x {N}, grid {grid} {tag}")
+    case = synth.dense_case(M, N, K, w8=w8, seed=M + grid)
+    r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+    qd, sd = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"])
+    wf, wsd = dev_u8(iu8.repack_weights(case["W"], w8)), dev_f32(case["ws"])
+    c = torch.full((M, N), 0x7FC0, dtype=torch.int16, device="cuda")
+    d = iu8.describe_raw(f"macaq_iu8_pf_{tag}_tn4_lbk64", (grid, 1, 1), 512, plugin="macaq_iu8", m=M, n=N, k=K)
+    bufs = dict(a=qd.data_ptr(), w=wf.data_ptr(), ws=wsd.data_ptr(), c=c.data_ptr())
+    bufs["as"] = sd.data_ptr()
+    ctx.launch(d, bufs)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(host_u16(c), r["C"])
