@@ -89,7 +89,7 @@ int ref_symbol_by_law(const std::string &kernel, int *w8, const char **note) {
   return 0;
 }
 
-// The linears the bands are written out for: BASELINE's 27B-class layer set, the reference's own
+// The linears the bands are written out for: the 27B-class layer set, the reference's own
 // 27B shapes at TP=1 and TP=2 (macaq_iu8.rs:931-947) and the routed layer's expert shapes.
 struct Shape {
   const char *op;
