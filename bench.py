@@ -419,6 +419,16 @@ def main():
     # ---- the other batch sizes of configs[1] (M = 4, 8, 16) through the same step: a linear is one fused
     # launch while its rows fit the fused form (M <= 4 and pow2(M) * K <= 20 KiB), else producer + GEMV;
     # graph replay, cold weights
+    # a host's workspaces for the launches whose descriptor shares K between workgroups (counters zeroed once)
+    split_part = torch.zeros(8 << 20, dtype=torch.uint8, device=dev)
+    split_cnt = torch.zeros(16384, dtype=torch.int32, device=dev)
+
+    def bind_split(d, b):
+        if d.ks > 1:
+            assert d.workspace("decode_partial").bytes <= split_part.numel() and d.workspace("decode_counter").bytes <= 4 * split_cnt.numel()
+            b.update(decode_partial=split_part.data_ptr(), decode_counter=split_cnt.data_ptr())
+        return b
+
     def decode_at(DM, nsteps=60):
         xs, qs, ss, cs = {}, {}, {}, {}
         for name, n, k in linears:
@@ -440,10 +450,9 @@ def main():
                 else:
                     ctx.launch(iu8.resolve_quant(DM, k), dict(x=xs[name].data_ptr(), q=qs[name].data_ptr(), scale=ss[name].data_ptr()), sh)
                     d = iu8.resolve(iu8.W4, DM, n, k)
-                    assert d.ks == 1
                     b = dict(a=qs[name].data_ptr(), w=w, ws=wsd, c=cs[name].data_ptr())
                     b["as"] = ss[name].data_ptr()
-                    ctx.launch(d, b, sh)
+                    ctx.launch(d, bind_split(d, b), sh)
 
         def graph_us(fn, reps_settle=8):
             """nsteps calls of fn(i) as one graph: replayed to settle, then one replay timed by HIP events"""
@@ -499,7 +508,7 @@ def main():
                 def gemv(i):
                     b = dict(a=qs[name].data_ptr(), w=dev_w[name][i % LAYERS].data_ptr(), ws=wsd, c=cs[name].data_ptr())
                     b["as"] = ss[name].data_ptr()
-                    ctx.launch(gd, b, sh)
+                    ctx.launch(gd, bind_split(gd, b), sh)
 
                 g_us = graph_us(gemv)
                 gb = alg_bytes(DM, n, k) - 2 * DM * k + DM * k + 4 * DM   # the GEMV reads codes and scales
@@ -749,10 +758,9 @@ def main():
             def run_seq():
                 for (name, n, k, w8), w in zip(seq, seq_w):
                     d = iu8.resolve(iu8.W8 if w8 else iu8.W4, SM, n, k)
-                    assert d.ks == 1
                     b = dict(a=acts[k][0].data_ptr(), w=w.data_ptr(), ws=dev_ws[name].data_ptr(), c=cbuf[n].data_ptr())
                     b["as"] = acts[k][1].data_ptr()
-                    ctx.launch(d, b, sh)
+                    ctx.launch(d, bind_split(d, b), sh)
 
             with torch.cuda.stream(stream):
                 run_seq()

@@ -427,6 +427,12 @@ static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint
   return nullptr;
 }
 
+bool law_split_stream(const saber_iu8_desc &d) {
+  int64_t m = 0, n = 0, k = 0;
+  return d.ks > 1 && dec_variant(d.kernel) && int_arg(d, "m", &m) && int_arg(d, "n", &n) && int_arg(d, "k", &k) &&
+         stream_split((uint32_t)m, (uint32_t)n, (uint32_t)k) == d.ks;
+}
+
 int unsplit_stream(saber_iu8_desc *d) {
   int64_t m = 0, n = 0, k = 0;
   if (d->ks <= 1 || !dec_variant(d->kernel) || !int_arg(*d, "m", &m) || !int_arg(*d, "n", &n) || !int_arg(*d, "k", &k)) return 0;

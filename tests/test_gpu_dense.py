@@ -512,3 +512,9 @@ def test_streamed_blocks_of_64_columns(ctx, M, N, K, w8):
             call(iu8.W8 if w8 else iu8.W4, codes.data_ptr(), s.data_ptr(), d["wf"].data_ptr(), d["ws"].data_ptr(), c.data_ptr(), M, N, K)
             torch.cuda.synchronize()
             np.testing.assert_array_equal(host_u16(c), r["C"])
+        c.zero_()
+        bufs = dict(a=codes.data_ptr(), w=d["wf"].data_ptr(), ws=d["ws"].data_ptr(), c=c.data_ptr())
+        bufs["as"] = s.data_ptr()
+        ctx.launch(run.desc, bufs)  # the law's own descriptor with neither workspace bound
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host_u16(c), r["C"])
