@@ -398,7 +398,8 @@ int saber_iu8_linear_prefill_fused(saber_iu8_ctx *ctx, int wkind, const void *x_
 /* Workspace bytes the resolved GEMM needs (both 0 when it does not split). Ask before every
  * saber_iu8_gemm of a new shape: the law splits K in two bands: tiles at 33..192 rows of K >= 16384
  * (few tiles), where a launch with `partial` / `counter` NULL is refused (SABER_IU8_E_ARG), and the streamed
- * cells at 9..48 rows of K >= 8192, which run in one piece without them. */
+ * cells at 9..48 rows of K >= 8192, which run in one piece without them (saber_iu8_launch of the resolved
+ * descriptor with neither bound too). */
 int saber_iu8_gemm_workspace(int wkind, uint32_t m, uint32_t n, uint32_t k, uint64_t *partial_bytes,
                              uint64_t *counter_bytes);
 

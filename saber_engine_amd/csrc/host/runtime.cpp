@@ -426,13 +426,15 @@ int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu
   if (!ctx || !d) return fail(SABER_IU8_E_ARG, "launch: null argument");
   // the law's own split of a streamed launch, with neither workspace bound: the launch in one piece, same bytes
   saber_iu8_desc whole;
-  bool has_partial = false, has_counter = false;
-  find_binding(bufs, n_bufs, "decode_partial", &has_partial);
-  find_binding(bufs, n_bufs, "decode_counter", &has_counter);
-  if (!has_partial && !has_counter && law_split_stream(*d)) {
-    whole = *d;
-    if (int rc = unsplit_stream(&whole)) return rc;
-    d = &whole;
+  if (d->ks > 1 && law_split_stream(*d)) {
+    bool has_partial = false, has_counter = false;
+    find_binding(bufs, n_bufs, "decode_partial", &has_partial);
+    find_binding(bufs, n_bufs, "decode_counter", &has_counter);
+    if (!has_partial && !has_counter) {
+      whole = *d;
+      if (int rc = unsplit_stream(&whole)) return rc;
+      d = &whole;
+    }
   }
   auto it = ctx->fn.find(d->kernel);
   if (it == ctx->fn.end()) return fail(SABER_IU8_E_NOTLOADED, std::string(d->kernel) + ": not in the loaded plugin set");
