@@ -424,17 +424,16 @@ static int launch_guard(const LoadedKernel &lk, const saber_iu8_desc *d) {
 int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu8_binding *bufs, uint32_t n_bufs,
                      void *stream) {
   if (!ctx || !d) return fail(SABER_IU8_E_ARG, "launch: null argument");
-  // the law's own split of a streamed launch, with neither workspace bound: the launch in one piece, same bytes
+  // the law's own split of a streamed launch without both of its workspaces: the launch in one piece, same bytes
   saber_iu8_desc whole;
-  if (d->ks > 1 && law_split_stream(*d)) {
-    bool has_partial = false, has_counter = false;
-    find_binding(bufs, n_bufs, "decode_partial", &has_partial);
-    find_binding(bufs, n_bufs, "decode_counter", &has_counter);
-    if (!has_partial && !has_counter) {
-      whole = *d;
-      if (int rc = unsplit_stream(&whole)) return rc;
-      d = &whole;
-    }
+  auto bound = [&](const char *name) {
+    bool found;
+    return bufs && find_binding(bufs, n_bufs, name, &found);
+  };
+  if (d->ks > 1 && !(bound("decode_partial") && bound("decode_counter")) && law_split_stream(*d)) {
+    whole = *d;
+    if (int rc = unsplit_stream(&whole)) return rc;
+    d = &whole;
   }
   auto it = ctx->fn.find(d->kernel);
   if (it == ctx->fn.end()) return fail(SABER_IU8_E_NOTLOADED, std::string(d->kernel) + ": not in the loaded plugin set");
@@ -560,7 +559,7 @@ int saber_iu8_gemm(saber_iu8_ctx *ctx, int wkind, const void *a, const float *as
                    void *c, uint32_t m, uint32_t n, uint32_t k, void *partial, void *counter, void *stream) {
   saber_iu8_desc d;
   if (int rc = resolve(wkind, m, n, k, &d)) return rc;
-  if (!partial && !counter)  // a streamed launch in one piece needs neither
+  if (!partial || !counter)  // a streamed launch in one piece needs neither
     if (int rc = unsplit_stream(&d)) return rc;
   return launch_gemm(ctx, d, a, as, w, ws, c, partial, counter, stream);
 }

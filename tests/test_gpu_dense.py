@@ -518,3 +518,29 @@ def test_streamed_blocks_of_64_columns(ctx, M, N, K, w8):
         ctx.launch(run.desc, bufs)  # the law's own descriptor with neither workspace bound
         torch.cuda.synchronize()
         np.testing.assert_array_equal(host_u16(c), r["C"])
+
+
+def test_streamed_split_without_both_workspaces_runs_in_one_piece(ctx):
+    """The law's own split with one workspace missing, or bound to NULL, needs neither: `gemm` and `launch` run it in one
+    piece, write the oracle's bytes and leave the workspace that is there alone."""
+    M, N, K = 16, 3024, 12288
+    case = synth.dense_case(M, N, K, seed=5)
+    r = ref.linear(case["X"], case["W"], case["ws"], False, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], False)), dev_f32(case["ws"])
+    d = iu8.resolve(iu8.W4, M, N, K)
+    assert d.ks == 4
+    part = torch.full((d.workspace("decode_partial").bytes // 4,), 0x5A5A5A5A, dtype=torch.int32, device="cuda")
+    cnt = torch.full((d.workspace("decode_counter").bytes // 4,), 77, dtype=torch.int32, device="cuda")
+    for p, n in ((part.data_ptr(), None), (None, cnt.data_ptr()), (None, None)):
+        bufs = {"a": codes.data_ptr(), "as": s.data_ptr(), "w": wf.data_ptr(), "ws": ws.data_ptr()}
+        only = {k: v for k, v in (("decode_partial", p), ("decode_counter", n)) if v}
+        null = {"decode_partial": p or 0, "decode_counter": n or 0}
+        for how in ("gemm", only, null):
+            c = torch.full((M, N), 0x7FC0, dtype=torch.int16, device="cuda")
+            if how == "gemm":
+                ctx.gemm(iu8.W4, bufs["a"], bufs["as"], bufs["w"], bufs["ws"], c.data_ptr(), M, N, K, p, n)
+            else:
+                ctx.launch(d, dict(bufs, c=c.data_ptr(), **how))
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(host_u16(c), r["C"])
+    assert (part.cpu().numpy() == 0x5A5A5A5A).all() and (cnt.cpu().numpy() == 77).all()
