@@ -427,10 +427,17 @@ static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint
   return nullptr;
 }
 
+// Which launch `a` and `b` are, whatever their workspaces.
+static bool same_launch(const saber_iu8_desc &a, const saber_iu8_desc &b) {
+  return !strcmp(a.kernel, b.kernel) && a.ks == b.ks && !memcmp(a.grid, b.grid, sizeof a.grid) && !memcmp(a.block, b.block, sizeof a.block);
+}
+
 bool law_split_stream(const saber_iu8_desc &d) {
   int64_t m = 0, n = 0, k = 0;
-  return d.ks > 1 && dec_variant(d.kernel) && int_arg(d, "m", &m) && int_arg(d, "n", &n) && int_arg(d, "k", &k) &&
-         stream_split((uint32_t)m, (uint32_t)n, (uint32_t)k) == d.ks;
+  const DecVariant *v = dec_variant(d.kernel);
+  if (d.ks <= 1 || !v || !int_arg(d, "m", &m) || !int_arg(d, "n", &n) || !int_arg(d, "k", &k)) return false;
+  saber_iu8_desc law;
+  return !resolve(v->w8 ? SABER_IU8_W8 : SABER_IU8_W4, (uint32_t)m, (uint32_t)n, (uint32_t)k, &law) && same_launch(d, law);
 }
 
 int unsplit_stream(saber_iu8_desc *d) {

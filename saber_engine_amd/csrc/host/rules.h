@@ -59,7 +59,7 @@ constexpr uint32_t T1024_SILU_ROWS = 512;
 constexpr uint32_t T1024_WIDE = 12288;
 
 int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out);
-bool law_split_stream(const saber_iu8_desc &d);  // d is a streamed cell on the law's own split of its shape
+bool law_split_stream(const saber_iu8_desc &d);  // d is what `resolve` gives its shape, a streamed cell on a split of K
 // The launch of a caller that binds no workspaces: `d` itself, or its streamed cell with K in one piece.
 int unsplit_stream(saber_iu8_desc *d);
 int describe(const std::string &kernel, uint32_t m, uint32_t n, uint32_t k, uint32_t ks, saber_iu8_desc *out);

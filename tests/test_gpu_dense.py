@@ -544,3 +544,20 @@ def test_streamed_split_without_both_workspaces_runs_in_one_piece(ctx):
             torch.cuda.synchronize()
             np.testing.assert_array_equal(host_u16(c), r["C"])
     assert (part.cpu().numpy() == 0x5A5A5A5A).all() and (cnt.cpu().numpy() == 77).all()
+
+
+def test_named_streamed_split_needs_its_workspaces(ctx):
+    """Only the launch that `resolve` gives a shape runs in one piece without workspaces: another streamed symbol, or the law's
+    own on an edited grid, with the same share count is refused by the missing buffer's name."""
+    M, N, K = 16, 3024, 12288
+    own = iu8.resolve(iu8.W4, M, N, K)
+    assert own.kernel == b"macaq_iu8_dec_w4_tm1_a0" and own.ks == 4
+    edited = iu8.resolve(iu8.W4, M, N, K)
+    edited.grid[0] += 1
+    buf = torch.zeros(N * K // 2, dtype=torch.uint8, device="cuda")
+    bufs = {name: buf.data_ptr() for name in ("a", "as", "w", "ws", "c")}
+    for d in (iu8.describe("macaq_iu8_dec_w4_tm2", M, N, K, ks=4), iu8.describe("macaq_iu8_dec_w4_tm1", M, N, K, ks=4),
+              iu8.describe("macaq_iu8_dec_w4_tm1_a0", M, N, K, ks=3), edited):
+        with pytest.raises(iu8.IU8Error, match="decode_partial") as e:
+            ctx.launch(d, bufs)
+        assert e.value.code == iu8.E_ARG
