@@ -446,6 +446,31 @@ int unsplit_stream(saber_iu8_desc *d) {
   return describe(std::string(d->kernel), (uint32_t)m, (uint32_t)n, (uint32_t)k, 1, d);
 }
 
+bool unsplit_pair(const saber_iu8_desc &d, bool bound, bool bound_b, saber_iu8_desc *out) {
+  const bool b_first = !strncmp(d.kernel, "macaq_iu8f_pairb_w4_", 20);
+  if (!b_first && strncmp(d.kernel, "macaq_iu8f_pair_w4_", 19)) return false;
+  static const char *const INTS[] = {"m", "k", "n", "ks", "nb", "n_b", "ks_b", "nb_b"};
+  int64_t v[8];
+  for (int i = 0; i < 8; ++i)
+    if (!int_arg(d, INTS[i], &v[i])) return false;
+  const uint32_t m = (uint32_t)v[0], k = (uint32_t)v[1];
+  const std::string name = std::string("macaq_iu8_dec_w4_") + (d.kernel + (b_first ? 20 : 19));
+  // the halves as the law gives them where they share K, and in one piece where a half shares K without its workspaces
+  saber_iu8_desc law[2], now[2], p;
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t n = (uint32_t)v[h ? 5 : 2], ks = (uint32_t)v[h ? 6 : 3];
+    if (ks > 1 ? resolve(SABER_IU8_W4, m, n, k, &law[h]) : describe(name, m, n, k, 1, &law[h])) return false;
+    if (law[h].ks != ks) return false;
+    now[h] = law[h];
+    if (!(h ? bound_b : bound) && unsplit_stream(&now[h])) return false;
+  }
+  if (pair(law[0], law[1], &p, b_first) || !same_launch(d, p)) return false;
+  int64_t w = 0;
+  for (int i = 0; i < 8; ++i)
+    if (!int_arg(p, INTS[i], &w) || w != v[i]) return false;
+  return !pair(now[0], now[1], out, b_first);
+}
+
 int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) {
   if (wkind != SABER_IU8_W4 && wkind != SABER_IU8_W8) return fail(SABER_IU8_E_ARG, "unknown weight kind");
   const bool w8 = wkind == SABER_IU8_W8;

@@ -62,6 +62,9 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out);
 bool law_split_stream(const saber_iu8_desc &d);  // d is what `resolve` gives its shape, a streamed cell on a split of K
 // The launch of a caller that binds no workspaces: `d` itself, or its streamed cell with K in one piece.
 int unsplit_stream(saber_iu8_desc *d);
+// The same for a pair whose halves that share K do so as `resolve` gave them: a half without both of its workspaces
+// (`bound`, `bound_b`: it has them) in one piece. False: no such pair.
+bool unsplit_pair(const saber_iu8_desc &d, bool bound, bool bound_b, saber_iu8_desc *out);
 int describe(const std::string &kernel, uint32_t m, uint32_t n, uint32_t k, uint32_t ks, saber_iu8_desc *out);
 // Two W4 decode descriptors of one M, K and kernel -> the one-dispatch pair (macaq_iu8.rs:632-704).
 // order: -1 the law's block order, 0 problem 0 first (`pair`), 1 the second problem first (`pairb`).

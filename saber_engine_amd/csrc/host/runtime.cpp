@@ -424,16 +424,19 @@ static int launch_guard(const LoadedKernel &lk, const saber_iu8_desc *d) {
 int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu8_binding *bufs, uint32_t n_bufs,
                      void *stream) {
   if (!ctx || !d) return fail(SABER_IU8_E_ARG, "launch: null argument");
-  // the law's own split of a streamed launch without both of its workspaces: the launch in one piece, same bytes
+  // the law's own split of a streamed launch, or of a half of a pair, without both of its workspaces: in one piece, same bytes
   saber_iu8_desc whole;
-  auto bound = [&](const char *name) {
+  auto bound = [&](const char *partial, const char *counter) {
     bool found;
-    return bufs && find_binding(bufs, n_bufs, name, &found);
+    return bufs && find_binding(bufs, n_bufs, partial, &found) && find_binding(bufs, n_bufs, counter, &found);
   };
-  if (d->ks > 1 && !(bound("decode_partial") && bound("decode_counter")) && law_split_stream(*d)) {
+  if (d->ks > 1 && !bound("decode_partial", "decode_counter") && law_split_stream(*d)) {
     whole = *d;
     if (int rc = unsplit_stream(&whole)) return rc;
     d = &whole;
+  } else if (d->n_workspaces && !strncmp(d->kernel, "macaq_iu8f_pair", 15)) {
+    const bool b0 = bound("decode_partial", "decode_counter"), b1 = bound("decode_partial_b", "decode_counter_b");
+    if (((i32_arg(d, "ks") > 1 && !b0) || (i32_arg(d, "ks_b") > 1 && !b1)) && unsplit_pair(*d, b0, b1, &whole)) d = &whole;
   }
   auto it = ctx->fn.find(d->kernel);
   if (it == ctx->fn.end()) return fail(SABER_IU8_E_NOTLOADED, std::string(d->kernel) + ": not in the loaded plugin set");

@@ -133,3 +133,54 @@ def test_both_block_orders_give_the_same_bytes(ctx, M, K, n0, n1):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(host_u16(c0), r0["C"])
         np.testing.assert_array_equal(host_u16(c1), r1["C"])
+
+
+def pair_case(ctx, M, K, n0, n1):
+    """Device operands of a pair, its outputs poisoned, and the oracle's bytes: (buffers, c0, c1, want0, want1)."""
+    rng = np.random.default_rng(M * 7 + n0 + K)
+    X, (W0, ws0), (W1, ws1) = halves(rng, M, K, n0, n1)
+    r0, r1 = ref.linear(X, W0, ws0, False, threads=8), ref.linear(X, W1, ws1, False, threads=8)
+    t = dict(a=dev_u8(iu8.repack_a(r0["q"])), w=dev_u8(iu8.repack_w4(W0)), ws=dev_f32(ws0), w_b=dev_u8(iu8.repack_w4(W1)), ws_b=dev_f32(ws1),
+             c=torch.full((M, n0), 0x7FC0, dtype=torch.int16, device="cuda"), c_b=torch.full((M, n1), 0x7FC0, dtype=torch.int16, device="cuda"))
+    t["as"] = dev_f32(r0["a_scale"])
+    return t, r0["C"], r1["C"]
+
+
+@pytest.mark.parametrize("M,K,n0,n1,ks", [(16, 17408, 5120, 96, (3, 1)),        # the second half is no shape the law shares K of
+                                          (20, 12288, 4096, 4112, (4, 3)),      # both halves on shares, `tm2_n1` and `tm2`
+                                          (40, 8192, 5120, 48, (3, 1))])        # `tm3_n2` and `tm3`
+def test_pair_of_resolved_halves_without_workspaces(ctx, M, K, n0, n1, ks):
+    """A pair of two descriptors of the law of which one shares K: launched without workspaces, or with those of one half
+    alone, a half without them runs in one piece; with all of them the counters end at zero. The oracle's bytes each time."""
+    say(f"pair of resolved halves M={M} K={K} N={n0}+{n1}")
+    t, want0, want1 = pair_case(ctx, M, K, n0, n1)
+    a, b = iu8.resolve(iu8.W4, M, n0, K), iu8.resolve(iu8.W4, M, n1, K)
+    assert (a.ks, b.ks) == ks
+    for second_first in (True, False):
+        d = iu8.pair_ordered(a, b, second_first)
+        ws = {}
+        for i in range(d.n_workspaces):
+            w = d.workspaces[i]
+            ws[w.name.decode()] = torch.full((w.bytes // 4,), 0 if w.zero_once else 0x5A5A5A5A, dtype=torch.int32, device="cuda")
+        spare = torch.zeros(64, dtype=torch.int32, device="cuda")     # bound for a half that has no use of it
+        for names in ((), ("decode_partial_b", "decode_counter_b"), ("decode_partial", "decode_counter"), ("decode_partial",), tuple(ws)):
+            t["c"].fill_(0x7FC0), t["c_b"].fill_(0x7FC0)
+            ctx.launch(d, {k: v.data_ptr() for k, v in {**t, **{n: ws.get(n, spare) for n in names}}.items()})
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(host_u16(t["c"]), want0)
+            np.testing.assert_array_equal(host_u16(t["c_b"]), want1)
+            assert not any(v.cpu().numpy().any() for n, v in ws.items() if "counter" in n)
+
+
+def test_pair_of_named_shares_needs_its_workspaces(ctx):
+    """A pair whose half was described on a share count of its own is refused without the workspaces, as that half is alone."""
+    M, K, n0, n1 = 16, 17408, 5120, 96
+    buf = torch.zeros(n0 * K // 2, dtype=torch.uint8, device="cuda")
+    bufs = {n: buf.data_ptr() for n in ("a", "as", "w", "ws", "c", "w_b", "ws_b", "c_b")}
+    one = iu8.describe("macaq_iu8_dec_w4_tm1_a0", M, n1, K)
+    for d in (iu8.pair(iu8.describe("macaq_iu8_dec_w4_tm1_a0", M, n0, K, ks=2), one),
+              iu8.pair(iu8.resolve(iu8.W4, M, n0, K), iu8.describe("macaq_iu8_dec_w4_tm1_a0", M, n1, K, ks=2)),
+              iu8.pair(iu8.describe("macaq_iu8_dec_w4_tm2", M, n0, K, ks=3), iu8.describe("macaq_iu8_dec_w4_tm2", M, n1, K))):
+        with pytest.raises(iu8.IU8Error, match="is not bound") as e:
+            ctx.launch(d, bufs)
+        assert e.value.code == iu8.E_ARG
