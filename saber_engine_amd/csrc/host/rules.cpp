@@ -637,7 +637,7 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
       cu_tiles = (double)q + (double)((4 * rem + grid - 1) / grid) * 0.25 * (c.tops_per_cu / quarter_rate);
     // ... and a few rows past the last whole 256 as thin tiles (int4 weights: the estimate of the int8 cells is drawn without)
     if (!strcmp(c.tile, "tn4_lbk64") && !w8 && tiles < (1u << 20) && k < (1u << 30)) {
-      const iu8_pf_plan plan = iu8_pf_plan256((int)m, (int)((n + 255) / 256), (int)grid, (int)k);
+      const iu8_pf_plan plan = iu8_pf_plan256((int)m, (int)((n + 255) / 256), (int)grid, (int)k, w8);
       if (plan.thin) cu_tiles = std::min(cu_tiles, plan.cost * 0.0108);  // (a margin: level picks stay as they were)
     }
     const double tile_bytes = bm * k + bn * k * (w8 ? 1.0 : 0.5);

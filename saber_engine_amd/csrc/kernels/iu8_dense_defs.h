@@ -54,7 +54,7 @@ static __device__ __forceinline__ int iu8_thin_tile_at(const iu8_pf_plan &p, int
       constexpr int LM = LB > LS ? LB : LS;                                                                        \
       __shared__ __attribute__((aligned(1024))) iu8_u8 lds[LM > LT ? LM : LT];                                     \
       const int G = gridDim.x;                                                                                     \
-      const iu8_pf_plan plan = G == 256 ? iu8_pf_plan256(m, gx, 256, k) : iu8_pf_plan256(m, gx, G, k);             \
+      const iu8_pf_plan plan = G == 256 ? iu8_pf_plan256(m, gx, 256, k, W8) : iu8_pf_plan256(m, gx, G, k, W8);        \
       iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP, false, false, true>(                                       \
           a, as, c, n, k,                                                                                          \
           [&](int r, iu8_tile &t) {                                                                                \

@@ -423,11 +423,14 @@ def test_config4_moe_prefill_shape(ctx):
     check_layer(layer, case, taps=False)
 
 
-@pytest.mark.parametrize("M,N,grid", [(257, 1008, 5), (288, 1296, 8), (384, 784, 6), (777, 1008, 6), (600, 3296, 8), (641, 2304, 11)])
+@pytest.mark.parametrize("M,N,grid", [(257, 1008, 5), (288, 1296, 8), (384, 784, 6), (777, 1008, 6), (600, 3296, 8), (641, 2304, 11),
+                                      (384, 1008, 4), (520, 1008, 8), (288, 3296, 13), (257, 1936, 4), (777, 1936, 10)])
 @pytest.mark.parametrize("tag,w8", [("w4", False), ("w8", True)])
 def test_rows_past_the_last_whole_256_run_as_thin_tiles(ctx, M, N, grid, tag, w8):
     """The 256 x 256 cell's thin tiles (1, 32, 128, 9, 88 and 129 -> whole rows past the last whole 256; a ragged last column block;
-    on the workgroups with a whole tile less, three and one each, on all of them, and behind quarter tiles): the oracle's bytes."""
+    on the workgroups with a whole tile less, three and one each, on all of them, and behind quarter tiles; the last five as int8
+    weights run them: behind whole rounds, also more thin tiles than workgroups, and two each on those with a tile less): the
+    oracle's bytes."""
     K = 1024
     say(f"256x256 cell, thin tiles: {M} x {N}, grid {grid} {tag}")
     case = synth.dense_case(M, N, K, w8=w8, seed=M + grid)

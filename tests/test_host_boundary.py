@@ -7,6 +7,7 @@ import os
 import re
 import shutil
 import struct
+import subprocess
 
 import numpy as np
 import pytest
@@ -786,3 +787,48 @@ def test_lines_of_the_streamed_cells_past_one_round():
                 iu8.describe(name, m, 160, 128)
     with pytest.raises(iu8.IU8Error):
         iu8.describe("macaq_iu8_pf_w4_t48x144_w", 48, 160, 256, ks=2)
+
+
+def test_thin_tiles_by_weight_kind(tmp_path):
+    """The layout rule of the 256 x 256 cell (csrc/kernels/iu8_pf_law.h, compiled here): which launches of 256 workgroups run
+    the rows past the last whole 256 as thin tiles -- int8 weights only where they measured no slower than whole tiles. Every
+    thin tile is dealt out once, whatever share the workgroups with a tile less take."""
+    src, so = tmp_path / "plan.cpp", tmp_path / "plan.so"
+    src.write_text(f'#include "{iu8.PKG}/csrc/kernels/iu8_pf_law.h"\n'
+                   'extern "C" void plan(int m, int gx, int G, int k, int w8, int *o) {\n'
+                   '  const iu8_pf_plan p = iu8_pf_plan256(m, gx, G, k, w8 != 0);\n'
+                   '  const int v[] = {p.thin, p.tail, p.gy, p.q, p.rem, p.own, p.own_wgs};\n'
+                   '  for (int i = 0; i < 7; ++i) o[i] = v[i];\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    lib, out = ctypes.CDLL(str(so)), (ctypes.c_int * 7)()
+
+    def plan(m, n, k, w8, G=256):
+        gx = -(-n // 256)
+        lib.plan(m, gx, min(G, gx * -(-m // 256)), k, int(w8), out)
+        return list(out)
+
+    for m, n, w4, w8 in ((520, 28672, 1, 0), (1030, 16384, 1, 0), (4105, 8192, 1, 0), (8212, 6144, 1, 0), (520, 34816, 1, 0), (600, 28672, 1, 0),
+                         (1290, 28672, 1, 0), (1540, 20480, 1, 0), (4105, 20480, 1, 1), (4200, 20480, 1, 1), (8212, 28672, 1, 1), (777, 34816, 1, 1),
+                         (800, 34816, 1, 1), (1030, 28672, 1, 1), (3100, 10240, 1, 1), (897, 34816, 0, 0), (2048, 34816, 0, 0)):
+        assert (plan(m, n, 5120, False)[0], plan(m, n, 5120, True)[0]) == (w4, w8), (m, n)
+        assert not plan(m, n, 896, False)[0] and not plan(m, n, 896, True)[0]
+    rng, seen = np.random.default_rng(7), 0
+    for _ in range(3000):
+        m, gx, G, w8 = int(rng.integers(257, 9000)), int(rng.integers(1, 140)), int(rng.integers(1, 257)), int(rng.integers(0, 2))
+        thin, tail, gy, q, rem, own, own_wgs = plan(m, gx * 256, 5120, w8, G)
+        if not thin:
+            continue
+        seen += 1
+        assert gy == m // 256 and 0 < m % 256 <= 128 and q * min(G, gx * -(-m // 256)) + rem == gx * gy
+        G, got = min(G, gx * -(-m // 256)), []
+        for at in range(G):          # the kernel's walk: iu8_dense_defs.h, iu8_thin_tile_at
+            for r in range(200):
+                if own_wgs > 0 and at >= rem and r < own:
+                    j = at - rem + r * own_wgs
+                else:
+                    j = own * own_wgs + (G - 1 - at) + (r - (own if own_wgs > 0 and at >= rem else 0)) * G
+                if j >= gx:
+                    break
+                got.append(j)
+        assert sorted(got) == list(range(gx)), (m, gx, G, w8)
+    assert seen > 200
