@@ -377,7 +377,24 @@ static int chain_guard(const LoadedKernel &lk, const saber_iu8_desc *d) {
   return 0;
 }
 
+// A launch that shares K counts its blocks' arrivals, a counter each: a descriptor whose grid has more blocks than its own
+// `decode_counter` has entries (another law's grid under this one's workspaces) would count past its end.
+static int counters_guard(const saber_iu8_desc *d) {
+  const bool is_pair = !strncmp(d->kernel, "macaq_iu8f_pair", 15);
+  if (!is_pair && (d->grid[2] <= 1 || strncmp(d->kernel, "macaq_iu8_dec_", 14))) return 0;
+  for (uint32_t i = 0; i < d->n_workspaces && i < 4; ++i) {
+    const saber_iu8_workspace &w = d->workspaces[i];
+    if (strncmp(w.name, "decode_counter", 14)) continue;
+    const uint64_t blocks = is_pair ? (uint64_t)std::max(i32_arg(d, w.name[14] ? "nb_b" : "nb"), 0) : d->grid[0];
+    if (w.bytes < blocks * 4)
+      return fail(SABER_IU8_E_RULE, fmt("%s: %llu column blocks count their arrivals in a `%s` of %llu B", d->kernel, (unsigned long long)blocks,
+                                        w.name, (unsigned long long)w.bytes));
+  }
+  return 0;
+}
+
 static int launch_guard(const LoadedKernel &lk, const saber_iu8_desc *d) {
+  if (int rc = counters_guard(d)) return rc;
   if (strncmp(d->kernel, "macaq_iu8f_mlp_", 15) == 0) return chain_guard(lk, d);
   if (strncmp(d->kernel, "macaq_iu8f_gateup_act_", 22) == 0) {
     const int64_t m = i32_arg(d, "m"), n = i32_arg(d, "n"), k = i32_arg(d, "k");

@@ -13,7 +13,8 @@
       const float *__restrict__ ws, int *__restrict__ decode_partial, int *__restrict__ decode_counter,           \
       unsigned short *__restrict__ c, int m, int n, int k) {                                                       \
     if constexpr (ALDS == 0) {                                                                                      \
-      iu8_stream_cells<TM, W8, NT, KW, D, ACC>(a, w, as, ws, decode_partial, decode_counter, c, m, n, k);           \
+      iu8_stream_cells<TM, W8, NT, KW, D, ACC>(a, w, as, ws, decode_partial, decode_counter, c, m, n, k,            \
+                                               iu8_blk_of_grid(), (int)gridDim.x);                                  \
     } else {                                                                                                       \
       iu8_dec_body<TM, W8, NT, KW, WPB, D, ALDS, ACC>(a, w, as, ws, decode_partial, decode_counter, c,              \
                                                       iu8_rows{nullptr, 0, m}, n, k);                               \

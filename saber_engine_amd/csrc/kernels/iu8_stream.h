@@ -273,17 +273,19 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
     for (int u = 0; u < NI; ++u) store(p, u);
 }
 
-// A symbol's two cells in one LDS block (iu8_stream_law.h).
+// A symbol's two cells in one LDS block. The launch's own grid says which runs: 64-column blocks where `nblk` blocks of the
+// symbol's own width would not reach the last column (iu8_stream_law.h is the host's rule for it). So the arrival counters are
+// as many as the grid's blocks, and a grid laid out in the symbol's own blocks stays right where the rule has changed since.
 template <int TM, bool W8, int NT, int KW, int D, bool ACC>
 __device__ __forceinline__ void iu8_stream_cells(const iu8_u8 *__restrict__ A, const iu8_u8 *__restrict__ W, const float *__restrict__ as,
                                                  const float *__restrict__ ws, int *__restrict__ P, int *__restrict__ cnt,
-                                                 void *__restrict__ Cv, int M, int N, int K, const iu8_blk B = iu8_blk_of_grid()) {
+                                                 void *__restrict__ Cv, int M, int N, int K, const iu8_blk B, int nblk) {
   constexpr int LDSK = 72;  // two workgroups a CU
   constexpr int NW = IU8_STREAM_WIDE_NT;
   constexpr int OWN = iu8_stream_geo<TM, NT, KW, LDSK>::BYTES, WIDE = iu8_stream_geo<TM, NW, KW, LDSK>::BYTES;
   __shared__ __attribute__((aligned(16))) iu8_u8 lds[KW == 8 && WIDE > OWN ? WIDE : OWN];
   if constexpr (KW == 8) {
-    if (iu8_stream_wide(KW, N, B.Z)) {
+    if (nblk < (N + NT * 16 - 1) / (NT * 16)) {
       iu8_stream_body<TM, W8, NW, KW, 1, ACC, LDSK, TM <= 2>(lds, A, W, as, ws, P, cnt, Cv, M, N, K, B);
       return;
     }

@@ -28,7 +28,7 @@
     const iu8_blk blk{bl % nbp, bl / nbp, p1 ? ks_b : ks};                                                          \
     if constexpr (ALDS == 0)                                                                                        \
       iu8_stream_cells<TM, false, NT, KW, D, false>(a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial, \
-                                                   p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, m, p1 ? n_b : n, k, blk); \
+                                                   p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, m, p1 ? n_b : n, k, blk, nbp); \
     else                                                                                                            \
       iu8_dec_body<TM, false, NT, KW, WPB, D, ALDS, false>(                                                         \
           a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial,                              \

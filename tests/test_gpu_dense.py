@@ -553,7 +553,7 @@ def test_named_streamed_split_needs_its_workspaces(ctx):
     own = iu8.resolve(iu8.W4, M, N, K)
     assert own.kernel == b"macaq_iu8_dec_w4_tm1_a0" and own.ks == 4
     edited = iu8.resolve(iu8.W4, M, N, K)
-    edited.grid[0] += 1
+    edited.grid[0] -= 1
     buf = torch.zeros(N * K // 2, dtype=torch.uint8, device="cuda")
     bufs = {name: buf.data_ptr() for name in ("a", "as", "w", "ws", "c")}
     for d in (iu8.describe("macaq_iu8_dec_w4_tm2", M, N, K, ks=4), iu8.describe("macaq_iu8_dec_w4_tm1", M, N, K, ks=4),
@@ -561,3 +561,37 @@ def test_named_streamed_split_needs_its_workspaces(ctx):
         with pytest.raises(iu8.IU8Error, match="decode_partial") as e:
             ctx.launch(d, bufs)
         assert e.value.code == iu8.E_ARG
+
+
+@pytest.mark.parametrize("kernel,M,N,K,ks,own", [("macaq_iu8_dec_w4_tm1_a0", 16, 3024, 1280, 3, 32), ("macaq_iu8_dec_w8_tm2_n1", 20, 272, 1152, 2, 16),
+                                                 ("macaq_iu8_dec_w4_tm2", 17, 8208, 384, 1, 32), ("macaq_iu8_dec_w8_tm3", 33, 12240, 256, 1, 16)])
+def test_streamed_launch_follows_its_grid(ctx, kernel, M, N, K, ks, own):
+    """A streamed symbol on the law's 64-column grid and on one of its own blocks (a plan laid out before the law had the wide
+    ones), with and without a split of K: the oracle's bytes and as many counters as blocks, left at zero. A grid of more blocks
+    than the descriptor's own counters is refused."""
+    w8 = "_w8_" in kernel
+    say(f"grids of {kernel} {M} x {N} x {K} ks={ks}")
+    case = synth.dense_case(M, N, K, w8=w8, seed=M + N)
+    r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], w8)), dev_f32(case["ws"])
+    for cols in (64, own):
+        d = iu8.describe(kernel, M, N, K, ks)
+        assert d.grid[0] == -(-N // 64)
+        d.grid[0] = -(-N // cols)
+        c = torch.full((M, N), 0x7FC0, dtype=torch.int16, device="cuda")
+        bufs = {"a": codes.data_ptr(), "as": s.data_ptr(), "w": wf.data_ptr(), "ws": ws.data_ptr(), "c": c.data_ptr()}
+        if ks > 1:
+            part = torch.full((d.workspace("decode_partial").bytes // 4,), 0x5A5A5A5A, dtype=torch.int32, device="cuda")
+            cnt = torch.zeros(d.grid[0] + 64, dtype=torch.int32, device="cuda")
+            cnt[d.grid[0]:] = 77                      # past the grid's blocks
+            bufs.update(decode_partial=part.data_ptr(), decode_counter=cnt.data_ptr())
+            if cols != 64:
+                with pytest.raises(iu8.IU8Error, match="decode_counter") as e:
+                    ctx.launch(d, bufs)
+                assert e.value.code == iu8.E_RULE
+                d.workspace("decode_counter").bytes = 4 * d.grid[0]
+        ctx.launch(d, bufs)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host_u16(c), r["C"])
+        if ks > 1:
+            assert not cnt[:d.grid[0]].cpu().numpy().any() and (cnt[d.grid[0]:].cpu().numpy() == 77).all()

@@ -184,3 +184,17 @@ def test_pair_of_named_shares_needs_its_workspaces(ctx):
         with pytest.raises(iu8.IU8Error, match="is not bound") as e:
             ctx.launch(d, bufs)
         assert e.value.code == iu8.E_ARG
+
+
+def test_pair_of_more_blocks_than_counters_is_refused(ctx):
+    """A pair descriptor whose half has more column blocks than its own counters have entries never reaches the GPU."""
+    M, K, n0, n1 = 17, 1152, 1040, 272
+    buf = torch.zeros(1 << 20, dtype=torch.uint8, device="cuda")
+    names = ("a", "as", "w", "ws", "c", "w_b", "ws_b", "c_b", "decode_partial", "decode_counter", "decode_partial_b", "decode_counter_b")
+    for arg in ("nb", "nb_b"):
+        d = iu8.pair(iu8.describe("macaq_iu8_dec_w4_tm2", M, n0, K, ks=3), iu8.describe("macaq_iu8_dec_w4_tm2", M, n1, K, ks=2))
+        d.grid[0] += d.arg(arg).ival * (3 if arg == "nb" else 2)
+        d.arg(arg).ival *= 2
+        with pytest.raises(iu8.IU8Error, match="decode_counter" + arg[2:]) as e:
+            ctx.launch(d, {n: buf.data_ptr() for n in names})
+        assert e.value.code == iu8.E_RULE
