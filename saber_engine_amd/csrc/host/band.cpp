@@ -262,9 +262,9 @@ std::string band_toml() {
       put(o, "regime", std::string("decode"));
       putb(o, "w8", v->w8 != 0);
       put(o, "rows_max", (uint64_t)v->tm * 16);
-      put(o, "block_n", v->block_n(1, 1));
-      if (v->block_n(1, 2) != v->block_n(1, 1)) {  // past one round of the own blocks, and for a split of K
-        put(o, "block_n_wide", v->block_n(1, 2));
+      put(o, "block_n", v->own_n());
+      if (v->block_n(1, 1, 128, 2) != v->own_n()) {  // past one round of the own blocks, and for a split of K
+        put(o, "block_n_wide", v->block_n(1, 1, 128, 2));
         put(o, "wide_from_n", 32 * 256 + 16);
       }
       put(o, "threads", v->threads());

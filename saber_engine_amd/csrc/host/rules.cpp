@@ -118,7 +118,7 @@ static int describe_dec(const DecVariant &v, uint32_t m, uint32_t n, uint32_t k,
   copy_name(d->op, sizeof d->op, op);
   copy_name(d->plugin, sizeof d->plugin, "macaq_iu8");
   copy_name(d->kernel, sizeof d->kernel, v.name);
-  const uint32_t bn = v.block_n(n, ks), nblk = (n + bn - 1) / bn;
+  const uint32_t bn = v.block_n(m, n, k, ks), nblk = (n + bn - 1) / bn;
   d->grid[0] = nblk, d->grid[1] = 1, d->grid[2] = ks;
   d->block[0] = v.threads(), d->block[1] = 1, d->block[2] = 1;
   d->n_launches = 1;
@@ -344,7 +344,10 @@ int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_de
   const DecVariant *pv = pair_variant(name);
   if (!pv) return fail(SABER_IU8_E_RULE, name + ": the fused object carries no such pair");
   const uint32_t ks0 = first.ks, ks1 = second.ks;
-  auto blocks = [&](int64_t n, uint32_t ks) { return (uint32_t)((n + pv->block_n((uint32_t)n, ks) - 1) / pv->block_n((uint32_t)n, ks)); };
+  auto blocks = [&](int64_t n, uint32_t ks) {
+    const int bn = pv->block_n((uint32_t)m0, (uint32_t)n, (uint32_t)kk0, ks);
+    return (uint32_t)((n + bn - 1) / bn);
+  };
   const uint32_t nb0 = blocks(n0, ks0), nb1 = blocks(n1, ks1);
   memset(out, 0, sizeof *out);
   copy_name(out->op, sizeof out->op, "gemm_i4a8_pair");

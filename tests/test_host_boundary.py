@@ -832,3 +832,19 @@ def test_thin_tiles_by_weight_kind(tmp_path):
                 got.append(j)
         assert sorted(got) == list(range(gx)), (m, gx, G, w8)
     assert seen > 200
+
+
+def test_64_column_blocks_where_they_halve_the_blocks_a_cu():
+    """The streamed symbols' block width on both sides of its lines: an even count of 32-column blocks on the busiest of the 256
+    CUs, the edges of such a count at up to eight rows, and a K of whole 8,192; the pair's halves by the same rule."""
+    for (m, n, k), blocks in {
+            (16, 8192, 5376): 256, (16, 8208, 5376): 129, (5, 16384, 5376): 256, (5, 16400, 5376): 513, (16, 24576, 5376): 768,
+            (16, 24592, 5376): 385, (16, 32768, 5376): 512, (16, 32784, 5376): 1025, (9, 41008, 5376): 641,
+            (8, 25088, 5376): 784, (8, 25104, 5376): 393, (9, 25088, 5376): 392, (8, 29696, 5376): 464, (8, 29712, 5376): 929, (9, 29712, 5376): 465,
+            (8, 13312, 8192): 208, (8, 13328, 8192): 417, (9, 13328, 8192): 209, (8, 13328, 8064): 209, (8, 13328, 16384): 417,
+            (8, 28672, 8192): 896, (9, 31744, 8192): 496, (9, 31760, 8192): 993, (16, 15360, 8192): 240, (16, 15376, 8192): 481}.items():
+        for wk, tag in ((iu8.W4, "w4"), (iu8.W8, "w8")):
+            d = iu8.resolve(wk, m, n, k)
+            assert (d.kernel.decode(), d.grid[0], d.ks) == (f"macaq_iu8_dec_{tag}_tm1_a0", blocks, 1), (m, n, k, d.grid[0])
+        p = iu8.pair(iu8.resolve(iu8.W4, m, n, k), iu8.resolve(iu8.W4, m, 48, k))
+        assert (p.arg("nb").ival, p.arg("nb_b").ival) == (blocks, 2), (m, n, k)
