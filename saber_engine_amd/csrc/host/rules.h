@@ -17,7 +17,7 @@ struct DecVariant {
   // columns a workgroup: a streamed symbol (no staged rows) holds 64-column blocks as well (iu8_stream_law.h)
   int own_n() const { return wpb / kw * nt * 16; }
   int block_n(uint32_t m, uint32_t n, uint32_t k, uint32_t ks) const {
-    return alds == 0 && iu8_stream_wide(kw, m, n, k, ks) ? IU8_STREAM_WIDE_NT * 16 : own_n();
+    return alds == 0 && iu8_stream_wide(kw, own_n(), m, n, k, ks) ? IU8_STREAM_WIDE_NT * 16 : own_n();
   }
   int threads() const { return wpb * 64; }
 };

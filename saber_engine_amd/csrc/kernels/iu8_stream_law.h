@@ -8,19 +8,22 @@
 // of 16384 x 5120 / 2048 / 1024 12.3 / 6.8 / 6.2 -> 10.2 / 6.1 / 4.8, 12288 x 5120 12.6 -> 11.2, 8208 x 5120 10.8 -> 9.9; W8 12288 x 5120
 // 17.1 -> 15.1, 16384 x 5120 17.4 -> 16.7. On three shares of K: 5120 x 17408 at 16 / 32 rows 12.8 / 14.5 -> 11.2 / 12.7.
 //
+// (Symbols whose own blocks are 16 columns wide, more than 32 rows: from 8,192 columns on, where they are more than two a CU.)
 // A 64-column block takes 1.75 times one of 32. The busiest CU of 256 runs ceil(n / 8,192) of those: an even count is half as
 // many wide ones, an odd one rounds up and loses. W4 at 5 / 16 rows: 17408 x 8192 15.9 / 18.2 -> 19.1 / 20.2, 17408 x 17408 30.2
 // -> 36.1, 34816 x 8192 24.9 -> 29.3, W8 18064 x 10112 33.2 -> 38.6 (three and five blocks a CU: own); 9600 x 8192 11.4 -> 9.9, W8 19.7
 // -> 16.0, 27648 x 5376 14.9 / 17.1 -> 14.4 / 15.4, W8 27648 x 12288 57.3 -> 52.9 (two and four: wide). Towards the last columns of an even
 // count the launch is bound by its bytes and up to eight rows have nothing left to share: 32752 x 12288 at 5 rows 0.97; in front of
 // them, past four blocks a CU, 24592 x 6144 0.95. A K of whole 8,192 puts a block's tiles 64 KiB apart and four of them on one channel:
-// 16384 / 28672 / 32752 x 8192 at 5 rows 0.93 / 0.97 / 0.90, at 16 rows 1.03 / 1.09 / 1.00, W8 0.97 / 1.04 / 0.97.
+// 16384 / 28672 / 32752 x 8192 at 5 rows 0.93 / 0.97 / 0.90, at 16 rows 1.03 / 1.09 / 1.00, W8 0.97 / 1.04 / 0.97
+// (at 24 rows 16384 x 8192 15.6 -> 13.9).
 constexpr int IU8_STREAM_WIDE_NT = 4;
-constexpr bool iu8_stream_wide(int kw, long m, long n, long k, long ks) {
+constexpr bool iu8_stream_wide(int kw, int own, long m, long n, long k, long ks) {
   if (kw != 8 || ks > 1) return kw == 8;
+  if (own < 32) return n > 8192;
   const long a_cu = (n + 8191) / 8192, last = n - (a_cu - 2) * 8192;  // own blocks on the busiest CU; columns of its last two
   const bool aligned = k % 8192 == 0;
   if (a_cu % 2) return false;
-  if (m > 8) return !aligned || last <= 15360;
+  if (m > 8) return m > 16 || !aligned || last <= 15360;
   return a_cu == 2 ? !aligned || last <= 13312 : !aligned && last > 8704 && last <= 13312;
 }

@@ -848,3 +848,9 @@ def test_64_column_blocks_where_they_halve_the_blocks_a_cu():
             assert (d.kernel.decode(), d.grid[0], d.ks) == (f"macaq_iu8_dec_{tag}_tm1_a0", blocks, 1), (m, n, k, d.grid[0])
         p = iu8.pair(iu8.resolve(iu8.W4, m, n, k), iu8.resolve(iu8.W4, m, 48, k))
         assert (p.arg("nb").ival, p.arg("nb_b").ival) == (blocks, 2), (m, n, k)
+    assert iu8.resolve(iu8.W4, 17, 16384, 8192).grid[0] == 256
+    for (m, n0, n1, k), blocks in {(16, 9600, 9600, 8192): (300, 300), (16, 9600, 96, 8192): (150, 3), (16, 16384, 16384, 5376): (256, 256),
+                                   (16, 16384, 8192, 5376): (256, 256), (8, 16384, 16384, 5376): (512, 512),
+                                   (40, 12288, 12288, 8192): (192, 192)}.items():
+        p = iu8.pair(iu8.resolve(iu8.W4, m, n0, k), iu8.resolve(iu8.W4, m, n1, k))
+        assert (p.arg("nb").ival, p.arg("nb_b").ival) == blocks, (m, n0, n1, k)
