@@ -149,25 +149,27 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
 #pragma unroll
         for (int h = 0; h < 2; ++h) ringa[slot][i][h] = *(const iu8_v4i *)(ab + h * 1024 + ao[i]);
     };
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-      issue(i, i);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    int t0 = 0;
-    for (; t0 + D < T; t0 += D) {
+    if (T > 0) {  // (a wave without a step: the first fragment, asked for by every such wave, is one line of one channel)
 #pragma unroll
       for (int i = 0; i < D; ++i) {
-        consume(i);
-        __builtin_amdgcn_sched_barrier(0);
-        issue(i, t0 + i + D);
+        issue(i, i);
         __builtin_amdgcn_sched_barrier(0);
       }
-    }
+      int t0 = 0;
+      for (; t0 + D < T; t0 += D) {
 #pragma unroll
-    for (int i = 0; i < D; ++i) {
-      if (t0 + i < T) consume(i);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < D; ++i) {
+          consume(i);
+          __builtin_amdgcn_sched_barrier(0);
+          issue(i, t0 + i + D);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        if (t0 + i < T) consume(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
 
