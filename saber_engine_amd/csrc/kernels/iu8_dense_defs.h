@@ -12,6 +12,7 @@
       const unsigned char *__restrict__ a, const unsigned char *__restrict__ w, const float *__restrict__ as,     \
       const float *__restrict__ ws, int *__restrict__ decode_partial, int *__restrict__ decode_counter,           \
       unsigned short *__restrict__ c, int m, int n, int k) {                                                       \
+    static_assert(ALDS > 0 ? TM == 1 : WPB == KW, "staged rows are one row tile; a streamed cell's waves its k-waves"); \
     if constexpr (ALDS == 0) {                                                                                      \
       iu8_stream_cells<TM, W8, NT, KW, D, ACC>(a, w, as, ws, decode_partial, decode_counter, c, m, n, k,            \
                                                iu8_blk_of_grid(), (int)gridDim.x);                                  \

@@ -26,6 +26,7 @@
     const bool p1 = BFIRST ? bx < b1 : bx >= b0;                                                                    \
     const int bl = BFIRST ? (p1 ? bx : bx - b1) : (p1 ? bx - b0 : bx), nbp = p1 ? nb_b : nb;                        \
     const iu8_blk blk{bl % nbp, bl / nbp, p1 ? ks_b : ks};                                                          \
+    static_assert(ALDS > 0 ? TM == 1 : WPB == KW, "staged rows are one row tile; a streamed cell's waves its k-waves"); \
     if constexpr (ALDS == 0)                                                                                        \
       iu8_stream_cells<TM, false, NT, KW, D, false>(a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial, \
                                                    p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, m, p1 ? n_b : n, k, blk, nbp); \
