@@ -346,7 +346,7 @@ def test_had_refusals(ctx):
 @pytest.mark.parametrize("W", [4096, 8064, 8192, 8320])
 def test_few_row_norm_producers_at_the_one_group_edge(ctx, W):
     """The 16-wave norms on both sides of one 8-element group a thread (8,192): rows that end inside the last wave, fill it
-    and pass it, with a row of infinities and NaN, against the oracle."""
+    and pass it, the GDN norm's with infinities and NaN (add_rms on them: the test below), against the oracle."""
     M = 3
     rng = np.random.default_rng(W)
     t = rng.choice([-1.0, 1.0], size=W).astype(np.float32)
@@ -372,3 +372,58 @@ def test_few_row_norm_producers_at_the_one_group_edge(ctx, W):
     np.testing.assert_array_equal(host_u16(ro), wro)
     np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32))
     np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, W), wq)
+
+
+@pytest.mark.parametrize("W", [2048, 4096, 8192, 8320, 12288])
+def test_add_rms_on_every_bf16_value(ctx, W):
+    """Every bf16 pattern of y -- infinities, NaNs and subnormal numbers among them -- beside a residual that is zero, one,
+    infinite or NaN, in each form of the producer (16-wave, 256 and 512 threads): res_out has the oracle's bits, but where
+    IEEE leaves them open: the sign of infinity - infinity's NaN, and which NaN of two is the sum. Codes and scales are the oracle's, rows of NaN included."""
+    M = 65536 // W + 2
+    say(f"add_rms on every bf16 value, W={W}")
+    rng = np.random.default_rng(W)
+    X = np.resize(np.arange(65536, dtype=np.uint16), (M, W))
+    X[-1] = synth.activations(rng, 1, W)[0]          # (an all-finite row)
+    wn = synth.f32_to_bf16_bits((rng.standard_normal(W) * 0.1).astype(np.float32))
+    t = rng.choice([-1.0, 1.0], size=W).astype(np.float32)
+    xd, wnd, td = dev_bf16_bits(X), dev_bf16_bits(wn), dev_f32(t)
+    for r in (0x0000, 0x8000, 0x3F80, 0x7F80, 0xFF80, 0x7FC0, 0xFF81):
+        res = np.full((M, W), r, dtype=np.uint16)
+        res[-1] = synth.activations(rng, 1, W)[0]
+        rd, ro = dev_bf16_bits(res), torch.zeros((M, W), dtype=torch.int16, device="cuda")
+        q, s = outs(M, W)
+        ctx.add_rms_quant_had(xd.data_ptr(), rd.data_ptr(), wnd.data_ptr(), q.data_ptr(), s.data_ptr(), ro.data_ptr(), M, W, 1e-6, td.data_ptr())
+        torch.cuda.synchronize()
+        with np.errstate(invalid="ignore"):
+            wq, wsc, wro = ref.add_rms_quant_had(X, res, wn, t, 1e-6, 256 if W <= 10240 else 512)
+        got = host_u16(ro)
+        nan, free = lambda v: (v & 0x7FFF) > 0x7F80, ((X & 0x7FFF) == 0x7F80) & (res == (X ^ 0x8000))
+        free |= nan(X) & nan(res)
+        assert nan(got[free]).all()
+        np.testing.assert_array_equal(got[~free], wro[~free], err_msg=hex(r))
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32), err_msg=hex(r))
+        np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, W), wq, err_msg=hex(r))
+
+
+@pytest.mark.parametrize("M,H", [(3, 64), (2, 65), (2, 136), (1, 320)])
+def test_attention_gate_rows_of_several_groups_by_name(ctx, M, H):
+    """The 16-wave attention gate launched by name on rows past what the entry point takes (6,144): one 8-element group a thread
+    at 8,192, more above it, five at 40,960; computed and table form, the oracle's bytes."""
+    W = H * 128
+    say(f"attention gate by name M={M} W={W}")
+    rng = np.random.default_rng(W)
+    core = synth.activations(rng, M, W)
+    block = synth.f32_to_bf16_bits((rng.standard_normal((M, 2 * W + 16)) * 3).astype(np.float32))
+    block[M // 2, 128:128 + 8] = [0x7F80, 0xFF80, 0x7FC0, 0x0000, 0x8000, 0x0001, 0x36FF, 0xC700]
+    t = rng.choice([-1.0, 1.0], size=W).astype(np.float32)
+    cd, bd, td = dev_bf16_bits(core), dev_bf16_bits(block), dev_f32(t)
+    sig = torch.zeros(65536, dtype=torch.int16, device="cuda")
+    ctx.sigmoid_table(sig.data_ptr())
+    wq, wsc = ref.attn_gate_quant_had(core, block, t, 128)
+    for name, tab in (("attn_gate_quant_hadi8_t1024", {}), ("attn_gate_quant_hadi8_lut_t1024", dict(lut=sig.data_ptr()))):
+        q, s = outs(M, W)
+        d = iu8.describe_raw(name, (M, 1, 1), 1024, plugin="attn_glue_hadi8", n=W, hd=128, gs=2 * W + 16)
+        ctx.launch(d, dict(core=cd.data_ptr(), gate=bd.data_ptr(), q=q.data_ptr(), scale=s.data_ptr(), had_t=td.data_ptr(), **tab))
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32), err_msg=name)
+        np.testing.assert_array_equal(iu8.unpack_a(q.cpu().numpy(), M, W), wq, err_msg=name)
