@@ -119,6 +119,7 @@ std::string band_toml() {
   put(o, "cu_count", CU_COUNT);
   put(o, "wavefront_size", 64);
   put(o, "decode_max_m", DECODE_MAX_M);
+  o += "# K shares of a decode launch outside the lines of [stream_split]\n";
   put(o, "decode_split", 1);
   put(o, "ks_max", KS_MAX);
   put(o, "a_layout_id", SABER_IU8_LAYOUT_A_TILED_I8_64);
@@ -150,6 +151,31 @@ std::string band_toml() {
     if (resolve_fused(SABER_IU8_W4, 1, sh.n, sh.k, &d)) continue;
     o += fmt("grid.%s = %u\n", sh.op, d.grid[0]);
   }
+  o += "\n[stream_split]\n";
+  o += "# K shares of a streamed decode launch: with b = ceil(n / 64), min(shares_max, cu_count / b) of them where that is shares_min\n";
+  o += "# at least and 4 * b at least three quarters of cu_count, from K = k_min (k_min_16_rows up to 16 rows, else k_min_4096_columns\n";
+  o += "# up to 4,096 columns). int4 from 33 rows: K >= 16384 is on tiles before this, where the bands say so\n";
+  put(o, "rows_over", STREAM_SPLIT_ROWS_OVER);
+  put(o, "rows_max", STREAM_SPLIT_ROWS_MAX);
+  put(o, "shares_min", STREAM_SPLIT_SHARES_MIN);
+  put(o, "shares_max", STREAM_SPLIT_SHARES_MAX);
+  put(o, "k_min", STREAM_SPLIT_K);
+  put(o, "k_min_16_rows", STREAM_SPLIT_K_16ROWS);
+  put(o, "k_min_4096_columns", STREAM_SPLIT_K_4096COLS);
+  o += "\n[decode_block_width]\n";
+  o += "# A decode cell with a block_n_wide has its grid laid out in blocks of that width (its kernel follows the grid, and the\n";
+  o += "# arrival counters are as many as the grid's blocks) where K is shared, and where\n";
+  o += "#   block_n = 16: n > round\n";
+  o += "#   block_n = 32: a = ceil(n / round) is even, and with last = n - (a - 2) * round\n";
+  o += "#     up to few_rows rows:  few_last_over < last <= few_last_max and K no multiple of aligned_k; a = 2: last <= few_last_max or such a K\n";
+  o += "#     up to aligned_rows:   last <= aligned_last_max, or K no multiple of aligned_k\n";
+  put(o, "round", IU8_STREAM_ROUND);
+  put(o, "few_rows", IU8_STREAM_FEW_ROWS);
+  put(o, "few_last_over", IU8_STREAM_FEW_LAST[0]);
+  put(o, "few_last_max", IU8_STREAM_FEW_LAST[1]);
+  put(o, "aligned_k", IU8_STREAM_ALIGNED_K);
+  put(o, "aligned_rows", IU8_STREAM_ALIGNED_ROWS);
+  put(o, "aligned_last_max", IU8_STREAM_ALIGNED_LAST);
   o += "\n[row_producers]\n# macaq_i8_quant_* / macaq_i8_silu_mul_quant_*: 16 waves a row (_t1024) for rows wider than\n";
   o += "# width_over while the row count leaves the card part idle, else the narrowest 256-thread form\n";
   put(o, "t1024_width_over", T1024_WIDTH_OVER);
@@ -263,12 +289,10 @@ std::string band_toml() {
       putb(o, "w8", v->w8 != 0);
       put(o, "rows_max", (uint64_t)v->tm * 16);
       put(o, "block_n", v->own_n());
-      if (v->block_n(1, 1, 128, 2) != v->own_n()) {  // past one round of the own blocks, and for a split of K
-        put(o, "block_n_wide", v->block_n(1, 1, 128, 2));
-        put(o, "wide_from_n", 32 * 256 + 16);
-      }
+      const bool wide = v->block_n(1, 1, 128, 2) != v->own_n();
+      if (wide) put(o, "block_n_wide", v->block_n(1, 1, 128, 2));
       put(o, "threads", v->threads());
-      put(o, "grid", std::string("[ceil(n / block_n), 1, ks]"));
+      put(o, "grid", std::string(wide ? "[ceil(n / (block_n or block_n_wide: [decode_block_width])), 1, ks]" : "[ceil(n / block_n), 1, ks]"));
       put(o, "kernarg", std::string("dec"));
     } else if (name.rfind("macaq_iu8_dec_w4_tm1_s80", 0) == 0 || name.rfind("macaq_iu8_dec_w8_tm1_s80", 0) == 0) {
       put(o, "regime", std::string("decode"));

@@ -396,9 +396,9 @@ static bool stream_wide_blocks(bool w8, uint32_t m, uint32_t n, uint32_t k) {
 // level at best. The static workspace holds it (3.9 MB), and a caller that binds no workspaces gets the launch in one piece.
 static uint32_t stream_split(uint32_t m, uint32_t n, uint32_t k) {
   const uint32_t blocks = (n + 16 * IU8_STREAM_WIDE_NT - 1) / (16 * IU8_STREAM_WIDE_NT);
-  const uint32_t z = blocks ? std::min(4u, CU_COUNT / blocks) : 0;
-  if (m <= 8 || m > 48 || z < 3 || blocks * 4 < CU_COUNT * 3 / 4) return 1;
-  return k >= (m <= 16 ? 10240u : n <= 4096 ? 12288u : 8192u) ? z : 1;
+  const uint32_t z = blocks ? std::min(STREAM_SPLIT_SHARES_MAX, CU_COUNT / blocks) : 0;
+  if (m <= STREAM_SPLIT_ROWS_OVER || m > STREAM_SPLIT_ROWS_MAX || z < STREAM_SPLIT_SHARES_MIN || blocks * 4 < CU_COUNT * 3 / 4) return 1;
+  return k >= (m <= 16 ? STREAM_SPLIT_K_16ROWS : n <= 4096 ? STREAM_SPLIT_K_4096COLS : STREAM_SPLIT_K) ? z : 1;
 }
 
 // The wide streamed cells: blocks of 64, 96 or 144 columns that give three quarters of the CUs and more one block each, from

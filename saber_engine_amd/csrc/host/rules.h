@@ -53,6 +53,9 @@ constexpr uint32_t FUSED_R1_MIN_K = 8192;   // rows at least this long take the 
 constexpr uint32_t MLP_CHAIN_PAYS_INTER_1 = 12288, MLP_CHAIN_PAYS_INTER_2 = 13824;  // one / two rows: the chain beats the three launches from here
 constexpr uint32_t S80_MIN_N = 24576;            // the staged persistent GEMV: columns from here at any row count
 constexpr uint64_t S80_MIN_BYTES = 64ull << 20;  // the staged persistent GEMV: weights from here at up to 8 rows, and for int8 weights
+// K shares of a streamed launch (rules.cpp:stream_split): rows, shares, the least K by rows and columns
+constexpr uint32_t STREAM_SPLIT_ROWS_OVER = 8, STREAM_SPLIT_ROWS_MAX = 48, STREAM_SPLIT_SHARES_MIN = 3, STREAM_SPLIT_SHARES_MAX = 4;
+constexpr uint32_t STREAM_SPLIT_K_16ROWS = 10240, STREAM_SPLIT_K_4096COLS = 12288, STREAM_SPLIT_K = 8192;
 constexpr uint32_t HAD_T1024_ROWS = 256, HAD_T1024_WIDTH = 4096;  // the Hadamard-basis producers' 16-wave forms: up to / from
 constexpr uint32_t T1024_WIDTH_OVER = 4096;
 constexpr uint32_t T1024_QUANT_ROWS = 256, T1024_QUANT_ROWS_WIDE = 512;

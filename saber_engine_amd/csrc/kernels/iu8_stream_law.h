@@ -18,12 +18,17 @@
 // 16384 / 28672 / 32752 x 8192 at 5 rows 0.93 / 0.97 / 0.90, at 16 rows 1.03 / 1.09 / 1.00, W8 0.97 / 1.04 / 0.97
 // (at 24 rows 16384 x 8192 15.6 -> 13.9).
 constexpr int IU8_STREAM_WIDE_NT = 4;
+constexpr long IU8_STREAM_ROUND = 8192;                                    // columns of one 32-column block a CU
+constexpr long IU8_STREAM_FEW_ROWS = 8, IU8_STREAM_FEW_LAST[2] = {8704, 13312};  // `last` in (8704, 13312] at up to eight rows
+constexpr long IU8_STREAM_ALIGNED_K = 8192, IU8_STREAM_ALIGNED_ROWS = 16, IU8_STREAM_ALIGNED_LAST = 15360;
 constexpr bool iu8_stream_wide(int kw, int own, long m, long n, long k, long ks) {
   if (kw != 8 || ks > 1) return kw == 8;
-  if (own < 32) return n > 8192;
-  const long a_cu = (n + 8191) / 8192, last = n - (a_cu - 2) * 8192;  // own blocks on the busiest CU; columns of its last two
-  const bool aligned = k % 8192 == 0;
+  if (own < 32) return n > IU8_STREAM_ROUND;
+  // own blocks on the busiest CU; columns of its last two
+  const long a_cu = (n + IU8_STREAM_ROUND - 1) / IU8_STREAM_ROUND, last = n - (a_cu - 2) * IU8_STREAM_ROUND;
+  const bool aligned = k % IU8_STREAM_ALIGNED_K == 0;
   if (a_cu % 2) return false;
-  if (m > 8) return m > 16 || !aligned || last <= 15360;
-  return a_cu == 2 ? !aligned || last <= 13312 : !aligned && last > 8704 && last <= 13312;
+  if (m > IU8_STREAM_FEW_ROWS) return m > IU8_STREAM_ALIGNED_ROWS || !aligned || last <= IU8_STREAM_ALIGNED_LAST;
+  if (a_cu == 2) return !aligned || last <= IU8_STREAM_FEW_LAST[1];
+  return !aligned && last > IU8_STREAM_FEW_LAST[0] && last <= IU8_STREAM_FEW_LAST[1];
 }

@@ -854,3 +854,50 @@ def test_64_column_blocks_where_they_halve_the_blocks_a_cu():
                                    (40, 12288, 12288, 8192): (192, 192)}.items():
         p = iu8.pair(iu8.resolve(iu8.W4, m, n0, k), iu8.resolve(iu8.W4, m, n1, k))
         assert (p.arg("nb").ival, p.arg("nb_b").ival) == blocks, (m, n0, n1, k)
+
+
+def test_band_table_grids_follow_their_cell_rows():
+    """Every decode and wide row of the shipped law table states the grid that its cell row and the table's own rules give: the
+    block width, the shares of K, one arrival counter a block."""
+    import tomli
+
+    t = tomli.loads(open(iu8.BAND_TABLE).read())
+    cells, sp, bw = {c["kernel"]: c for c in t["cell"]}, t["stream_split"], t["decode_block_width"]
+
+    def shares(m, n, k):
+        b = -(-n // 64)
+        z = min(sp["shares_max"], t["cu_count"] // b)
+        k_min = sp["k_min_16_rows"] if m <= 16 else sp["k_min_4096_columns"] if n <= 4096 else sp["k_min"]
+        return z if sp["rows_over"] < m <= sp["rows_max"] and z >= sp["shares_min"] and 16 * b >= 3 * t["cu_count"] and k >= k_min else t["decode_split"]
+
+    def width(c, m, n, k, ks):
+        if "block_n_wide" not in c or (ks == 1 and c["block_n"] == 16 and n <= bw["round"]):
+            return c["block_n"]
+        a = -(-n // bw["round"])
+        last, aligned = n - (a - 2) * bw["round"], k % bw["aligned_k"] == 0
+        if m <= bw["few_rows"]:
+            edge = (not aligned or last <= bw["few_last_max"]) if a == 2 else not aligned and bw["few_last_over"] < last <= bw["few_last_max"]
+        else:
+            edge = m > bw["aligned_rows"] or not aligned or last <= bw["aligned_last_max"]
+        return c["block_n_wide"] if ks > 1 or c["block_n"] == 16 or (a % 2 == 0 and edge) else c["block_n"]
+
+    seen = set()
+    for b in t["band"]:
+        c = cells[b["kernel"]]
+        if c["regime"] not in ("decode", "wide") or "persistent" in c["grid"]:
+            continue
+        for m, grid in ((b["first_m"], b["grid_first"]), (b["last_m"], b["grid_last"])):
+            ks = shares(m, b["n"], b["k"]) if "block_n_wide" in c else 1     # (the streamed symbols have one)
+            w = width(c, m, b["n"], b["k"], ks) if c["regime"] == "decode" else c["block_n"]
+            assert b["ks"] == ks and grid == [-(-b["n"] // w), 1, ks], (b, m, ks, w)
+            seen.add((c["regime"], w, ks > 1))
+            if ks > 1:
+                assert iu8.gemm_workspace(iu8.W8 if b["w8"] else iu8.W4, m, b["n"], b["k"])[1] == 4 * grid[0]
+    assert {("decode", 64, True), ("decode", 64, False), ("decode", 32, False), ("decode", 16, False), ("wide", 144, False)} <= seen
+    # the width rule away from the table's shapes
+    rng = np.random.default_rng(11)
+    for _ in range(2000):
+        name = str(rng.choice([c for c in cells if cells[c]["regime"] == "decode" and "block_n_wide" in cells[c]]))
+        c, n, k, ks = cells[name], int(rng.integers(1, 3500)) * 16, int(rng.choice([128, 5376, 8192, 16384])), int(rng.integers(1, 3))
+        m, ks = int(rng.integers(1, c["rows_max"] + 1)), min(ks, k // 128)
+        assert iu8.describe(name, m, n, k, ks).grid[0] == -(-n // width(c, m, n, k, ks)), (name, m, n, k, ks)
