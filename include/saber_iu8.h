@@ -307,6 +307,8 @@ int saber_iu8_attn_gate_quant_had(saber_iu8_ctx *ctx, const void *core_bf16, con
  * GEMMs that read one A operand, one dispatch of the fused object's `macaq_iu8f_pair_w4_tm*`
  * (kernarg list abi.rs:3411-3432). Each half is the descriptor saber_iu8_resolve / _describe gave
  * it alone; the grids go end to end, the second half's buffers and workspaces take the suffix `_b`.
+ * A resolved half of 9..48 rows of a deep linear shares K and brings its two workspaces along (saber_iu8_gemm_workspace);
+ * saber_iu8_launch runs such a half in one piece where they are not both bound.
  * Refused (SABER_IU8_E_RULE) unless both halves are W4 decode cells of one kernel, M and K. */
 int saber_iu8_pair(const saber_iu8_desc *first, const saber_iu8_desc *second, saber_iu8_desc *out);
 /* The same with the block order named instead of taken from the law (PAIR_BA_FIRST,
@@ -314,7 +316,7 @@ int saber_iu8_pair(const saber_iu8_desc *first, const saber_iu8_desc *second, sa
  * (macaq_iu8f_pairb_w4_tm*), 0 problem 0's (macaq_iu8f_pair_w4_tm*). Same bytes either way. */
 int saber_iu8_pair_ordered(const saber_iu8_desc *first, const saber_iu8_desc *second, int second_first,
                            saber_iu8_desc *out);
-/* resolve x 2 + pair + launch for the unsplit decode law: c [m,n] and c_b [m,n_b] from one a / a_scale. */
+/* resolve x 2 + pair + launch, every half in one piece (no workspaces): c [m,n] and c_b [m,n_b] from one a / a_scale. */
 int saber_iu8_gemm_pair(saber_iu8_ctx *ctx, const void *a, const float *a_scale, const void *w, const float *w_scale, void *c,
                         uint32_t n, const void *w_b, const float *w_scale_b, void *c_b, uint32_t n_b, uint32_t m, uint32_t k,
                         void *stream);
@@ -398,8 +400,9 @@ int saber_iu8_linear_prefill_fused(saber_iu8_ctx *ctx, int wkind, const void *x_
 /* Workspace bytes the resolved GEMM needs (both 0 when it does not split). Ask before every
  * saber_iu8_gemm of a new shape: the law splits K in two bands: tiles at 33..192 rows of K >= 16384
  * (few tiles), where a launch with `partial` / `counter` NULL is refused (SABER_IU8_E_ARG), and the streamed
- * cells at 9..48 rows of K >= 8192, which run in one piece without them (saber_iu8_launch of the resolved
- * descriptor with neither bound too). */
+ * cells at 9..48 rows of K >= 8192, which run in one piece unless both are given (saber_iu8_launch of the resolved
+ * descriptor too; a descriptor on a share count of the caller's own needs them). Launches that share a `partial` /
+ * `counter` pair must not overlap in time. */
 int saber_iu8_gemm_workspace(int wkind, uint32_t m, uint32_t n, uint32_t k, uint64_t *partial_bytes,
                              uint64_t *counter_bytes);
 
@@ -418,7 +421,9 @@ int saber_iu8_gemm(saber_iu8_ctx *ctx, int wkind, const void *a, const float *as
  * every allocation (include/saber_abi.h:163-174). The split-K workspaces of the launch (`partial`,
  * `counter`) are not arguments: they live in one static device array of the library, 8 MiB of
  * partials + 64 KiB of counters (saber_iu8_static_workspace_bytes), present once on every GPU a context
- * was opened on and held until the process ends. Same kernels, same bytes as saber_iu8_gemm. Allocates,
+ * was opened on and held until the process ends. Same bytes as saber_iu8_gemm; the streamed cells' split (9..48
+ * rows of K >= 8192) runs in one piece here, so saber_iu8_gemm with workspaces is the faster call there (16 rows of
+ * 5120 x 17408 11.2 against 13.7 us). Allocates,
  * clears and synchronises nothing: the counters are zero from set-up and every kernel leaves them
  * zero. A shape whose split needs more than the array holds is refused (SABER_IU8_E_RULE): use
  * saber_iu8_gemm with caller-owned workspaces. All calls on one GPU share that GPU's array: calls

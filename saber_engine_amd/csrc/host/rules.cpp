@@ -393,7 +393,9 @@ static bool stream_wide_blocks(bool w8, uint32_t m, uint32_t n, uint32_t k) {
 // K = 10240 / 12288 / 17408 9.0 / 10.0 / 13.7 -> 8.6 / 9.5 / 11.2 (8192: 7.5 -> 8.0), 32 rows of 8192 / 12288 / 17408 9.1 / 12.5 / 17.4 -> 8.4 /
 // 10.3 / 12.7, 48 rows of 8192 / 12288 10.6 / 14.8 -> 9.6 / 11.5 (6144 level); W8 16 / 32 / 48 rows of 12288 14.7 / 17.8 / 20.2 -> 14.2 / 15.2 /
 // 16.4. 4096 columns on four shares, 16 / 32 rows of 16384 12.2 / 13.2 -> 11.3 / 11.9, 20 rows of 10240 level. Up to eight rows it is
-// level at best. The static workspace holds it (3.9 MB), and a caller that binds no workspaces gets the launch in one piece.
+// level at 5,120 columns and pays on narrower ones of a longer K, which no line takes yet (6 rows, W4 / W8: 3072 x 17408 10.5 / 16.0 -> 8.9 / 12.5,
+// 4096 x 17408 10.8 / 16.8 -> 10.1 / 15.0, 3072 x 10240 level / 10.4 -> 9.3). The partials are 3.1 MB at most; a caller without both
+// workspaces, saber_iu8_gemm_static and saber_iu8_gemm_pair get the launch in one piece.
 static uint32_t stream_split(uint32_t m, uint32_t n, uint32_t k) {
   const uint32_t blocks = (n + 16 * IU8_STREAM_WIDE_NT - 1) / (16 * IU8_STREAM_WIDE_NT);
   const uint32_t z = blocks ? std::min(STREAM_SPLIT_SHARES_MAX, CU_COUNT / blocks) : 0;
@@ -490,7 +492,9 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // A deep, narrow linear of int4 weights leaves the band at 33 rows already: where the tile law shares K over workgroups
   // (pf_split), its 64 x 128 cell overtakes the streaming form (5120 x 17408 at 33 / 45 rows on four shares 18.6 / 18.9 us,
   // 21.0 / 22.5 on `tm3_n2`; up to 32 rows streaming wins, 15.5 against 17.5 at 17. A narrower one would stay: 3072 x 16384 at
-  // 33 / 45 rows 17.3 / 17.7 shared, 13.7 / 15.0 on `tm3`).
+  // 33 / 45 rows 17.3 / 17.7 shared, 13.7 / 15.0 on `tm3`). The streaming cells' own K shares, which are newer than this line, are faster
+  // all over this band at up to 48 rows (stream_split's shares at 40 / 48 rows of 5120 x 17408 14.4 / 15.1, 4096 x 17408 12.8 / 13.3, 3072 x 20480
+  // 12.9 / 13.6, on tiles 18.3 / 18.4, 18.0 / 18.0, 19.5 / 19.6): below K = 16,384 they are what the law takes, the line itself has not moved.
   const PfVariant *split_cell = nullptr;
   const uint32_t tile_ks = pf_split(wkind == SABER_IU8_W8, m, n, k, &split_cell);
   const bool narrow = n <= 16 * CU_COUNT, two_wide = !narrow && n <= 32 * CU_COUNT;  // a 16- / 32-column block a CU

@@ -616,8 +616,8 @@ int saber_iu8_static_workspace_reset(saber_iu8_ctx *ctx, void *stream) {
 
 uint64_t saber_iu8_static_workspace_bytes(void) { return STATIC_WS_BYTES; }
 
-// Two W4 linears on one activation operand in one dispatch (decode band; the launch law's own
-// descriptors, which do not split K, so no workspace is bound).
+// Two W4 linears on one activation operand in one dispatch (decode band): the launch law's own
+// descriptors, a streamed half that shares K in one piece, so no workspace is bound.
 int saber_iu8_gemm_pair(saber_iu8_ctx *ctx, const void *a, const float *as, const void *w, const float *ws, void *c, uint32_t n,
                         const void *w_b, const float *ws_b, void *c_b, uint32_t n_b, uint32_t m, uint32_t k, void *stream) {
   saber_iu8_desc d0, d1, d;
@@ -712,7 +712,7 @@ int saber_iu8_silu_mul_quant_had_lut(saber_iu8_ctx *ctx, const void *gu, void *q
 int saber_iu8_add_rms_quant_had(saber_iu8_ctx *ctx, const void *y, const void *res, const void *w, void *q, float *scale,
                                 void *res_out, uint32_t m, uint32_t k, float eps, const float *had_t, void *stream) {
   saber_iu8_desc d;
-  // the 16-wave form carries the 256-thread form's sum order (a chain handed through LDS): one group a thread, K <= 8192
+  // the 16-wave form carries the 256-thread form's sum order (its chains run from LDS): one group a thread, K <= 8192
   if (int rc = had_desc("add_rms_quant_had_i8", "add_rms_quant", m, k, &d, k <= 8192)) return rc;
   set_i32(&d, "k", k);
   set_f32(&d, "eps", eps);
