@@ -17,7 +17,7 @@
       iu8_stream_cells<TM, W8, NT, KW, D, ACC>(a, w, as, ws, decode_partial, decode_counter, c, m, n, k,            \
                                                iu8_blk_of_grid(), (int)gridDim.x);                                  \
     } else {                                                                                                       \
-      iu8_dec_body<TM, W8, NT, KW, WPB, D, ALDS, ACC>(a, w, as, ws, decode_partial, decode_counter, c,              \
+      iu8_dec_body<W8, NT, KW, WPB, D, ALDS, ACC>(a, w, as, ws, decode_partial, decode_counter, c,              \
                                                       iu8_rows{nullptr, 0, m}, n, k);                               \
     }                                                                                                              \
   }

@@ -46,16 +46,15 @@ static __device__ __forceinline__ iu8_blk iu8_blk_of_grid() {
 // EXACT (the staged forms): the first ring issued by every wave and the last steps as straight-line code, so that
 // the compiler counts the loads in flight at each consume (see the streamed form's ring below). It costs registers:
 // the grouped launches, held to 64 a lane for eight waves a SIMD, keep the plain loops.
-template <int TM, bool W8, int NT, int KW, int WPB, int D, int ALDS, bool ACC, int MODE = 0, bool EXACT = true>
+template <bool W8, int NT, int KW, int WPB, int D, int ALDS, bool ACC, int MODE = 0, bool EXACT = true>
 __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const iu8_u8 *__restrict__ W,
                                              const float *__restrict__ as, const float *__restrict__ ws,
                                              int *__restrict__ P, int *__restrict__ cnt, void *__restrict__ Cv,
                                              const iu8_rows R, int N, int K, const iu8_blk B = iu8_blk_of_grid()) {
   const int M = R.rows;
   static_assert(WPB % KW == 0, "k-waves divide the workgroup");
-  static_assert(ALDS == 0 || TM == 1, "LDS staging of A is the M <= 16 form");
   constexpr bool PAIR = MODE == 1, AQ = MODE == 2;
-  static_assert(!PAIR || (NT % 2 == 0 && TM == 1 && !W8 && !ACC), "the paired form: gate tiles and their up tiles a wave");
+  static_assert(!PAIR || (NT % 2 == 0 && !W8 && !ACC), "the paired form: gate tiles and their up tiles a wave");
   constexpr int NP = PAIR ? NT / 2 : 1;  // tiles of p a wave (paired: tiles [0, NP) are gate tiles, [NP, NT) their up tiles)
   static_assert(!AQ || (ALDS > 0 && !ACC), "rows quantised here are staged in LDS");
   constexpr int WN = WPB / KW;
@@ -63,7 +62,7 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
   constexpr int WSTEP = W8 ? 2048 : 1024;  // bytes of one 16-row weight tile per 128-deep K step
   constexpr int WV = W8 ? 2 : 1;           // 16-byte loads a lane per step per tile
   constexpr int BN = WN * NT * 16;         // columns a workgroup
-  constexpr int RED = (KW > 1 ? KW - 1 : 1) * WN * TM * NT * 1024;
+  constexpr int RED = (KW > 1 ? KW - 1 : 1) * WN * NT * 1024;
   constexpr int ABYTES = ALDS * 1024;
   // one LDS block: the staged activation rows, re-used for the k-waves' partials at the end
   __shared__ __attribute__((aligned(16))) iu8_u8 s_mem[ABYTES > RED ? ABYTES : RED];
@@ -91,11 +90,9 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
     wp[j] = W + ((size_t)ntj * steps + (EXACT && ALDS > 0 ? min(s_lo + wk, steps - 1) : s_lo + wk)) * WSTEP + lane * 16;
   }
 
-  iu8_v4i acc[TM][NT];
+  iu8_v4i acc[NT];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = iu8_v4i{0, 0, 0, 0};
+  for (int j = 0; j < NT; ++j) acc[j] = iu8_v4i{0, 0, 0, 0};
 
   // ---- LDS staging of the live activation rows (issued before the weight ring, waited after it)
   // MR = staged rows (a power of two >= M); piece p = ((kt*4 + g)*MR + r) holds row r's 16 bytes
@@ -147,18 +144,14 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
 
   // ---- the weight ring
   iu8_v4u ring[D][NT][WV];
-  iu8_v4i ringa[ALDS ? 1 : D][TM][2];  // direct-from-L2 activation operands when not staged
-  // this lane's row of every activation tile, at the wave's first K step. A lane past the live rows reads the
+  iu8_v4i ringa[ALDS ? 1 : D][2];  // direct-from-L2 activation operands when not staged
+  // this lane's row of the activation tile, at the wave's first K step. A lane past the live rows reads the
   // last live row again (the piece a live lane of the same load already touches: no line more from L2), and
   // what it multiplies lands in output rows that are never stored. The loads are unconditional on purpose:
   // under a per-lane test the compiler cannot count them and waits for every load in flight (`vmcnt(0)`) at
   // each consume, which makes a ring of any depth a ring of one.
-  const iu8_u8 *ap[TM];
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int ar = iu8_arow(R, min(i * 16 + ml, M - 1));
-    ap[i] = A + ((size_t)(ar >> 4) * ktiles + (size_t)(s_lo + wk) * 2) * 1024 + ((ar & 15) + 16 * lg) * 16;
-  }
+  const int arow = iu8_arow(R, min(ml, M - 1));
+  const iu8_u8 *ap = A + ((size_t)(arow >> 4) * ktiles + (size_t)(s_lo + wk) * 2) * 1024 + ((arow & 15) + 16 * lg) * 16;
   auto issue = [&](int slot, int t) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
@@ -166,10 +159,7 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
       for (int v = 0; v < WV; ++v) ring[slot][j][v] = iu8_ldg_nt(wp[j] + (size_t)t * (KW * WSTEP) + v * 1024);
     if (!staged) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          ringa[ALDS ? 0 : slot][i][h] = *(const iu8_v4i *)(ap[i] + ((size_t)t * (2 * KW) + h) * 1024);
+      for (int h = 0; h < 2; ++h) ringa[ALDS ? 0 : slot][h] = *(const iu8_v4i *)(ap + ((size_t)t * (2 * KW) + h) * 1024);
     }
   };
   auto issue_w = [&](int slot, int t) {  // the staged ring: weights alone, no run-time test around a load
@@ -180,17 +170,14 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
   };
   const int a_lane = (((lg << mr_shift) + min(ml, (1 << mr_shift) - 1)) << 4);
   auto consume = [&](int slot, int t) {
-    iu8_v4i a0[TM], a1[TM];
+    iu8_v4i a0, a1;
     if (ALDS > 0 && staged) {
       const int kt = 2 * (wk + t * KW);
-      a0[0] = *(const iu8_v4i *)&s_mem[((kt * 4) << (mr_shift + 4)) + a_lane];
-      a1[0] = *(const iu8_v4i *)&s_mem[(((kt + 1) * 4) << (mr_shift + 4)) + a_lane];
+      a0 = *(const iu8_v4i *)&s_mem[((kt * 4) << (mr_shift + 4)) + a_lane];
+      a1 = *(const iu8_v4i *)&s_mem[(((kt + 1) * 4) << (mr_shift + 4)) + a_lane];
     } else {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        a0[i] = ringa[ALDS ? 0 : slot][i][0];
-        a1[i] = ringa[ALDS ? 0 : slot][i][1];
-      }
+      a0 = ringa[ALDS ? 0 : slot][0];
+      a1 = ringa[ALDS ? 0 : slot][1];
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
@@ -201,11 +188,8 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
       } else {
         iu8_unpack_w4(ring[slot][j][0], w0, w1);
       }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        acc[i][j] = iu8_mfma(w0, a0[i], acc[i][j]);
-        acc[i][j] = iu8_mfma(w1, a1[i], acc[i][j]);
-      }
+      acc[j] = iu8_mfma(w0, a0, acc[j]);
+      acc[j] = iu8_mfma(w1, a1, acc[j]);
     }
   };
 
@@ -372,20 +356,14 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
   if constexpr (KW > 1) {
     if (wk > 0) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-          *(iu8_v4i *)&s_red[((((wk - 1) * WN + wn) * TM + i) * NT + j) * 256 + lane * 4] = acc[i][j];
+      for (int j = 0; j < NT; ++j) *(iu8_v4i *)&s_red[(((wk - 1) * WN + wn) * NT + j) * 256 + lane * 4] = acc[j];
     }
     __syncthreads();
     if (wk == 0) {
 #pragma unroll
       for (int q = 0; q < KW - 1; ++q)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-            acc[i][j] += *(const iu8_v4i *)&s_red[(((q * WN + wn) * TM + i) * NT + j) * 256 + lane * 4];
+        for (int j = 0; j < NT; ++j) acc[j] += *(const iu8_v4i *)&s_red[((q * WN + wn) * NT + j) * 256 + lane * 4];
     }
   }
 
@@ -403,8 +381,8 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
       unsigned h[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float g = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[0][jj][r], am, iu8_wsu<W8>(ws, n + r))));
-        const float u = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[0][NP + jj][r], am, iu8_wsu<W8>(ws, half + n + r))));
+        const float g = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[jj][r], am, iu8_wsu<W8>(ws, n + r))));
+        const float u = iu8_bf16_f32((unsigned short)iu8_bf16_bits(iu8_epi(acc[NP + jj][r], am, iu8_wsu<W8>(ws, half + n + r))));
         h[r] = iu8_bf16_bits(iu8_silu_bf16(g) * u);
       }
       *(iu8_v2u *)((unsigned short *)Cv + (size_t)(R.row0 + ml) * half + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
@@ -420,20 +398,16 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
       float wsu[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) wsu[r] = iu8_wsu<W8>(ws, n + r);
+      if (ml >= M) continue;
+      const size_t crow = (size_t)(R.row0 + ml) * N;
+      if constexpr (ACC) {
+        *(iu8_v4i *)((int *)Cv + crow + n) = acc[j];
+      } else {
+        const float am = AQ ? s_rsc[ml] : as[iu8_arow(R, ml)];
+        unsigned h[4];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = i * 16 + ml;
-        if (m >= M) continue;
-        const size_t crow = (size_t)(R.row0 + m) * N;
-        if constexpr (ACC) {
-          *(iu8_v4i *)((int *)Cv + crow + n) = acc[i][j];
-        } else {
-          const float am = AQ ? s_rsc[m] : as[iu8_arow(R, m)];
-          unsigned h[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(acc[i][j][r], am, wsu[r]));
-          *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-        }
+        for (int r = 0; r < 4; ++r) h[r] = iu8_bf16_bits(iu8_epi(acc[j][r], am, wsu[r]));
+        *(iu8_v2u *)((unsigned short *)Cv + crow + n) = iu8_v2u{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
       }
     }
     return;
@@ -446,11 +420,7 @@ __device__ __forceinline__ void iu8_dec_body(const iu8_u8 *__restrict__ A, const
     for (int j = 0; j < NT; ++j) {
       if (nt0 + j >= ntiles) continue;
       const int n = (nt0 + j) * 16 + nq;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = i * 16 + ml;
-        if (m < M) iu8_store_through(&P[((size_t)z * M + m) * N + n], acc[i][j]);
-      }
+      if (ml < M) iu8_store_through(&P[((size_t)z * M + ml) * N + n], acc[j]);
     }
     iu8_stores_done();
   }

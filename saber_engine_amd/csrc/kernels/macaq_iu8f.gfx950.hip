@@ -31,7 +31,7 @@
       iu8_stream_cells<TM, false, NT, KW, D, false>(a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial, \
                                                    p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, m, p1 ? n_b : n, k, blk, nbp); \
     else                                                                                                            \
-      iu8_dec_body<TM, false, NT, KW, WPB, D, ALDS, false>(                                                         \
+      iu8_dec_body<false, NT, KW, WPB, D, ALDS, false>(                                                         \
           a, p1 ? w_b : w, as, p1 ? ws_b : ws, p1 ? decode_partial_b : decode_partial,                              \
           p1 ? decode_counter_b : decode_counter, p1 ? c_b : c, iu8_rows{nullptr, 0, m}, p1 ? n_b : n, k, blk);     \
   }
