@@ -25,7 +25,7 @@ struct iu8_stream_geo {
 // common head; which is faster differs by cell. us, loop / exact: W4 5 rows of 5120 x 5120 5.6 / 5.1, 20 rows 7.1 / 6.5, 64 rows of
 // 4096 x 4096 7.5 / 7.1, 45 rows of 34816 x 5120 22.0 / 21.3; W8 16 rows of 5120 x 6144 9.6 / 8.4; the other way W8 64 rows 12.6 / 12.9, W4
 // 72 rows of 20480 x 5120 21.4 / 22.7, W8 45 rows of 20480 x 5120 22.4 / 23.7.
-template <int TM, bool W8, int NT, int KW, int D, bool ACC, int LDSK, bool EXACT>
+template <int TM, bool W8, int NT, int KW, int D, bool ACC, int LDSK, bool EXACT, bool SHORT = false>
 __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const iu8_u8 *__restrict__ A, const iu8_u8 *__restrict__ W,
                                                 const float *__restrict__ as, const float *__restrict__ ws, int *__restrict__ P,
                                                 int *__restrict__ cnt, void *__restrict__ Cv, int M, int N, int K, const iu8_blk B) {
@@ -149,9 +149,10 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
 #pragma unroll
         for (int h = 0; h < 2; ++h) ringa[slot][i][h] = *(const iu8_v4i *)(ab + h * 1024 + ao[i]);
     };
-    // a wave without a step asks for nothing: the matrix's first fragment, read by every such wave of the grid, is one line of one
-    // channel (W8, 33 rows of 8192 x 256 / 384 / 640 4.8 / 5.0 / 5.5 -> 3.6 / 4.1 / 4.5 us)
-    if (T > 0) {
+    // SHORT, a symbol's own cell, which the law takes at any K: a wave without a step asks for nothing. The matrix's first fragment,
+    // read by every such wave of the grid, is one line of one channel (W8, 33 rows of 8192 x 256 / 384 / 640 4.8 / 5.0 / 5.5 -> 3.6 /
+    // 4.1 / 4.5 us). The wider cells start at a K that gives every wave a step.
+    if (!SHORT || T > 0) {
 #pragma unroll
       for (int i = 0; i < D; ++i) {
         issue(i, i);
@@ -294,5 +295,5 @@ __device__ __forceinline__ void iu8_stream_cells(const iu8_u8 *__restrict__ A, c
       return;
     }
   }
-  iu8_stream_body<TM, W8, NT, KW, D, ACC, LDSK, !(W8 && TM >= 3)>(lds, A, W, as, ws, P, cnt, Cv, M, N, K, B);
+  iu8_stream_body<TM, W8, NT, KW, D, ACC, LDSK, !(W8 && TM >= 3), true>(lds, A, W, as, ws, P, cnt, Cv, M, N, K, B);
 }
