@@ -1,5 +1,5 @@
 // The parity suite's taps: the code object `iu8_taps`. Test infrastructure, not part of the plugin
-// set a host loads: it is built beside the plugin directory (in `taps/`) and a checker adds it to a
+// set a host loads: it is built beside the plugin directory (in `taps/`) and a test adds it to a
 // context by its manifest.
 //
 //   macaq_iu8_dec_{w4,w8}_tm1_acc, macaq_iu8_dec_w4_tm4_acc, macaq_iu8_pf_{w4,w8}_acc

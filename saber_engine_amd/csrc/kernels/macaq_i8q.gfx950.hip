@@ -20,7 +20,7 @@
 //                                 a wave a row, four rows a workgroup (grid M/4, block 256)
 //   macaq_i8_silu_mul_quant_lut_w64   the second with the bf16 silu read from a 65,536-entry table in
 //                                 LDS: persistent, 16 waves, a wave a row (grid <= 256, block 1024)
-//   macaq_silu_bf16_table         the bf16 silu of all 65,536 bf16 inputs (a checker's tap)
+//   macaq_silu_bf16_table         the bf16 silu of all 65,536 bf16 inputs (a test's tap)
 //
 // One workgroup a row; a thread owns 16-element groups g = tid + i*256 (one 16-byte store each).
 // A kernel holds its row in registers, so each comes in forms for rows of up to 4,096 (_g1), 8,192

@@ -21,7 +21,7 @@
 // ulp off now and then, which showed as a bf16 value of a row flipped once in a few million elements). gdn_norm's
 // gate silu_f32(z) = z / (1 + expf(-z)) stays in f32 and so carries the device's expf: a function of
 // a bf16 input, it is tabled by a tap kernel of the test-only object `iu8_taps` (had_silu_f32 lives
-// in iu8_had.h for both) for a checker to hold against a host's.
+// in iu8_had.h for both) for a test to hold against a host's.
 #include "iu8_had.h"
 
 template <int T>

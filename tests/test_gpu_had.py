@@ -140,7 +140,7 @@ def test_add_rms_quant_had_rows_of_many_magnitudes(ctx, M, K):
 
 
 def tap(ctx, kernel, plugin, dtype):
-    """A checker's tap kernel: one value for each of the 65,536 bf16 inputs."""
+    """A test's tap kernel: one value for each of the 65,536 bf16 inputs."""
     out = torch.zeros(65536, dtype=dtype, device="cuda")
     ctx.launch(iu8.describe_raw(kernel, (256, 1, 1), 256, plugin=plugin), dict(out=out.data_ptr()))
     torch.cuda.synchronize()
