@@ -122,7 +122,7 @@ uint32_t pack(const Signature &sig, std::vector<std::pair<uint32_t, uint32_t>> &
   out.clear();
   uint32_t off = 0;
   for (const SigArg &a : sig) {
-    off = (off + a.align() - 1) / a.align() * a.align();
+    off = pack_at(a, off);
     out.emplace_back(off, a.size());
     off += a.size();
   }

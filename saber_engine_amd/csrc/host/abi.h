@@ -23,6 +23,8 @@ using Signature = std::vector<SigArg>;
 // The declared signature of a kernel symbol of the gfx950 objects, or nullptr.
 const Signature *signature_for(const std::string &kernel);
 
+// Where an argument goes in the kernarg block that holds `off` bytes so far: natural alignment.
+inline uint32_t pack_at(const SigArg &a, uint32_t off) { return (off + a.align() - 1) / a.align() * a.align(); }
 // (offset, size) per argument by natural alignment; returns the explicit kernarg bytes.
 uint32_t pack(const Signature &sig, std::vector<std::pair<uint32_t, uint32_t>> &out);
 

@@ -1,5 +1,6 @@
 #include "rules.h"
 
+#include <array>
 #include <cmath>
 #include <cstring>
 
@@ -49,28 +50,25 @@ const PfVariant *pf_variant(const std::string &name) {
   return nullptr;
 }
 
-static void copy_name(char *dst, size_t cap, const std::string &s) {
-  snprintf(dst, cap, "%s", s.c_str());
-}
-
 int fill_slots(const std::string &kernel, saber_iu8_desc *d) {
   const Signature *sig = signature_for(kernel);
   if (!sig) return fail(SABER_IU8_E_RULE, kernel + ": no declared signature");
-  std::vector<std::pair<uint32_t, uint32_t>> packed;
-  d->kernarg_bytes = pack(*sig, packed);
   if (sig->size() > sizeof(d->args) / sizeof(d->args[0])) return fail(SABER_IU8_E_RULE, kernel + ": too many arguments");
   d->n_args = (uint32_t)sig->size();
+  uint32_t off = 0;
   for (size_t i = 0; i < sig->size(); ++i) {
     saber_iu8_slot &s = d->args[i];
     memset(&s, 0, sizeof s);
     copy_name(s.name, sizeof s.name, (*sig)[i].name);
-    s.offset = packed[i].first;
-    s.size = packed[i].second;
+    s.offset = off = pack_at((*sig)[i], off);
+    s.size = (*sig)[i].size();
+    off += s.size;
     s.kind = (*sig)[i].kind == ArgKind::Buffer ? SABER_IU8_ARG_BUFFER
              : (*sig)[i].kind == ArgKind::F32  ? SABER_IU8_ARG_F32
              : (*sig)[i].kind == ArgKind::I64  ? SABER_IU8_ARG_I64
                                                : SABER_IU8_ARG_I32;
   }
+  d->kernarg_bytes = off;
   return 0;
 }
 
@@ -625,13 +623,23 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
   static const Law W8 = {4.419, 75.175, 18.116, 1.782, 5.234, 1.935,
                          {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t256x224", 11.270, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}}};
   const Law &law = w8 ? W8 : W4;
+  // the cells' variants, looked up once
+  constexpr size_t NCELL = sizeof(Law::cells) / sizeof(Cell);
+  using Variants = std::array<const PfVariant *, NCELL>;
+  auto variants = [](const Law &l, const char *tag) {
+    Variants v;
+    for (size_t i = 0; i < NCELL; ++i) v[i] = pf_variant(fmt("macaq_iu8_pf_%s_%s", tag, l.cells[i].tile));
+    return v;
+  };
+  static const Variants V4 = variants(W4, "w4"), V8 = variants(W8, "w8");
   double quarter_rate = 0;
   for (const auto &c : law.cells)
     if (!strcmp(c.tile, "t128x128")) quarter_rate = c.tops_per_cu;
   const PfVariant *best = nullptr;
   double best_t = 0;
-  for (const auto &c : law.cells) {
-    const PfVariant *v = pf_variant(fmt("macaq_iu8_pf_%s_%s", w8 ? "w8" : "w4", c.tile));
+  for (size_t i = 0; i < NCELL; ++i) {
+    const Cell &c = law.cells[i];
+    const PfVariant *v = (w8 ? V8 : V4)[i];
     if (!v) continue;
     const double bm = v->block_m(), bn = v->block_n();
     const uint64_t tiles = (uint64_t)((n + v->block_n() - 1) / v->block_n()) * ((m + v->block_m() - 1) / v->block_m());

@@ -28,7 +28,7 @@ struct saber_iu8_ctx {
   int device = 0;
   std::string arch;
   std::vector<hipModule_t> modules;
-  std::map<std::string, LoadedKernel> fn;
+  std::map<std::string, LoadedKernel, std::less<>> fn;  // (found by a name in place, without a string of its own)
   saber_iu8_counters counters{};
   std::string static_ws_error;  // why this device has no static workspace (empty: it has one)
 };
@@ -159,9 +159,9 @@ int saber_iu8_describe_raw(const char *kernel, const char *plugin, const uint32_
   if (!kernel || !grid || !out) return fail(SABER_IU8_E_ARG, "describe_raw: null argument");
   if (!grid[0] || !grid[1] || !grid[2] || !block || block > 1024) return fail(SABER_IU8_E_RULE, std::string(kernel) + ": empty or oversized launch");
   memset(out, 0, sizeof *out);
-  snprintf(out->op, sizeof out->op, "raw");
-  snprintf(out->plugin, sizeof out->plugin, "%s", plugin ? plugin : "");
-  snprintf(out->kernel, sizeof out->kernel, "%s", kernel);
+  copy_name(out->op, sizeof out->op, "raw");
+  copy_name(out->plugin, sizeof out->plugin, plugin ? plugin : "");
+  copy_name(out->kernel, sizeof out->kernel, kernel);
   for (int i = 0; i < 3; ++i) out->grid[i] = grid[i];
   out->block[0] = block, out->block[1] = 1, out->block[2] = 1;
   out->n_launches = 1;
@@ -346,7 +346,7 @@ int saber_iu8_get_counters(const saber_iu8_ctx *ctx, saber_iu8_counters *out) {
 }
 
 int saber_iu8_has_kernel(const saber_iu8_ctx *ctx, const char *kernel) {
-  return ctx && kernel && ctx->fn.count(kernel) ? 1 : 0;
+  return ctx && kernel && ctx->fn.count(std::string_view(kernel)) ? 1 : 0;
 }
 
 // What a hand-edited descriptor could get wrong for a kernel whose bounds depend on its grid: the
@@ -455,7 +455,7 @@ int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu
     const bool b0 = bound("decode_partial", "decode_counter"), b1 = bound("decode_partial_b", "decode_counter_b");
     if (((i32_arg(d, "ks") > 1 && !b0) || (i32_arg(d, "ks_b") > 1 && !b1)) && unsplit_pair(*d, b0, b1, &whole)) d = &whole;
   }
-  auto it = ctx->fn.find(d->kernel);
+  const auto it = ctx->fn.find(std::string_view(d->kernel));
   if (it == ctx->fn.end()) return fail(SABER_IU8_E_NOTLOADED, std::string(d->kernel) + ": not in the loaded plugin set");
   if (d->shared_bytes != 0) return fail(SABER_IU8_E_RULE, std::string(d->kernel) + ": dynamic LDS is not part of this ABI");
   if (!d->grid[0] || !d->grid[1] || !d->grid[2] || !d->block[0]) return fail(SABER_IU8_E_RULE, std::string(d->kernel) + ": empty grid");
@@ -666,7 +666,7 @@ static int had_desc(const char *op, const char *stem, uint32_t rows, uint32_t wi
   const std::string name = wide ? fmt("%s_hadi8_t1024", stem) : fmt("%s_hadi8_t%u_tiled1", stem, t);
   const uint32_t grid[3] = {rows, 1, 1};
   if (int rc = saber_iu8_describe_raw(name.c_str(), "mxfp4_hadi8", grid, t, d)) return rc;
-  snprintf(d->op, sizeof d->op, "%s", op);
+  copy_name(d->op, sizeof d->op, op);
   return 0;
 }
 static void set_f32(saber_iu8_desc *d, const char *name, float v) {
@@ -703,7 +703,7 @@ int saber_iu8_silu_mul_quant_had_lut(saber_iu8_ctx *ctx, const void *gu, void *q
   const std::string name = fmt("silu_mul_quant_hadi8_lut_t%u", d.block[0]);
   const uint32_t grid[3] = {m, 1, 1};
   if (int rc = saber_iu8_describe_raw(name.c_str(), "mxfp4_hadi8", grid, d.block[0], &d)) return rc;
-  snprintf(d.op, sizeof d.op, "silu_mul_quant_had_i8");
+  copy_name(d.op, sizeof d.op, "silu_mul_quant_had_i8");
   set_i32(&d, "n", n);
   const saber_iu8_binding b[] = {{"gu", (void *)gu}, {"q", q}, {"scale", scale}, {"had_t", (void *)had_t}, {"lut", (void *)silu_lut}};
   return saber_iu8_launch(ctx, &d, b, 5, stream);
@@ -733,7 +733,7 @@ int saber_iu8_gdn_norm_quant_had(saber_iu8_ctx *ctx, const void *x, const void *
   const uint32_t grid[3] = {m, 1, 1};
   const bool wide = had_t1024(m, n);  // a head's sum is its 16 lanes' whatever the workgroup's size
   if (int rc = saber_iu8_describe_raw(wide ? "gdn_norm_quant_hadi8_t1024" : "gdn_norm_quant_hadi8_t256_tiled1", "mxfp4_hadi8", grid, wide ? 1024 : 256, &d)) return rc;
-  snprintf(d.op, sizeof d.op, "gdn_norm_quant_had_i8");
+  copy_name(d.op, sizeof d.op, "gdn_norm_quant_had_i8");
   set_i32(&d, "n", n);
   set_i32(&d, "zs", z_stride);
   set_f32(&d, "eps", eps);
@@ -758,7 +758,7 @@ static int attn_gate_launch(saber_iu8_ctx *ctx, const void *core, const void *ga
   const char *name = wide ? (lut ? "attn_gate_quant_hadi8_lut_t1024" : "attn_gate_quant_hadi8_t1024")
                           : (lut ? "attn_gate_quant_hadi8_lut_t256" : "attn_gate_quant_hadi8_t256_tiled1");
   if (int rc = saber_iu8_describe_raw(name, "attn_glue_hadi8", grid, wide ? 1024 : 256, &d)) return rc;
-  snprintf(d.op, sizeof d.op, "attn_gate_quant_had_i8");
+  copy_name(d.op, sizeof d.op, "attn_gate_quant_had_i8");
   set_i32(&d, "n", n);
   set_i32(&d, "hd", head_dim);
   set_i32(&d, "gs", gate_stride);

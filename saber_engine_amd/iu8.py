@@ -168,7 +168,7 @@ def lib():
 
 
 def _check(rc):
-    if rc != 0:
+    if rc:
         raise IU8Error(rc, lib().saber_iu8_last_error().decode())
 
 
@@ -368,17 +368,48 @@ def manifest_validate(path, arch="gfx950"):
 
 # ---------------------------------------------------------------------------- device side
 
+_ops = None
+
+
+class _CtypesOperators:
+    """The operators through ctypes alone, for an interpreter that `_fastcall` was not built for."""
+
+    def __getattr__(self, name):
+        return getattr(lib(), "saber_iu8_" + name)
+
+
+def operators():
+    """The operator entry points by name: `_fastcall`'s (csrc/python/fastcall.cpp), which take ints and None as they are and
+    give everything else to the ctypes function, else the ctypes functions."""
+    global _ops
+    if _ops is None:
+        L = lib()  # first: _fastcall links to the same library
+        try:
+            from . import _fastcall
+        except ImportError:
+            _ops = _CtypesOperators()
+            return _ops
+        _fastcall.bind({n: getattr(L, "saber_iu8_" + n) for n in dir(_fastcall) if not n.startswith("_") and n != "bind"})
+        _ops = _fastcall
+    return _ops
+
+
+def _tables(t):
+    return C.addressof(t) if type(t) is MoeTables else C.byref(t)
+
+
 class Context:
     """A loaded plugin set on one device (PluginSet + Launcher)."""
 
     def __init__(self, prebuilt_dir=PREBUILT, device=0):
         self._h = C.c_void_p()
         _check(lib().saber_iu8_open(prebuilt_dir.encode(), device, C.byref(self._h)))
+        self._op, self._addr = operators(), self._h.value
 
     def close(self):
         if self._h:
             lib().saber_iu8_close(self._h)
-            self._h = C.c_void_p()
+            self._h, self._addr = C.c_void_p(), None
 
     def __del__(self):
         try:
@@ -405,26 +436,26 @@ class Context:
         _check(lib().saber_iu8_launch(self._h, C.byref(desc), _bindings(bufs), len(bufs), stream))
 
     def quant(self, x, q, scale, m, k, stream=0):
-        _check(lib().saber_iu8_quant(self._h, x, q, scale, m, k, stream))
+        _check(self._op.quant(self._addr, x, q, scale, m, k, stream))
 
     def quant_rowmajor(self, x, q, scale, m, k, stream=0):
-        _check(lib().saber_iu8_quant_rowmajor(self._h, x, q, scale, m, k, stream))
+        _check(self._op.quant_rowmajor(self._addr, x, q, scale, m, k, stream))
 
     def gemm(self, wkind, a, a_scale, w, w_scale, c, m, n, k, partial=None, counter=None, stream=0):
-        _check(lib().saber_iu8_gemm(self._h, wkind, a, a_scale, w, w_scale, c, m, n, k, partial, counter, stream))
+        _check(self._op.gemm(self._addr, wkind, a, a_scale, w, w_scale, c, m, n, k, partial, counter, stream))
 
     def gate_up_act(self, a, a_scale, w_gu, ws_gu, gu, p, m, hidden, inter, stream=0):
-        _check(lib().saber_iu8_gate_up_act(self._h, a, a_scale, w_gu, ws_gu, gu, p, m, hidden, inter, stream))
+        _check(self._op.gate_up_act(self._addr, a, a_scale, w_gu, ws_gu, gu, p, m, hidden, inter, stream))
 
     def rowscale(self, x, scale, m, k, stream=0):
-        _check(lib().saber_iu8_rowscale(self._h, x, scale, m, k, stream))
+        _check(self._op.rowscale(self._addr, x, scale, m, k, stream))
 
     def linear_prefill_fused(self, wkind, x, a_scale, w, w_scale, c, m, n, k, stream=0):
-        _check(lib().saber_iu8_linear_prefill_fused(self._h, wkind, x, a_scale, w, w_scale, c, m, n, k, stream))
+        _check(self._op.linear_prefill_fused(self._addr, wkind, x, a_scale, w, w_scale, c, m, n, k, stream))
 
     def gemm_static(self, wkind, a, a_scale, w, w_scale, c, m, n, k, stream=0):
         """gemm() with the split-K workspaces in the library's static device array: allocates nothing."""
-        _check(lib().saber_iu8_gemm_static(self._h, wkind, a, a_scale, w, w_scale, c, m, n, k, stream))
+        _check(self._op.gemm_static(self._addr, wkind, a, a_scale, w, w_scale, c, m, n, k, stream))
 
     def static_workspace_reset(self, stream=0):
         """The static array's arrival counters back to zero (a fill kernel on `stream`): recovery after a split
@@ -432,37 +463,37 @@ class Context:
         _check(lib().saber_iu8_static_workspace_reset(self._h, stream))
 
     def gemm_pair(self, a, a_scale, w, w_scale, c, n, w_b, w_scale_b, c_b, n_b, m, k, stream=0):
-        _check(lib().saber_iu8_gemm_pair(self._h, a, a_scale, w, w_scale, c, n, w_b, w_scale_b, c_b, n_b, m, k, stream))
+        _check(self._op.gemm_pair(self._addr, a, a_scale, w, w_scale, c, n, w_b, w_scale_b, c_b, n_b, m, k, stream))
 
     def linear_fused(self, wkind, x, w, w_scale, c, m, n, k, q=None, scale=None, stream=0):
-        _check(lib().saber_iu8_linear_fused(self._h, wkind, x, w, w_scale, c, q, scale, m, n, k, stream))
+        _check(self._op.linear_fused(self._addr, wkind, x, w, w_scale, c, q, scale, m, n, k, stream))
 
     def mlp_chain(self, x, w_gu, ws_gu, w_dn, ws_dn, gu, p, state, c, m, hidden, inter, spin=0, stream=0):
         """gate+up -> SiLU * up + requant -> down in one persistent launch; `state` (MLP_CHAIN_STATE_BYTES)
         zero before the first use. A non-zero word at state + MLP_CHAIN_STATUS_OFFSET after the launch:
         a meeting timed out, c is undefined."""
-        _check(lib().saber_iu8_mlp_chain(self._h, x, w_gu, ws_gu, w_dn, ws_dn, gu, p, state, c, m, hidden, inter, spin, stream))
+        _check(self._op.mlp_chain(self._addr, x, w_gu, ws_gu, w_dn, ws_dn, gu, p, state, c, m, hidden, inter, spin, stream))
 
     def quant_had(self, x, q, scale, m, k, had_t, stream=0):
-        _check(lib().saber_iu8_quant_had(self._h, x, q, scale, m, k, had_t, stream))
+        _check(self._op.quant_had(self._addr, x, q, scale, m, k, had_t, stream))
 
     def silu_mul_quant_had(self, gu, q, scale, m, n, had_t, stream=0):
-        _check(lib().saber_iu8_silu_mul_quant_had(self._h, gu, q, scale, m, n, had_t, stream))
+        _check(self._op.silu_mul_quant_had(self._addr, gu, q, scale, m, n, had_t, stream))
 
     def silu_mul_quant_had_lut(self, gu, q, scale, m, n, had_t, silu_lut, stream=0):
-        _check(lib().saber_iu8_silu_mul_quant_had_lut(self._h, gu, q, scale, m, n, had_t, silu_lut, stream))
+        _check(self._op.silu_mul_quant_had_lut(self._addr, gu, q, scale, m, n, had_t, silu_lut, stream))
 
     def add_rms_quant_had(self, y, res, w, q, scale, res_out, m, k, eps, had_t, stream=0):
-        _check(lib().saber_iu8_add_rms_quant_had(self._h, y, res, w, q, scale, res_out, m, k, eps, had_t, stream))
+        _check(self._op.add_rms_quant_had(self._addr, y, res, w, q, scale, res_out, m, k, eps, had_t, stream))
 
     def gdn_norm_quant_had(self, x, z, z_stride, w, q, scale, m, n, eps, had_t, stream=0):
-        _check(lib().saber_iu8_gdn_norm_quant_had(self._h, x, z, z_stride, w, q, scale, m, n, eps, had_t, stream))
+        _check(self._op.gdn_norm_quant_had(self._addr, x, z, z_stride, w, q, scale, m, n, eps, had_t, stream))
 
     def attn_gate_quant_had(self, core, gate, q, scale, m, n, head_dim, gate_stride, had_t, stream=0):
-        _check(lib().saber_iu8_attn_gate_quant_had(self._h, core, gate, q, scale, m, n, head_dim, gate_stride, had_t, stream))
+        _check(self._op.attn_gate_quant_had(self._addr, core, gate, q, scale, m, n, head_dim, gate_stride, had_t, stream))
 
     def attn_gate_quant_had_lut(self, core, gate, q, scale, m, n, head_dim, gate_stride, had_t, sigmoid_lut, stream=0):
-        _check(lib().saber_iu8_attn_gate_quant_had_lut(self._h, core, gate, q, scale, m, n, head_dim, gate_stride, had_t, sigmoid_lut, stream))
+        _check(self._op.attn_gate_quant_had_lut(self._addr, core, gate, q, scale, m, n, head_dim, gate_stride, had_t, sigmoid_lut, stream))
 
     def sigmoid_table(self, out, stream=0):
         _check(lib().saber_iu8_sigmoid_table(self._h, out, stream))
@@ -473,32 +504,32 @@ class Context:
 
     # ---- routed experts
     def moe_route(self, logits, tokens, experts, topk, tile_blocks, tables, stream=0):
-        _check(lib().saber_iu8_moe_route(self._h, logits, tokens, experts, topk, tile_blocks, C.byref(tables), stream))
+        _check(self._op.moe_route(self._addr, logits, tokens, experts, topk, tile_blocks, _tables(tables), stream))
 
     def moe_route_quant(self, logits, x, q, scale, tokens, experts, topk, k, tile_blocks, tables, stream=0):
-        _check(lib().saber_iu8_moe_route_quant(self._h, logits, x, q, scale, tokens, experts, topk, k, tile_blocks,
-                                               C.byref(tables), stream))
+        _check(self._op.moe_route_quant(self._addr, logits, x, q, scale, tokens, experts, topk, k, tile_blocks,
+                                               _tables(tables), stream))
 
     def moe_grouped(self, a, a_scale, xptr, c, n, k, gather, tokens, experts, topk, tile_blocks, tables, stream=0):
-        _check(lib().saber_iu8_moe_grouped(self._h, a, a_scale, xptr, c, n, k, int(gather), tokens, experts, topk,
-                                           tile_blocks, C.byref(tables), stream))
+        _check(self._op.moe_grouped(self._addr, a, a_scale, xptr, c, n, k, int(gather), tokens, experts, topk,
+                                           tile_blocks, _tables(tables), stream))
 
     def moe_gate_up_act(self, a, a_scale, xptr, p, inter, k, tokens, experts, topk, tile_blocks, tables, stream=0):
-        _check(lib().saber_iu8_moe_gate_up_act(self._h, a, a_scale, xptr, p, inter, k, tokens, experts, topk, tile_blocks,
-                                               C.byref(tables), stream))
+        _check(self._op.moe_gate_up_act(self._addr, a, a_scale, xptr, p, inter, k, tokens, experts, topk, tile_blocks,
+                                               _tables(tables), stream))
 
     def moe_down_rows(self, p, xptr, y, n, inter, tokens, experts, topk, tile_blocks, tables, stream=0):
-        _check(lib().saber_iu8_moe_down_rows(self._h, p, xptr, y, n, inter, tokens, experts, topk, tile_blocks,
-                                             C.byref(tables), stream))
+        _check(self._op.moe_down_rows(self._addr, p, xptr, y, n, inter, tokens, experts, topk, tile_blocks,
+                                             _tables(tables), stream))
 
     def moe_quant_rows(self, x, q, scale, k, rows_cap, tables, stream=0):
-        _check(lib().saber_iu8_moe_quant_rows(self._h, x, q, scale, k, rows_cap, C.byref(tables), stream))
+        _check(self._op.moe_quant_rows(self._addr, x, q, scale, k, rows_cap, _tables(tables), stream))
 
     def moe_silu_mul_quant(self, gu, q, scale, n, rows_cap, tables, stream=0):
-        _check(lib().saber_iu8_moe_silu_mul_quant(self._h, gu, q, scale, n, rows_cap, C.byref(tables), stream))
+        _check(self._op.moe_silu_mul_quant(self._addr, gu, q, scale, n, rows_cap, _tables(tables), stream))
 
     def moe_combine(self, y, tables, out, tokens, topk, h, stream=0):
-        _check(lib().saber_iu8_moe_combine(self._h, y, C.byref(tables), out, tokens, topk, h, stream))
+        _check(self._op.moe_combine(self._addr, y, _tables(tables), out, tokens, topk, h, stream))
 
     def silu_table(self, out, stream=0):
         _check(lib().saber_iu8_silu_table(self._h, out, stream))

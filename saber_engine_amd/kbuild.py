@@ -18,6 +18,7 @@ import hashlib
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -26,6 +27,7 @@ HOST = os.path.join(PKG, "csrc", "host")
 ARCH = "gfx950"
 PREBUILT = os.path.join(ROOT, "prebuilt", ARCH)
 LIB = os.path.join(PKG, "libsaber_iu8.so")
+FASTCALL = os.path.join(PKG, "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # -ffp-contract=off: every product and sum rounds where the source says (the epilogue contract);
@@ -84,7 +86,19 @@ def build_lib():
               "-packed-fp32-ops", inc, "-c", src, "-o", obj])
         objs.append(obj)
     _run([HIPCC, "-shared", "-fPIC", "-o", LIB] + objs)
+    build_fastcall(inc)
     return LIB
+
+
+def build_fastcall(inc):
+    """The operators' entry points for this interpreter without ctypes' conversions (iu8.py uses ctypes where it is not built:
+    an interpreter without its headers)."""
+    py = sysconfig.get_path("include")
+    if not os.path.exists(os.path.join(py, "Python.h")):
+        return None
+    _run([HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-fvisibility=hidden", "-I" + py, inc, "-shared", os.path.join(PKG, "csrc", "python", "fastcall.cpp"),
+          "-o", FASTCALL, "-L" + PKG, "-lsaber_iu8", "-Wl,-rpath,$ORIGIN"])
+    return FASTCALL
 
 
 def _lib():

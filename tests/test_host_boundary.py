@@ -663,6 +663,27 @@ def test_open_without_a_gpu_fails_loudly():
     assert e.value.code == iu8.E_HIP and "no CPU fallback" in str(e.value)
 
 
+def test_operator_entry_points_take_what_ctypes_takes():
+    """The binding's own entry points (csrc/python/fastcall.cpp): ints and None as they are, everything else -- ctypes objects,
+    other integer types, a wrong type or count -- as the ctypes function has it. Without a context every call is refused by
+    the library itself, before anything is launched."""
+    op, L = iu8.operators(), iu8.lib()
+    assert op.__name__.endswith("_fastcall")
+    args = (0, 1 << 40, 1 << 40, 1 << 40, 1 << 40, None, None, 1, 5120, 5120)
+    for a in ((None,) + args + (0,), (None,) + args + (None,), (ctypes.c_void_p(),) + args + (ctypes.c_void_p(0),), (None, True) + args[1:] + (0,),
+              (None,) + args[:-1] + (np.int64(5120), 0), (None,) + args[:-1] + ((1 << 32) + 5120, 0), (None, 7) + args[1:] + (0,),
+              (None,) + args[:-1] + (5121, 0)):
+        assert op.linear_fused(*a) == L.saber_iu8_linear_fused(*a) != 0, a
+    assert op.linear_fused(None, 0, -1, 1, 1, 1, None, None, 1, 5120, 5121, 0) == iu8.E_RULE and "5121" in L.saber_iu8_last_error().decode()
+    assert op.add_rms_quant_had(None, 1, 1, 1, 1, 1, 1, 4, 5120, 1e-6, 1, 0) == iu8.E_ARG
+    assert op.add_rms_quant_had(None, 1, 1, 1, 1, 1, 1, 4, 5120, 1, 1, 0) == iu8.E_ARG      # an int for a float: ctypes takes it
+    for bad in ((None,) + args[:-1] + (1.5, 0), (None,) + args[:-1] + ("5120", 0), (None,) + args):
+        with pytest.raises((ctypes.ArgumentError, TypeError)):
+            op.linear_fused(*bad)
+        with pytest.raises((ctypes.ArgumentError, TypeError)):
+            L.saber_iu8_linear_fused(*bad)
+
+
 # ------------------------------------------------------------------ operand orders
 
 def test_a_order_is_a_bijection_with_16_byte_lane_pieces():
