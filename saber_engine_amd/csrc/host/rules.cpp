@@ -16,8 +16,8 @@ static const DecVariant DEC_VARIANTS[] = {
 #include "../kernels/iu8_variants.def"
 };
 static const PfVariant PF_VARIANTS[] = {
-#define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) {#name, W8, WMW, WNW, TM, TN, ACC, OCC},
-#define IU8_PF_TAP(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) {#name, W8, WMW, WNW, TM, TN, ACC, OCC},
+#define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW) {#name, W8, WMW, WNW, TM, TN, ACC, OCC, KW},
+#define IU8_PF_TAP(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW) {#name, W8, WMW, WNW, TM, TN, ACC, OCC, KW},
 #include "../kernels/iu8_variants.def"
 };
 static const WideVariant WIDE_VARIANTS[] = {

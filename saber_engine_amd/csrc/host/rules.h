@@ -30,10 +30,10 @@ struct WideVariant {  // the streamed cell on the prefill kernarg list: one bloc
 };
 struct PfVariant {
   const char *name;
-  int w8, wmw, wnw, tm, tn, acc, occ;  // waves, 32 x 32 MFMA tiles a wave, workgroups a CU
+  int w8, wmw, wnw, tm, tn, acc, occ, kw;  // waves, 32 x 32 MFMA tiles a wave, workgroups a CU, k-waves a wave tile
   int block_m() const { return wmw * tm * 32; }
   int block_n() const { return wnw * tn * 32; }
-  int threads() const { return wmw * wnw * 64; }
+  int threads() const { return wmw * wnw * kw * 64; }
 };
 
 const DecVariant *dec_variant(const std::string &name);

@@ -41,9 +41,9 @@ static __device__ __forceinline__ int iu8_thin_tile_at(const iu8_pf_plan &p, int
 // 128 x 128 cell, which take 0.42 (one round) or 0.84 (two) of a big tile's time, and a few rows past the last whole 256 run as
 // thin tiles on a 128 x 256 cell whose waves skip row blocks without a row. Same bytes: every output element is one exact
 // integer sum and one epilogue, whichever cell computes it.
-#define IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP)                                                        \
-  extern "C" __global__ __launch_bounds__(WMW * WNW * 64)                                                         \
-      __attribute__((amdgpu_waves_per_eu(WMW * WNW * OCC / 4, WMW * WNW * OCC / 4))) void name(                    \
+#define IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW)                                                    \
+  extern "C" __global__ __launch_bounds__(WMW * WNW * KW * 64)                                                    \
+      __attribute__((amdgpu_waves_per_eu(WMW * WNW * KW * OCC / 4, WMW * WNW * KW * OCC / 4))) void name(          \
       const unsigned char *__restrict__ a, const unsigned char *__restrict__ w, const float *__restrict__ as,     \
       const float *__restrict__ ws, unsigned short *__restrict__ c, int m, int n, int k) {                         \
     constexpr int BM = WMW * TM * 32, BN = WNW * TN * 32;                                                          \
@@ -93,7 +93,7 @@ static __device__ __forceinline__ int iu8_thin_tile_at(const iu8_pf_plan &p, int
             nullptr, nullptr, lds);                                                                                \
       }                                                                                                            \
     } else {                                                                                                       \
-      iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP>(a, as, c, n, k, [&](int r, iu8_tile &t) {                  \
+      iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP, false, false, false, false, false, KW>(a, as, c, n, k, [&](int r, iu8_tile &t) { \
         int bx, by;                                                                                                \
         if (!iu8_dense_tile_at(r, gx, gy, bx, by)) return false;                                                   \
         t = iu8_tile{R, by * BM, bx * (BN / 16), w, ws, by * gx + bx};                                             \

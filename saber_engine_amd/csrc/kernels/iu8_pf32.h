@@ -24,6 +24,13 @@
 // for NST-1 steps ahead leave, the next step's operands are read from its stage and this step's
 // MFMAs run from registers filled a step ago.
 //
+// KW = 2 (two k-waves a wave tile). A wave tile is as wide as its accumulators' registers allow, a workgroup of such tiles has
+// four waves, one a SIMD, and nothing runs while that wave waits for LDS or unpacks; eight waves of half the tile read the
+// weights' fragments from LDS and unpack them twice as often. Here two waves hold the same tile and each multiplies two of a
+// step's four sub-steps: a wave reads half the step's operands and unpacks each of its weight pieces once, and a SIMD has two
+// waves. Their sums meet in LDS at the tile's end, each storing half of the row blocks (some 1 us a tile). Before / after:
+// iu8_variants.def.
+//
 // D[n][m]: src0 = weight operand (lane: row n = l%32), src1 = activation operand (lane: row
 // m = l%32); lane l, register e holds n = 8*(e/4) + 4*(l/32) + e%4, m = l%32.
 #pragma once
@@ -123,13 +130,13 @@ constexpr int iu8_pf32_lds_bytes() {
 // a fragment), turns them into codes by the law's own routine (iu8_code4_rcp: the bytes of the
 // producer kernel) one step later and writes the fragment into its stage; the weights keep their
 // LDS-DMA stream. One conversion a workgroup and step, whatever the columns of the tile.
-template <bool W8, int WMW, int WNW, int TM, int TN, bool ACC, int STMAX, bool DEEP = false, bool SPARSE = false, bool ARM = false, bool EXT_LDS = false, bool AQ = false, bool TAB = false, class TileAt>
+template <bool W8, int WMW, int WNW, int TM, int TN, bool ACC, int STMAX, bool DEEP = false, bool SPARSE = false, bool ARM = false, bool EXT_LDS = false, bool AQ = false, bool TAB = false, int KW = 1, class TileAt>
 __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const float *__restrict__ as,
                                              void *__restrict__ Cv, int N, int K, TileAt tile_at,
                                              int *__restrict__ P = nullptr, int *__restrict__ cnt = nullptr,
                                              iu8_u8 *ext_lds = nullptr, iu8_tabs tabs = {}) {
   // tile_at(r, t): fills the workgroup's r-th tile, false when it has none
-  constexpr int NWAVE = WMW * WNW;
+  constexpr int NWAVE = WMW * WNW * KW, TME = TM / KW;  // TME: row blocks a wave stores
   constexpr int BMT = WMW * TM * 2, BNT = WNW * TN * 2;  // 16-row tiles a workgroup, both ways
   constexpr int WSTEP = W8 ? 2048 : 1024;                // bytes of a 16-row weight tile per K step
   constexpr int A_BYTES = BMT * 2048, W_BYTES = BNT * WSTEP, STAGE = A_BYTES + W_BYTES;
@@ -146,6 +153,7 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
   static_assert((NST - 2) * (PER + (A_X > 0) + (W_X > 0)) <= 63, "the in-flight count fits s_waitcnt's vmcnt field");
   static_assert(!DEEP || NST >= 3, "the deep form reads a stage a step ahead of its MFMAs");
   static_assert(!(DEEP && SPARSE), "the sparse forms exist for the phased loop only");
+  static_assert(KW == 1 || (KW == 2 && TM % 2 == 0 && !DEEP && !SPARSE && !AQ && !TAB), "two k-waves a wave tile: phased loop, whole row blocks each");
   static_assert(!AQ || (!DEEP && !SPARSE && !ARM && A_FR % NWAVE == 0), "the fused-quant form: phased loop, whole A fragments a wave");
   // EXT_LDS: the stages live in the caller's LDS block (1-KiB aligned, iu8_pf32_lds_bytes of this cell),
   // for a kernel that runs two cells one after the other in the same memory
@@ -173,7 +181,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WNW, wn = wave % WNW;
+  const int kw = KW == 1 ? 0 : wave / (WMW * WNW), wt = KW == 1 ? wave : wave % (WMW * WNW);  // k-wave, wave tile
+  const int wm = wt / WNW, wn = wt % WNW;
   const int ntiles = N >> 4, ksteps = K >> 7, ktiles = K >> 6;
   // this workgroup's share of the K steps
   const int Z = P != nullptr ? (int)gridDim.z : 1, z = P != nullptr ? (int)blockIdx.z : 0;
@@ -353,10 +362,13 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
   // this lane's operand addresses inside a stage, at sub-step 0
   const int r32 = lane & 31, h = lane >> 5;
   // A: fragment (mt, kt2) at (mt*2 + kt2) KiB; piece (chunk*16 + row%16)
-  const int a_lane = (((wm * TM * 2 + (r32 >> 4)) * 2) * 64 + h * 16 + (r32 & 15)) * 16;
+  const int a_lane = (((wm * TM * 2 + (r32 >> 4)) * 2) * 64 + h * 16 + (r32 & 15)) * 16 + kw * 512;
+  // (two k-waves: a wave's first row blocks are those it stores, the rest the ones it hands over)
+  const int a_own = a_lane + kw * TME * 4096, a_give = a_lane + (1 - kw) * TME * 4096;
   // W4: fragment nt at nt KiB; W8: the A form
   const int w_lane = W8 ? (((wn * TN * 2 + (r32 >> 4)) * 2) * 64 + h * 16 + (r32 & 15)) * 16
                         : ((wn * TN * 2 + (r32 >> 4)) * 64 + h * 16 + (r32 & 15)) * 16;
+  const int w_at = w_lane + kw * 512;  // (k-wave kw: sub-steps 2 kw, 2 kw + 1)
 
   // ---- the pipelined K loop. A step is four phases (sub-steps) f = 2p + kt2. Nothing is consumed
   // in the phase that fetched it: a phase's MFMAs multiply A operands read from LDS one phase
@@ -373,18 +385,24 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
   using Full = std::integral_constant<int, TM>;
   auto fetch_a = [&](const iu8_u8 *sA, int buf, int p, int kt2, auto nl) {  // the first nl row blocks
 #pragma unroll
-    for (int i = 0; i < decltype(nl)::value; ++i) af[buf][i] = *(const iu8_v4i *)&sA[a_lane + i * 4096 + kt2 * 1024 + p * 512];
+    for (int i = 0; i < decltype(nl)::value; ++i) af[buf][i] = *(const iu8_v4i *)&sA[(KW == 1 ? a_lane + i * 4096 : i < TME ? a_own + i * 4096 : a_give + (i - TME) * 4096) + kt2 * 1024 + p * 512];
   };
   auto fetch_w8 = [&](const iu8_u8 *sW, int buf, int p, int kt2) {  // W8: a whole operand a phase
     if constexpr (W8) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) wf[buf][j] = *(const iu8_v4i *)&sW[w_lane + j * 4096 + kt2 * 1024 + p * 512];
+      for (int j = 0; j < TN; ++j) wf[buf][j] = *(const iu8_v4i *)&sW[w_at + j * 4096 + kt2 * 1024 + p * 512];
     }
   };
   auto fetch_w4 = [&](const iu8_u8 *sW, int p) {  // W4: the packed pieces of sub-steps 2p, 2p+1
     if constexpr (!W8) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) wpk[p][j] = *(const iu8_v4u *)&sW[w_lane + j * 2048 + p * 512];
+      for (int j = 0; j < TN; ++j) wpk[p][j] = *(const iu8_v4u *)&sW[w_at + j * 2048 + p * 512];
+    }
+  };
+  auto fetch_w4_set = [&](const iu8_u8 *sW, int set) {  // W4, a k-wave: the pieces of its two sub-steps
+    if constexpr (!W8) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) wpk[set][j] = *(const iu8_v4u *)&sW[w_at + j * 2048];
     }
   };
   auto mfmas = [&](int buf, int p, int kt2, auto nl) {
@@ -449,12 +467,12 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
         if constexpr (W8) {
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            wfd[set][2 * p + kt2][j] = *(const iu8_v4i *)&sW[w_lane + j * 4096 + kt2 * 1024 + p * 512];
+            wfd[set][2 * p + kt2][j] = *(const iu8_v4i *)&sW[w_at + j * 4096 + kt2 * 1024 + p * 512];
         }
       }
       if constexpr (!W8) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) wpd[set][p][j] = *(const iu8_v4u *)&sW[w_lane + j * 2048 + p * 512];
+        for (int j = 0; j < TN; ++j) wpd[set][p][j] = *(const iu8_v4u *)&sW[w_at + j * 2048 + p * 512];
       }
     }
   };
@@ -463,7 +481,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
   } else {
     fetch_a(smem, 0, 0, 0, Full{});
     fetch_w8(smem + A_BYTES, 0, 0, 0);
-    fetch_w4(smem + A_BYTES, 0);
+    if constexpr (KW == 1) fetch_w4(smem + A_BYTES, 0);
+    else fetch_w4_set(smem + A_BYTES, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -535,6 +554,73 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
 #pragma unroll
             for (int j = 0; j < TN; ++j) wpd[0][p][j] = wpd[1][p][j];
         }
+      }
+    } else if constexpr (KW == 2) {
+      // Two k-waves: a step's two phases are this wave's sub-steps (kt2 = 0, 1); the weights' pieces serve both, so the next
+      // step's go to the other register set.
+      auto kw_step = [&](int set) {
+        const int st1 = st == NST - 1 ? 0 : st + 1, stl = st == 0 ? NST - 1 : st - 1;
+        const iu8_u8 *sA = smem + st * STAGE, *sW = sA + A_BYTES;
+        const iu8_u8 *nA = smem + st1 * STAGE, *nW = nA + A_BYTES;
+        fetch_a(sA, 1, 0, 1, Full{});
+        fetch_w8(sW, 1, 0, 1);
+        issue(stl);
+        mfmas(0, set, 0, Full{});
+        IU8_PHASE_ORDER(TM + (W8 ? TN : 0), TM);
+        wait_step(true);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_a(nA, 0, 0, 0, Full{});
+        fetch_w8(nW, 0, 0, 0);
+        fetch_w4_set(nW, set ^ 1);
+        mfmas(1, set, 1, Full{});
+        IU8_PHASE_ORDER(TM + TN, TM);
+        advance();
+        st = st1;
+      };
+      int s = 0;
+      for (; s + 2 <= steps; s += 2) {
+        kw_step(0);
+        kw_step(1);
+      }
+      if (s < steps) {  // an odd step count: one more step, then the sets are renamed back
+        kw_step(0);
+        if constexpr (!W8) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) wpk[0][j] = wpk[1][j];
+        }
+      }
+      // The k-waves of a wave tile each hold a sum over half of K. They meet in the stage the last step drained: each hands
+      // over the row blocks that the other stores, JC column blocks at a time (int32: exact, in any order).
+      constexpr int JC = STAGE / (NWAVE * TME * 4096) < TN ? STAGE / (NWAVE * TME * 4096) : TN;
+      static_assert(JC >= 1, "a column block's sums fit the stage");
+      iu8_u8 *meet = smem + (st == 0 ? NST - 1 : st - 1) * STAGE + lane * 16;
+      const int other = wave + (kw ? -(WMW * WNW) : WMW * WNW);
+#pragma unroll
+      for (int j0 = 0; j0 < TN; j0 += JC) {
+        auto each = [&](auto f) {
+#pragma unroll
+          for (int jj = 0; jj < JC && j0 + jj < TN; ++jj)
+#pragma unroll
+            for (int i = 0; i < TME; ++i)
+#pragma unroll
+              for (int g = 0; g < 4; ++g) f(i, j0 + jj, g, ((jj * TME + i) * 4 + g) * 1024);
+        };
+        auto met = [&]() {
+          wait_vm(std::integral_constant<int, 63>{}, true);
+          __builtin_amdgcn_s_barrier();
+        };
+        each([&](int i, int j, int g, int at) {
+          const iu8_v16i &a = acc[TME + i][j];
+          *(iu8_v4i *)&meet[wave * (JC * TME * 4096) + at] = iu8_v4i{a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]};
+        });
+        met();
+        each([&](int i, int j, int g, int at) {
+          const iu8_v4i v = *(const iu8_v4i *)&meet[other * (JC * TME * 4096) + at];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][g * 4 + e] += v[e];
+        });
+        met();  // (the next blocks', or the epilogue's own, regions lie in the same stage)
       }
     } else {
       // the phased loop with the first `nl` of this wave's TM row blocks live
@@ -616,8 +702,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
       // now 18.5 / 19.3 / 22.8 / 28.5, the wave layout included.)
       auto part = [&](int zq, int m, int n) { return P + (((size_t)zq * (N >> 2) + (n >> 2)) * M + m) * 4; };
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = C.mbase + (wm * TM + i) * 32 + r32;
+      for (int i = 0; i < TME; ++i) {
+        const int m = C.mbase + (wm * TM + kw * TME + i) * 32 + r32;
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -638,8 +724,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
         if (tid == 0) __hip_atomic_store(&cnt[C.id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         constexpr int SH = 3;  // shares asked for at a time
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int m = C.mbase + (wm * TM + i) * 32 + r32;
+        for (int i = 0; i < TME; ++i) {
+          const int m = C.mbase + (wm * TM + kw * TME + i) * 32 + r32;
           const float am = as[iu8_arow(C.R, min(m, M - 1))];
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
@@ -692,8 +778,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
           const int n = ncol0 + j * 32 + g * 8 + nq;
           if (n >= N) continue;
 #pragma unroll
-          for (int i = 0; i < TM; ++i) {
-            const int m = C.mbase + (wm * TM + i) * 32 + r32;
+          for (int i = 0; i < TME; ++i) {
+            const int m = C.mbase + (wm * TM + kw * TME + i) * 32 + r32;
             if (m >= M) continue;
             *(iu8_v4i *)((int *)Cv + (size_t)(C.R.row0 + m) * N + n) =
                 iu8_v4i{acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
@@ -704,8 +790,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
       // its 4 consecutive columns of a row (8 bytes; lane halves side by side) -- such a tile's output
       // is small.
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = C.mbase + (wm * TM + i) * 32 + r32;
+      for (int i = 0; i < TME; ++i) {
+        const int m = C.mbase + (wm * TM + kw * TME + i) * 32 + r32;
         float am = TAB ? tabs.am[C.tab * BM + m - C.mbase] : as[iu8_arow(C.R, min(m, M - 1))];
         iu8_taken(am);
 #pragma unroll
@@ -730,15 +816,15 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
       constexpr int ROWB = CB * 64 + 16, LPR = CB * 4, PIECES = 32 * LPR;
       static_assert(NWAVE * 32 * ROWB <= STAGE, "the epilogue region fits one stage");
       iu8_u8 *reg = smem + (st == 0 ? NST - 1 : st - 1) * STAGE + wave * (32 * ROWB);
-      float am[TM];
+      float am[TME];
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-        am[i] = TAB       ? tabs.am[C.tab * BM + (wm * TM + i) * 32 + r32]
-                : stashed ? s_am[r & 1][(wm * TM + i) * 32 + r32]
-                          : as[iu8_arow(C.R, min(C.mbase + (wm * TM + i) * 32 + r32, M - 1))];
+      for (int i = 0; i < TME; ++i)
+        am[i] = TAB       ? tabs.am[C.tab * BM + (wm * TM + kw * TME + i) * 32 + r32]
+                : stashed ? s_am[r & 1][(wm * TM + kw * TME + i) * 32 + r32]
+                          : as[iu8_arow(C.R, min(C.mbase + (wm * TM + kw * TME + i) * 32 + r32, M - 1))];
       if constexpr (DEEP) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) iu8_taken(am[i]);
+        for (int i = 0; i < TME; ++i) iu8_taken(am[i]);
       }
       // a column block's weight scales are read once, for all the wave's row blocks
 #pragma unroll
@@ -761,8 +847,8 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
             for (int g = 0; g < 4; ++g) iu8_taken(wsu[jj][g]);
         }
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          if (C.mbase + (wm * TM + i) * 32 >= M) continue;  // a row block past the tile's rows (the whole wave)
+        for (int i = 0; i < TME; ++i) {
+          if (C.mbase + (wm * TM + kw * TME + i) * 32 >= M) continue;  // a row block past the tile's rows (the whole wave)
 #pragma unroll
           for (int jj = 0; jj < CB; ++jj) {
             const int j = jb * CB + jj;
@@ -779,7 +865,7 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
 #pragma unroll
           for (int q0 = 0; q0 < PIECES; q0 += 64) {
             const int q = q0 + lane, row = q / LPR, pc = q % LPR;
-            const int mm = C.mbase + (wm * TM + i) * 32 + row, nn = ncol0 + jb * (CB * 32) + pc * 8;
+            const int mm = C.mbase + (wm * TM + kw * TME + i) * 32 + row, nn = ncol0 + jb * (CB * 32) + pc * 8;
             if ((PIECES % 64 == 0 || q < PIECES) && mm < M && nn < N)
               *(iu8_v4u *)((unsigned short *)Cv + (size_t)(C.R.row0 + mm) * N + nn) =
                   *(const iu8_v4u *)&reg[row * ROWB + pc * 16];

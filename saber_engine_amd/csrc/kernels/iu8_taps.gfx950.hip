@@ -12,7 +12,7 @@
 #include "iu8_had.h"
 
 #define IU8_DEC_TAP(name, TM, W8, NT, KW, WPB, D, ALDS, ACC) IU8_DEC(name, TM, W8, NT, KW, WPB, D, ALDS, ACC)
-#define IU8_PF_TAP(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP)
+#define IU8_PF_TAP(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW) IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW)
 #include "iu8_variants.def"
 
 extern "C" __global__ __launch_bounds__(256) void mxfp4_hadi8_silu_f32_table(float *__restrict__ out) {

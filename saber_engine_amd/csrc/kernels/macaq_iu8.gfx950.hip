@@ -139,7 +139,7 @@ IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 1, 4, 2, 1, 5, 2, true)
     iu8_stream_body<TM, W8, NT, KW, D, false, 144, W8 ? NT == 4 : NT == 9 && TM >= 3>(                             \
         lds, a, w, as, ws, nullptr, nullptr, c, m, n, k, iu8_blk{(int)blockIdx.x, 0, 1});                          \
   }
-#define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP) IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP)
+#define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW) IU8_PF32(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW)
 #include "iu8_variants.def"
 
 // The tile GEMM with the per-token quantisation fused into its A-tile load (symbols `macaq_iu8_pfq_*`,

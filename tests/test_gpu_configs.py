@@ -247,6 +247,28 @@ def test_last_round_of_the_256x256_cell_runs_as_quarter_tiles(ctx, grid, tag, w8
     np.testing.assert_array_equal(host_u16(c), r["C"])
 
 
+@pytest.mark.parametrize("cell", ["w4_t256x160", "w4_t128x320", "w4_t128x256", "w8_t128x256"])
+@pytest.mark.parametrize("M,N,K,grid", [(1, 16, 128, 1), (33, 336, 256, 2), (129, 656, 384, 3), (257, 1040, 640, 2), (300, 272, 1152, 1)])
+def test_tile_cells_of_two_k_waves(ctx, cell, M, N, K, grid):
+    """The cells whose wave tile two k-waves sum: one and an odd count of K steps, ragged rows and columns, a row block or a
+    column block without an element, several tiles a workgroup; the oracle's bytes, and nothing stored past them."""
+    w8 = cell.startswith("w8")
+    say(f"two k-waves: {cell} {M} x {N} x {K} on {grid} workgroups")
+    case = synth.dense_case(M, N, K, w8=w8, seed=M + K)
+    r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], w8)), dev_f32(case["ws"])
+    d = iu8.describe(f"macaq_iu8_pf_{cell}", M, N, K)
+    d.grid[0] = min(d.grid[0], grid)
+    c = torch.full((M + 1, N), 0x7FC0, dtype=torch.int16, device="cuda")
+    bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr())
+    bufs["as"] = s.data_ptr()
+    ctx.launch(d, bufs)
+    torch.cuda.synchronize()
+    got = host_u16(c)
+    np.testing.assert_array_equal(got[:M], r["C"])
+    assert (got[M] == 0x7FC0).all()
+
+
 def test_split_counter_is_reusable_across_launches(ctx):
     say("explicit split, two launches on one counter")
     case = synth.dense_case(3, 256, 2048, seed=23)
