@@ -590,38 +590,41 @@ __device__ __forceinline__ void iu8_pf32_run(const iu8_u8 *__restrict__ A, const
           for (int j = 0; j < TN; ++j) wpk[0][j] = wpk[1][j];
         }
       }
-      // The k-waves of a wave tile each hold a sum over half of K. They meet in the stage the last step drained: each hands
-      // over the row blocks that the other stores, JC column blocks at a time (int32: exact, in any order).
-      constexpr int JC = STAGE / (NWAVE * TME * 4096) < TN ? STAGE / (NWAVE * TME * 4096) : TN;
-      static_assert(JC >= 1, "a column block's sums fit the stage");
+      // The k-waves of a wave tile each hold a sum over their part of K. They meet in the stage the last step drained: each
+      // hands over the row blocks that the other stores, JC column blocks or GC quads of one at a time (int32: exact, in
+      // any order).
+      constexpr int FIT = STAGE / (NWAVE * TME * 1024);  // quads that fit
+      constexpr int JC = FIT < 4 ? 1 : FIT / 4 < TN ? FIT / 4 : TN, GC = FIT < 4 ? 2 : 4, PART = JC * GC * TME * 1024;
+      static_assert(FIT >= 2, "half a column block's sums fit the stage");
       iu8_u8 *meet = smem + (st == 0 ? NST - 1 : st - 1) * STAGE + lane * 16;
       const int other = wave + (kw ? -(WMW * WNW) : WMW * WNW);
 #pragma unroll
-      for (int j0 = 0; j0 < TN; j0 += JC) {
-        auto each = [&](auto f) {
+      for (int j0 = 0; j0 < TN; j0 += JC)
 #pragma unroll
-          for (int jj = 0; jj < JC && j0 + jj < TN; ++jj)
+        for (int g0 = 0; g0 < 4; g0 += GC) {
+          auto each = [&](auto f) {
 #pragma unroll
-            for (int i = 0; i < TME; ++i)
+            for (int jj = 0; jj < JC && j0 + jj < TN; ++jj)
 #pragma unroll
-              for (int g = 0; g < 4; ++g) f(i, j0 + jj, g, ((jj * TME + i) * 4 + g) * 1024);
-        };
-        auto met = [&]() {
-          wait_vm(std::integral_constant<int, 63>{}, true);
-          __builtin_amdgcn_s_barrier();
-        };
-        each([&](int i, int j, int g, int at) {
-          const iu8_v16i &a = acc[TME + i][j];
-          *(iu8_v4i *)&meet[wave * (JC * TME * 4096) + at] = iu8_v4i{a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]};
-        });
-        met();
-        each([&](int i, int j, int g, int at) {
-          const iu8_v4i v = *(const iu8_v4i *)&meet[other * (JC * TME * 4096) + at];
+              for (int i = 0; i < TME; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][j][g * 4 + e] += v[e];
-        });
-        met();  // (the next blocks', or the epilogue's own, regions lie in the same stage)
-      }
+                for (int g = 0; g < GC; ++g) f(i, j0 + jj, g0 + g, ((jj * TME + i) * GC + g) * 1024);
+          };
+          auto met = [&]() {
+            wait_vm(std::integral_constant<int, 63>{}, true);
+            __builtin_amdgcn_s_barrier();
+          };
+          auto put = [&](iu8_u8 *to, const iu8_v16i &a, int g) { *(iu8_v4i *)to = iu8_v4i{a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]}; };
+          auto add = [&](iu8_v16i &a, int g, const iu8_u8 *from) {
+            const iu8_v4i v = *(const iu8_v4i *)from;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[g * 4 + e] += v[e];
+          };
+          each([&](int i, int j, int g, int at) { put(&meet[wave * PART + at], acc[TME + i][j], g); });
+          met();
+          each([&](int i, int j, int g, int at) { add(acc[i][j], g, &meet[other * PART + at]); });
+          met();  // (the next part's, or the epilogue's own, regions lie in the same stage)
+        }
     } else {
       // the phased loop with the first `nl` of this wave's TM row blocks live
       auto run_steps = [&](auto nl) {

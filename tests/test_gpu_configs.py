@@ -247,7 +247,7 @@ def test_last_round_of_the_256x256_cell_runs_as_quarter_tiles(ctx, grid, tag, w8
     np.testing.assert_array_equal(host_u16(c), r["C"])
 
 
-@pytest.mark.parametrize("cell", ["w4_t256x160", "w4_t128x320", "w4_t128x256", "w8_t128x256"])
+@pytest.mark.parametrize("cell", ["w4_t256x160", "w4_t128x320", "w4_t128x256", "w4_t128x128", "w8_t128x256"])
 @pytest.mark.parametrize("M,N,K,grid", [(1, 16, 128, 1), (33, 336, 256, 2), (129, 656, 384, 3), (257, 1040, 640, 2), (300, 272, 1152, 1)])
 def test_tile_cells_of_two_k_waves(ctx, cell, M, N, K, grid):
     """The cells whose wave tile two k-waves sum: one and an odd count of K steps, ragged rows and columns, a row block or a
