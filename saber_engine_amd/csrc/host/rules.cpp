@@ -607,22 +607,32 @@ uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant *
 // cold (successive launches walk copies that exceed the memory-side cache; with warm weights the 64 x 64
 // cell overtakes the 64 x 128 one at 256 rows, which no layer of a model sees), and checked on shapes the fit had
 // not seen -- the served 27B graph's own 16384 x 5120, 14336 x 5120, 5120 x 6144 and 96 x 5120 at eight row counts,
-// which moved three small-cell rates and took the side-by-side term off the 64-row cells. The W4 64 x 128 cell has
-// since moved to four waves side by side and is 12-16 % faster than its constants here say; with it the pick is within
-// 0.6 % of the fastest cell on 105 of 111 points (eight shapes, 65 to 8,192 rows) and within 3 % on 108; off are 300 rows
-// of 7168 x 5120 (23.5 us on 128 x 128, 20.5 on 64 x 128) and of 34816 x 5120 (76.6 on 256 x 320, 69.9). W8, output-side shapes
+// which moved three small-cell rates and took the side-by-side term off the 64-row cells. The W4 rates were drawn again when
+// the 128- and 256-row cells got their k-waves (iu8_pf32.h): 1,336 shapes of 65 to 8,192 rows, 256 to 35,200 columns and K to
+// 17,408, every cell timed on weights from memory, half of them the grid of the served widths and half drawn at random. The
+// pick moved on 172 of them, 7 % faster there on average and none more than 1.6 % slower; on 116 of 1,200 further shapes, 6 %
+// faster, 7 of them 2-5 % slower (843 rows of 17232 x 3456 54.7 on 256 x 320, 57.6 on 128 x 128 two a CU). 128 x 256 has constants of
+// its own at 65 to 1,023 rows, where it is one round: from 1,024 rows of 5,120 columns the pick stays 128 x 128 two a CU although
+// 128 x 256 has become 5-7 % faster there (1,100 / 1,300 rows of 5120 x 17408 102 / 113 against 97 / 106). W8, output-side shapes
 // from 2,048 rows: every pick the fastest; at 1,025 to 1,280 rows up to 7 % off (256 x 160, 128 x 128 two a CU). The
 // reference keeps its band tables the same way
 // (crates/saber-kernels/src/macaq_iu8.rs:150-212). One table for both kinds had sent the int8-weight
 // O and down projections at 2,048 rows to the 128 x 320 cell, 17-22 % behind the 256 x 160 cell there.
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
   struct Cell { const char *tile; double tops_per_cu, tile_us; };
-  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, hbm_tbps, side_cap; Cell cells[11]; };
-  static const Law W4 = {0.974, 90.000, 19.875, 1.422, 3.113, 2.116,
-                         {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t256x224", 13.814, 14.000}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}}};
-  static const Law W8 = {4.419, 75.175, 18.116, 1.782, 5.234, 1.935,
-                         {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t256x224", 11.270, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}}};
-  const Law &law = w8 ? W8 : W4;
+  // quarter: the rate of the 128 x 128 tiles in the 256 x 256 cell's last round; few: a cell's constants at 65 to 1,023 rows
+  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, hbm_tbps, side_cap, quarter; Cell cells[11], few; };
+  static const Law W4 = {0.974, 90.000, 19.875, 1.422, 3.113, 2.116, 8.799,
+                         {{"tn4_lbk64", 13.797, 3.223}, {"t256x320", 13.314, 6.002}, {"t256x224", 12.693, 14.000}, {"t128x320", 11.675, 2.893}, {"t256x160", 11.618, 7.995}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.905, 2.045}, {"t128x128_o2", 10.703, 2.096}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 5.698, 1.372}, {"t64x64_s", 5.504, 1.829}},
+                         {"t128x256", 10.078, 1.844}};
+  // up to 64 rows, which the lines above this estimate in `resolve` are drawn against
+  static const Law W4_64 = {0.974, 90.000, 19.875, 1.422, 3.113, 2.116, 8.799,
+                            {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t256x224", 13.814, 14.000}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}},
+                            {"", 0.000, 0.000}};
+  static const Law W8 = {4.419, 75.175, 18.116, 1.782, 5.234, 1.935, 8.069,
+                         {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t256x224", 11.270, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}},
+                         {"", 0.000, 0.000}};
+  const Law &law = w8 ? W8 : m <= 64 ? W4_64 : W4;
   // the cells' variants, looked up once
   constexpr size_t NCELL = sizeof(Law::cells) / sizeof(Cell);
   using Variants = std::array<const PfVariant *, NCELL>;
@@ -632,13 +642,10 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
     return v;
   };
   static const Variants V4 = variants(W4, "w4"), V8 = variants(W8, "w8");
-  double quarter_rate = 0;
-  for (const auto &c : law.cells)
-    if (!strcmp(c.tile, "t128x128")) quarter_rate = c.tops_per_cu;
   const PfVariant *best = nullptr;
   double best_t = 0;
   for (size_t i = 0; i < NCELL; ++i) {
-    const Cell &c = law.cells[i];
+    const Cell &c = m < 1024 && !strcmp(law.cells[i].tile, law.few.tile) ? law.few : law.cells[i];
     const PfVariant *v = (w8 ? V8 : V4)[i];
     if (!v) continue;
     const double bm = v->block_m(), bn = v->block_n();
@@ -650,7 +657,7 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
     // 128 x 128 cell, each a quarter of the work at that cell's rate
     const uint64_t q = tiles / grid, rem = tiles - q * grid;
     if (!strcmp(c.tile, "tn4_lbk64") && q >= 1 && rem > 0 && 2 * rem <= grid)
-      cu_tiles = (double)q + (double)((4 * rem + grid - 1) / grid) * 0.25 * (c.tops_per_cu / quarter_rate);
+      cu_tiles = (double)q + (double)((4 * rem + grid - 1) / grid) * 0.25 * (c.tops_per_cu / law.quarter);
     // ... and a few rows past the last whole 256 as thin tiles (int4 weights: the estimate of the int8 cells is drawn without)
     if (!strcmp(c.tile, "tn4_lbk64") && !w8 && tiles < (1u << 20) && k < (1u << 30)) {
       const iu8_pf_plan plan = iu8_pf_plan256((int)m, (int)((n + 255) / 256), (int)grid, (int)k, w8);
