@@ -463,7 +463,14 @@ int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu
   // max_flat_workgroup_size): a descriptor from another launch law -- the reference's 256-thread
   // blocks under its own names -- would run and give wrong bytes, so it is refused here by name.
   const uint64_t threads = (uint64_t)d->block[0] * std::max(d->block[1], 1u) * std::max(d->block[2], 1u);
-  if (threads != it->second.max_threads)
+  uint32_t block[3] = {d->block[0], d->block[1], d->block[2]};
+  if (threads != it->second.max_threads) {
+    // A tile cell derives all it does from its grid and m, n, k: a descriptor of 128 x 320 or 128 x 256 laid out when their wave
+    // tiles had one wave each (256 threads) runs on the k-waves they have now.
+    const PfVariant *v = pf_variant(d->kernel);
+    if (v && v->kw > 1 && v->block_m() == 128 && v->block_n() >= 256 && threads * v->kw == it->second.max_threads) block[0] = it->second.max_threads, block[1] = block[2] = 1;
+  }
+  if ((uint64_t)block[0] * std::max(block[1], 1u) * std::max(block[2], 1u) != it->second.max_threads)
     return fail(SABER_IU8_E_RULE, fmt("%s: a block of %llu threads; the gfx950 kernel is written for %u (use this object's launch law)",
                                       d->kernel, (unsigned long long)threads, it->second.max_threads));
   if (int rc = launch_guard(it->second, d)) return rc;
@@ -472,8 +479,8 @@ int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu
   if (int rc = saber_iu8_pack_kernarg(d, bufs, n_bufs, image, sizeof image, &bytes)) return rc;
   size_t sz = bytes;
   void *extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, image, HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz, HIP_LAUNCH_PARAM_END};
-  const hipError_t e = hipModuleLaunchKernel(it->second.fn, d->grid[0], d->grid[1], d->grid[2], d->block[0], d->block[1],
-                                             d->block[2], 0, (hipStream_t)stream, nullptr, extra);
+  const hipError_t e = hipModuleLaunchKernel(it->second.fn, d->grid[0], d->grid[1], d->grid[2], block[0], block[1],
+                                             block[2], 0, (hipStream_t)stream, nullptr, extra);
   if (e != hipSuccess) return hip_fail(d->kernel, e);
   ctx->counters.launches++;
   return 0;

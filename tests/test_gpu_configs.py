@@ -262,11 +262,18 @@ def test_tile_cells_of_two_k_waves(ctx, cell, M, N, K, grid):
     c = torch.full((M + 1, N), 0x7FC0, dtype=torch.int16, device="cuda")
     bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr())
     bufs["as"] = s.data_ptr()
-    ctx.launch(d, bufs)
-    torch.cuda.synchronize()
-    got = host_u16(c)
-    np.testing.assert_array_equal(got[:M], r["C"])
-    assert (got[M] == 0x7FC0).all()
+    # ... also from a descriptor laid out for one wave a wave tile
+    for threads in (512, 256) if cell.split("_")[1] in ("t128x320", "t128x256") else (512,):
+        d.block[0] = threads
+        c.fill_(0x7FC0)
+        ctx.launch(d, bufs)
+        torch.cuda.synchronize()
+        got = host_u16(c)
+        np.testing.assert_array_equal(got[:M], r["C"])
+        assert (got[M] == 0x7FC0).all()
+    d.block[0] = 128 if cell.split("_")[1] in ("t128x320", "t128x256") else 256
+    with pytest.raises(iu8.IU8Error, match="threads"):
+        ctx.launch(d, bufs)
 
 
 def test_split_counter_is_reusable_across_launches(ctx):
