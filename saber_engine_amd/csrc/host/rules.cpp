@@ -610,8 +610,8 @@ uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant *
 // which moved three small-cell rates and took the side-by-side term off the 64-row cells. The W4 rates were drawn again when
 // the 128- and 256-row cells got their k-waves (iu8_pf32.h): 1,336 shapes of 65 to 8,192 rows, 256 to 35,200 columns and K to
 // 17,408, every cell timed on weights from memory, half of them the grid of the served widths and half drawn at random. The
-// pick moved on 172 of them, 7 % faster there on average and none more than 1.6 % slower; on 116 of 1,200 further shapes, 6 %
-// faster, 7 of them 2-5 % slower (843 rows of 17232 x 3456 54.7 on 256 x 320, 57.6 on 128 x 128 two a CU). 128 x 256 has constants of
+// pick moved on 158 of them, 7 % faster there on average and none more than 1.6 % slower; on 109 of 1,200 further shapes, 6 %
+// faster, 3 of them 2-7 % slower (634 rows of 12160 x 2688 23.4 on 128 x 256, 25.0 on 128 x 128 two a CU). 128 x 256 has constants of
 // its own at 65 to 1,023 rows, where it is one round: from 1,024 rows of 5,120 columns the pick stays 128 x 128 two a CU although
 // 128 x 256 has become 5-7 % faster there (1,100 / 1,300 rows of 5120 x 17408 102 / 113 against 97 / 106). W8, output-side shapes
 // from 2,048 rows: every pick the fastest; at 1,025 to 1,280 rows up to 7 % off (256 x 160, 128 x 128 two a CU). The
@@ -621,15 +621,15 @@ uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant *
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
   struct Cell { const char *tile; double tops_per_cu, tile_us; };
   // quarter: the rate of the 128 x 128 tiles in the 256 x 256 cell's last round; few: a cell's constants at 65 to 1,023 rows
-  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, hbm_tbps, side_cap, quarter; Cell cells[11], few; };
-  static const Law W4 = {0.974, 90.000, 19.875, 1.422, 3.113, 2.116, 8.799,
+  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, again, hbm_tbps, side_cap, quarter; Cell cells[11], few; };
+  static const Law W4 = {0.974, 90.000, 19.875, 1.422, 1.050, 3.113, 2.116, 8.799,
                          {{"tn4_lbk64", 13.797, 3.223}, {"t256x320", 13.314, 6.002}, {"t256x224", 12.693, 14.000}, {"t128x320", 11.675, 2.893}, {"t256x160", 11.618, 7.995}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.905, 2.045}, {"t128x128_o2", 10.703, 2.096}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 5.698, 1.372}, {"t64x64_s", 5.504, 1.829}},
                          {"t128x256", 10.078, 1.844}};
   // up to 64 rows, which the lines above this estimate in `resolve` are drawn against
-  static const Law W4_64 = {0.974, 90.000, 19.875, 1.422, 3.113, 2.116, 8.799,
+  static const Law W4_64 = {0.974, 90.000, 19.875, 1.422, 1.000, 3.113, 2.116, 8.799,
                             {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t256x224", 13.814, 14.000}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}},
                             {"", 0.000, 0.000}};
-  static const Law W8 = {4.419, 75.175, 18.116, 1.782, 5.234, 1.935, 8.069,
+  static const Law W8 = {4.419, 75.175, 18.116, 1.782, 1.000, 5.234, 1.935, 8.069,
                          {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t256x224", 11.270, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}},
                          {"", 0.000, 0.000}};
   const Law &law = w8 ? W8 : m <= 64 ? W4_64 : W4;
@@ -668,8 +668,11 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
     const double t_cu = cu_tiles * tile_bytes / (law.cu_gbps * 1e3);
     const double t_l2 = (double)tiles * tile_bytes / (law.l2_tbps * 1e6);
     // the two-a-CU 128 x 128 cell alone on a CU (no more workgroups than CUs) has four waves to hide
-    // its latencies with and measured well behind the eight-wave 128 x 128 cell there
-    const double lone = (!strcmp(c.tile, "t128x128_o2") && grid <= CU_COUNT) ? law.lone : 1.0;
+    // its latencies with and measured well behind the eight-wave 128 x 128 cell there; a second round of it (`again`, int4
+    // weights: 5 %) is dearer than its rate says: without the factor 300-384 rows of 34816 x 5120 went to it from 256 x 320, and
+    // a layer of 300 rows took 360 us (348 with the rates before; with the factor 337 against 344 in another run)
+    const bool o2 = !strcmp(c.tile, "t128x128_o2");
+    const double lone = o2 && grid <= CU_COUNT ? law.lone : o2 && per_wg > 1 ? law.again : 1.0;
     // cold weights: the row tiles that run side by side on one column block each fetch it from memory -- those of the
     // 128- and 256-row cells; the 64-row cells' neighbours share a column block's lines (fetch over operands 1.5-1.65 at
     // four row tiles by the counters, and the wide projections of the served graph at 65-128 rows: 16.5-18.8 us on
