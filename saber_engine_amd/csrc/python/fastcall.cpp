@@ -5,9 +5,10 @@
 // a call; here an argument is read by the type the header declares, 0.7 us with the descriptor's layout. (With the layout's
 // share, util.h: a one-row linear of 5120 x 5120 in a loop of calls 8.4 -> 7.4 us, its kernel 5.3; 16 rows, quantiser and GEMM,
 // 13.0 -> 11.3.) The conversions are ctypes' own for what a caller
-// passes: a pointer is an int or None, a number an int, a float a float, each taken modulo its width. Anything else in an
-// argument's place (a ctypes object, a bool, another count of arguments) goes to the ctypes function of the same name,
-// which converts or refuses it. The interpreter lock is released around the call, as ctypes does.
+// passes: a pointer is an int or None, a number an int, a float a float, each taken modulo its width; the routed operators'
+// tables are the structure itself (an address in their place is refused, as ctypes refuses it). Anything else in an argument's
+// place (a ctypes object, a bool, another count of arguments) sends the whole call, its arguments as they came, to the ctypes
+// function of the same name, which converts or refuses them. The interpreter lock is released around the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -19,9 +20,19 @@
 
 namespace {
 
+PyObject *tables_type = nullptr;  // the binding's saber_iu8_moe_tables
+
 template <class T>
 bool take(PyObject *o, T &v) {
-  if constexpr (std::is_floating_point_v<T>) {
+  if constexpr (std::is_same_v<T, const saber_iu8_moe_tables *>) {
+    if ((PyObject *)Py_TYPE(o) != tables_type) return false;
+    Py_buffer b;
+    if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE)) return false;
+    const bool whole = b.len == (Py_ssize_t)sizeof *v;
+    v = (T)b.buf;
+    PyBuffer_Release(&b);  // (the structure's own memory: it lives as long as the caller's reference)
+    return whole;
+  } else if constexpr (std::is_floating_point_v<T>) {
     if (!PyFloat_CheckExact(o)) return false;
     v = (T)PyFloat_AS_DOUBLE(o);
   } else {
@@ -71,9 +82,12 @@ struct Entry<F> {
   X(attn_gate_quant_had) X(attn_gate_quant_had_lut) X(moe_route) X(moe_route_quant) X(moe_grouped) X(moe_quant_rows)              \
   X(moe_silu_mul_quant) X(moe_gate_up_act) X(moe_down_rows) X(moe_combine)
 
-// bind(functions): {name: ctypes function}
-PyObject *bind(PyObject *, PyObject *functions) {
-  if (!PyDict_Check(functions)) return PyErr_Format(PyExc_TypeError, "bind takes a dict");
+// bind(functions, tables): {name: ctypes function}, the ctypes structure of the routed operators' tables
+PyObject *bind(PyObject *, PyObject *args) {
+  PyObject *functions, *tables;
+  if (!PyArg_ParseTuple(args, "O!O!", &PyDict_Type, &functions, &PyType_Type, &tables)) return nullptr;
+  Py_INCREF(tables);
+  Py_XSETREF(tables_type, tables);
 #define BIND(name)                                                  \
   if (PyObject *f = PyDict_GetItemString(functions, #name)) {       \
     Py_INCREF(f);                                                   \
@@ -88,7 +102,7 @@ PyMethodDef methods[] = {
 #define METHOD(name) {#name, (PyCFunction)(void (*)())Entry<saber_iu8_##name>::call, METH_FASTCALL, nullptr},
     OPERATORS(METHOD)
 #undef METHOD
-    {"bind", bind, METH_O, nullptr},
+    {"bind", bind, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fastcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -379,8 +379,8 @@ class _CtypesOperators:
 
 
 def operators():
-    """The operator entry points by name: `_fastcall`'s (csrc/python/fastcall.cpp), which take ints and None as they are and
-    give everything else to the ctypes function, else the ctypes functions."""
+    """The operator entry points by name: `_fastcall`'s (csrc/python/fastcall.cpp), which take ints, None and `MoeTables` as they
+    are and give everything else to the ctypes function, else the ctypes functions."""
     global _ops
     if _ops is None:
         L = lib()  # first: _fastcall links to the same library
@@ -389,13 +389,14 @@ def operators():
         except ImportError:
             _ops = _CtypesOperators()
             return _ops
-        _fastcall.bind({n: getattr(L, "saber_iu8_" + n) for n in dir(_fastcall) if not n.startswith("_") and n != "bind"})
+        _fastcall.bind({n: getattr(L, "saber_iu8_" + n) for n in dir(_fastcall) if not n.startswith("_") and n != "bind"}, MoeTables)
         _ops = _fastcall
     return _ops
 
 
 def _tables(t):
-    return C.addressof(t) if type(t) is MoeTables else C.byref(t)
+    """The routed operators' tables as both kinds of entry points take them (never as an address, which ctypes refuses)."""
+    return t if type(t) is MoeTables else C.byref(t)
 
 
 class Context:

@@ -663,12 +663,22 @@ def test_open_without_a_gpu_fails_loudly():
     assert e.value.code == iu8.E_HIP and "no CPU fallback" in str(e.value)
 
 
-def test_operator_entry_points_take_what_ctypes_takes():
+@pytest.fixture(params=["fastcall", "ctypes"])
+def op(request):
+    """The operators' entry points: the extension's (where this interpreter has it) and those of an interpreter without it."""
+    if request.param == "ctypes":
+        return iu8._CtypesOperators()
+    o = iu8.operators()
+    if isinstance(o, iu8._CtypesOperators):
+        pytest.skip("_fastcall is not built for this interpreter")
+    return o
+
+
+def test_operator_entry_points_take_what_ctypes_takes(op):
     """The binding's own entry points (csrc/python/fastcall.cpp): ints and None as they are, everything else -- ctypes objects,
     other integer types, a wrong type or count -- as the ctypes function has it. Without a context every call is refused by
     the library itself, before anything is launched."""
-    op, L = iu8.operators(), iu8.lib()
-    assert op.__name__.endswith("_fastcall")
+    L = iu8.lib()
     args = (0, 1 << 40, 1 << 40, 1 << 40, 1 << 40, None, None, 1, 5120, 5120)
     for a in ((None,) + args + (0,), (None,) + args + (None,), (ctypes.c_void_p(),) + args + (ctypes.c_void_p(0),), (None, True) + args[1:] + (0,),
               (None,) + args[:-1] + (np.int64(5120), 0), (None,) + args[:-1] + ((1 << 32) + 5120, 0), (None, 7) + args[1:] + (0,),
@@ -682,6 +692,72 @@ def test_operator_entry_points_take_what_ctypes_takes():
             op.linear_fused(*bad)
         with pytest.raises((ctypes.ArgumentError, TypeError)):
             L.saber_iu8_linear_fused(*bad)
+
+
+OPERATORS = ("quant quant_rowmajor gemm rowscale linear_prefill_fused gemm_static gemm_pair linear_fused mlp_chain gate_up_act quant_had "
+             "silu_mul_quant_had silu_mul_quant_had_lut add_rms_quant_had gdn_norm_quant_had attn_gate_quant_had attn_gate_quant_had_lut "
+             "moe_route moe_route_quant moe_grouped moe_quant_rows moe_silu_mul_quant moe_gate_up_act moe_down_rows moe_combine").split()
+
+
+class OtherTables(iu8.MoeTables):
+    pass
+
+
+@pytest.mark.parametrize("name", OPERATORS)
+def test_every_operator_takes_the_forms_ctypes_takes(op, name):
+    """Every operator, every argument in turn in every form a caller may have it in (the routed ones' tables among them): the
+    ctypes function's result, message or exception. Without a context: the library refuses each call before a launch."""
+    f, g, T = getattr(op, name), getattr(iu8.lib(), "saber_iu8_" + name), iu8.MoeTables()
+    base, forms = [], []
+    for t in g.argtypes:
+        if t is ctypes.c_void_p:
+            base.append(1 << 40 if base else None)
+            forms.append([None] if len(base) == 1 else [None, 0, -1, 1 << 63, ctypes.c_void_p(0), ctypes.c_void_p(64), ctypes.byref(T), b"x", True, np.int64(64), 1.5])
+        elif t is ctypes.c_float:
+            base.append(1e-6)
+            forms.append([1, ctypes.c_float(2.0), np.float32(3.0), np.float64(3.0), True, None, "1"])
+        elif t is ctypes.POINTER(iu8.MoeTables):
+            base.append(T)
+            forms.append([ctypes.byref(T), ctypes.pointer(T), (iu8.MoeTables * 1)(), OtherTables(), None, ctypes.addressof(T), ctypes.byref(iu8.Counters()),
+                          iu8.Counters(), ctypes.c_void_p(0), bytearray(ctypes.sizeof(T))])
+        else:
+            base.append(128 if len(base) > 1 else 0)
+            forms.append([8, 1, 0, 128 - (1 << 32), (1 << 32) + 128, 1 << 70, np.int64(128), np.uint32(8), True, t(128), 1.5, None, "128"])
+
+    def outcome(fn, a):
+        try:
+            return fn(*a), iu8.lib().saber_iu8_last_error()
+        except Exception as e:
+            return type(e), str(e)
+
+    calls = [base, base[:-1], base + [0], []] + [base[:i] + [v] + base[i + 1:] for i, vs in enumerate(forms) for v in vs]
+    refused = sum(isinstance(outcome(g, a)[0], int) for a in calls)
+    assert refused > len(base)      # the library's own refusals, not the conversions' alone
+    for a in calls:
+        want = outcome(g, a)
+        assert want[0] != 0 and outcome(f, a) == want, (name, a)
+
+
+def test_routed_operators_of_a_context_take_any_form(op):
+    """The routed layer's methods with a count or a stream that is not a plain int (refused for the missing context, by the
+    library), on the extension and on ctypes alone; what is not a table is refused as ctypes refuses it."""
+    ctx, P = iu8.Context.__new__(iu8.Context), 1 << 40
+    ctx._h, ctx._op, ctx._addr = ctypes.c_void_p(), op, None
+    calls = (("moe_route", (P, 16, 128, 8, 1), ()), ("moe_route_quant", (P, P, P, P, 16, 128, 8, 4096, 1), ()),
+             ("moe_grouped", (P, P, P, P, 4096, 1536, True, 16, 128, 8, 1), ()), ("moe_gate_up_act", (P, P, P, P, 1536, 4096, 16, 128, 8, 1), ()),
+             ("moe_down_rows", (P, P, P, 4096, 1536, 16, 128, 8, 1), ()), ("moe_quant_rows", (P, P, P, 4096, 64), ()),
+             ("moe_silu_mul_quant", (P, P, P, 1536, 64), ()), ("moe_combine", (P,), (P, 16, 8, 4096)))
+    for name, before, after in calls:
+        for tables in (iu8.MoeTables(), OtherTables()):
+            full = before + (tables,) + after
+            ints = [i for i, a in enumerate(full) if type(a) is int and a != P]
+            for a in [full] + [full[:i] + (np.int64(full[i]),) + full[i + 1:] for i in ints]:
+                for stream in (0, None, ctypes.c_void_p(0)):
+                    with pytest.raises(iu8.IU8Error, match="null argument"):
+                        getattr(ctx, name)(*a, stream=stream)
+        for bad in (None, 0, iu8.Counters()):
+            with pytest.raises((ctypes.ArgumentError, TypeError)):
+                getattr(ctx, name)(*before, bad, *after)
 
 
 # ------------------------------------------------------------------ operand orders
