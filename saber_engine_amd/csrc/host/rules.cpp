@@ -104,6 +104,9 @@ static int check_shape(const char *op, uint32_t m, uint32_t n, uint32_t k) {
   if (n % 16 != 0 || k % 128 != 0)
     return fail(SABER_IU8_E_RULE,
                 fmt("%s: N=%u must be a multiple of 16 (whole fragments) and K=%u of 128 (the slab)", op, n, k));
+  // the kernels take their sizes as int; and a count of blocks or tiles, (size + block - 1) / block in 32 bits, wraps to none
+  if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX)
+    return fail(SABER_IU8_E_RULE, fmt("%s: %u x %u x %u is past the kernels' 32-bit sizes", op, m, n, k));
   return 0;
 }
 

@@ -694,6 +694,31 @@ def test_operator_entry_points_take_what_ctypes_takes(op):
             L.saber_iu8_linear_fused(*bad)
 
 
+def test_sizes_at_the_end_of_32_bits_are_refused_not_divided_by():
+    """Row and column counts whose tile counts used to wrap to none: refused with a message, and no descriptor without a workgroup."""
+    top = 1 << 32
+    sizes = [(top - 1, 5120, 128), (top - 15, 16, 128), (top - 16, 5120, 5120), (top - 63, 16, 128), (top - 255, 256, 16384), (1 << 31, 5120, 5120),
+             (100, top - 16, 128), (17, top - 128, 16384), (192, top - 16, 16384), (1, top - 16, 16384), (16, top - 32, 5120), (2048, top - 256, 128),
+             (top - 1, top - 16, top - 128), (40, top - 48, 4096), (64, top - 16, 6144), (1 << 27, 16, 128)]
+    names = [f"macaq_iu8_pf_{t}" for t in ("w4_tn4_lbk64", "w8_tn4_lbk64", "w4_t256x160", "w4_t128x320", "w4_t64x64_s", "w8_t128x160", "w4_t64x128_s_ks")]
+    names += ["macaq_iu8_pfq_w4_t128x128", "macaq_iu8_dec_w4_tm1", "macaq_iu8_pf_w4_t48x144_w"]
+    calls = [lambda m, n, k, wk=wk, f=f: f(wk, m, n, k) for wk in (iu8.W4, iu8.W8) for f in (iu8.resolve, iu8.resolve_fused, iu8.resolve_prefill_fused)]
+    calls += [lambda m, n, k, name=name: iu8.describe(name, m, n, k) for name in names]
+    calls += [lambda m, n, k: iu8.resolve_gate_up_act(m, k, n), lambda m, n, k: iu8.resolve_mlp_chain(m, k, n), lambda m, n, k: iu8.resolve_quant(m, k)]
+    for m, n, k in sizes:
+        for f in calls:
+            try:
+                d = f(m, n, k)
+            except iu8.IU8Error as e:
+                assert e.code == iu8.E_RULE and str(e)
+            else:
+                assert d.grid[0] and d.grid[1] and d.grid[2], (m, n, k, d.kernel)
+    for m, n, k in ((top - 1, 5120, 128), (1, 1 << 31, 128), (1, 16, 1 << 31)):
+        with pytest.raises(iu8.IU8Error, match="32-bit sizes"):
+            iu8.resolve(iu8.W4, m, n, k)
+    assert iu8.resolve(iu8.W4, 1, (1 << 31) - 16, 128).grid[0]
+
+
 OPERATORS = ("quant quant_rowmajor gemm rowscale linear_prefill_fused gemm_static gemm_pair linear_fused mlp_chain gate_up_act quant_had "
              "silu_mul_quant_had silu_mul_quant_had_lut add_rms_quant_had gdn_norm_quant_had attn_gate_quant_had attn_gate_quant_had_lut "
              "moe_route moe_route_quant moe_grouped moe_quant_rows moe_silu_mul_quant moe_gate_up_act moe_down_rows moe_combine").split()
@@ -722,7 +747,7 @@ def test_every_operator_takes_the_forms_ctypes_takes(op, name):
                           iu8.Counters(), ctypes.c_void_p(0), bytearray(ctypes.sizeof(T))])
         else:
             base.append(128 if len(base) > 1 else 0)
-            forms.append([8, 1, 0, 128 - (1 << 32), (1 << 32) + 128, 1 << 70, np.int64(128), np.uint32(8), True, t(128), 1.5, None, "128"])
+            forms.append([8, 1, 0, -1, 128 - (1 << 32), (1 << 32) + 128, 1 << 70, np.int64(128), np.uint32(8), True, t(128), 1.5, None, "128"])
 
     def outcome(fn, a):
         try:
