@@ -35,6 +35,54 @@ static __device__ __forceinline__ int iu8_thin_tile_at(const iu8_pf_plan &p, int
   return j < gx ? j : -1;
 }
 
+// The form a cell of BM x BN rows and columns, OCC workgroups a CU, takes on a short K: wave tiles, stages and k-waves (the launch,
+// its threads and its tiles are the cell's own). Most cells have one form: a second one costs 128 x 256 and 128 x 320 (three
+// stages for four below K = 3,072) 3-7 % of the time of their long K, and gives them 1-3 % of the short one's.
+template <bool W8, int BM, int BN, int OCC>
+struct iu8_pf_short {
+  static constexpr bool HAS = false;
+};
+// W4 128 x 128, two k-waves and five stages (iu8_pf32.h): their meeting, some 1 us a tile, and the stages to fill are more than the
+// halved reads save on a few K steps. us, cold weights, 4 x 2 wave tiles of one wave and three stages / k-waves: 512 rows of
+// 7168 x 1024 8.7 / 9.8, 768 of 5120 x 2048 12.5 / 13.3, 96 of 28672 x 2048 13.5 / 15.0, 430 of 7728 x 384 6.6 / 7.5; over 63 shapes the
+// k-waves are 16 % slower below K = 512, 12 % below 1,024, 9 % below 2,048. From K = 2,176 they gain: 71 rows of 18048 x 2432
+// 13.6 / 12.7, 700 of 4096 x 4096 19.4 / 17.9; 46 shapes of 4,096-6,143 7 %, 38 from 9,000 14 %.
+template <>
+struct iu8_pf_short<false, 128, 128, 1> {
+  static constexpr bool HAS = true;
+  static constexpr int WMW = 4, WNW = 2, TM = 1, TN = 2, ST = 3, KW = 1;
+  static __device__ __forceinline__ bool takes(int k, int) { return k <= 2048; }
+};
+
+// The tiles of a dense launch on the cell, or on its form for a short K.
+template <bool W8, int WMW, int WNW, int TM, int TN, bool ACC, int ST, int OCC, bool DEEP, int KW>
+static __device__ __forceinline__ void iu8_pf32_dense(const unsigned char *__restrict__ a, const unsigned char *__restrict__ w,
+                                                      const float *__restrict__ as, const float *__restrict__ ws,
+                                                      unsigned short *__restrict__ c, int m, int n, int k) {
+  constexpr int BM = WMW * TM * 32, BN = WNW * TN * 32;
+  const int gx = (n + BN - 1) / BN, gy = (m + BM - 1) / BM;
+  const iu8_rows R{nullptr, 0, m};
+  auto tile_at = [&](int r, iu8_tile &t) {
+    int bx, by;
+    if (!iu8_dense_tile_at(r, gx, gy, bx, by)) return false;
+    t = iu8_tile{R, by * BM, bx * (BN / 16), w, ws, by * gx + bx};
+    return true;
+  };
+  using S = iu8_pf_short<W8, BM, BN, OCC>;
+  if constexpr (S::HAS) {
+    static_assert(S::WMW * S::TM * 32 == BM && S::WNW * S::TN * 32 == BN && S::WMW * S::WNW * S::KW == WMW * WNW * KW, "one launch");
+    constexpr int L = iu8_pf32_lds_bytes<W8, WMW, WNW, TM, TN, ST>();
+    static_assert(iu8_pf32_lds_bytes<W8, S::WMW, S::WNW, S::TM, S::TN, S::ST>() <= L, "the short form runs in the cell's stages");
+    __shared__ __attribute__((aligned(1024))) iu8_u8 lds[L];
+    if (S::takes(k, (int)gridDim.x))
+      iu8_pf32_run<W8, S::WMW, S::WNW, S::TM, S::TN, ACC, S::ST, DEEP, false, false, true, false, false, S::KW>(a, as, c, n, k, tile_at, nullptr, nullptr, lds);
+    else
+      iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP, false, false, true, false, false, KW>(a, as, c, n, k, tile_at, nullptr, nullptr, lds);
+  } else {
+    iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP, false, false, false, false, false, KW>(a, as, c, n, k, tile_at);
+  }
+}
+
 // Persistent launch: gridDim.x workgroups (one or OCC a CU) walk the tiles of the m x n output.
 //
 // The 256 x 256 cell's last round and its ragged rows (iu8_pf_law.h): a thin last round is cut into quarter tiles on the
@@ -93,11 +141,6 @@ static __device__ __forceinline__ int iu8_thin_tile_at(const iu8_pf_plan &p, int
             nullptr, nullptr, lds);                                                                                \
       }                                                                                                            \
     } else {                                                                                                       \
-      iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP, false, false, false, false, false, KW>(a, as, c, n, k, [&](int r, iu8_tile &t) { \
-        int bx, by;                                                                                                \
-        if (!iu8_dense_tile_at(r, gx, gy, bx, by)) return false;                                                   \
-        t = iu8_tile{R, by * BM, bx * (BN / 16), w, ws, by * gx + bx};                                             \
-        return true;                                                                                               \
-      });                                                                                                          \
+      iu8_pf32_dense<W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW>(a, w, as, ws, c, m, n, k);                       \
     }                                                                                                              \
   }

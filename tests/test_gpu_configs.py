@@ -276,6 +276,28 @@ def test_tile_cells_of_two_k_waves(ctx, cell, M, N, K, grid):
         ctx.launch(d, bufs)
 
 
+@pytest.mark.parametrize("cell,K", [("w4_t128x128", 2048), ("w4_t128x128", 2176)])
+@pytest.mark.parametrize("M,N,grid", [(130, 272, 6), (257, 1040, 8), (300, 400, 7)])
+def test_tile_cells_either_side_of_their_short_k(ctx, cell, K, M, N, grid):
+    """The cells that take another form on a short K, either side of the line, on grids in the order by XCD and out of it and on
+    fewer workgroups than tiles: the oracle's bytes, nothing stored past them."""
+    w8 = cell.startswith("w8")
+    say(f"short K: {cell} {M} x {N} x {K} on {grid} workgroups")
+    case = synth.dense_case(M, N, K, w8=w8, seed=M + K)
+    r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], w8)), dev_f32(case["ws"])
+    d = iu8.describe(f"macaq_iu8_pf_{cell}", M, N, K)
+    d.grid[0] = min(d.grid[0], grid)
+    c = torch.full((M + 1, N), 0x7FC0, dtype=torch.int16, device="cuda")
+    bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr())
+    bufs["as"] = s.data_ptr()
+    ctx.launch(d, bufs)
+    torch.cuda.synchronize()
+    got = host_u16(c)
+    np.testing.assert_array_equal(got[:M], r["C"])
+    assert (got[M] == 0x7FC0).all()
+
+
 def test_split_counter_is_reusable_across_launches(ctx):
     say("explicit split, two launches on one counter")
     case = synth.dense_case(3, 256, 2048, seed=23)
