@@ -53,6 +53,25 @@ struct iu8_pf_short<false, 128, 128, 1> {
   static constexpr int WMW = 4, WNW = 2, TM = 1, TN = 2, ST = 3, KW = 1;
   static __device__ __forceinline__ bool takes(int k, int) { return k <= 2048; }
 };
+// Int8 weights 128 x 128, four stages: three up to K = 2,048, and up to 6,143 on a count of tiles that leaves the order by XCD
+// (iu8_dense_tile_at), where the fourth makes neighbours' loads miss each other in the L2. us on three / four: 143 rows of 14352 x
+// 1664 13.0 / 15.5, of 14208 x 3840 21.9 / 26.0, 584 of 6256 x 1152 12.0 / 13.6, 638 of 5312 x 256 6.2 / 6.5; 415 of 6832 x 2688 16.2 /
+// 14.7, 304 of 9872 x 9856 53.4 / 48.0.
+template <>
+struct iu8_pf_short<true, 128, 128, 1> {
+  static constexpr bool HAS = true;
+  static constexpr int WMW = 4, WNW = 2, TM = 1, TN = 2, ST = 3, KW = 1;
+  static __device__ __forceinline__ bool takes(int k, int wgs) { return k <= 2048 || (k < 6144 && wgs % 8 != 0); }
+};
+// Int8 weights 64 x 64, five stages: four below K = 3,072. us on four / five: 511 rows of 2784 x 256 4.6 / 5.0, 675 of 2096 x 1024 8.4 /
+// 8.9, 2,025 of 560 x 2304 10.4 / 10.7; 89 of 2112 x 5376 13.7 / 12.5, 142 of 1648 x 8960 20.8 / 17.7. (Between 1,536 and 3,071 the
+// two are level on the whole: 160-256 tiles gain up to 6 %, more than 256 lose up to 6 %.)
+template <>
+struct iu8_pf_short<true, 64, 64, 2> {
+  static constexpr bool HAS = true;
+  static constexpr int WMW = 2, WNW = 2, TM = 1, TN = 1, ST = 4, KW = 1;
+  static __device__ __forceinline__ bool takes(int k, int) { return k < 3072; }
+};
 
 // The tiles of a dense launch on the cell, or on its form for a short K.
 template <bool W8, int WMW, int WNW, int TM, int TN, bool ACC, int ST, int OCC, bool DEEP, int KW>

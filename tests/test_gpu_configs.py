@@ -276,7 +276,8 @@ def test_tile_cells_of_two_k_waves(ctx, cell, M, N, K, grid):
         ctx.launch(d, bufs)
 
 
-@pytest.mark.parametrize("cell,K", [("w4_t128x128", 2048), ("w4_t128x128", 2176)])
+@pytest.mark.parametrize("cell,K", [("w4_t128x128", 2048), ("w4_t128x128", 2176), ("w8_t128x128", 2048), ("w8_t128x128", 2176),
+                                    ("w8_t128x128", 6144), ("w8_t64x64_s", 2944), ("w8_t64x64_s", 3072)])
 @pytest.mark.parametrize("M,N,grid", [(130, 272, 6), (257, 1040, 8), (300, 400, 7)])
 def test_tile_cells_either_side_of_their_short_k(ctx, cell, K, M, N, grid):
     """The cells that take another form on a short K, either side of the line, on grids in the order by XCD and out of it and on
