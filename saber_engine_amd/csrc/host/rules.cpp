@@ -624,16 +624,16 @@ uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant *
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
   struct Cell { const char *tile; double tops_per_cu, tile_us; };
   // quarter: the rate of the 128 x 128 tiles in the 256 x 256 cell's last round; few: a cell's constants at 65 to 1,023 rows
-  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, again, hbm_tbps, side_cap, quarter; Cell cells[11], few; };
+  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, again, hbm_tbps, side_cap, quarter; Cell cells[10], few; };
   static const Law W4 = {0.974, 90.000, 19.875, 1.422, 1.050, 3.113, 2.116, 8.799,
-                         {{"tn4_lbk64", 13.797, 3.223}, {"t256x320", 13.314, 6.002}, {"t256x224", 12.693, 14.000}, {"t128x320", 11.675, 2.893}, {"t256x160", 11.618, 7.995}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.905, 2.045}, {"t128x128_o2", 10.703, 2.096}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 5.698, 1.372}, {"t64x64_s", 5.504, 1.829}},
+                         {{"tn4_lbk64", 13.797, 3.223}, {"t256x320", 13.314, 6.002}, {"t128x320", 11.675, 2.893}, {"t256x160", 11.618, 7.995}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.905, 2.045}, {"t128x128_o2", 10.703, 2.096}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 5.698, 1.372}, {"t64x64_s", 5.504, 1.829}},
                          {"t128x256", 10.078, 1.844}};
   // up to 64 rows, which the lines above this estimate in `resolve` are drawn against
   static const Law W4_64 = {0.974, 90.000, 19.875, 1.422, 1.000, 3.113, 2.116, 8.799,
-                            {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t256x224", 13.814, 14.000}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}},
+                            {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}},
                             {"", 0.000, 0.000}};
   static const Law W8 = {4.419, 75.175, 18.116, 1.782, 1.000, 5.234, 1.935, 8.069,
-                         {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t256x224", 11.270, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}},
+                         {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}},
                          {"", 0.000, 0.000}};
   const Law &law = w8 ? W8 : m <= 64 ? W4_64 : W4;
   // the cells' variants, looked up once

@@ -490,6 +490,14 @@ def test_prefill_cells_of_the_benchmark_shapes():
         iu8.describe("macaq_iu8_pf_w4_tn4_lbk64", 256, 5120, 5120, ks=2)   # the prefill tile does not split K
 
 
+def test_256x224_cell_is_reached_by_name_only():
+    """The estimate does not hold the 256 x 224 cell, which lost to 256 x 256 wherever it was picked, last at a K past 24,000."""
+    for m, n, k in ((718, 13712, 27520), (2270, 4832, 24448), (8221, 1184, 25344), (1317, 16496, 26112), (786, 3632, 29056), (2404, 6032, 29568)):
+        assert iu8.resolve(iu8.W4, m, n, k).kernel != b"macaq_iu8_pf_w4_t256x224", (m, n, k)
+    d = iu8.describe("macaq_iu8_pf_w4_t256x224", 718, 13712, 27520)
+    assert d.block[0] == 512 and d.grid[0] == 186
+
+
 # ------------------------------------------------------------------ kernarg ABI
 
 def test_signatures_pack_exactly_like_the_reference_manifest():
