@@ -610,47 +610,52 @@ uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant *
 // cold (successive launches walk copies that exceed the memory-side cache; with warm weights the 64 x 64
 // cell overtakes the 64 x 128 one at 256 rows, which no layer of a model sees), and checked on shapes the fit had
 // not seen -- the served 27B graph's own 16384 x 5120, 14336 x 5120, 5120 x 6144 and 96 x 5120 at eight row counts,
-// which moved three small-cell rates and took the side-by-side term off the 64-row cells. The W4 rates were drawn again when
-// the 128- and 256-row cells got their k-waves (iu8_pf32.h): 1,336 shapes of 65 to 8,192 rows, 256 to 35,200 columns and K to
-// 17,408, every cell timed on weights from memory, half of them the grid of the served widths and half drawn at random. The
-// pick moved on 158 of them, 7 % faster there on average and none more than 1.6 % slower; on 109 of 1,200 further shapes, 6 %
-// faster, 3 of them 2-7 % slower (634 rows of 12160 x 2688 23.4 on 128 x 256, 25.0 on 128 x 128 two a CU). 128 x 256 has constants of
-// its own at 65 to 1,023 rows, where it is one round: from 1,024 rows of 5,120 columns the pick stays 128 x 128 two a CU although
-// 128 x 256 has become 5-7 % faster there (1,100 / 1,300 rows of 5120 x 17408 102 / 113 against 97 / 106). W8, output-side shapes
+// which moved three small-cell rates and took the side-by-side term off the 64-row cells.
+// The W4 rates are a fit to 2,549 shapes of 65 to 8,192 rows, 256 to 35,200 columns and K of 128 to 17,408, spread over the logarithm of
+// each and over the served widths, every cell timed on weights from memory; what it minimises is the time of the cell it picks
+// over the fastest one's, with three times the weight on what a shape loses against its pick before. The pick takes 0.9 % more than
+// the fastest cell over them (3.4 % with the rates before, which were drawn when the 128- and 256-row cells got their k-waves from
+// shapes with few short K among them, and took slower cells than the ones in use there: 611 rows of 14368 x 768 20.2 us on 128 x
+// 320 for 16.0 on 256 x 256, 125 of 288 x 128 3.6 on 64 x 128 for 3.2 on 64 x 64, 217 of 25984 x 2304 26.5 on 128 x 128 for 24.0). On 814
+// other shapes where the pick has moved it is 5 % faster than those rates' and 6 % than the ones' before the k-waves; slower than
+// either by more than 4 % on nine, three of them past a K of 17,408 (3,324 rows of 2016 x 18688 123 -> 140) and two of about 1,350 rows
+// of 14336 x 1024 (31 -> 33). 634 rows of 12160 x 2688 take 28.3 on 128 x 128 two a CU (28.5 on 128 x 256 as it was, 24.6 as it is).
+// 128 x 256 is held up to 1,023 rows (600 rows of 34816 x 5120 113 there, 119 on the pick, 126 before; 777 of 5120 x 17408 92 for 96):
+// from 1,024 the pick of a narrow output is 128 x 128 two a CU as before, although 128 x 256 has become 5 % faster (1,024 / 1,100 /
+// 1,300 rows of 5120 x 17408 100 / 103 / 119 against 95 / 98 / 110): there one rate cannot keep both. W8, output-side shapes
 // from 2,048 rows: every pick the fastest; at 1,025 to 1,280 rows up to 7 % off (256 x 160, 128 x 128 two a CU). The
 // reference keeps its band tables the same way
 // (crates/saber-kernels/src/macaq_iu8.rs:150-212). One table for both kinds had sent the int8-weight
 // O and down projections at 2,048 rows to the 128 x 320 cell, 17-22 % behind the 256 x 160 cell there.
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
-  struct Cell { const char *tile; double tops_per_cu, tile_us; };
-  // quarter: the rate of the 128 x 128 tiles in the 256 x 256 cell's last round; few: a cell's constants at 65 to 1,023 rows
-  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, again, hbm_tbps, side_cap, quarter; Cell cells[10], few; };
-  static const Law W4 = {0.974, 90.000, 19.875, 1.422, 1.050, 3.113, 2.116, 8.799,
-                         {{"tn4_lbk64", 13.797, 3.223}, {"t256x320", 13.314, 6.002}, {"t128x320", 11.675, 2.893}, {"t256x160", 11.618, 7.995}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.905, 2.045}, {"t128x128_o2", 10.703, 2.096}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 5.698, 1.372}, {"t64x64_s", 5.504, 1.829}},
-                         {"t128x256", 10.078, 1.844}};
+  // rows: the cell is held for launches of fewer (0: of any count)
+  struct Cell { const char *tile; double tops_per_cu, tile_us; uint32_t rows; };
+  // quarter: the rate of the 128 x 128 tiles in the 256 x 256 cell's last round (held while the others were fitted)
+  struct Law { double fixed_us, cu_gbps, l2_tbps, lone, hbm_tbps, side_cap, quarter; Cell cells[10]; };
+  static const Law W4 = {1.729, 90.000, 14.830, 23.134, 4.944, 2.018, 8.799,
+                         {{"tn4_lbk64", 13.270, 1.444}, {"t256x320", 12.890, 2.969}, {"t128x320", 12.932, 5.553}, {"t256x160", 11.387, 3.577}, {"t128x128", 7.955, 0.429}, {"t128x128_o2", 9.929, 0.709}, {"t64x128_s", 7.719, 0.442}, {"t64x64_s", 4.276, 0.226}, {"t128x256", 13.391, 9.456, 1024}}};
   // up to 64 rows, which the lines above this estimate in `resolve` are drawn against
-  static const Law W4_64 = {0.974, 90.000, 19.875, 1.422, 1.000, 3.113, 2.116, 8.799,
-                            {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}},
-                            {"", 0.000, 0.000}};
-  static const Law W8 = {4.419, 75.175, 18.116, 1.782, 1.000, 5.234, 1.935, 8.069,
-                         {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}},
-                         {"", 0.000, 0.000}};
+  static const Law W4_64 = {0.974, 90.000, 19.875, 1.422, 3.113, 2.116, 8.799,
+                            {{"tn4_lbk64", 14.007, 3.223}, {"t256x320", 13.568, 4.138}, {"t128x320", 11.147, 7.968}, {"t256x160", 11.173, 8.857}, {"t128x256", 9.046, 1.844}, {"t128x128", 8.799, 2.045}, {"t128x128_o2", 9.622, 3.231}, {"t128x64_s", 4.711, 1.952}, {"t64x128_s", 6.085, 2.027}, {"t64x64_s", 5.582, 1.829}}};
+  static const Law W8 = {4.419, 75.175, 18.116, 1.782, 5.234, 1.935, 8.069,
+                         {{"tn4_lbk64", 13.145, 0.244}, {"t256x320", 12.800, 0.000}, {"t128x320", 6.328, 2.194}, {"t256x160", 11.499, 0.000}, {"t128x256", 10.761, 3.251}, {"t128x128", 8.069, 0.427}, {"t128x128_o2", 8.619, 0.229}, {"t128x64_s", 4.123, 0.073}, {"t64x128_s", 6.003, 2.817}, {"t64x64_s", 5.960, 0.000}}};
   const Law &law = w8 ? W8 : m <= 64 ? W4_64 : W4;
   // the cells' variants, looked up once
   constexpr size_t NCELL = sizeof(Law::cells) / sizeof(Cell);
   using Variants = std::array<const PfVariant *, NCELL>;
   auto variants = [](const Law &l, const char *tag) {
-    Variants v;
-    for (size_t i = 0; i < NCELL; ++i) v[i] = pf_variant(fmt("macaq_iu8_pf_%s_%s", tag, l.cells[i].tile));
+    Variants v{};
+    for (size_t i = 0; i < NCELL && l.cells[i].tile; ++i) v[i] = pf_variant(fmt("macaq_iu8_pf_%s_%s", tag, l.cells[i].tile));
     return v;
   };
-  static const Variants V4 = variants(W4, "w4"), V8 = variants(W8, "w8");
+  static const Variants V4 = variants(W4, "w4"), V4_64 = variants(W4_64, "w4"), V8 = variants(W8, "w8");
+  const Variants &cells = w8 ? V8 : m <= 64 ? V4_64 : V4;
   const PfVariant *best = nullptr;
   double best_t = 0;
   for (size_t i = 0; i < NCELL; ++i) {
-    const Cell &c = m < 1024 && !strcmp(law.cells[i].tile, law.few.tile) ? law.few : law.cells[i];
-    const PfVariant *v = (w8 ? V8 : V4)[i];
-    if (!v) continue;
+    const Cell &c = law.cells[i];
+    const PfVariant *v = cells[i];
+    if (!v || (c.rows && m >= c.rows)) continue;
     const double bm = v->block_m(), bn = v->block_n();
     const uint64_t tiles = (uint64_t)((n + v->block_n() - 1) / v->block_n()) * ((m + v->block_m() - 1) / v->block_m());
     const uint64_t grid = std::min<uint64_t>(tiles, (uint64_t)CU_COUNT * v->occ);
@@ -664,18 +669,15 @@ const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k) {
     // ... and a few rows past the last whole 256 as thin tiles (int4 weights: the estimate of the int8 cells is drawn without)
     if (!strcmp(c.tile, "tn4_lbk64") && !w8 && tiles < (1u << 20) && k < (1u << 30)) {
       const iu8_pf_plan plan = iu8_pf_plan256((int)m, (int)((n + 255) / 256), (int)grid, (int)k, w8);
-      if (plan.thin) cu_tiles = std::min(cu_tiles, plan.cost * 0.0108);  // (a margin: level picks stay as they were)
+      if (plan.thin) cu_tiles = std::min(cu_tiles, plan.cost * 0.0101);  // (in tiles, with the fit's factor)
     }
     const double tile_bytes = bm * k + bn * k * (w8 ? 1.0 : 0.5);
     const double t_mfma = cu_tiles * bm * bn * k * 2.0 / (c.tops_per_cu * 1e6);
     const double t_cu = cu_tiles * tile_bytes / (law.cu_gbps * 1e3);
     const double t_l2 = (double)tiles * tile_bytes / (law.l2_tbps * 1e6);
     // the two-a-CU 128 x 128 cell alone on a CU (no more workgroups than CUs) has four waves to hide
-    // its latencies with and measured well behind the eight-wave 128 x 128 cell there; a second round of it (`again`, int4
-    // weights: 5 %) is dearer than its rate says: without the factor 300-384 rows of 34816 x 5120 went to it from 256 x 320, and
-    // a layer of 300 rows took 360 us (348 with the rates before; with the factor 337 against 344 in another run)
-    const bool o2 = !strcmp(c.tile, "t128x128_o2");
-    const double lone = o2 && grid <= CU_COUNT ? law.lone : o2 && per_wg > 1 ? law.again : 1.0;
+    // its latencies with and measured well behind the eight-wave 128 x 128 cell there
+    const double lone = !strcmp(c.tile, "t128x128_o2") && grid <= CU_COUNT ? law.lone : 1.0;
     // cold weights: the row tiles that run side by side on one column block each fetch it from memory -- those of the
     // 128- and 256-row cells; the 64-row cells' neighbours share a column block's lines (fetch over operands 1.5-1.65 at
     // four row tiles by the counters, and the wide projections of the served graph at 65-128 rows: 16.5-18.8 us on

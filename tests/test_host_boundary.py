@@ -490,6 +490,18 @@ def test_prefill_cells_of_the_benchmark_shapes():
         iu8.describe("macaq_iu8_pf_w4_tn4_lbk64", 256, 5120, 5120, ks=2)   # the prefill tile does not split K
 
 
+def test_int4_tile_cells_that_a_refit_had_slowed():
+    """Shapes, most of a short K, that rates drawn from long ones gave slower cells than the ones before them (us there / on the pick
+    here): the launch law is back on the earlier cell, or on one at least as fast."""
+    for m, n, k, tile in ((611, 14368, 768, "tn4_lbk64"), (1397, 6784, 640, "tn4_lbk64"),      # 20.2 / 16.0, 17.0 / 14.6
+                          (125, 288, 128, "t64x64_s"), (192, 4032, 256, "t64x64_s"),           # 3.6 / 3.2, 4.2 / 3.8
+                          (420, 7856, 128, "t128x128"), (66, 30864, 512, "t128x128"), (191, 14080, 384, "t128x128"),  # 5.8 / 5.1, 7.9 / 6.7, 7.1 / 6.3
+                          (802, 18368, 256, "t128x128_o2"), (573, 14192, 256, "t64x128_s"),    # 15.7 / 12.7, 12.0 / 9.7
+                          (217, 25984, 2304, "t128x128_o2"), (149, 23440, 10368, "t128x256"),  # 26.5 / 21.6, 78.2 / 61.6
+                          (777, 5120, 17408, "t128x256"), (200, 34816, 5120, "t256x160")):     # 96.0 / 92.4; as before
+        assert iu8.resolve(iu8.W4, m, n, k).kernel.decode() == "macaq_iu8_pf_w4_" + tile, (m, n, k)
+
+
 def test_256x224_cell_is_reached_by_name_only():
     """The estimate does not hold the 256 x 224 cell, which lost to 256 x 256 wherever it was picked, last at a K past 24,000."""
     for m, n, k in ((718, 13712, 27520), (2270, 4832, 24448), (8221, 1184, 25344), (1317, 16496, 26112), (786, 3632, 29056), (2404, 6032, 29568)):
