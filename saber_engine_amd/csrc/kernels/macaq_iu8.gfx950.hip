@@ -101,14 +101,27 @@ IU8_DECQ1(macaq_iu8_decq_w4_r1, false, 8, 16, 4)
 IU8_DECQ1(macaq_iu8_decq_w8_r1, true, 8, 16, 2)
 #undef IU8_DECQ1
 
+// The launch law gives the split and the fused-quant forms the tile, threads and workgroups a CU of the cell they are named after,
+// whatever k-waves that cell has: their own geometry has to be the same.
+struct iu8_geo {
+  int bm, bn, threads, occ;
+  constexpr bool operator==(const iu8_geo &o) const { return bm == o.bm && bn == o.bn && threads == o.threads && occ == o.occ; }
+};
+#define IU8_PF_VARIANT(name, W8, WMW, WNW, TM, TN, ACC, ST, OCC, DEEP, KW) \
+  constexpr iu8_geo name##_geo{WMW * TM * 32, WNW * TN * 32, WMW * WNW * KW * 64, OCC};
+#include "iu8_variants.def"
+#define IU8_SAME_LAUNCH(cell, WMW, WNW, TM, TN, OCC) \
+  static_assert(macaq_iu8_pf_##cell##_geo == iu8_geo{WMW * TM * 32, WNW * TN * 32, WMW * WNW * 64, OCC}, "the launch law's geometry for the cell");
+
 // Cells with K split over gridDim.z (symbol suffix `_ks`, the decode kernarg list: the two workspaces
 // in front of c), for the rows between the regimes, where few tiles leave CUs idle. Measured, the
 // partials' way through memory (ks * M * N * 4 bytes out and back) costs more than the idle CUs on
 // every shape but deep, narrow linears at 49-128 rows, the one band where the launch law picks a
 // split form (the 64 x 128 cell); the others are kept, tested and reachable by name like the decode split.
-#define IU8_PF32K(name, W8, WMW, WNW, TM, TN, ST, OCC, DEEP)                                                       \
+#define IU8_PF32K(cell, W8, WMW, WNW, TM, TN, ST, OCC, DEEP)                                                       \
+  IU8_SAME_LAUNCH(cell, WMW, WNW, TM, TN, OCC)                                                                     \
   extern "C" __global__ __launch_bounds__(WMW * WNW * 64)                                                         \
-      __attribute__((amdgpu_waves_per_eu(WMW * WNW * OCC / 4, WMW * WNW * OCC / 4))) void name(                    \
+      __attribute__((amdgpu_waves_per_eu(WMW * WNW * OCC / 4, WMW * WNW * OCC / 4))) void macaq_iu8_pf_##cell##_ks(                    \
       const unsigned char *__restrict__ a, const unsigned char *__restrict__ w, const float *__restrict__ as,     \
       const float *__restrict__ ws, int *__restrict__ decode_partial, int *__restrict__ decode_counter,           \
       unsigned short *__restrict__ c, int m, int n, int k) {                                                       \
@@ -125,11 +138,11 @@ IU8_DECQ1(macaq_iu8_decq_w8_r1, true, 8, 16, 2)
         },                                                                                                         \
         gridDim.z > 1 ? decode_partial : nullptr, decode_counter);                                                 \
   }
-IU8_PF32K(macaq_iu8_pf_w4_t128x128_ks, false, 4, 2, 1, 2, 3, 1, false)
-IU8_PF32K(macaq_iu8_pf_w8_t128x128_ks, true, 4, 2, 1, 2, 3, 1, false)
-IU8_PF32K(macaq_iu8_pf_w4_t256x160_ks, false, 8, 1, 1, 5, 3, 1, false)
-IU8_PF32K(macaq_iu8_pf_w8_t256x160_ks, true, 8, 1, 1, 5, 3, 1, false)
-IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 1, 4, 2, 1, 5, 2, true)
+IU8_PF32K(w4_t128x128, false, 4, 2, 1, 2, 3, 1, false)
+IU8_PF32K(w8_t128x128, true, 4, 2, 1, 2, 3, 1, false)
+IU8_PF32K(w4_t256x160, false, 8, 1, 1, 5, 3, 1, false)
+IU8_PF32K(w8_t256x160, true, 8, 1, 1, 5, 3, 1, false)
+IU8_PF32K(w4_t64x128_s, false, 1, 4, 2, 1, 5, 2, true)
 #undef IU8_PF32K
 #define IU8_WIDE_VARIANT(name, TM, W8, NT, KW, D)                                                                     \
   extern "C" __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4, KW / 4))) void name(  \
@@ -154,9 +167,10 @@ IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 1, 4, 2, 1, 5, 2, true)
 // does not pick them: they are kept, tested and reachable by name. The 256 x 256 cell has no registers
 // left for the pieces in flight (it spilt, and still was the least slow at 2.05-2.3x), so it has no
 // fused form here.
-#define IU8_PFQ(name, W8, WMW, WNW, TM, TN, ST, OCC)                                                               \
+#define IU8_PFQ(cell, W8, WMW, WNW, TM, TN, ST, OCC)                                                               \
+  IU8_SAME_LAUNCH(cell, WMW, WNW, TM, TN, OCC)                                                                     \
   extern "C" __global__ __launch_bounds__(WMW * WNW * 64)                                                         \
-      __attribute__((amdgpu_waves_per_eu(WMW * WNW * OCC / 4, WMW * WNW * OCC / 4))) void name(                    \
+      __attribute__((amdgpu_waves_per_eu(WMW * WNW * OCC / 4, WMW * WNW * OCC / 4))) void macaq_iu8_pfq_##cell(                    \
       const unsigned short *__restrict__ x, const unsigned char *__restrict__ w, const float *__restrict__ as,    \
       const float *__restrict__ ws, unsigned short *__restrict__ c, int m, int n, int k) {                         \
     constexpr int BM = WMW * TM * 32, BN = WNW * TN * 32;                                                          \
@@ -170,9 +184,9 @@ IU8_PF32K(macaq_iu8_pf_w4_t64x128_s_ks, false, 1, 4, 2, 1, 5, 2, true)
           return true;                                                                                             \
         });                                                                                                        \
   }
-IU8_PFQ(macaq_iu8_pfq_w4_t128x128, false, 4, 2, 1, 2, 3, 1)
-IU8_PFQ(macaq_iu8_pfq_w8_t128x128, true, 4, 2, 1, 2, 3, 1)
-IU8_PFQ(macaq_iu8_pfq_w4_t128x128_o2, false, 2, 2, 2, 2, 3, 2)
-IU8_PFQ(macaq_iu8_pfq_w4_t256x160, false, 8, 1, 1, 5, 3, 1)
-IU8_PFQ(macaq_iu8_pfq_w8_t256x160, true, 8, 1, 1, 5, 3, 1)
+IU8_PFQ(w4_t128x128, false, 4, 2, 1, 2, 3, 1)
+IU8_PFQ(w8_t128x128, true, 4, 2, 1, 2, 3, 1)
+IU8_PFQ(w4_t128x128_o2, false, 2, 2, 2, 2, 3, 2)
+IU8_PFQ(w4_t256x160, false, 8, 1, 1, 5, 3, 1)
+IU8_PFQ(w8_t256x160, true, 8, 1, 1, 5, 3, 1)
 #undef IU8_PFQ
