@@ -465,8 +465,8 @@ int saber_iu8_launch(saber_iu8_ctx *ctx, const saber_iu8_desc *d, const saber_iu
   const uint64_t threads = (uint64_t)d->block[0] * std::max(d->block[1], 1u) * std::max(d->block[2], 1u);
   uint32_t block[3] = {d->block[0], d->block[1], d->block[2]};
   if (threads != it->second.max_threads) {
-    // A tile cell derives all it does from its grid and m, n, k: a descriptor of 128 x 320 or 128 x 256 laid out when their wave
-    // tiles had one wave each (256 threads) runs on the k-waves they have now.
+    // A tile cell derives all it does from its grid and m, n, k. Descriptors of 256 threads, laid out when every wave tile had one
+    // wave, run on the k-waves of today: W4 128 x 320 and 128 x 256, W8 128 x 256. (The other cells with k-waves kept their 512.)
     const PfVariant *v = pf_variant(d->kernel);
     if (v && v->kw > 1 && v->block_m() == 128 && v->block_n() >= 256 && threads * v->kw == it->second.max_threads) block[0] = it->second.max_threads, block[1] = block[2] = 1;
   }

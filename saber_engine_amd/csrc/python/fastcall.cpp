@@ -3,8 +3,8 @@
 // An operator is a launch, 5 us on the card for a decode linear, and is called from a serving loop: a call that takes longer
 // on the host than its kernel is what the loop waits for. ctypes converts a dozen arguments one Python object at a time, 1.7 us
 // a call; here an argument is read by the type the header declares, 0.7 us with the descriptor's layout. (With the layout's
-// share, util.h: a one-row linear of 5120 x 5120 in a loop of calls 8.4 -> 7.4 us, its kernel 5.3; 16 rows, quantiser and GEMM,
-// 13.0 -> 11.3.) The conversions are ctypes' own for what a caller
+// share, util.h: a one-row linear of 5120 x 5120 in a loop of calls 7.5-8.1 -> 6.5-7.2 us, its kernel 5; 16 rows, quantiser and
+// GEMM, 11.6-12.7 -> 9.7-11.0.) The conversions are ctypes' own for what a caller
 // passes: a pointer is an int or None, a number an int, a float a float, each taken modulo its width; the routed operators'
 // tables are the structure itself (an address in their place is refused, as ctypes refuses it). Anything else in an argument's
 // place (a ctypes object, a bool, another count of arguments) sends the whole call, its arguments as they came, to the ctypes

@@ -387,20 +387,31 @@ PF_CELLS = {  # tile suffix -> (rows, columns, workgroups a CU, threads)
     "tn4_lbk64": (256, 256, 1, 512), "t256x224": (256, 224, 1, 512), "t256x160": (256, 160, 1, 512),
     "t128x128": (128, 128, 1, 512), "t128x128_o2": (128, 128, 2, 256), "t128x64_o2": (128, 64, 2, 256),
     "t128x64_s": (128, 64, 1, 256), "t64x128_s": (64, 128, 2, 256), "t64x64_s": (64, 64, 2, 256),
-    "t256x320": (256, 320, 1, 512), "t128x320": (128, 320, 1, 256), "t128x256": (128, 256, 1, 256)}
+    "t256x320": (256, 320, 1, 512), "t128x320": (128, 320, 1, 512), "t128x256": (128, 256, 1, 512)}
+PF_CELLS_W8 = dict(PF_CELLS, t128x320=(128, 320, 1, 256), t128x160=(128, 160, 1, 256))  # (one wave a wave tile)
+
 
 
 def test_prefill_launch_is_persistent_and_covers_the_output():
     for wk, tag in ((iu8.W4, "w4"), (iu8.W8, "w8")):
-        for (m, n, k) in [(256, 5120, 5120), (2048, 34816, 5120), (300, 304, 640), (8192, 7168, 5120), (65, 16, 128)]:
+        for (m, n, k) in [(256, 5120, 5120), (2048, 34816, 5120), (300, 304, 640), (8192, 7168, 5120), (65, 16, 128), (2048, 5120, 5120),
+                          (777, 5120, 17408), (1024, 5120, 17408), (256, 34816, 5120)]:
             d = iu8.resolve(wk, m, n, k)
             name = d.kernel.decode()
             assert name.startswith(f"macaq_iu8_pf_{tag}_")
-            bm, bn, occ, thr = PF_CELLS[name[len(f"macaq_iu8_pf_{tag}_"):]]
+            bm, bn, occ, thr = (PF_CELLS_W8 if wk == iu8.W8 else PF_CELLS)[name[len(f"macaq_iu8_pf_{tag}_"):]]
             tiles = -(-n // bn) * -(-m // bm)
             # one workgroup (or two) a CU walks the tiles; the kernel derives the tile grid from m, n
             assert d.grid[0] == min(tiles, 256 * occ) and d.grid[1] == 1 and d.grid[2] == 1 and d.block[0] == thr
             assert d.n_workspaces == 0 and d.ks == 1
+
+
+def test_every_tile_cell_has_its_threads():
+    """By name, the threads a workgroup of every cell of the table, those with k-waves among them."""
+    for tag, cells in (("w4", PF_CELLS), ("w8", {c: v for c, v in PF_CELLS_W8.items() if c != "t256x224"})):
+        for cell, (bm, bn, occ, thr) in cells.items():
+            d = iu8.describe(f"macaq_iu8_pf_{tag}_{cell}", 300, 5120, 2176)
+            assert d.block[0] == thr and d.grid[0] == min(-(-300 // bm) * -(-5120 // bn), 256 * occ), (tag, cell)
 
 
 def test_lines_of_the_launch_law_at_17_to_64_rows():
