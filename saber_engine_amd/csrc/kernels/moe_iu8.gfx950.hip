@@ -23,6 +23,7 @@
 //        one rounding (crates/saber-kernels/hip/moe_route.hip:287-329; abi.rs:377-385).
 #include "iu8_gemm.h"
 #include "iu8_pf32.h"
+#include "moe_deal.h"
 
 #define MOE_E 128
 #define MOE_TOPK 8
@@ -728,19 +729,19 @@ MOE_GROUPED_DEC(moe_iu8_grouped_w4_decpb_g1, true, 4, 8, 8, 2, 0, 1, 5)
 // (tile, column block) of the live tiles, column blocks of one tile on neighbouring workgroups, the
 // load stream running across items (iu8_pf32.h). grid [256, 1, 1]. Every workgroup first sorts the
 // tiles the same way, those of more than MOE_LIGHT_ROWS rows first in table order, the light ones
-// after them; the walk is static (item = workgroup + r * gridDim.x), so each kind is dealt evenly.
+// after them; the walk is static, each kind dealt by moe_deal.h.
 //
 // An expert's last tile is often nearly empty. On the tile cell such a tile still moves whole stages
 // of mostly dead rows behind a barrier a step: measured, some 70 % of a full tile's time for a
-// twentieth of its work. The two-cell form (LIGHT) runs the light tiles on a second cell in the same
-// LDS, 64 rows x 256 columns, whose small stages keep four steps of loads in flight and move no dead
+// twentieth of its work. So the light tiles run on a second cell in the same LDS, 64 rows x 256
+// columns, whose small stages keep four steps of loads in flight and move no dead
 // rows; its K steps start at a depth that differs from item to item (iu8_tile::rot), which spreads
 // the weight streams of the light items over the memory channels (512 tokens, gate+up: 187 -> 160 us).
 // The light cell's eight waves stand side by side, each 64 rows x 32 columns: a W4 operand is unpacked
 // once and serves both row blocks (on 2 x 4 waves every weight fragment was read from LDS and unpacked
 // twice, and an item of mostly few rows is bound by that issue work once its weights arrive), and rows,
-// activation scales and weight scales of the light items come from tables in LDS (iu8_tabs), filled
-// beside the item table: no ordinary load stands between two items and drains the stream (a layer at
+// activation scales and weight scales of the light items come from tables in LDS (iu8_tabs):
+// no ordinary load stands between two items and drains the stream (a layer at
 // 120 / 300 / 1,000 / 2,000 tokens: 269 / 277 / 337 / 493 us on 2 x 4 waves in the deep form, 259 / 266 /
 // 335 / 482 on 8 waves side by side, 252 / 261 / 329 / 479 with the tables). Light tiles together are bound by the memory rate,
 // the heavy ones by the matrix pipes, so a workgroup runs its light items between two parts of its
@@ -748,26 +749,43 @@ MOE_GROUPED_DEC(moe_iu8_grouped_w4_decpb_g1, true, 4, 8, 8, 2, 0, 1, 5)
 // workgroup down: at any time a slice of every XCD's CUs streams light tiles under the others'
 // matrix work (2,048 tokens on 128-row tiles: 633 -> 577 us a layer against 639 with the light items
 // last). An item's descriptor hangs on a chain of dependent loads (order -> tile table -> expert
-// pointers), so a workgroup resolves its items up front, one lane an item, into a table in LDS.
-// The 128-row kernels are two-cell (256 to 2,048 tokens: 3 to 9 % a layer). The 256-row kernels are
-// not: at 4,096 tokens the light tiles' weights come from memory a second time whichever cell asks
-// (timestamps: a light item takes 20-28 us there against 4 with its weights cached, a heavy round
-// 62-82 us with light items beside it against 63 without), the layer gained 2 %, and launches with no
-// light tile (1,536 to 2,048 tokens) lost 2 to 4 % to the two-cell kernel's heavier item switch.
+// pointers), so a workgroup resolves its items up front, one lane an item, into a table in LDS, and
+// takes one over in two 16-byte reads at a crossing (eight dwords one after another, and the walk's numbers
+// beside them: a layer at 300 / 1,300 / 1,792 / 2,048 tokens 262 / 405 / 416 / 477 us, now 258 / 395 / 411 / 465).
+//
+// The 256-row kernels are two-cell as well. At 4,096 tokens half of the experts have a light remainder tile, whose
+// weights come from memory a second time: on the tile cell, two steps ahead, an item waited 20-28 us for its 512 KB,
+// the light cell has twice the bytes in flight (a layer at 4,096 / 4,000 tokens with a shared expert 816 / 866 -> 766 / 817 us).
+// With the light cell's state in registers beside the 256 x 256 tile cell's the compiler spills, and every crossing between two
+// heavy items paid for it (2,048 tokens, no light tile at all: 468 -> 489). It has two registers of spills left: everything that
+// is made of the thread's index in front of the walk is opaque to the optimiser, the light items' tables lie
+// behind their cell's stages and are filled when they are due, and a launch of more items than the table holds
+// (64 heavy or 12 light a workgroup) does not pass over it again and again but runs on the tile cell alone.
+// (Row maps of the heavy items in LDS as well, so that a crossing reads no row map from memory: 32 more registers of spills, 1 % slower.)
 #define MOE_ORDER_CAP 4096  // tiles the ordering holds in LDS; beyond, table order on the big cell
 #define MOE_LIGHT_ROWS 64
 #define MOE_LIGHT_ST 5
-#define MOE_HEAVY_ROUNDS 8  // rounds of items a workgroup resolves at a time: the item table in LDS
-#define MOE_LIGHT_ROUNDS 8
-struct moe_item {
-  int row0, rows, nt0, rot;  // rows < 0: no item
+#define MOE_HEAVY_ROUNDS 8  // rounds of items a workgroup of the 128-row kernels resolves at a time: the item table in LDS
+#define MOE_LIGHT_ROUNDS 12
+struct __attribute__((aligned(16))) moe_item {
+  int row0, rows, nt0, rot;  // rows < 0: no item, and the end of a list of them
   const unsigned char *W;
   const float *ws;
 };
+// threadIdx.x, opaque to the optimiser: what is made of it in front of a K loop is not carried through that loop in registers
+static __device__ __forceinline__ int moe_tid() {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+// Up to NTHR tiles their descriptors come along (`desc`, by place in the order): a thread asks for its tile's three table entries
+// at once and for the expert's pointers while the counts meet, so an item costs one round trip to memory less.
 template <int NTHR>
-static __device__ __forceinline__ int moe_tile_order(const int *__restrict__ tile_rows, int nt, unsigned short *s_order) {
+static __device__ __forceinline__ int moe_tile_order(const int *__restrict__ tile_rows, const int *__restrict__ tile_expert,
+                                                     const int *__restrict__ tile_row0, const unsigned long long *__restrict__ xptr,
+                                                     int nt, unsigned short *s_order, moe_item *desc) {
   __shared__ int s_w[NTHR / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = moe_tid(), lane = tid & 63, wave = tid >> 6;
   auto block_sum = [&](int v, int &before) {  // sum over the workgroup; `before` = the waves ahead of this one
     if (lane == 0) s_w[wave] = v;
     __syncthreads();
@@ -782,11 +800,27 @@ static __device__ __forceinline__ int moe_tile_order(const int *__restrict__ til
     __syncthreads();
     return all;
   };
+  if (nt <= NTHR) {
+    const int t = min(tid, nt - 1);
+    const int rows = tile_rows[t], row0 = tile_row0[t], e = tile_expert[t];
+    const unsigned long long wp = xptr[2 * e], sp = xptr[2 * e + 1];
+    const bool h = tid < nt && rows > MOE_LIGHT_ROWS;
+    const unsigned long long b = __ballot(h);
+    int before;
+    const int total = __builtin_amdgcn_readfirstlane(block_sum(__popcll(b), before));
+    const int hb = before + __popcll(b & ((1ull << lane) - 1ull)), slot = h ? hb : total + (tid - hb);
+    if (tid < nt) {
+      s_order[slot] = (unsigned short)tid;
+      desc[slot] = moe_item{row0, rows, 0, 0, (const unsigned char *)wp, (const float *)sp};
+    }
+    __syncthreads();
+    return total;
+  }
   int mine = 0, unused;
   for (int t = tid; t < nt; t += NTHR) mine += tile_rows[t] > MOE_LIGHT_ROWS;
 #pragma unroll
   for (int o = 32; o; o >>= 1) mine += __shfl_xor(mine, o, 64);
-  const int heavy_total = block_sum(mine, unused);
+  const int heavy_total = __builtin_amdgcn_readfirstlane(block_sum(mine, unused));
   int run = 0;  // heavy tiles before this chunk
   for (int base = 0; base < nt; base += NTHR) {
     const int t = base + tid;
@@ -801,186 +835,140 @@ static __device__ __forceinline__ int moe_tile_order(const int *__restrict__ til
   __syncthreads();
   return heavy_total;
 }
-// one cell, items in the sorted order
 // Workgroup b of a grid of G in the order in which an XCD's workgroups follow each other: b % 8 is the XCD (the
 // hardware deals consecutive ids round-robin), so XCD x holds positions x * G/8 ... of the walk. A grid that is not
 // whole eighths keeps its ids.
 static __device__ __forceinline__ int moe_xcd_run(unsigned b, int G) {
   return (G & 7) == 0 ? (int)(b & 7) * (G >> 3) + (int)(b >> 3) : (int)b;
 }
-#define MOE_ONE_ITEMS 64  // items a workgroup resolves up front (16,384 items a launch of 256 workgroups)
-template <int GATHER, int WMW, int WNW, int TM, int TN, int ST>
-static __device__ __forceinline__ void moe_grouped_pf_one(
+// two cells: heavy items on the tile cell, light ones on the small cell between two parts of them. A workgroup resolves HR heavy
+// and MOE_LIGHT_ROUNDS light items at a time; a launch of more runs in as many passes (PASSES), or as a whole on the tile cell
+// with its items resolved as it goes.
+template <int GATHER, int WMW, int WNW, int TM, int TN, int ST, int HR, int COST, bool PASSES>
+static __device__ __forceinline__ void moe_grouped_pf(
     const unsigned char *__restrict__ a, const unsigned long long *__restrict__ xptr, const int *__restrict__ tile_expert,
     const int *__restrict__ tile_row0, const int *__restrict__ tile_rows, const int *__restrict__ row_tok,
     const int *__restrict__ meta, const float *__restrict__ as, unsigned short *__restrict__ c, int n, int k) {
-  constexpr int BN = WNW * TN * 32;
-  static_assert(BN == 256 && WMW * WNW == 8, "both cells are 8 waves and 256 columns wide");
-  __shared__ unsigned short s_order[MOE_ORDER_CAP];
-  __shared__ moe_item s_item[MOE_ONE_ITEMS];
-  __shared__ __attribute__((aligned(1024))) iu8_u8 lds[iu8_pf32_lds_bytes<false, WMW, WNW, TM, TN, ST, true>()];  // one block for both walks below
-  const int nt = meta[0], gx = (n + BN - 1) / BN, total = nt * gx;
-  const bool ordered = nt <= MOE_ORDER_CAP;
-  if (ordered) moe_tile_order<WMW * WNW * 64>(tile_rows, nt, s_order);
-  // Consecutive workgroup ids are dealt round-robin over the 8 XCDs, consecutive item ids are the column blocks of
-  // one tile. With a grid of whole eighths an XCD's workgroups take a run of item ids (`moe_xcd_run`), so a tile's
-  // column blocks share the tile's rows in one L2, or two (dealt by workgroup id they spread over all eight and
-  // every XCD fetched the rows for itself: the L2-miss fetch of a launch at 4,096 tokens was twice its operands).
-  const int G = gridDim.x, wv = moe_xcd_run(blockIdx.x, G);
-  const int rounds = (total + G - 1) / G;
-  auto resolve = [&](int q, moe_item &it) {  // this workgroup's item of round q; false past its last
-    const int j = wv + q * G;
-    const int slot = j / gx, bx = j % gx;
-    if (slot >= nt) return false;
-    const int tile = ordered ? (int)s_order[slot] : slot;
-    const int e = tile_expert[tile];
-    it = moe_item{tile_row0[tile], min(tile_rows[tile], WMW * TM * 32), bx * (BN / 16), 0,
-                  (const unsigned char *)xptr[2 * e], (const float *)xptr[2 * e + 1]};
-    return true;
-  };
-  if (rounds <= MOE_ONE_ITEMS) {
-    // An item's descriptor hangs on a chain of dependent loads (order -> tile table -> expert pointers);
-    // fetched where the load stream crosses into the item, every link drains the stream. The
-    // workgroup's items are resolved here instead, one lane an item, into a table in LDS.
-    const int q = threadIdx.x;
-    if (q < rounds) {
-      moe_item it{0, -1, 0, 0, nullptr, nullptr};
-      resolve(q, it);
-      s_item[q] = it;
-    }
-    __syncthreads();
-    iu8_pf32_run<false, WMW, WNW, TM, TN, false, ST, false, true, GATHER == 2, true>(a, as, c, n, k, [&](int r, iu8_tile &t) {
-      if (r >= rounds) return false;
-      const volatile int *p32 = (const volatile int *)&s_item[r];
-      auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(p32[i]); };
-      if (u(1) < 0) return false;
-      const unsigned long long wp = (unsigned)u(4) | ((unsigned long long)(unsigned)u(5) << 32);
-      const unsigned long long sp = (unsigned)u(6) | ((unsigned long long)(unsigned)u(7) << 32);
-      t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, u(0), u(1)}, 0, u(2), (const unsigned char *)wp, (const float *)sp};
-      return true;
-    }, nullptr, nullptr, lds);
-    return;
-  }
-  iu8_pf32_run<false, WMW, WNW, TM, TN, false, ST, false, true, GATHER == 2, true>(a, as, c, n, k, [&](int r, iu8_tile &t) {
-    moe_item it;
-    if (r >= rounds || !resolve(r, it)) return false;
-    t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, it.row0, it.rows}, 0, it.nt0, it.W, it.ws};
-    return true;
-  }, nullptr, nullptr, lds);
-}
-// two cells: heavy items on the tile cell, light ones on the small cell between two parts of them
-template <int GATHER, int WMW, int WNW, int TM, int TN, int ST>
-static __device__ __forceinline__ void moe_grouped_pf_two(
-    const unsigned char *__restrict__ a, const unsigned long long *__restrict__ xptr, const int *__restrict__ tile_expert,
-    const int *__restrict__ tile_row0, const int *__restrict__ tile_rows, const int *__restrict__ row_tok,
-    const int *__restrict__ meta, const float *__restrict__ as, unsigned short *__restrict__ c, int n, int k) {
-  constexpr int BN = WNW * TN * 32;
+  constexpr int BN = WNW * TN * 32, NTHR = WMW * WNW * 64;
   static_assert(BN == 256 && WMW * WNW == 8, "both cells are 8 waves and 256 columns wide");
   constexpr int LB = iu8_pf32_lds_bytes<false, WMW, WNW, TM, TN, ST, true>();
   constexpr int LL = iu8_pf32_lds_bytes<false, 1, 8, 2, 1, MOE_LIGHT_ST>();
-  __shared__ __attribute__((aligned(1024))) iu8_u8 lds[LB > LL ? LB : LL];
+  constexpr int LT = MOE_LIGHT_ROUNDS * (2 * MOE_LIGHT_ROWS + BN) * 4;  // the light items' tables, behind the light cell's stages
+  __shared__ __attribute__((aligned(1024))) iu8_u8 lds[LB > LL + LT ? LB : LL + LT];
   __shared__ unsigned short s_order[MOE_ORDER_CAP];
-  /* the walk's numbers and this workgroup's resolved items live in LDS */
-  __shared__ int s_par[4];
-  __shared__ moe_item s_item[MOE_HEAVY_ROUNDS + MOE_LIGHT_ROUNDS];
-  __shared__ int s_row[MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS];
-  __shared__ float s_am[MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS];
-  __shared__ __attribute__((aligned(16))) float s_ws[MOE_LIGHT_ROUNDS * BN];
-  auto par = [&](int i) { return __builtin_amdgcn_readfirstlane(((volatile int *)s_par)[i]); };
+  __shared__ moe_item s_item[HR + MOE_LIGHT_ROUNDS + 3];  // this workgroup's resolved items
+  float *const s_ws = (float *)(lds + LL), *const s_am = s_ws + MOE_LIGHT_ROUNDS * BN;
+  int *const s_row = (int *)(s_am + MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS);
+  // s_item: the heavy items of part 0, an end, those of part 1, an end, the light items, an end
   auto item = [&](int q, iu8_tile &t, int tab = 0) {
-    const volatile int *p32 = (const volatile int *)&s_item[q];
-    auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(p32[i]); };
-    if (u(1) < 0) return false;
-    const unsigned long long wp = (unsigned)u(4) | ((unsigned long long)(unsigned)u(5) << 32);
-    const unsigned long long sp = (unsigned)u(6) | ((unsigned long long)(unsigned)u(7) << 32);
-    t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, u(0), u(1)}, 0, u(2), (const unsigned char *)wp, (const float *)sp, 0, u(3), tab};
+    const iu8_v4i lo = *(const iu8_v4i *)&s_item[q].row0, hi = *(const iu8_v4i *)&s_item[q].W;
+    auto u = [&](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    if (u(lo[1]) < 0) return false;
+    const unsigned long long wp = (unsigned)u(hi[0]) | ((unsigned long long)(unsigned)u(hi[1]) << 32);
+    const unsigned long long sp = (unsigned)u(hi[2]) | ((unsigned long long)(unsigned)u(hi[3]) << 32);
+    t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, u(lo[0]), u(lo[1])}, 0, u(lo[2]), (const unsigned char *)wp, (const float *)sp, 0, u(lo[3]), tab};
     return true;
   };
   const int nt = meta[0];
+  if (nt <= 0) return;
   const bool ordered = nt <= MOE_ORDER_CAP;
-  const int heavy = ordered ? moe_tile_order<WMW * WNW * 64>(tile_rows, nt, s_order) : nt;
-  /* a launch of more rounds than the item table holds runs in epochs of that many */
+  const int heavy = ordered ? moe_tile_order<NTHR>(tile_rows, tile_expert, tile_row0, xptr, nt, s_order, (moe_item *)lds) : nt;
+  const int gx = (n + BN - 1) / BN;
+  if constexpr (!PASSES) {
+    const int G = gridDim.x;
+    const moe_deal deal = moe_deal_of(heavy * gx, (nt - heavy) * gx, G, COST);
+    if ((heavy * gx + G - 1) / G > HR || deal.l_rest > MOE_LIGHT_ROUNDS) {
+      iu8_pf32_run<false, WMW, WNW, TM, TN, false, ST, false, true, GATHER == 2, true>(a, as, c, n, k, [&](int r, iu8_tile &t) {
+        const int j = moe_xcd_run(blockIdx.x, gridDim.x) + r * (int)gridDim.x;
+        const int slot = j / gx, bx = j % gx;
+        if (slot >= nt) return false;
+        const int tile = ordered ? (int)s_order[slot] : slot;
+        const int e = tile_expert[tile];
+        t = iu8_tile{iu8_rows{GATHER ? row_tok : nullptr, tile_row0[tile], min(tile_rows[tile], WMW * TM * 32)}, 0, bx * (BN / 16),
+                     (const unsigned char *)xptr[2 * e], (const float *)xptr[2 * e + 1]};
+        return true;
+      }, nullptr, nullptr, lds);
+      return;
+    }
+  }
   for (int ep = 0;; ++ep) {
+    int at1, atl, lrounds;  // where part 1 and the light items begin; this pass's light items
     {
-      const int gx = (n + BN - 1) / BN, G = gridDim.x, w = moe_xcd_run(blockIdx.x, G);
+      const int G = gridDim.x, w = moe_xcd_run(blockIdx.x, G);
       const int hi = heavy * gx, li = (nt - heavy) * gx;
-      const int h0 = ep * MOE_HEAVY_ROUNDS, l0 = ep * MOE_LIGHT_ROUNDS;
-      const int rounds = max(0, min((hi + G - 1) / G - h0, MOE_HEAVY_ROUNDS));
-      const int lrounds = max(0, min((li + G - 1) / G - l0, MOE_LIGHT_ROUNDS));
+      const moe_deal deal = moe_deal_of(hi, li, G, COST);
+      const int h0 = ep * HR, l0 = ep * MOE_LIGHT_ROUNDS;
+      const int rounds = max(0, min(hi / G + (w < deal.more) - h0, HR));
+      lrounds = max(0, min((w < deal.more ? deal.l_more : deal.l_rest) - l0, MOE_LIGHT_ROUNDS));
       if (rounds + lrounds == 0) break;
       /* a workgroup's heavy items run in two parts, its light items between them, after `first` rounds */
-      if (threadIdx.x == 0) {
-        s_par[0] = rounds, s_par[1] = lrounds;
-        s_par[2] = lrounds > 0 ? (w >> 3) % (rounds + 1) : rounds;
-      }
-      const int q = threadIdx.x;
-      if (q < rounds + lrounds) {
-        const bool light = q >= rounds;
-        const int id = light ? G - 1 - w + (l0 + q - rounds) * G : w + (h0 + q) * G;
+      const int first = lrounds > 0 ? (w >> 3) % (rounds + 1) : rounds;
+      at1 = first + 1, atl = rounds + 2;
+      const int q = moe_tid();
+      if (q < atl + lrounds + 1) {
+        const bool light = q >= atl, end = q == first || q == atl - 1 || q == atl + lrounds;
+        const int id = light ? deal.light_id(l0 + q - atl, w, G) : w + (h0 + q - (q > first)) * G;
         moe_item it{0, -1, 0, 0, nullptr, nullptr};
-        if (id < (light ? li : hi)) {
+        if (!end && id < (light ? li : hi)) {
           const int slot = (light ? heavy : 0) + id / gx, tile = ordered ? (int)s_order[slot] : slot;
-          const int e = tile_expert[tile];
-          it = moe_item{tile_row0[tile], min(tile_rows[tile], light ? MOE_LIGHT_ROWS : WMW * TM * 32),
-                        id % gx * (BN / 16), light ? (int)(((unsigned)id * 2654435761u >> 10) % (unsigned)(k >> 7)) : 0,
-                        (const unsigned char *)xptr[2 * e], (const float *)xptr[2 * e + 1]};
+          if (ep == 0 && nt <= NTHR) {
+            it = ((const moe_item *)lds)[slot];
+          } else {
+            const int e = tile_expert[tile];
+            it = moe_item{tile_row0[tile], tile_rows[tile], 0, 0, (const unsigned char *)xptr[2 * e], (const float *)xptr[2 * e + 1]};
+          }
+          it.rows = min(it.rows, light ? MOE_LIGHT_ROWS : WMW * TM * 32);
+          it.nt0 = id % gx * (BN / 16);
+          it.rot = light ? (int)(((unsigned)id * 2654435761u >> 10) % (unsigned)(k >> 7)) : 0;
         }
         s_item[q] = it;
       }
       __syncthreads();
-      /* the light items' tables: rows of A, their scales, the columns' scales */
-      static_assert(MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS == WMW * WNW * 64 && MOE_LIGHT_ROUNDS * BN == WMW * WNW * 64 * 4, "a thread an entry");
-      if (lrounds > 0) {
-        const int ri = threadIdx.x / MOE_LIGHT_ROWS, m = threadIdx.x % MOE_LIGHT_ROWS;
-        const int ci = threadIdx.x / (BN / 4), col = threadIdx.x % (BN / 4) * 4;
-        if (ri < lrounds && s_item[rounds + ri].rows > 0) {
-          const moe_item &it = s_item[rounds + ri];
-          const int ar = iu8_arow(iu8_rows{GATHER ? row_tok : nullptr, it.row0, it.rows}, m);
-          s_row[threadIdx.x] = ar;
-          s_am[threadIdx.x] = as[GATHER ? ar : min(ar, it.row0 + it.rows - 1)];
-        }
-        if (ci < lrounds && s_item[rounds + ci].rows > 0) {
-          const moe_item &it = s_item[rounds + ci];
-          *(float4 *)&s_ws[threadIdx.x * 4] = *(const float4 *)(it.ws + min(it.nt0 * 16 + col, n - 4));
-        }
-        __syncthreads();
-      }
     }
     for (int part = 0; part < 2; ++part) {
       if (part == 1) {
-        if (par(1) == 0) break;
+        if (lrounds == 0) break;
+        /* the light items' tables: rows of A, their scales, the columns' scales */
+        for (int i = moe_tid(); i < lrounds * MOE_LIGHT_ROWS; i += NTHR) {
+          const moe_item &it = s_item[atl + i / MOE_LIGHT_ROWS];
+          if (it.rows <= 0) continue;
+          const int ar = iu8_arow(iu8_rows{GATHER ? row_tok : nullptr, it.row0, it.rows}, i % MOE_LIGHT_ROWS);
+          s_row[i] = ar;
+          s_am[i] = as[GATHER ? ar : min(ar, it.row0 + it.rows - 1)];
+        }
+        for (int i = moe_tid(); i < lrounds * (BN / 4); i += NTHR) {
+          const moe_item &it = s_item[atl + i / (BN / 4)];
+          if (it.rows > 0) *(float4 *)&s_ws[i * 4] = *(const float4 *)(it.ws + min(it.nt0 * 16 + i % (BN / 4) * 4, n - 4));
+        }
+        __syncthreads();
         iu8_pf32_run<false, 1, 8, 2, 1, false, MOE_LIGHT_ST, false, true, GATHER == 2, true, false, true>(
-            a, as, c, n, k, [&](int r, iu8_tile &t) { return r < par(1) && item(par(0) + r, t, r); }, nullptr, nullptr, lds,
-            iu8_tabs{s_row, s_am, s_ws});
+            a, as, c, n, k, [&](int r, iu8_tile &t) { return item(atl + r, t, r); }, nullptr, nullptr, lds, iu8_tabs{s_row, s_am, s_ws});
         __syncthreads();
       }
+      const int at = part ? at1 : 0;
       iu8_pf32_run<false, WMW, WNW, TM, TN, false, ST, false, true, GATHER == 2, true>(
-          a, as, c, n, k,
-          [&](int r, iu8_tile &t) {
-            const int first = par(2), rr = part ? first + r : r;
-            return rr < (part ? par(0) : first) && item(rr, t);
-          },
-          nullptr, nullptr, lds);
+          a, as, c, n, k, [&](int r, iu8_tile &t) { return item(at + r, t); }, nullptr, nullptr, lds);
       __syncthreads();
     }
+    if constexpr (!PASSES) break;
   }
 }
-#define MOE_GROUPED_PF(name, BODY, GATHER, WMW, WNW, TM, TN, ST)                                                     \
+#define MOE_GROUPED_PF(name, GATHER, WMW, WNW, TM, TN, ST, HR, COST, PASSES)                                                  \
   extern "C" __global__ __launch_bounds__(WMW * WNW * 64) void name(                                              \
       const unsigned char *__restrict__ a, const unsigned long long *__restrict__ xptr,                           \
       const int *__restrict__ tile_expert, const int *__restrict__ tile_row0, const int *__restrict__ tile_rows,  \
       const int *__restrict__ row_tok, const int *__restrict__ meta, const float *__restrict__ as,                \
       int *__restrict__ p, int *__restrict__ cnt, unsigned short *__restrict__ c, int n, int k, int pmax) {        \
-    BODY<GATHER, WMW, WNW, TM, TN, ST>(a, xptr, tile_expert, tile_row0, tile_rows, row_tok, meta, as, c, n, k);    \
+    moe_grouped_pf<GATHER, WMW, WNW, TM, TN, ST, HR, COST, PASSES>(a, xptr, tile_expert, tile_row0, tile_rows, row_tok, meta, as, c, n, k);    \
   }
 // tiles of up to 128 rows (tile_blocks 8) on the 128 x 256 tile of 2 x 4 waves
-MOE_GROUPED_PF(moe_iu8_grouped_w4_pf_g2, moe_grouped_pf_two, 2, 2, 4, 2, 2, 4)
-MOE_GROUPED_PF(moe_iu8_grouped_w4_pf_g1, moe_grouped_pf_two, 1, 2, 4, 2, 2, 4)
-MOE_GROUPED_PF(moe_iu8_grouped_w4_pf_g0, moe_grouped_pf_two, 0, 2, 4, 2, 2, 4)
+MOE_GROUPED_PF(moe_iu8_grouped_w4_pf_g2, 2, 2, 4, 2, 2, 4, MOE_HEAVY_ROUNDS, 2, true)
+MOE_GROUPED_PF(moe_iu8_grouped_w4_pf_g1, 1, 2, 4, 2, 2, 4, MOE_HEAVY_ROUNDS, 2, true)
+MOE_GROUPED_PF(moe_iu8_grouped_w4_pf_g0, 0, 2, 4, 2, 2, 4, MOE_HEAVY_ROUNDS, 2, true)
 // tiles of up to 256 rows (tile_blocks 16) on the 256 x 256 tile, the dense GEMM's fastest cell
-MOE_GROUPED_PF(moe_iu8_grouped_w4_pf16_g2, moe_grouped_pf_one, 2, 2, 4, 4, 2, 3)
-MOE_GROUPED_PF(moe_iu8_grouped_w4_pf16_g1, moe_grouped_pf_one, 1, 2, 4, 4, 2, 3)
-MOE_GROUPED_PF(moe_iu8_grouped_w4_pf16_g0, moe_grouped_pf_one, 0, 2, 4, 4, 2, 3)
+MOE_GROUPED_PF(moe_iu8_grouped_w4_pf16_g2, 2, 2, 4, 4, 2, 3, 64, 4, false)
+MOE_GROUPED_PF(moe_iu8_grouped_w4_pf16_g1, 1, 2, 4, 4, 2, 3, 64, 4, false)
+MOE_GROUPED_PF(moe_iu8_grouped_w4_pf16_g0, 0, 2, 4, 4, 2, 3, 64, 4, false)
 #undef MOE_GROUPED_PF
 
 // ---------------------------------------------------------------------------- combine

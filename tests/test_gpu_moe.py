@@ -343,6 +343,36 @@ def test_light_tiles_at_their_edges(ctx, counts):
     assert sorted(layer.buf["expert_cnt"].tolist())[-16:] == sorted(list(counts) + [T - c for c in counts])
 
 
+@pytest.mark.parametrize("tb,kern", [(16, "moe_iu8_grouped_w4_pf16_g2"), (8, "moe_iu8_grouped_w4_pf_g2")])
+def test_light_and_heavy_items_of_one_workgroup(ctx, tb, kern):
+    """Full, ragged and nearly empty tiles of one launch: the layer against the oracle, and its gate+up on grids whose workgroups
+    walk several items of both kinds (16), more light ones than an item table holds (2) or more heavy ones as well (1),
+    and light ones on some workgroups only (61: no whole eighths)."""
+    say(f"light and heavy items of one workgroup: {kern}")
+    counts, T, E, k, H, I = (1, 31, 64, 65, 255, 257, 300, 330), 330, 128, 8, 640, 1152
+    case = synth.moe_case(T=T, E=E, topk=k, H=H, I=I, seed=tb, experts=4)
+    lg = np.zeros((T, E), np.float32)
+    for s, c in enumerate(counts):
+        lg[:c, s] = 8.0 - 0.5 * s       # the first c tokens' route s
+        lg[c:, 8 + s] = 8.0 - 0.5 * s   # the others': a second set of experts
+    case["logits"] = synth.f32_to_bf16_bits(lg)
+    layer = run_layer(ctx, case, tile_blocks=tb)
+    check_layer(layer, case)
+    want, rows = layer.gu.clone(), int(layer.buf["meta"][1].item())
+    live = layer.buf["row_tok"][:rows] >= 0
+    bufs = dict(a=layer.q1.data_ptr(), xptr=layer.xptr_gu.data_ptr(), c=layer.gu.data_ptr(),
+                **{n_: layer.buf[n_].data_ptr() for n_ in ("tile_expert", "tile_row0", "tile_rows", "row_tok", "meta")})
+    bufs["as"] = layer.s1.data_ptr()
+    for grid in (61, 16, 2, 1):
+        d = iu8.describe_raw(kern, (grid, 1, 1), 512, plugin="moe_iu8", n=2 * I, k=H, pmax=0)
+        for name in ("p", "cnt"):
+            d.arg(name).kind = iu8.ARG_NULL_BUFFER
+        layer.gu.fill_(0x7FC0)
+        ctx.launch(d, bufs)
+        torch.cuda.synchronize()
+        assert torch.equal(layer.gu[:rows][live], want[:rows][live]), grid
+
+
 def test_moe_router_ties_and_skew(ctx):
     say("moe router: ties and one hot expert")
     case = synth.moe_case(T=40, E=128, topk=8, H=512, I=256, seed=5, experts=4)

@@ -1054,3 +1054,31 @@ def test_band_table_grids_follow_their_cell_rows():
         c, n, k, ks = cells[name], int(rng.integers(1, 3500)) * 16, int(rng.choice([128, 5376, 8192, 16384])), int(rng.integers(1, 3))
         m, ks = int(rng.integers(1, c["rows_max"] + 1)), min(ks, k // 128)
         assert iu8.describe(name, m, n, k, ks).grid[0] == -(-n // width(c, m, n, k, ks)), (name, m, n, k, ks)
+
+
+def test_routed_items_are_dealt_once_and_level(tmp_path):
+    """The deal of the routed tile launches (csrc/kernels/moe_deal.h, compiled here): every light item goes to one position
+    once, and no position's share (a heavy item counts `cost`) is more than one heavy item above another's that has light ones."""
+    src, so = tmp_path / "deal.cpp", tmp_path / "deal.so"
+    src.write_text(f'#include "{iu8.PKG}/csrc/kernels/moe_deal.h"\n'
+                   'extern "C" int share(int hi, int li, int G, int cost, int w, int *ids) {\n'
+                   '  const moe_deal d = moe_deal_of(hi, li, G, cost);\n'
+                   '  int n = 0;\n'
+                   '  for (int r = 0; r < (w < d.more ? d.l_more : d.l_rest); ++r)\n'
+                   '    if (d.light_id(r, w, G) < li) ids[n++] = d.light_id(r, w, G);\n'
+                   '  return n;\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    lib, ids = ctypes.CDLL(str(so)), (ctypes.c_int * 4096)()
+    rng = np.random.default_rng(3)
+    cases = [(0, 1, 256, 2), (24, 1548, 256, 2), (256, 0, 256, 2), (255, 1, 256, 4), (1, 256, 256, 2), (1, 255, 256, 2), (1536, 700, 256, 4),
+             (0, 2048, 256, 2), (5, 3, 3, 2), (1, 2, 1, 4)]
+    cases += [(int(rng.integers(0, 3000)), int(rng.integers(0, 3000)), int(rng.choice([1, 3, 16, 255, 256])), int(rng.choice([2, 4]))) for _ in range(60)]
+    for hi, li, G, cost in cases:
+        got, load = [], []
+        for w in range(G):
+            n = lib.share(hi, li, G, cost, w, ids) if (li // G + cost + 2) < 4096 else 0
+            got += ids[:n]
+            load.append((cost * (hi // G + (w < hi % G)) + n, n))
+        assert sorted(got) == list(range(li)), (hi, li, G, cost)
+        top = max(x for x, n in load if n) if li else 0
+        assert all(x >= top - 1 - cost for x, _ in load), (hi, li, G, cost)
