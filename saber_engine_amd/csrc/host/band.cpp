@@ -176,6 +176,25 @@ std::string band_toml() {
   put(o, "aligned_k", IU8_STREAM_ALIGNED_K);
   put(o, "aligned_rows", IU8_STREAM_ALIGNED_ROWS);
   put(o, "aligned_last_max", IU8_STREAM_ALIGNED_LAST);
+  o += "\n[row_tiles]\n";
+  o += "# macaq_iu8_pf_{w4,w8}_t*_r, before the other lines but the shares of K of tiles, from K = k_min, over rows_over up to rows_max rows. 16x16 up to few_rows rows of few_n\n";
+  o += "# columns (from K = few_deep_k few_deep_n, int8 w8_few_n), and above, from n_64_rows columns up to 64 rows, with cu_count blocks at\n";
+  o += "# most. int4 alone: 16x32 over few_rows rows with cu_count blocks; from 65 rows 32x32 with cu_count\n";
+  o += "# (blocks_32 below K = k_min_32) and 32x64 from K = k_min_64 with blocks_64 (up to rows_64 rows cu_count)\n";
+  put(o, "rows_over", ROWS_CELL_ROWS_OVER);
+  put(o, "rows_max", ROWS_CELL_ROWS_MAX);
+  put(o, "k_min", ROWS_CELL_K);
+  put(o, "few_rows", ROWS_CELL_FEW_ROWS);
+  put(o, "few_n", ROWS_CELL_FEW_N);
+  put(o, "few_deep_n", ROWS_CELL_FEW_DEEP_N);
+  put(o, "few_deep_k", ROWS_CELL_FEW_DEEP_K);
+  put(o, "w8_few_n", ROWS_CELL_W8_FEW_N);
+  put(o, "n_64_rows", ROWS_CELL_64_ROWS_N);
+  put(o, "k_min_32", ROWS_CELL_32_K);
+  put(o, "blocks_32", ROWS_CELL_32_BLOCKS);
+  put(o, "k_min_64", ROWS_CELL_64_K);
+  put(o, "rows_64", ROWS_CELL_64_ROWS);
+  put(o, "blocks_64", ROWS_CELL_64_BLOCKS);
   o += "\n[row_producers]\n# macaq_i8_quant_* / macaq_i8_silu_mul_quant_*: 16 waves a row (_t1024) for rows wider than\n";
   o += "# width_over while the row count leaves the card part idle, else the narrowest 256-thread form\n";
   put(o, "t1024_width_over", T1024_WIDTH_OVER);
@@ -311,6 +330,14 @@ std::string band_toml() {
       put(o, "block_n", v->block_n());
       put(o, "threads", v->threads());
       put(o, "grid", std::string("[ceil(n / block_n), 1, 1]"));
+      put(o, "kernarg", std::string("pf"));
+    } else if (const RowsVariant *v = rows_variant(name)) {
+      put(o, "regime", std::string("rows"));
+      putb(o, "w8", v->w8 != 0);
+      put(o, "block_m", v->block_m());
+      put(o, "block_n", v->block_n());
+      put(o, "threads", v->threads());
+      put(o, "grid", std::string("[ceil(n / block_n) * ceil(m / block_m) rounded up to 8, 1, 1]"));
       put(o, "kernarg", std::string("pf"));
     } else if (const PfVariant *v = pf_variant(ks_form ? name.substr(0, name.size() - 3) : name)) {
       put(o, "regime", std::string("prefill"));

@@ -24,6 +24,10 @@ static const WideVariant WIDE_VARIANTS[] = {
 #define IU8_WIDE_VARIANT(name, TM, W8, NT, KW, D) {#name, TM, W8, NT, KW},
 #include "../kernels/iu8_variants.def"
 };
+static const RowsVariant ROWS_VARIANTS[] = {
+#define IU8_ROWS_VARIANT(name, TM, W8, NT, KW, D) {#name, TM, W8, NT, KW},
+#include "../kernels/iu8_variants.def"
+};
 static const DecVariant PAIR_VARIANTS[] = {
 #define IU8_PAIR_VARIANT(name, TM, NT, KW, WPB, D, ALDS, BFIRST) {#name, TM, false, NT, KW, WPB, D, ALDS, false},
 #include "../kernels/iu8_variants.def"
@@ -41,6 +45,11 @@ const DecVariant *pair_variant(const std::string &name) {
 }
 const WideVariant *wide_variant(const std::string &name) {
   for (const WideVariant &v : WIDE_VARIANTS)
+    if (name == v.name) return &v;
+  return nullptr;
+}
+const RowsVariant *rows_variant(const std::string &name) {
+  for (const RowsVariant &v : ROWS_VARIANTS)
     if (name == v.name) return &v;
   return nullptr;
 }
@@ -199,6 +208,28 @@ static int describe_wide(const WideVariant &v, uint32_t m, uint32_t n, uint32_t 
   return 0;
 }
 
+// Blocks in whole eighths: the kernel gives an XCD a run of them, column blocks of one row tile side by side.
+static int describe_rows_cell(const RowsVariant &v, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *d) {
+  const char *op = v.w8 ? "gemm_i8a8" : "gemm_i4a8";
+  if (int rc = check_shape(op, m, n, k)) return rc;
+  const uint64_t blocks = (uint64_t)((n + v.block_n() - 1) / v.block_n()) * ((m + v.block_m() - 1) / v.block_m());
+  if (blocks > ROWS_CELL_BLOCKS_MAX || (uint64_t)v.block_m() * k > INT32_MAX)
+    return fail(SABER_IU8_E_RULE, fmt("%s: %s holds %u blocks of rows under 2 GiB, %u x %u x %u", op, v.name, ROWS_CELL_BLOCKS_MAX, m, n, k));
+  memset(d, 0, sizeof *d);
+  copy_name(d->op, sizeof d->op, op);
+  copy_name(d->plugin, sizeof d->plugin, "macaq_iu8");
+  copy_name(d->kernel, sizeof d->kernel, v.name);
+  d->grid[0] = (uint32_t)((blocks + 7) / 8 * 8), d->grid[1] = 1, d->grid[2] = 1;
+  d->block[0] = v.threads(), d->block[1] = 1, d->block[2] = 1;
+  d->n_launches = 1;
+  d->ks = 1;
+  if (int rc = fill_slots(v.name, d)) return rc;
+  set_i32(d, "m", m);
+  set_i32(d, "n", n);
+  set_i32(d, "k", k);
+  return 0;
+}
+
 static uint64_t staged_bytes(uint32_t m, uint32_t k);
 // The streaming decode cell of M rows: tm 16-row tiles; one tile's live rows staged in LDS when they fit the 20 KiB
 // form, else streamed from L2 beside the weights.
@@ -252,6 +283,10 @@ int describe(const std::string &kernel, uint32_t m, uint32_t n, uint32_t k, uint
   if (const WideVariant *v = wide_variant(kernel)) {
     if (ks != 1) return fail(SABER_IU8_E_RULE, kernel + ": the wide streamed cell does not split K");
     return describe_wide(*v, m, n, k, out);
+  }
+  if (const RowsVariant *v = rows_variant(kernel)) {
+    if (ks != 1) return fail(SABER_IU8_E_RULE, kernel + ": the streamed cell on row tiles does not split K");
+    return describe_rows_cell(*v, m, n, k, out);
   }
   if (const PfVariant *v = pf_variant(kernel)) {
     if (ks != 1) return fail(SABER_IU8_E_RULE, kernel + ": the prefill tile does not split K (its `_ks` form does)");
@@ -308,7 +343,10 @@ int pair(const saber_iu8_desc &first, const saber_iu8_desc &second, saber_iu8_de
   static const char PREFIX[] = "macaq_iu8_dec_w4_";
   // a half the law gave the staged persistent form, or 17 to 48 rows at another block width, is paired as its streamed
   // form, which is the pair kernels' geometry, on the split count it was given
+  // (and up to 48 rows the streamed cell on row tiles)
   auto other_form = [](const saber_iu8_desc &h) {
+    int64_t hm = 0;
+    if (const RowsVariant *v = rows_variant(h.kernel)) return !v->w8 && int_arg(h, "m", &hm) && hm <= ROWS_CELL_FEW_ROWS;
     return !strncmp(h.kernel, "macaq_iu8_dec_w4_tm1_s80", 24) || !strcmp(h.kernel, "macaq_iu8_dec_w4_tm2_n1") ||
            !strcmp(h.kernel, "macaq_iu8_dec_w4_tm3_n2");
   };
@@ -434,6 +472,39 @@ static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint
   return nullptr;
 }
 
+// The streamed cells on row tiles: outputs of so few 64 x 64 tiles that most CUs idle while a tile goes through its K steps (0.22 us
+// each, int4), and streamed launches of so few column blocks that a CU reads every row for one of them. The smallest block that
+// is one round of the CUs: 16 x 16, then for int4 16 x 32 and from 65 rows 32 x 32 and 32 x 64. us, the law's pick without these / here, int4,
+// K = 5,120: 96 columns at 33 / 64 / 100 / 400 / 777 / 1,500 rows 4.1 / 5.4 / 11.7 / 12.0 / 11.9 / 12.0 -> 3.3 / 4.1 / 5.0 / 5.3 / 6.5 / 8.0, 256 at 200 /
+// 777 11.8 / 11.9 -> 5.9 / 8.4, 1024 at 45 / 100 / 200 6.4 / 11.9 / 11.8 -> 5.1 / 7.5 / 8.8, 2048 at 100 11.9 -> 7.9, 5120 at 80 / 96 12.4 / 12.4
+// -> 10.2 / 10.4, 512 at 777 12.0 -> 10.4; 96 x 17408 at 400 32.6 -> 11.4, 256 x 1024 at 100 / 777 4.8 / 4.8 -> 3.7 / 3.7.
+// Int8: 96 x 5120 at 64 / 200 8.0 / 9.2 -> 5.8 / 6.8, 512 x 5120 at 100 9.3 -> 7.7. Over 240 shapes drawn over the whole of it 16 x 16 1.83 times
+// faster, 16 x 32 1.62, 32 x 32 1.45, 32 x 64 1.22, int8 16 x 16 1.32; none slower by more than 3 % but an int8 launch of 52 rows of 64 columns (5).
+// Where the lines lie: up to 48 rows the streamed law has a cell of few columns already: 512 x 2048 at 17 / 45 rows 3.0 / 3.2, here 3.2 /
+// 3.5, but 512 x 5120 4.5 / 5.9 -> 4.4 / 5.0 (int8 1024 x 5120 level, 80 x 2432 at 17 rows 3.4 -> 3.5). A second round loses: 16 x 16 on 1024 x 2048
+// at 200 rows (832 blocks) 1.02, on 1024 x 5120 at 400 0.64. 32 x 32 on more than 200 blocks at K = 1,024 0.95-1.06; 32 x 64 at K = 2,048 0.93-1.11, at
+// 5,120 1.06-1.20, at 17,408 1.23-1.50, on more than 208 blocks 0.96 where the 64-row tiles are full (190 rows of 2288 x 5632) and 1.2 where they are
+// not (up to 96 rows). Int8 64 x 64 tiles have nothing to unpack: 16 x 32 on 88-160 blocks 0.91-1.32, 7 % on average, not built. Below K = 768 a
+// launch is mostly its start (96 x 512 at 100 / 777 rows 3.8 -> 2.8, not taken). Three lines are held: 2,048 rows of 96 x 5120 would gain
+// as 1,500 do, 49-64 rows of fewer than 64 columns as 64 columns do, and the tile launches that share K (96 x 17408 at 45 rows 17.0 -> 9.5).
+static const RowsVariant *rows_cell(bool w8, uint32_t m, uint32_t n, uint32_t k, bool tile_split) {
+  if (m <= ROWS_CELL_ROWS_OVER || m > ROWS_CELL_ROWS_MAX || k < ROWS_CELL_K || k > ROWS_CELL_K_MAX || n > 64 * CU_COUNT || tile_split) return nullptr;
+  auto blocks = [&](uint32_t bm, uint32_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn); };
+  auto cell = [&](const char *block) { return rows_variant(fmt("macaq_iu8_pf_%s_t%s_r", w8 ? "w8" : "w4", block)); };
+  if (m <= ROWS_CELL_FEW_ROWS) {
+    const bool deep = k >= ROWS_CELL_FEW_DEEP_K;
+    const uint32_t widest = w8 ? (deep ? ROWS_CELL_W8_FEW_N : 0) : deep ? ROWS_CELL_FEW_DEEP_N : ROWS_CELL_FEW_N;
+    return n <= widest ? cell("16x16") : nullptr;
+  }
+  if (m <= DECODE_MAX_M && n < ROWS_CELL_64_ROWS_N) return nullptr;
+  if (blocks(16, 16) <= CU_COUNT) return cell("16x16");
+  if (w8) return nullptr;
+  if (blocks(16, 32) <= CU_COUNT) return cell("16x32");
+  if (m <= DECODE_MAX_M) return nullptr;
+  if (blocks(32, 32) <= (k >= ROWS_CELL_32_K ? CU_COUNT : ROWS_CELL_32_BLOCKS)) return cell("32x32");
+  return blocks(32, 64) <= (m <= ROWS_CELL_64_ROWS ? CU_COUNT : ROWS_CELL_64_BLOCKS) && k >= ROWS_CELL_64_K ? cell("32x64") : nullptr;
+}
+
 // Which launch `a` and `b` are, whatever their workspaces.
 static bool same_launch(const saber_iu8_desc &a, const saber_iu8_desc &b) {
   return !strcmp(a.kernel, b.kernel) && a.ks == b.ks && !memcmp(a.grid, b.grid, sizeof a.grid) && !memcmp(a.block, b.block, sizeof a.block);
@@ -498,6 +569,7 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // 12.9 / 13.6, on tiles 18.3 / 18.4, 18.0 / 18.0, 19.5 / 19.6): below K = 16,384 they are what the law takes, the line itself has not moved.
   const PfVariant *split_cell = nullptr;
   const uint32_t tile_ks = pf_split(wkind == SABER_IU8_W8, m, n, k, &split_cell);
+  if (const RowsVariant *v = rows_cell(w8, m, n, k, tile_ks && m > 32)) return describe_rows_cell(*v, m, n, k, out);
   const bool narrow = n <= 16 * CU_COUNT, two_wide = !narrow && n <= 32 * CU_COUNT;  // a 16- / 32-column block a CU
   const bool stream = m <= 16 || (m <= 32 && n <= 16384) || (m <= 48 && n <= 8192 && tile_ks == 0) ||
                       (tile_ks == 0 && m <= 64 && stream_wide_blocks(w8, m, n, k)) ||

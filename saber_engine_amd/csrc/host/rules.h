@@ -28,6 +28,13 @@ struct WideVariant {  // the streamed cell on the prefill kernarg list: one bloc
   int block_n() const { return nt * 16; }
   int threads() const { return kw * 64; }
 };
+struct RowsVariant {  // the streamed cell on row tiles of its own: a workgroup a block of block_m rows and block_n columns
+  const char *name;
+  int tm, w8, nt, kw;
+  int block_m() const { return tm * 16; }
+  int block_n() const { return nt * 16; }
+  int threads() const { return kw * 64; }
+};
 struct PfVariant {
   const char *name;
   int w8, wmw, wnw, tm, tn, acc, occ, kw;  // waves, 32 x 32 MFMA tiles a wave, workgroups a CU, k-waves a wave tile
@@ -39,6 +46,7 @@ struct PfVariant {
 const DecVariant *dec_variant(const std::string &name);
 const PfVariant *pf_variant(const std::string &name);
 const WideVariant *wide_variant(const std::string &name);
+const RowsVariant *rows_variant(const std::string &name);
 // The prefill cell (tile shape) the launch law picks for a shape.
 const PfVariant *pf_cell(bool w8, uint32_t m, uint32_t n, uint32_t k);
 uint32_t pf_split(bool w8, uint32_t m, uint32_t n, uint32_t k, const PfVariant **cell);
@@ -56,6 +64,12 @@ constexpr uint64_t S80_MIN_BYTES = 64ull << 20;  // the staged persistent GEMV: 
 // K shares of a streamed launch (rules.cpp:stream_split): rows, shares, the least K by rows and columns
 constexpr uint32_t STREAM_SPLIT_ROWS_OVER = 8, STREAM_SPLIT_ROWS_MAX = 48, STREAM_SPLIT_SHARES_MIN = 3, STREAM_SPLIT_SHARES_MAX = 4;
 constexpr uint32_t STREAM_SPLIT_K_16ROWS = 10240, STREAM_SPLIT_K_4096COLS = 12288, STREAM_SPLIT_K = 8192;
+// the streamed cells on row tiles (rules.cpp:rows_cell): rows, K; up to 48 rows the columns; 32-row blocks by K
+constexpr uint32_t ROWS_CELL_BLOCKS_MAX = 1u << 16;  // blocks a launch of them holds
+constexpr uint32_t ROWS_CELL_ROWS_OVER = 16, ROWS_CELL_ROWS_MAX = 2047, ROWS_CELL_K = 768, ROWS_CELL_K_MAX = 1u << 24;
+constexpr uint32_t ROWS_CELL_FEW_ROWS = 48, ROWS_CELL_FEW_N = 256, ROWS_CELL_FEW_DEEP_N = 1024, ROWS_CELL_FEW_DEEP_K = 4096;
+constexpr uint32_t ROWS_CELL_W8_FEW_N = 512, ROWS_CELL_64_ROWS_N = 64;
+constexpr uint32_t ROWS_CELL_32_K = 2048, ROWS_CELL_32_BLOCKS = 200, ROWS_CELL_64_K = 4096, ROWS_CELL_64_ROWS = 96, ROWS_CELL_64_BLOCKS = 208;
 constexpr uint32_t HAD_T1024_ROWS = 256, HAD_T1024_WIDTH = 4096;  // the Hadamard-basis producers' 16-wave forms: up to / from
 constexpr uint32_t T1024_WIDTH_OVER = 4096;
 constexpr uint32_t T1024_QUANT_ROWS = 256, T1024_QUANT_ROWS_WIDE = 512;

@@ -493,6 +493,27 @@ def test_wide_streamed_cells(ctx, kernel, rows, cols):
         assert_dense_matches(run, ref.linear(case["X"], case["W"], case["ws"], w8), w8)
 
 
+ROWS = re.findall(r"^IU8_ROWS_VARIANT\((macaq_iu8_pf_w\d_t(\d+)x(\d+)_r),", open(os.path.join(iu8.PKG, "csrc", "kernels", "iu8_variants.def")).read(), flags=re.M)
+
+
+@pytest.mark.parametrize("kernel,rows,cols", ROWS, ids=lambda v: str(v))
+def test_streamed_cells_on_row_tiles(ctx, kernel, rows, cols):
+    """Every streamed cell on row tiles by name: one block and counts that are no multiple of eight, a last row tile of one
+    and of all but one row, a last column block of one and of all but one column tile, fewer K steps than k-waves, odd counts,
+    and the launch that the law makes of such a shape."""
+    w8, rows, cols = "_w8_" in kernel, int(rows), int(cols)
+    for M, N, K in [(1, 16, 128), (rows + 1, cols + 16, 128 * 7), (3 * rows, 2 * cols - 16 if cols > 16 else 16, 128 * 8),
+                    (5 * rows - 1, 3 * cols, 128 * 9), (9 * rows + 1, 96, 128 * 21)]:
+        case = synth.dense_case(M, N, K, w8=w8, seed=M + N + K)
+        run = DenseRun(ctx, case, kernel=kernel, want_acc=False)
+        assert_dense_matches(run, ref.linear(case["X"], case["W"], case["ws"], w8), w8)
+    M, N, K = {"16x16": (100, 96, 1024), "16x32": (301, 304, 896), "32x32": (200, 1008, 2048), "32x64": (97, 3008, 4096)}[f"{rows}x{cols}"]
+    case = synth.dense_case(M, N, K, w8=w8, seed=5)
+    run = DenseRun(ctx, case, want_acc=False)
+    assert run.desc.kernel.decode() == kernel
+    np.testing.assert_array_equal(run.C, ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)["C"])
+
+
 @pytest.mark.parametrize("M,N,K,w8", [(16, 5120, 10240, False), (9, 3024, 12288, True), (31, 5424, 8192, False), (48, 4096, 12288, True),
                                       (20, 8208, 384, False), (33, 12240, 2048, False), (50, 12256, 3072, False), (32, 16384, 256, True)])
 def test_streamed_blocks_of_64_columns(ctx, M, N, K, w8):

@@ -942,6 +942,41 @@ def test_lines_of_the_streamed_cells_past_one_round():
         iu8.describe("macaq_iu8_pf_w4_t48x144_w", 48, 160, 256, ks=2)
 
 
+def test_lines_of_the_streamed_cells_on_row_tiles():
+    """Either side of the lines in rows, columns, K and blocks; such a launch needs no workspace, its grid is whole eighths that
+    hold every block, and a half of a pair is described again in the pair's form wherever it was one before."""
+    for (w8, m, n, k), want in {
+            (0, 16, 96, 5120): None, (0, 17, 96, 5120): "16x16", (0, 17, 96, 640): None, (0, 17, 96, 768): "16x16", (0, 48, 256, 768): "16x16",
+            (0, 48, 272, 3968): None, (0, 48, 272, 4096): "16x16", (0, 48, 1024, 4096): "16x16", (0, 48, 1040, 4096): None,
+            (1, 48, 512, 4096): "16x16", (1, 48, 512, 3968): None, (1, 48, 528, 5120): None, (1, 17, 96, 3968): None,
+            (0, 49, 48, 2048): None, (0, 49, 64, 2048): "16x16", (1, 64, 48, 5120): None, (1, 64, 64, 768): "16x16", (0, 65, 16, 768): "16x16",
+            (0, 49, 1024, 768): "16x16", (0, 49, 1040, 768): "16x32", (0, 64, 2048, 768): "16x32", (0, 64, 2064, 5120): None,
+            (0, 400, 160, 1024): "16x16", (0, 416, 160, 1024): "16x32", (0, 777, 160, 1024): "16x32", (0, 800, 192, 2048): "32x32",
+            (0, 800, 256, 1920): "32x32", (0, 800, 288, 1920): None, (0, 800, 320, 2048): "32x32", (0, 800, 336, 3968): None,
+            (0, 800, 336, 4096): "32x64", (0, 800, 512, 4096): "32x64", (0, 800, 528, 4096): None, (0, 97, 3328, 4096): "32x64", (0, 97, 3344, 4096): None, (0, 2047, 96, 5120): "32x32", (0, 2048, 96, 5120): None,
+            (0, 96, 5440, 4096): "32x64", (0, 96, 5456, 4096): None, (0, 96, 1024, 16256): "16x32", (0, 96, 1024, 16384): None, (0, 32, 96, 17408): "16x16", (0, 33, 96, 17408): None,
+            (0, 193, 96, 17408): "16x16",
+            (1, 100, 576, 768): "16x16", (1, 100, 592, 768): None, (1, 200, 304, 5120): "16x16", (1, 200, 320, 5120): None}.items():
+        d = iu8.resolve(iu8.W8 if w8 else iu8.W4, m, n, k)
+        name = d.kernel.decode()
+        assert (name[len("macaq_iu8_pf_w4_t"):-2] if name.endswith("_r") else None) == want, (w8, m, n, k, name)
+        if want:
+            bm, bn = map(int, want.split("x"))
+            assert d.grid[0] % 8 == 0 and 0 <= d.grid[0] - -(-m // bm) * -(-n // bn) < 8 and d.block[0] == 512 and d.n_workspaces == 0 and d.ks == 1
+    for m, twin in ((17, "tm2"), (32, "tm2"), (48, "tm3")):
+        wide, ba = iu8.resolve(iu8.W4, m, 16384, 5120), iu8.resolve(iu8.W4, m, 96, 5120)
+        assert ba.kernel.endswith(b"_r")
+        want = iu8.pair(wide, iu8.describe(f"macaq_iu8_dec_w4_{twin}", m, 96, 5120))
+        assert bytes(iu8.pair(wide, ba)) == bytes(want)
+    for m, k in ((49, 5120), (64, 5120), (33, 16384)):     # no half of a pair before, and none now
+        with pytest.raises(iu8.IU8Error):
+            iu8.pair(iu8.describe(f"macaq_iu8_dec_w4_tm{-(-m // 16)}", m, 96, k), iu8.resolve(iu8.W4, m, 96, k))
+    with pytest.raises(iu8.IU8Error):
+        iu8.describe("macaq_iu8_pf_w4_t16x16_r", 100, 96, 1024, ks=2)
+    with pytest.raises(iu8.IU8Error):
+        iu8.describe("macaq_iu8_pf_w4_t16x16_r", 1 << 20, 96, 1024)   # more blocks than a launch holds
+
+
 def test_thin_tiles_by_weight_kind(tmp_path):
     """The layout rule of the 256 x 256 cell (csrc/kernels/iu8_pf_law.h, compiled here): which launches of 256 workgroups run
     the rows past the last whole 256 as thin tiles -- int8 weights only where they measured no slower than whole tiles. Every
