@@ -51,6 +51,7 @@ template <>
 struct iu8_pf_short<false, 128, 128, 1> {
   static constexpr bool HAS = true;
   static constexpr int WMW = 4, WNW = 2, TM = 1, TN = 2, ST = 3, KW = 1;
+  static constexpr bool DEEP = false;
   static __device__ __forceinline__ bool takes(int k, int) { return k <= 2048; }
 };
 // Int8 weights 128 x 128, four stages: three up to K = 2,048, and up to 6,143 on a count of tiles that leaves the order by XCD
@@ -61,7 +62,18 @@ template <>
 struct iu8_pf_short<true, 128, 128, 1> {
   static constexpr bool HAS = true;
   static constexpr int WMW = 4, WNW = 2, TM = 1, TN = 2, ST = 3, KW = 1;
+  static constexpr bool DEEP = false;
   static __device__ __forceinline__ bool takes(int k, int wgs) { return k <= 2048 || (k < 6144 && wgs % 8 != 0); }
+};
+// W4 64 x 64, two k-waves: the deep form of one wave a wave tile up to K = 512, where the k-waves' meeting and their fuller prologue are what a
+// launch is. us, deep / k-waves: 600 rows of 4096 x 128 6.1 / 6.5, 200 of 4096 x 128 3.5 / 3.6; over 140 shapes the k-waves are 3 % slower at K = 128, 2 %
+// at 256, level at 384 and 512, 2 % faster at 640, 5 % at 1,536, 9 % at 3,072 and 15 % past 8,192.
+template <>
+struct iu8_pf_short<false, 64, 64, 2> {
+  static constexpr bool HAS = true;
+  static constexpr int WMW = 2, WNW = 2, TM = 1, TN = 1, ST = 6, KW = 1;
+  static constexpr bool DEEP = true;
+  static __device__ __forceinline__ bool takes(int k, int) { return k <= 512; }
 };
 // Int8 weights 64 x 64, five stages: four below K = 3,072. us on four / five: 511 rows of 2784 x 256 4.6 / 5.0, 675 of 2096 x 1024 8.4 /
 // 8.9, 2,025 of 560 x 2304 10.4 / 10.7; 89 of 2112 x 5376 13.7 / 12.5, 142 of 1648 x 8960 20.8 / 17.7. (Between 1,536 and 3,071 the
@@ -70,6 +82,7 @@ template <>
 struct iu8_pf_short<true, 64, 64, 2> {
   static constexpr bool HAS = true;
   static constexpr int WMW = 2, WNW = 2, TM = 1, TN = 1, ST = 4, KW = 1;
+  static constexpr bool DEEP = true;
   static __device__ __forceinline__ bool takes(int k, int) { return k < 3072; }
 };
 
@@ -94,7 +107,7 @@ static __device__ __forceinline__ void iu8_pf32_dense(const unsigned char *__res
     static_assert(iu8_pf32_lds_bytes<W8, S::WMW, S::WNW, S::TM, S::TN, S::ST>() <= L, "the short form runs in the cell's stages");
     __shared__ __attribute__((aligned(1024))) iu8_u8 lds[L];
     if (S::takes(k, (int)gridDim.x))
-      iu8_pf32_run<W8, S::WMW, S::WNW, S::TM, S::TN, ACC, S::ST, DEEP, false, false, true, false, false, S::KW>(a, as, c, n, k, tile_at, nullptr, nullptr, lds);
+      iu8_pf32_run<W8, S::WMW, S::WNW, S::TM, S::TN, ACC, S::ST, S::DEEP, false, false, true, false, false, S::KW>(a, as, c, n, k, tile_at, nullptr, nullptr, lds);
     else
       iu8_pf32_run<W8, WMW, WNW, TM, TN, ACC, ST, DEEP, false, false, true, false, false, KW>(a, as, c, n, k, tile_at, nullptr, nullptr, lds);
   } else {
