@@ -635,11 +635,25 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // estimate, whose table does not hold this cell: not for its speed at 1,024 rows themselves, where it is as many tiles as
   // at 1,000 (5120 x 5120 / 17408 32.6 / 99 us, 128 x 256 41.2 / 118); from 1,025 rows of 5,120 columns it is two rounds
   // (55.4 / 174 against 42.4 / 124).
-  if (w8 && m > 64 && m < 1024) {
-    auto tiles = [&](uint32_t bn) { return (uint64_t)((n + bn - 1) / bn) * ((m + 127) / 128); };
+  // Int8 weights where the estimate, whose rates rank a 64-row cell too high past one round of it, has such a cell: 128 x 64 where that is one
+  // round and 64 x 64 is not (a 64 x 128 tile, the estimate's pick of a long K, has as many bytes and half the rows to share a weight stage), else
+  // 128 x 128 where that is one and 64 x 128 is not. us, the estimate's pick / here: 200 rows of 5120 x 17408 / 6144 / 5120 62.8 / 23.4 / 21.2 -> 47.0 /
+  // 18.7 / 17.0, 300 of 4096 x 17408 61.5 -> 46.3, 160 of 7168 x 5120 22.0 -> 17.3, 777 of 2048 x 17408 59.8 -> 48.0, 300 of 5120 x 3072 14.7 -> 11.6; 160 / 256 of
+  // 16384 x 5120 36.9 / 39.4 -> 29.3 / 32.4, 227 of 16384 x 4096 1.25, 152 of 14336 x 256 1.26 times faster. From K = 2,048 (2,048 level to 1.11, 3,072 1.07-1.27, 5,120
+  // and more 1.05-1.38, 1,024 0.95-1.05), from 4,096 on a count that is not whole eighths (854 rows of 1776 x 3072 0.88); with no more 64 x 64 tiles than
+  // CUs those stay (160 of 5120 x 3072 0.80). Over 305 shapes of 65 to 4,096 rows that moved, drawn after the lines, 128 x 64 1.20 times faster, 128 x 128 1.26, the
+  // slowest 0.99. 256 rows are held on the 64 x 128 cell (5120 x 5120 21.3 for 18.6).
+  if (w8 && m > 64) {
+    auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)((n + bn - 1) / bn) * ((m + bm - 1) / bm); };
     const PfVariant *est = pf_cell(w8, m, n, k);
-    const bool pays = est->block_m() == 64 ? k >= 5120 : m <= 128 || k < 512 || k >= 3072 || tiles(160) % 8 == 0;
-    if (pays && tiles(160) <= CU_COUNT && tiles(128) > CU_COUNT) return describe_pf(*pf_variant("macaq_iu8_pf_w8_t128x160"), m, n, k, 0, out);
+    const bool small = est->block_m() == 64;
+    const bool pays = small ? k >= 5120 : m <= 128 || k < 512 || k >= 3072 || tiles(128, 160) % 8 == 0;
+    if (m < 1024 && pays && tiles(128, 160) <= CU_COUNT && tiles(128, 128) > CU_COUNT) est = pf_variant("macaq_iu8_pf_w8_t128x160");
+    else if (small && tiles(128, 64) <= CU_COUNT) {
+      if (m != 256 && tiles(64, 64) > CU_COUNT && k >= (tiles(128, 64) % 8 ? 4096u : 2048u)) est = pf_variant("macaq_iu8_pf_w8_t128x64_s");
+    } else if (small && tiles(128, 128) <= CU_COUNT && tiles(64, 128) > CU_COUNT) {
+      est = pf_variant("macaq_iu8_pf_w8_t128x128");
+    }
     return describe_pf(*est, m, n, k, 0, out);
   }
   return describe_pf(*pf_cell(wkind == SABER_IU8_W8, m, n, k), m, n, k, 0, out);

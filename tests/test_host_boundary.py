@@ -459,6 +459,18 @@ def test_int8_128x160_cell_only_where_it_measured_faster():
             assert iu8.resolve(iu8.W8, m, n, k).kernel.decode().startswith(("macaq_iu8_pf_w8_t64x", "macaq_iu8_pf_w8_t256x160")), (m, n, k)
 
 
+def test_int8_cells_of_one_round_in_place_of_two_of_a_64_row_cell():
+    """Int8 weights: 128 x 64 where it is one round and 64 x 64 is not, by K and by whole eighths; else 128 x 128 where that is one and
+    64 x 128 is not. 256 rows and launches of no more 64 x 64 tiles than CUs stay with the estimate."""
+    for m, n, k, tile in ((200, 5120, 5120, "t128x64_s"), (200, 5120, 2048, "t128x64_s"), (200, 5120, 1920, None), (256, 5120, 17408, None),
+                          (257, 5120, 5120, "t128x64_s"), (160, 5120, 5120, None), (192, 5120, 5120, None), (193, 5120, 5120, "t128x64_s"),
+                          (384, 5440, 5120, "t128x64_s"), (384, 5456, 5120, "t128x128"), (200, 5136, 4096, "t128x64_s"), (200, 5136, 3968, None),
+                          (777, 2048, 17408, "t128x64_s"), (1500, 1152, 5120, "t128x64_s"), (65, 10240, 6144, "t128x64_s"),
+                          (160, 16384, 5120, "t128x128"), (256, 16384, 4096, "t128x128"), (160, 16400, 5120, None), (129, 11008, 6144, "t128x128")):
+        name = iu8.resolve(iu8.W8, m, n, k).kernel.decode()[len("macaq_iu8_pf_w8_"):]
+        assert (name == tile) if tile else name not in ("t128x64_s", "t128x128"), (m, n, k, name)
+
+
 def test_prefill_cells_of_the_benchmark_shapes():
     # speed data of this card: the cell that was fastest in the sustained sweep of each shape, weights cold (every cell on
     # the four 27B-class shapes x 14 row counts; the law's tables are fitted to those timings, one a weight kind)
