@@ -80,6 +80,8 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out);
 bool law_split_stream(const saber_iu8_desc &d);  // d is what `resolve` gives its shape, a streamed cell on a split of K
 // The launch of a caller that binds no workspaces: `d` itself, or its streamed cell with K in one piece.
 int unsplit_stream(saber_iu8_desc *d);
+// The streamed launch on its own K shares that `saber_iu8_gemm` makes of the law's tile launch `d`, in that launch's workspaces.
+bool stream_in_tile_workspaces(const saber_iu8_desc &d, saber_iu8_desc *out);
 // The same for a pair whose halves that share K do so as `resolve` gave them: a half without both of its workspaces
 // (`bound`, `bound_b`: it has them) in one piece. False: no such pair.
 bool unsplit_pair(const saber_iu8_desc &d, bool bound, bool bound_b, saber_iu8_desc *out);

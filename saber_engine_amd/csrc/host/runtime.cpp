@@ -586,8 +586,12 @@ int saber_iu8_gemm(saber_iu8_ctx *ctx, int wkind, const void *a, const float *as
                    void *c, uint32_t m, uint32_t n, uint32_t k, void *partial, void *counter, void *stream) {
   saber_iu8_desc d;
   if (int rc = resolve(wkind, m, n, k, &d)) return rc;
-  if (!partial || !counter)  // a streamed launch in one piece needs neither
+  saber_iu8_desc streamed;
+  if (!partial || !counter) {  // a streamed launch in one piece needs neither
     if (int rc = unsplit_stream(&d)) return rc;
+  } else if (stream_in_tile_workspaces(d, &streamed)) {
+    d = streamed;
+  }
   return launch_gemm(ctx, d, a, as, w, ws, c, partial, counter, stream);
 }
 

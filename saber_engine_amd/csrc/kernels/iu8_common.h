@@ -220,8 +220,8 @@ static __device__ __forceinline__ iu8_v4i iu8_load_through(const int *p) {
 }
 static __device__ __forceinline__ void iu8_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // one lane, after the workgroup met behind its completed stores: count the arrival
-static __device__ __forceinline__ int iu8_arrive(int *counter) {
-  return __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+static __device__ __forceinline__ int iu8_arrive(int *counter, int by = 1) {
+  return __hip_atomic_fetch_add(counter, by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 static __device__ __forceinline__ iu8_v4u iu8_ldg_nt(const iu8_u8 *p) {

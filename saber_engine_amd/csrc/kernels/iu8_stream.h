@@ -244,10 +244,14 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
     }
   iu8_stores_done();
   __syncthreads();
-  if (tid == 0) s_last = (iu8_arrive(&cnt[B.bx]) == Z - 1);
+  // two blocks count in one word, 16 bits each: a 64-column launch's counters fit where a 128-column tile launch's would
+  // (rules.cpp:stream_in_tile_workspaces). Z is a grid's z, at most 65,535, so a half never carries into the other.
+  int *const word = &cnt[B.bx >> 1];
+  const unsigned half = (B.bx & 1) * 16;
+  if (tid == 0) s_last = (((unsigned)iu8_arrive(word, (int)(1u << half)) >> half) & 0xFFFFu) == (unsigned)(Z - 1);
   __syncthreads();
   if (!s_last) return;
-  if (tid == 0) __hip_atomic_store(&cnt[B.bx], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) iu8_arrive(word, (int)(0u - ((unsigned)Z << half)));
   constexpr int SH = PASSES * NI <= 2 ? 3 : PASSES * NI <= 9 ? 2 : 1;  // shares asked for at a time
   for (int q0 = 1; q0 < Z; q0 += SH) {
     iu8_v4i v[SH][PASSES][NI];

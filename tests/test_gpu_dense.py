@@ -541,6 +541,35 @@ def test_streamed_blocks_of_64_columns(ctx, M, N, K, w8):
         np.testing.assert_array_equal(host_u16(c), r["C"])
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 3024, 16384), (48, 4096, 16512), (45, 5136, 17408), (40, 5440, 16384), (48, 5456, 16384)])
+def test_gemm_streams_in_the_workspaces_of_a_tile_launch(ctx, M, N, K):
+    """33 to 48 rows of a deep, narrow linear: the descriptor is the tile launch that shares K, the call with its workspaces
+    streams (up to 5,440 columns) -- the oracle's bytes every time, nothing written past the workspaces and the counters left at zero, also on
+    workspaces that the tile launch itself has used between; without workspaces it is refused as it was."""
+    case = synth.dense_case(M, N, K, seed=M + N)
+    r = ref.linear(case["X"], case["W"], case["ws"], False, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], False)), dev_f32(case["ws"])
+    d = iu8.resolve(iu8.W4, M, N, K)
+    assert d.kernel == b"macaq_iu8_pf_w4_t64x128_s_ks"
+    pb, cb = iu8.gemm_workspace(iu8.W4, M, N, K)
+    part, cnt = torch.full((pb + 64,), 0x5A, dtype=torch.uint8, device="cuda"), torch.full((cb + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    cnt[:cb] = 0
+    c = torch.zeros((M, N), dtype=torch.int16, device="cuda")
+    bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr(), decode_partial=part.data_ptr(), decode_counter=cnt.data_ptr())
+    bufs["as"] = s.data_ptr()
+    for tiles in (False, True, False, False):
+        c.zero_()
+        if tiles:
+            ctx.launch(d, bufs)
+        else:
+            ctx.gemm(iu8.W4, codes.data_ptr(), s.data_ptr(), wf.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K, part.data_ptr(), cnt.data_ptr())
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host_u16(c), r["C"])
+        assert not cnt[:cb].any() and (cnt[cb:] == 0x5A).all() and (part[pb:] == 0x5A).all()
+    with pytest.raises(iu8.IU8Error):
+        ctx.gemm(iu8.W4, codes.data_ptr(), s.data_ptr(), wf.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K)
+
+
 def test_streamed_split_without_both_workspaces_runs_in_one_piece(ctx):
     """The law's own split with one workspace missing, or bound to NULL, needs neither: `gemm` and `launch` run it in one
     piece, write the oracle's bytes and leave the workspace that is there alone."""
