@@ -518,14 +518,17 @@ bool law_split_stream(const saber_iu8_desc &d) {
   return !resolve(v->w8 ? SABER_IU8_W8 : SABER_IU8_W4, (uint32_t)m, (uint32_t)n, (uint32_t)k, &law) && same_launch(d, law);
 }
 
-// 33 to 48 rows of a deep, narrow int4 linear: the descriptor is the tile launch that shares K (pf_split), and the call that has both
+// 33 to 64 rows of a deep, narrow int4 linear: the descriptor is the tile launch that shares K (pf_split), and the call that has both
 // workspaces in hand streams instead, on as many shares or one fewer: its partials are no more than the tiles', and its arrival
 // counters, 16 bits a 64-column block, are a word a 128-column tile. us, tiles / streamed, 33 / 45 / 48 rows of 5120 x 17408 18.2 / 18.8 / 18.4 -> 14.0 /
-// 15.3 / 15.1, 40 of 4096 x 17408 18.0 -> 12.8, of 3072 x 20480 19.5 -> 12.9.
+// 15.3 / 15.1, 50 / 64 19.4 / 19.0 -> 15.9 / 16.4; 40 of 4096 x 17408 18.0 -> 12.8, 64 18.4 -> 14.2; 40 of 3072 x 20480 19.5 -> 12.9. In a pass, behind other kernels, the
+// tiles lose 2 us more (four layers of the served graph at 45 rows 372.7 -> 346.2).
 bool stream_in_tile_workspaces(const saber_iu8_desc &d, saber_iu8_desc *out) {
   int64_t m = 0, n = 0, k = 0;
-  if (strcmp(d.kernel, "macaq_iu8_pf_w4_t64x128_s_ks") || !int_arg(d, "m", &m) || !int_arg(d, "n", &n) || !int_arg(d, "k", &k) || m > 48) return false;
-  const uint32_t z = stream_split((uint32_t)m, (uint32_t)n, (uint32_t)k);
+  if (strcmp(d.kernel, "macaq_iu8_pf_w4_t64x128_s_ks") || !int_arg(d, "m", &m) || !int_arg(d, "n", &n) || !int_arg(d, "k", &k)) return false;
+  if (m > DECODE_MAX_M) return false;
+  // (past the rows that the law's own shares end at the lines in columns and K are the same)
+  const uint32_t z = stream_split(std::min((uint32_t)m, STREAM_SPLIT_ROWS_MAX), (uint32_t)n, (uint32_t)k);
   if (z <= 1 || z > d.ks) return false;
   std::string name = dec_stream_name("w4", (uint32_t)m, (uint32_t)k);
   if (n > 16 * CU_COUNT) name += "_n2";

@@ -541,9 +541,10 @@ def test_streamed_blocks_of_64_columns(ctx, M, N, K, w8):
         np.testing.assert_array_equal(host_u16(c), r["C"])
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 3024, 16384), (48, 4096, 16512), (45, 5136, 17408), (40, 5440, 16384), (48, 5456, 16384)])
+@pytest.mark.parametrize("M,N,K", [(33, 3024, 16384), (48, 4096, 16512), (45, 5136, 17408), (40, 5440, 16384), (48, 5456, 16384),
+                                   (49, 4096, 16384), (64, 5120, 17408)])
 def test_gemm_streams_in_the_workspaces_of_a_tile_launch(ctx, M, N, K):
-    """33 to 48 rows of a deep, narrow linear: the descriptor is the tile launch that shares K, the call with its workspaces
+    """33 to 64 rows of a deep, narrow linear: the descriptor is the tile launch that shares K, the call with its workspaces
     streams (up to 5,440 columns) -- the oracle's bytes every time, nothing written past the workspaces and the counters left at zero, also on
     workspaces that the tile launch itself has used between; without workspaces it is refused as it was."""
     case = synth.dense_case(M, N, K, seed=M + N)
