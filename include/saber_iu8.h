@@ -408,7 +408,8 @@ int saber_iu8_gemm_workspace(int wkind, uint32_t m, uint32_t n, uint32_t k, uint
 
 /* C[m,n] bf16 = epilogue(A . W^T): a/as from the producer, w in the gfx950 fragment order, ws f32
  * [n]. `partial` (scratch) and `counter` (zeroed once by the caller, left zero) may be NULL when
- * saber_iu8_gemm_workspace reports 0.
+ * saber_iu8_gemm_workspace reports 0. (33 to 64 rows of a deep, narrow int4 linear: the resolved launch shares K over tiles; the call
+ * streams on K shares in the same workspaces, which is faster. saber_iu8_launch runs the descriptor as it is.)
  * Non-finite rows: a row whose scale is infinite (an infinity among its activations) gives infinities
  * where its accumulator is not zero and NaNs where it is (0 * inf), exactly where the contract's two
  * multiplies make them (crates/saber-kernels/hip/macaq_iu8.hip:20-24); that an element of c is a NaN is

@@ -583,7 +583,8 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // 21.0 / 22.5 on `tm3_n2`; up to 32 rows streaming wins, 15.5 against 17.5 at 17. A narrower one would stay: 3072 x 16384 at
   // 33 / 45 rows 17.3 / 17.7 shared, 13.7 / 15.0 on `tm3`). The streaming cells' own K shares, which are newer than this line, are faster
   // all over this band at up to 48 rows (stream_split's shares at 40 / 48 rows of 5120 x 17408 14.4 / 15.1, 4096 x 17408 12.8 / 13.3, 3072 x 20480
-  // 12.9 / 13.6, on tiles 18.3 / 18.4, 18.0 / 18.0, 19.5 / 19.6): below K = 16,384 they are what the law takes, the line itself has not moved.
+  // 12.9 / 13.6, on tiles 18.3 / 18.4, 18.0 / 18.0, 19.5 / 19.6): below K = 16,384 they are what the law takes; from there the descriptor
+  // stays and saber_iu8_gemm streams in its workspaces (stream_in_tile_workspaces).
   const PfVariant *split_cell = nullptr;
   const uint32_t tile_ks = pf_split(wkind == SABER_IU8_W8, m, n, k, &split_cell);
   if (const RowsVariant *v = rows_cell(w8, m, n, k, tile_ks && m > 32)) return describe_rows_cell(*v, m, n, k, out);
