@@ -148,16 +148,21 @@ static int describe_dec(const DecVariant &v, uint32_t m, uint32_t n, uint32_t k,
   return 0;
 }
 
+// The tile GEMM addresses its operands with 32-bit byte offsets from a per-step base.
+static uint64_t a_operand_bytes(uint32_t m, uint32_t k) { return (uint64_t)((m + 15) / 16 * 16) * k; }
+static uint64_t w_operand_bytes(bool w8, uint32_t n, uint32_t k) { return (uint64_t)n * k / (w8 ? 1 : 2); }
+static bool tile_operands_hold(bool w8, uint32_t m, uint32_t n, uint32_t k) {
+  return a_operand_bytes(m, k) <= 0xFFFFFFFFull && w_operand_bytes(w8, n, k) <= 0xFFFFFFFFull;
+}
+
 // `ks` > 0 names the cell's split form (`<cell>_ks`, the decode kernarg list): gridDim.z shares of the
 // K steps, none of them empty, `grid[0]` persistent workgroups a share.
 static int describe_pf(const PfVariant &v, uint32_t m, uint32_t n, uint32_t k, uint32_t ks, saber_iu8_desc *d) {
   const char *op = v.w8 ? "gemm_i8a8" : "gemm_i4a8";
   if (int rc = check_shape(op, m, n, k)) return rc;
-  // the tile GEMM addresses its operands with 32-bit byte offsets from a per-step base
-  const uint64_t a_bytes = (uint64_t)((m + 15) / 16 * 16) * k, w_bytes = (uint64_t)n * k / (v.w8 ? 1 : 2);
-  if (a_bytes > 0xFFFFFFFFull || w_bytes > 0xFFFFFFFFull)
+  if (!tile_operands_hold(v.w8, m, n, k))
     return fail(SABER_IU8_E_RULE, fmt("%s: %u x %u x %u puts an operand past 4 GiB (A %llu B, W %llu B), more than the tile GEMM addresses",
-                                      op, m, n, k, (unsigned long long)a_bytes, (unsigned long long)w_bytes));
+                                      op, m, n, k, (unsigned long long)a_operand_bytes(m, k), (unsigned long long)w_operand_bytes(v.w8, n, k)));
   const std::string name = std::string(v.name) + (ks ? "_ks" : "");
   if (ks) {
     const uint32_t steps = k / 128, spb = (steps + ks - 1) / ks;
@@ -489,6 +494,8 @@ static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint
 // as 1,500 do, 49-64 rows of fewer than 64 columns as 64 columns do, and the tile launches that share K (96 x 17408 at 45 rows 17.0 -> 9.5).
 static const RowsVariant *rows_cell(bool w8, uint32_t m, uint32_t n, uint32_t k, bool tile_split) {
   if (m <= ROWS_CELL_ROWS_OVER || m > ROWS_CELL_ROWS_MAX || k < ROWS_CELL_K || k > ROWS_CELL_K_MAX || n > 64 * CU_COUNT || tile_split) return nullptr;
+  // an operand past 4 GiB keeps the answer it has without these cells: the streamed form or the tiles' refusal
+  if (!tile_operands_hold(w8, m, n, k)) return nullptr;
   auto blocks = [&](uint32_t bm, uint32_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn); };
   auto cell = [&](const char *block) { return rows_variant(fmt("macaq_iu8_pf_%s_t%s_r", w8 ? "w8" : "w4", block)); };
   if (m <= ROWS_CELL_FEW_ROWS) {

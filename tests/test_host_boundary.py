@@ -989,6 +989,21 @@ def test_lines_of_the_streamed_cells_on_row_tiles():
         iu8.describe("macaq_iu8_pf_w4_t16x16_r", 1 << 20, 96, 1024)   # more blocks than a launch holds
 
 
+def test_row_tiles_leave_operands_past_4_gib_to_the_other_cells():
+    """An operand past 4 GiB, which the tile GEMM refuses by name, is refused for an output of few tiles as for any other, on either
+    side of the limit in rows, columns and K; up to 64 rows the streamed form, which has no such limit, has it."""
+    for kind, m, n, k in ((iu8.W4, 1518, 112, 13019776), (iu8.W8, 425, 48, 10425088), (iu8.W8, 1181, 48, 4639872), (iu8.W4, 65, 1024, 1 << 23),
+                          (iu8.W4, 256, 64, 1 << 24), (iu8.W8, 65, 256, 1 << 24), (iu8.W4, 2000, 16, 1 << 22)):
+        with pytest.raises(iu8.IU8Error, match="4 GiB") as e:
+            iu8.resolve(kind, m, n, k)
+        assert e.value.code == iu8.E_RULE
+    for kind, m, n, k in ((iu8.W4, 256, 64, (1 << 24) - 128), (iu8.W4, 2000, 16, 2147328), (iu8.W8, 65, 240, 1 << 24)):
+        assert iu8.resolve(kind, m, n, k).kernel.endswith(b"_r"), (m, n, k)
+    assert iu8.resolve(iu8.W4, 17, 1024, 1 << 23).kernel == b"macaq_iu8_dec_w4_tm2_n1"
+    for m, name in ((48, b"macaq_iu8_dec_w8_tm3"), (49, b"macaq_iu8_dec_w8_tm4_k16"), (64, b"macaq_iu8_dec_w8_tm4_k16")):
+        assert iu8.resolve(iu8.W8, m, 256, 1 << 24).kernel == name
+
+
 def test_thin_tiles_by_weight_kind(tmp_path):
     """The layout rule of the 256 x 256 cell (csrc/kernels/iu8_pf_law.h, compiled here): which launches of 256 workgroups run
     the rows past the last whole 256 as thin tiles -- int8 weights only where they measured no slower than whole tiles. Every
