@@ -244,14 +244,12 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
     }
   iu8_stores_done();
   __syncthreads();
-  // two blocks count in one word, 16 bits each: a 64-column launch's counters fit where a 128-column tile launch's would
-  // (rules.cpp:stream_in_tile_workspaces). Z is a grid's z, at most 65,535, so a half never carries into the other.
-  int *const word = &cnt[B.bx >> 1];
-  const unsigned half = (B.bx & 1) * 16;
-  if (tid == 0) s_last = (((unsigned)iu8_arrive(word, (int)(1u << half)) >> half) & 0xFFFFu) == (unsigned)(Z - 1);
+  const iu8_arrival arrival = iu8_arrival_of(B.bx, Z);
+  int *const word = &cnt[arrival.word];
+  if (tid == 0) s_last = arrival.last((unsigned)iu8_arrive(word, (int)arrival.one()), Z);
   __syncthreads();
   if (!s_last) return;
-  if (tid == 0) iu8_arrive(word, (int)(0u - ((unsigned)Z << half)));
+  if (tid == 0) iu8_arrive(word, (int)(0u - arrival.all(Z)));
   constexpr int SH = PASSES * NI <= 2 ? 3 : PASSES * NI <= 9 ? 2 : 1;  // shares asked for at a time
   for (int q0 = 1; q0 < Z; q0 += SH) {
     iu8_v4i v[SH][PASSES][NI];
@@ -283,8 +281,8 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
 }
 
 // A symbol's two cells in one LDS block. The launch's own grid says which runs: 64-column blocks where `nblk` blocks of the
-// symbol's own width would not reach the last column (iu8_stream_law.h is the host's rule for it). So the arrival counters are
-// as many as the grid's blocks, and a grid laid out in the symbol's own blocks stays right where the rule has changed since.
+// symbol's own width would not reach the last column (iu8_stream_law.h is the host's rule for it). So the arrivals are counted
+// by the grid's blocks (iu8_arrival_of: in no more words than blocks), and a grid laid out in the symbol's own blocks stays right where the rule has changed since.
 template <int TM, bool W8, int NT, int KW, int D, bool ACC>
 __device__ __forceinline__ void iu8_stream_cells(const iu8_u8 *__restrict__ A, const iu8_u8 *__restrict__ W, const float *__restrict__ as,
                                                  const float *__restrict__ ws, int *__restrict__ P, int *__restrict__ cnt,

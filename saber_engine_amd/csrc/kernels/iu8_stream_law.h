@@ -1,5 +1,5 @@
 // The block width of the streamed decode cells (iu8_stream.h): the host's launch law lays the grid out by it, and the kernels
-// follow the grid. Plain C++: the host includes it as it is.
+// follow the grid; and where a launch that shares K counts. Plain C++: the host includes it as it is.
 #pragma once
 
 // A symbol of eight k-waves carries two cells: its own (NT 16-column tiles a block, D steps in flight), and 64-column blocks
@@ -31,4 +31,18 @@ constexpr bool iu8_stream_wide(int kw, int own, long m, long n, long k, long ks)
   if (m > IU8_STREAM_FEW_ROWS) return m > IU8_STREAM_ALIGNED_ROWS || !aligned || last <= IU8_STREAM_ALIGNED_LAST;
   if (a_cu == 2) return !aligned || last <= IU8_STREAM_FEW_LAST[1];
   return !aligned && last > IU8_STREAM_FEW_LAST[0] && last <= IU8_STREAM_FEW_LAST[1];
+}
+
+// Where a block of a launch that shares K counts its arrivals: two blocks in one word, 16 bits each, so that a 64-column launch's
+// counters fit where a 128-column tile launch's would (rules.cpp:stream_in_tile_workspaces); a word a block where the shares pass
+// 16 bits (a K of 8.4 million and more, which a pair's halves and a symbol by name take).
+struct iu8_arrival {
+  int word;
+  unsigned shift, mask;
+  constexpr unsigned one() const { return 1u << shift; }
+  constexpr bool last(unsigned before, int shares) const { return ((before >> shift) & mask) == (unsigned)(shares - 1); }
+  constexpr unsigned all(int shares) const { return (unsigned)shares << shift; }
+};
+constexpr iu8_arrival iu8_arrival_of(int block, int shares) {
+  return shares <= 0xFFFF ? iu8_arrival{block >> 1, (block & 1) * 16u, 0xFFFFu} : iu8_arrival{block, 0u, ~0u};
 }

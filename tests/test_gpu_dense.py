@@ -614,6 +614,34 @@ def test_named_streamed_split_needs_its_workspaces(ctx):
         assert e.value.code == iu8.E_ARG
 
 
+@pytest.mark.parametrize("ks", [3, 65535, 65536, 66000])
+def test_pair_of_more_shares_than_16_bits(ctx, ks):
+    """A pair whose halves share a very long K: arrivals past 16 bits are counted too -- the bytes of the launches in one piece,
+    three column blocks of one half beside one of the other, the counters left at zero."""
+    say(f"pair on {ks} shares of K")
+    M, N, NB, K = 5, 144, 16, 128 * 66000
+    g = torch.Generator(device="cuda").manual_seed(ks)
+    rnd = lambda n: torch.randint(0, 256, (n,), generator=g, dtype=torch.uint8, device="cuda")
+    a, w, wb = rnd(iu8.a_bytes(M, K)), rnd(N * K // 2), rnd(NB * K // 2)
+    s, ws, wsb = (torch.rand(n, generator=g, device="cuda") for n in (M, N, NB))
+    want, got = ([torch.full((M, n), 0x7FC0, dtype=torch.int16, device="cuda") for n in (N, NB)] for _ in range(2))
+    for w_, ws_, c_, n in ((w, ws, want[0], N), (wb, wsb, want[1], NB)):
+        d = iu8.describe("macaq_iu8_dec_w4_tm1_a0", M, n, K)
+        ctx.launch(d, {"a": a.data_ptr(), "as": s.data_ptr(), "w": w_.data_ptr(), "ws": ws_.data_ptr(), "c": c_.data_ptr()})
+    d = iu8.pair(*[iu8.describe("macaq_iu8_dec_w4_tm1_a0", M, n, K, ks) for n in (N, NB)])
+    part, partb = (torch.full((ks * M * n,), 0x5A5A5A5A, dtype=torch.int32, device="cuda") for n in (N, NB))
+    cnt, cntb = (torch.zeros(d.workspace(n).bytes // 4, dtype=torch.int32, device="cuda") for n in ("decode_counter", "decode_counter_b"))
+    bufs = {"a": a, "as": s, "w": w, "ws": ws, "c": got[0], "w_b": wb, "ws_b": wsb, "c_b": got[1], "decode_partial": part, "decode_counter": cnt,
+            "decode_partial_b": partb, "decode_counter_b": cntb}
+    bufs = {name: t.data_ptr() for name, t in bufs.items()}
+    for _ in range(2):
+        for c_ in got:
+            c_.fill_(0x7FC0)
+        ctx.launch(d, bufs)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want)) and not cnt.any() and not cntb.any()
+
+
 @pytest.mark.parametrize("kernel,M,N,K,ks,own", [("macaq_iu8_dec_w4_tm1_a0", 16, 3024, 1280, 3, 32), ("macaq_iu8_dec_w8_tm2_n1", 20, 272, 1152, 2, 16),
                                                  ("macaq_iu8_dec_w4_tm2", 17, 8208, 384, 1, 32), ("macaq_iu8_dec_w8_tm3", 33, 12240, 256, 1, 16)])
 def test_streamed_launch_follows_its_grid(ctx, kernel, M, N, K, ks, own):

@@ -1071,6 +1071,36 @@ def test_64_column_blocks_where_they_halve_the_blocks_a_cu():
         assert (p.arg("nb").ival, p.arg("nb_b").ival) == blocks, (m, n0, n1, k)
 
 
+def test_arrivals_of_shared_launches_are_counted_at_any_share_count(tmp_path):
+    """The arrival counters of a streamed launch that shares K (csrc/kernels/iu8_stream_law.h, compiled here), the blocks' arrivals
+    in any order: one last arrival a block, behind all its others, and every word back at zero, in no more words than blocks
+    (half of them up to 16 bits of shares, which is what a tile launch's workspaces hold)."""
+    src, so = tmp_path / "arrival.cpp", tmp_path / "arrival.so"
+    src.write_text(f'#include "{iu8.PKG}/csrc/kernels/iu8_stream_law.h"\n'
+                   'extern "C" int run(int blocks, int shares, int odd_first, unsigned *words) {\n'
+                   '  for (int i = 0; i < blocks; ++i) {\n'
+                   '    const iu8_arrival a = iu8_arrival_of(i, shares);\n'
+                   '    if (a.word < 0 || a.word >= (shares <= 0xFFFF ? (blocks + 1) / 2 : blocks)) return 1;\n'
+                   '  }\n'
+                   '  for (int s = 0; s < shares; ++s)\n'       # the last arrivals of two blocks of a word either way round
+                   '    for (int j = 0; j < blocks; ++j) {\n'
+                   '      const int i = odd_first ? blocks - 1 - j : j;\n'
+                   '      const iu8_arrival a = iu8_arrival_of(i, shares);\n'
+                   '      const unsigned before = words[a.word];\n'
+                   '      words[a.word] += a.one();\n'
+                   '      if (a.last(before, shares) != (s == shares - 1)) return 2;\n'
+                   '      if (s == shares - 1) words[a.word] -= a.all(shares);\n'
+                   '    }\n'
+                   '  return 0;\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    lib = ctypes.CDLL(str(so))
+    for blocks in (1, 2, 3, 80):
+        for shares in (2, 3, 4, 0xFFFE, 0xFFFF, 0x10000, 0x10001, 70000, 1 << 17):
+            for odd_first in (0, 1):
+                words = (ctypes.c_uint * (blocks + 1))()
+                assert lib.run(blocks, shares, odd_first, words) == 0 and not any(words), (blocks, shares, odd_first)
+
+
 def test_band_table_grids_follow_their_cell_rows():
     """Every decode and wide row of the shipped law table states the grid that its cell row and the table's own rules give: the
     block width, the shares of K, one arrival counter a block."""
