@@ -20,3 +20,8 @@ constexpr moe_deal moe_deal_of(int hi, int li, int G, int cost) {
   const int l = li <= rest * cost ? (li + rest - 1) / rest : (li + more * cost + G - 1) / G;
   return moe_deal{more, l > cost ? l - cost : 0, l};
 }
+// How many of nt tiles, `heavy` of them heavy, run on the tile cell in a kernel that does not pass over its item table again and
+// again: all of them, the light ones behind the heavy ones, where the light items are more a position than the table holds.
+constexpr int moe_tile_cell_tiles(int heavy, int nt, int gx, int G, int cost, int light_rounds) {
+  return moe_deal_of(heavy * gx, (nt - heavy) * gx, G, cost).l_rest > light_rounds ? nt : heavy;
+}

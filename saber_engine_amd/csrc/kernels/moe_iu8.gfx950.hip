@@ -757,15 +757,19 @@ MOE_GROUPED_DEC(moe_iu8_grouped_w4_decpb_g1, true, 4, 8, 8, 2, 0, 1, 5)
 // weights come from memory a second time: on the tile cell, two steps ahead, an item waited 20-28 us for its 512 KB,
 // the light cell has twice the bytes in flight (a layer at 4,096 / 4,000 tokens with a shared expert 816 / 866 -> 766 / 817 us).
 // With the light cell's state in registers beside the 256 x 256 tile cell's the compiler spills, and every crossing between two
-// heavy items paid for it (2,048 tokens, no light tile at all: 468 -> 489). It has two registers of spills left: everything that
+// heavy items paid for it (2,048 tokens, no light tile at all: 468 -> 489). It has two or three registers of spills left: everything that
 // is made of the thread's index in front of the walk is opaque to the optimiser, the light items' tables lie
-// behind their cell's stages and are filled when they are due, and a launch of more items than the table holds
-// (64 heavy or 12 light a workgroup) does not pass over it again and again but runs on the tile cell alone.
+// behind their cell's stages and are filled when they are due, and a launch does not pass over the item table again and again. One of
+// more light items than the light cell's block has room for (18 a workgroup: 128 experts of a light tile each on outputs past 9,216
+// columns) has all its tiles on the tile cell, its items still resolved in front up to 64 a workgroup. (With the 12 light items
+// that a 4,096-wide layer needs, and nothing resolved in front past them, a wider one had little or no gain; experts of 272 rows, one cell /
+// that / now: down 8192 x 1536 545 / 536 / 481 us, gate+up 2 x 4096 x 8192 2,612 / 2,625 / 2,429, down 7168 x 4096 1,046 / 1,038 / 962.)
 // (Row maps of the heavy items in LDS as well, so that a crossing reads no row map from memory: 32 more registers of spills, 1 % slower.)
 #define MOE_ORDER_CAP 4096  // tiles the ordering holds in LDS; beyond, table order on the big cell
 #define MOE_LIGHT_ROWS 64
 #define MOE_LIGHT_ST 5
-#define MOE_HEAVY_ROUNDS 8  // rounds of items a workgroup of the 128-row kernels resolves at a time: the item table in LDS
+// rounds of items a workgroup of the 128-row kernels resolves at a time: the item table in LDS
+#define MOE_HEAVY_ROUNDS 8
 #define MOE_LIGHT_ROUNDS 12
 struct __attribute__((aligned(16))) moe_item {
   int row0, rows, nt0, rot;  // rows < 0: no item, and the end of a list of them
@@ -842,8 +846,8 @@ static __device__ __forceinline__ int moe_xcd_run(unsigned b, int G) {
   return (G & 7) == 0 ? (int)(b & 7) * (G >> 3) + (int)(b >> 3) : (int)b;
 }
 // two cells: heavy items on the tile cell, light ones on the small cell between two parts of them. A workgroup resolves HR heavy
-// and MOE_LIGHT_ROUNDS light items at a time; a launch of more runs in as many passes (PASSES), or as a whole on the tile cell
-// with its items resolved as it goes.
+// and LR light items at a time; a launch of more runs in as many passes (PASSES), or as a whole on the tile cell, its items
+// resolved as it goes if they are more than HR a workgroup.
 template <int GATHER, int WMW, int WNW, int TM, int TN, int ST, int HR, int COST, bool PASSES>
 static __device__ __forceinline__ void moe_grouped_pf(
     const unsigned char *__restrict__ a, const unsigned long long *__restrict__ xptr, const int *__restrict__ tile_expert,
@@ -853,12 +857,14 @@ static __device__ __forceinline__ void moe_grouped_pf(
   static_assert(BN == 256 && WMW * WNW == 8, "both cells are 8 waves and 256 columns wide");
   constexpr int LB = iu8_pf32_lds_bytes<false, WMW, WNW, TM, TN, ST, true>();
   constexpr int LL = iu8_pf32_lds_bytes<false, 1, 8, 2, 1, MOE_LIGHT_ST>();
-  constexpr int LT = MOE_LIGHT_ROUNDS * (2 * MOE_LIGHT_ROWS + BN) * 4;  // the light items' tables, behind the light cell's stages
+  // the light items' tables, behind the light cell's stages: without passes as many as fit there in the tile cell's block
+  constexpr int LT1 = (2 * MOE_LIGHT_ROWS + BN) * 4, LR = PASSES ? MOE_LIGHT_ROUNDS : (LB - LL) / LT1, LT = LR * LT1;
+  static_assert(LR >= MOE_LIGHT_ROUNDS, "room for the light items' tables");
   __shared__ __attribute__((aligned(1024))) iu8_u8 lds[LB > LL + LT ? LB : LL + LT];
   __shared__ unsigned short s_order[MOE_ORDER_CAP];
-  __shared__ moe_item s_item[HR + MOE_LIGHT_ROUNDS + 3];  // this workgroup's resolved items
-  float *const s_ws = (float *)(lds + LL), *const s_am = s_ws + MOE_LIGHT_ROUNDS * BN;
-  int *const s_row = (int *)(s_am + MOE_LIGHT_ROUNDS * MOE_LIGHT_ROWS);
+  __shared__ moe_item s_item[HR + LR + 3];  // this workgroup's resolved items
+  float *const s_ws = (float *)(lds + LL), *const s_am = s_ws + LR * BN;
+  int *const s_row = (int *)(s_am + LR * MOE_LIGHT_ROWS);
   // s_item: the heavy items of part 0, an end, those of part 1, an end, the light items, an end
   auto item = [&](int q, iu8_tile &t, int tab = 0) {
     const iu8_v4i lo = *(const iu8_v4i *)&s_item[q].row0, hi = *(const iu8_v4i *)&s_item[q].W;
@@ -872,12 +878,12 @@ static __device__ __forceinline__ void moe_grouped_pf(
   const int nt = meta[0];
   if (nt <= 0) return;
   const bool ordered = nt <= MOE_ORDER_CAP;
-  const int heavy = ordered ? moe_tile_order<NTHR>(tile_rows, tile_expert, tile_row0, xptr, nt, s_order, (moe_item *)lds) : nt;
+  int heavy = ordered ? moe_tile_order<NTHR>(tile_rows, tile_expert, tile_row0, xptr, nt, s_order, (moe_item *)lds) : nt;
   const int gx = (n + BN - 1) / BN;
   if constexpr (!PASSES) {
     const int G = gridDim.x;
-    const moe_deal deal = moe_deal_of(heavy * gx, (nt - heavy) * gx, G, COST);
-    if ((heavy * gx + G - 1) / G > HR || deal.l_rest > MOE_LIGHT_ROUNDS) {
+    heavy = moe_tile_cell_tiles(heavy, nt, gx, G, COST, LR);
+    if ((heavy * gx + G - 1) / G > HR) {
       iu8_pf32_run<false, WMW, WNW, TM, TN, false, ST, false, true, GATHER == 2, true>(a, as, c, n, k, [&](int r, iu8_tile &t) {
         const int j = moe_xcd_run(blockIdx.x, gridDim.x) + r * (int)gridDim.x;
         const int slot = j / gx, bx = j % gx;
@@ -897,9 +903,9 @@ static __device__ __forceinline__ void moe_grouped_pf(
       const int G = gridDim.x, w = moe_xcd_run(blockIdx.x, G);
       const int hi = heavy * gx, li = (nt - heavy) * gx;
       const moe_deal deal = moe_deal_of(hi, li, G, COST);
-      const int h0 = ep * HR, l0 = ep * MOE_LIGHT_ROUNDS;
+      const int h0 = ep * HR, l0 = ep * LR;
       const int rounds = max(0, min(hi / G + (w < deal.more) - h0, HR));
-      lrounds = max(0, min((w < deal.more ? deal.l_more : deal.l_rest) - l0, MOE_LIGHT_ROUNDS));
+      lrounds = max(0, min((w < deal.more ? deal.l_more : deal.l_rest) - l0, LR));
       if (rounds + lrounds == 0) break;
       /* a workgroup's heavy items run in two parts, its light items between them, after `first` rounds */
       const int first = lrounds > 0 ? (w >> 3) % (rounds + 1) : rounds;

@@ -373,6 +373,43 @@ def test_light_and_heavy_items_of_one_workgroup(ctx, tb, kern):
         assert torch.equal(layer.gu[:rows][live], want[:rows][live]), grid
 
 
+def test_light_items_past_the_table_of_the_256_row_kernel(ctx):
+    """The 256-row kernels on grids that give a workgroup 13 to 18 light items (the table's last entries), more than the table holds
+    (all tiles on the tile cell, resolved in front) and more than 64 of those (resolved as it goes): one launch's bytes."""
+    say("light items past the table: moe_iu8_grouped_w4_pf16")
+    counts, T, E, k, H, I = (1, 31, 64, 65, 255, 257, 300, 330), 330, 128, 8, 640, 1152
+    case = synth.moe_case(T=T, E=E, topk=k, H=H, I=I, seed=3, experts=4)
+    lg = np.zeros((T, E), np.float32)
+    for s, c in enumerate(counts):
+        lg[:c, s] = 8.0 - 0.5 * s       # the first c tokens' route s
+        lg[c:, 8 + s] = 8.0 - 0.5 * s   # the others': a second set of experts
+    case["logits"] = synth.f32_to_bf16_bits(lg)
+    layer = run_layer(ctx, case, tile_blocks=16)
+    check_layer(layer, case)
+    nt, rows = (int(layer.buf["meta"][i].item()) for i in (0, 1))
+    tile_rows = layer.buf["tile_rows"][:nt].cpu().numpy()
+    live = layer.buf["row_tok"][:rows] >= 0
+    tables = {n_: layer.buf[n_].data_ptr() for n_ in ("tile_expert", "tile_row0", "tile_rows", "row_tok", "meta")}
+    for kern, a, s_, xptr, out, n, kk in (("g2", layer.q1, layer.s1, layer.xptr_gu, layer.gu, 2 * I, H), ("g0", layer.q2, layer.s2, layer.xptr_dn, layer.y, H, I)):
+        want, gx = out.clone(), -(-n // 256)
+        hi, li = (tile_rows > 64).sum() * gx, (tile_rows <= 64).sum() * gx
+        seen = set()
+        for grid in (8, 6, 5, 4, 3, 2, 1):
+            more = hi % grid
+            light = -(-li // (grid - more)) if li <= (grid - more) * 4 else -(-(li + more * 4) // grid)
+            seen.add("table" if 12 < light <= 18 else "tiles" if light > 18 and nt * gx <= 64 * grid else "walk" if light > 18 else "")
+            d = iu8.describe_raw(f"moe_iu8_grouped_w4_pf16_{kern}", (grid, 1, 1), 512, plugin="moe_iu8", n=n, k=kk, pmax=0)
+            for name in ("p", "cnt"):
+                d.arg(name).kind = iu8.ARG_NULL_BUFFER
+            bufs = dict(a=a.data_ptr(), xptr=xptr.data_ptr(), c=out.data_ptr(), **tables)
+            bufs["as"] = s_.data_ptr()
+            out.fill_(0x7FC0)
+            ctx.launch(d, bufs)
+            torch.cuda.synchronize()
+            assert torch.equal(out[:rows][live], want[:rows][live]), (kern, grid)
+        assert {"table", "tiles", "walk"} <= seen or kern == "g0", seen
+
+
 def test_moe_router_ties_and_skew(ctx):
     say("moe router: ties and one hot expert")
     case = synth.moe_case(T=40, E=128, topk=8, H=512, I=256, seed=5, experts=4)

@@ -1174,3 +1174,25 @@ def test_routed_items_are_dealt_once_and_level(tmp_path):
         assert sorted(got) == list(range(li)), (hi, li, G, cost)
         top = max(x for x, n in load if n) if li else 0
         assert all(x >= top - 1 - cost for x, _ in load), (hi, li, G, cost)
+
+
+def test_routed_launches_keep_both_cells_on_wide_experts(tmp_path):
+    """Which tiles of a 256-row routed launch run on the tile cell (csrc/kernels/moe_deal.h, compiled here; a table of 18 light items a
+    workgroup): 128 experts of a full tile and a light one keep both cells up to outputs of 9,216 columns, and past the
+    table all tiles run on the tile cell, where a launch of up to 64 of its items a workgroup still has them resolved in front."""
+    src, so = tmp_path / "cells.cpp", tmp_path / "cells.so"
+    src.write_text(f'#include "{iu8.PKG}/csrc/kernels/moe_deal.h"\n'
+                   'extern "C" int tiles(int heavy, int nt, int gx, int G, int cost, int lr) { return moe_tile_cell_tiles(heavy, nt, gx, G, cost, lr); }\n'
+                   'extern "C" int rounds(int hi, int li, int G, int cost) { return moe_deal_of(hi, li, G, cost).l_rest; }\n')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    lib = ctypes.CDLL(str(so))
+    for columns, tiles in ((3072, 128), (4096, 128), (7168, 128), (8192, 128), (9216, 128), (9472, 256), (16384, 256)):
+        assert lib.tiles(128, 256, columns // 256, 256, 4, 18) == tiles, columns
+    assert 256 * (16384 // 256) <= 64 * 256
+    rng = np.random.default_rng(11)
+    for _ in range(2000):
+        nt, gx, G, lr = int(rng.integers(1, 900)), int(rng.integers(1, 70)), int(rng.choice([1, 3, 8, 61, 256])), int(rng.choice([12, 18]))
+        heavy = int(rng.integers(0, nt + 1))
+        kept = lib.tiles(heavy, nt, gx, G, 4, lr)
+        assert kept == (heavy if lib.rounds(heavy * gx, (nt - heavy) * gx, G, 4) <= lr else nt)
+        assert lib.rounds(kept * gx, (nt - kept) * gx, G, 4) <= lr           # what the light table is asked to hold
