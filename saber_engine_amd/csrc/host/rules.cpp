@@ -497,19 +497,23 @@ static const RowsVariant *rows_cell(bool w8, uint32_t m, uint32_t n, uint32_t k,
   // an operand past 4 GiB keeps the answer it has without these cells: the streamed form or the tiles' refusal
   if (!tile_operands_hold(w8, m, n, k)) return nullptr;
   auto blocks = [&](uint32_t bm, uint32_t bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn); };
-  auto cell = [&](const char *block) { return rows_variant(fmt("macaq_iu8_pf_%s_t%s_r", w8 ? "w8" : "w4", block)); };
+  // (the variants looked up once)
+  static const RowsVariant *const W4_16X16 = rows_variant("macaq_iu8_pf_w4_t16x16_r"), *const W8_16X16 = rows_variant("macaq_iu8_pf_w8_t16x16_r"),
+                           *const W4_16X32 = rows_variant("macaq_iu8_pf_w4_t16x32_r"), *const W4_32X32 = rows_variant("macaq_iu8_pf_w4_t32x32_r"),
+                           *const W4_32X64 = rows_variant("macaq_iu8_pf_w4_t32x64_r");
+  const RowsVariant *const smallest = w8 ? W8_16X16 : W4_16X16;
   if (m <= ROWS_CELL_FEW_ROWS) {
     const bool deep = k >= ROWS_CELL_FEW_DEEP_K;
     const uint32_t widest = w8 ? (deep ? ROWS_CELL_W8_FEW_N : 0) : deep ? ROWS_CELL_FEW_DEEP_N : ROWS_CELL_FEW_N;
-    return n <= widest ? cell("16x16") : nullptr;
+    return n <= widest ? smallest : nullptr;
   }
   if (m <= DECODE_MAX_M && n < ROWS_CELL_64_ROWS_N) return nullptr;
-  if (blocks(16, 16) <= CU_COUNT) return cell("16x16");
+  if (blocks(16, 16) <= CU_COUNT) return smallest;
   if (w8) return nullptr;
-  if (blocks(16, 32) <= CU_COUNT) return cell("16x32");
+  if (blocks(16, 32) <= CU_COUNT) return W4_16X32;
   if (m <= DECODE_MAX_M) return nullptr;
-  if (blocks(32, 32) <= (k >= ROWS_CELL_32_K ? CU_COUNT : ROWS_CELL_32_BLOCKS)) return cell("32x32");
-  return blocks(32, 64) <= (m <= ROWS_CELL_64_ROWS ? CU_COUNT : ROWS_CELL_64_BLOCKS) && k >= ROWS_CELL_64_K ? cell("32x64") : nullptr;
+  if (blocks(32, 32) <= (k >= ROWS_CELL_32_K ? CU_COUNT : ROWS_CELL_32_BLOCKS)) return W4_32X32;
+  return blocks(32, 64) <= (m <= ROWS_CELL_64_ROWS ? CU_COUNT : ROWS_CELL_64_BLOCKS) && k >= ROWS_CELL_64_K ? W4_32X64 : nullptr;
 }
 
 // Which launch `a` and `b` are, whatever their workspaces.
@@ -537,9 +541,11 @@ bool stream_in_tile_workspaces(const saber_iu8_desc &d, saber_iu8_desc *out) {
   // (past the rows that the law's own shares end at the lines in columns and K are the same)
   const uint32_t z = stream_split(std::min((uint32_t)m, STREAM_SPLIT_ROWS_MAX), (uint32_t)n, (uint32_t)k);
   if (z <= 1 || z > d.ks) return false;
-  std::string name = dec_stream_name("w4", (uint32_t)m, (uint32_t)k);
-  if (n > 16 * CU_COUNT) name += "_n2";
-  return !describe(name, (uint32_t)m, (uint32_t)n, (uint32_t)k, z, out);
+  // the streamed symbol of the rows and columns (looked up once)
+  static const DecVariant *const TM3 = dec_variant("macaq_iu8_dec_w4_tm3"), *const TM3_N2 = dec_variant("macaq_iu8_dec_w4_tm3_n2"),
+                          *const TM4 = dec_variant("macaq_iu8_dec_w4_tm4"), *const TM4_N2 = dec_variant("macaq_iu8_dec_w4_tm4_n2");
+  const DecVariant *v = n > 16 * CU_COUNT ? (m <= 48 ? TM3_N2 : TM4_N2) : (m <= 48 ? TM3 : TM4);
+  return !describe_dec(*v, (uint32_t)m, (uint32_t)n, (uint32_t)k, z, out);
 }
 
 int unsplit_stream(saber_iu8_desc *d) {
@@ -670,14 +676,16 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // slowest 0.99. 256 rows are held on the 64 x 128 cell (5120 x 5120 21.3 for 18.6).
   if (w8 && m > 64) {
     auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)((n + bn - 1) / bn) * ((m + bm - 1) / bm); };
+    static const PfVariant *const T128X160 = pf_variant("macaq_iu8_pf_w8_t128x160"), *const T128X64 = pf_variant("macaq_iu8_pf_w8_t128x64_s"),
+                           *const T128X128 = pf_variant("macaq_iu8_pf_w8_t128x128");
     const PfVariant *est = pf_cell(w8, m, n, k);
     const bool small = est->block_m() == 64;
     const bool pays = small ? k >= 5120 : m <= 128 || k < 512 || k >= 3072 || tiles(128, 160) % 8 == 0;
-    if (m < 1024 && pays && tiles(128, 160) <= CU_COUNT && tiles(128, 128) > CU_COUNT) est = pf_variant("macaq_iu8_pf_w8_t128x160");
+    if (m < 1024 && pays && tiles(128, 160) <= CU_COUNT && tiles(128, 128) > CU_COUNT) est = T128X160;
     else if (small && tiles(128, 64) <= CU_COUNT) {
-      if (m != 256 && tiles(64, 64) > CU_COUNT && k >= (tiles(128, 64) % 8 ? 4096u : 2048u)) est = pf_variant("macaq_iu8_pf_w8_t128x64_s");
+      if (m != 256 && tiles(64, 64) > CU_COUNT && k >= (tiles(128, 64) % 8 ? 4096u : 2048u)) est = T128X64;
     } else if (small && tiles(128, 128) <= CU_COUNT && tiles(64, 128) > CU_COUNT) {
-      est = pf_variant("macaq_iu8_pf_w8_t128x128");
+      est = T128X128;
     }
     return describe_pf(*est, m, n, k, 0, out);
   }
