@@ -299,6 +299,14 @@ def test_tile_cells_either_side_of_their_short_k(ctx, cell, K, M, N, grid):
     assert (got[M] == 0x7FC0).all()
 
 
+@pytest.mark.parametrize("K", [128, 512, 640, 768, 1152, 2176])
+@pytest.mark.parametrize("M,N,grid", [(1, 16, 1), (33, 48, 1), (130, 272, 6), (300, 400, 7)])
+def test_int4_64x64_cell_of_two_k_waves(ctx, K, M, N, grid):
+    """Its form of one wave a wave tile up to K = 512 and its two k-waves from there: odd and even counts of K steps, fewer than
+    the stages and more, a row block and a column block without an element, several tiles a workgroup."""
+    test_tile_cells_either_side_of_their_short_k(ctx, "w4_t64x64_s", K, M, N, grid)
+
+
 def test_split_counter_is_reusable_across_launches(ctx):
     say("explicit split, two launches on one counter")
     case = synth.dense_case(3, 256, 2048, seed=23)

@@ -558,8 +558,12 @@ def test_gemm_streams_in_the_workspaces_of_a_tile_launch(ctx, M, N, K):
     c = torch.zeros((M, N), dtype=torch.int16, device="cuda")
     bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr(), decode_partial=part.data_ptr(), decode_counter=cnt.data_ptr())
     bufs["as"] = s.data_ptr()
+    # a streamed launch on fewer shares than the tile launch has leaves the last shares' slab as it was
+    shares = min(4, 256 // -(-N // 64))
+    slab, streams = shares * M * N * 4, N <= 5440
     for tiles in (False, True, False, False):
         c.zero_()
+        part[:pb] = 0x5A
         if tiles:
             ctx.launch(d, bufs)
         else:
@@ -567,6 +571,9 @@ def test_gemm_streams_in_the_workspaces_of_a_tile_launch(ctx, M, N, K):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(host_u16(c), r["C"])
         assert not cnt[:cb].any() and (cnt[cb:] == 0x5A).all() and (part[pb:] == 0x5A).all()
+        if shares < d.ks:
+            assert (part[slab:pb] == 0x5A).all().item() == (streams and not tiles)
+    assert shares < d.ks or N <= 4096
     with pytest.raises(iu8.IU8Error):
         ctx.gemm(iu8.W4, codes.data_ptr(), s.data_ptr(), wf.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K)
 

@@ -410,6 +410,41 @@ def test_light_items_past_the_table_of_the_256_row_kernel(ctx):
         assert {"table", "tiles", "walk"} <= seen or kern == "g0", seen
 
 
+@pytest.mark.parametrize("kern", ["moe_iu8_grouped_w4_pf", "moe_iu8_grouped_w4_pf16"])
+def test_tile_tables_of_more_tiles_than_threads(ctx, kern):
+    """Tables of more tiles than a workgroup has threads (a prompt of some 12,300 tokens on 256-row tiles), light and heavy ones: the
+    ordering runs in chunks and an item's entries are read when it is resolved. The table is the router's at 80 rows a tile; the
+    rows are those of the layer that the oracle checks, whatever the tiles."""
+    say(f"more than 512 tiles: {kern}")
+    T, E, k, H, I = 5200, 128, 8, 128, 384
+    case = synth.moe_case(T=T, E=E, topk=k, H=H, I=I, seed=7, experts=4)
+    layer = run_layer(ctx, case, tile_blocks=8)
+    check_layer(layer, case)
+    rows = int(layer.buf["meta"][1].item())
+    live = layer.buf["row_tok"][:rows] >= 0
+    fine = MoeLayerIU8(ctx, T, E, k, H, I, tile_blocks=5)
+    lg = dev_bf16_bits(case["logits"])
+    ctx.moe_route(lg.data_ptr(), T, E, k, 5, fine.tables)
+    torch.cuda.synchronize()
+    nt = int(fine.buf["meta"][0].item())
+    tile_rows = fine.buf["tile_rows"][:nt].cpu().numpy()
+    assert nt > 512 and (tile_rows > 64).sum() > 256 and (tile_rows <= 64).sum() > 64
+    assert torch.equal(fine.buf["row_tok"][:rows], layer.buf["row_tok"][:rows])
+    tables = {n_: fine.buf[n_].data_ptr() for n_ in ("tile_expert", "tile_row0", "tile_rows", "row_tok", "meta")}
+    for gather, a, s_, xptr, out, n, kk in (("g2", layer.q1, layer.s1, layer.xptr_gu, layer.gu, 2 * I, H), ("g0", layer.q2, layer.s2, layer.xptr_dn, layer.y, H, I)):
+        want = out.clone()
+        for grid in (256, 61, 8):
+            d = iu8.describe_raw(f"{kern}_{gather}", (grid, 1, 1), 512, plugin="moe_iu8", n=n, k=kk, pmax=0)
+            for name in ("p", "cnt"):
+                d.arg(name).kind = iu8.ARG_NULL_BUFFER
+            bufs = dict(a=a.data_ptr(), xptr=xptr.data_ptr(), c=out.data_ptr(), **tables)
+            bufs["as"] = s_.data_ptr()
+            out.fill_(0x7FC0)
+            ctx.launch(d, bufs)
+            torch.cuda.synchronize()
+            assert torch.equal(out[:rows][live], want[:rows][live]), (gather, grid)
+
+
 def test_moe_router_ties_and_skew(ctx):
     say("moe router: ties and one hot expert")
     case = synth.moe_case(T=40, E=128, topk=8, H=512, I=256, seed=5, experts=4)

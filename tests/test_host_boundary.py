@@ -1148,9 +1148,51 @@ def test_band_table_grids_follow_their_cell_rows():
         assert iu8.describe(name, m, n, k, ks).grid[0] == -(-n // width(c, m, n, k, ks)), (name, m, n, k, ks)
 
 
+def test_lines_of_the_calls_that_stream_in_a_tile_launchs_workspaces(tmp_path):
+    """What saber_iu8_gemm makes of the law's tile launches that share K (rules.cpp:stream_in_tile_workspaces, called in the library):
+    which shapes stream, on which symbol and shares, either side of the lines in rows, columns and K; partials and
+    counters are never more than the tile launch's, counting as the kernel does."""
+    src, so = tmp_path / "streams.cpp", tmp_path / "streams.so"
+    src.write_text(f'#include "{iu8.ROOT}/include/saber_iu8.h"\n#include "{iu8.PKG}/csrc/host/rules.h"\n#include "{iu8.PKG}/csrc/kernels/iu8_stream_law.h"\n'
+                   'extern "C" int streams(const saber_iu8_desc *d, saber_iu8_desc *out) { return iu8::stream_in_tile_workspaces(*d, out); }\n'
+                   'extern "C" int words(int blocks, int shares) {\n'
+                   '  int n = 0;\n'
+                   '  for (int i = 0; i < blocks; ++i) n = iu8_arrival_of(i, shares).word + 1;\n'
+                   '  return n;\n}\n')
+    lib_dir = os.path.dirname(iu8.lib()._name)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so), f"-L{lib_dir}", "-lsaber_iu8", f"-Wl,-rpath,{lib_dir}"], check=True)
+    lib = ctypes.CDLL(str(so))
+
+    def streamed(m, n, k):
+        tiles, out = iu8.resolve(iu8.W4, m, n, k), iu8.Desc()
+        return tiles, out if lib.streams(ctypes.byref(tiles), ctypes.byref(out)) else None
+
+    for (m, n, k), want in {(33, 5120, 16384): ("tm3_n2", 3), (48, 5120, 17408): ("tm3_n2", 3), (49, 5120, 17408): ("tm4_n2", 3), (64, 5120, 17408): ("tm4_n2", 3),
+                            (65, 5120, 17408): None, (33, 4096, 16384): ("tm3", 4), (48, 4112, 16384): ("tm3_n2", 3), (64, 4096, 16384): ("tm4", 4),
+                            (33, 3024, 16384): ("tm3", 4), (33, 3008, 16384): None, (64, 3008, 16384): None, (48, 5440, 16384): ("tm3_n2", 3),
+                            (48, 5456, 16384): None, (64, 5456, 16384): None, (45, 8192, 16384): None, (32, 5120, 17408): None, (45, 5120, 16256): None}.items():
+        tiles, d = streamed(m, n, k)
+        assert (tiles.kernel == b"macaq_iu8_pf_w4_t64x128_s_ks") == (33 <= m and k >= 16384), (m, n, k)
+        assert (d and (d.kernel.decode()[len("macaq_iu8_dec_w4_"):], d.ks)) == want, (m, n, k)
+    rng = np.random.default_rng(2)
+    taken = 0
+    for _ in range(4000):
+        m, n, k = int(rng.integers(33, 65)), 16 * int(rng.integers(180, 360)), 128 * int(rng.integers(120, 300))
+        tiles, d = streamed(m, n, k)
+        if d is None:
+            continue
+        taken += 1
+        assert d.grid[2] == d.ks and d.grid[0] == -(-n // 64) and d.ks <= tiles.ks
+        assert d.workspace("decode_partial").bytes <= tiles.workspace("decode_partial").bytes
+        assert 4 * lib.words(d.grid[0], d.ks) <= tiles.workspace("decode_counter").bytes
+    assert taken > 1000
+
+
 def test_routed_items_are_dealt_once_and_level(tmp_path):
     """The deal of the routed tile launches (csrc/kernels/moe_deal.h, compiled here): every light item goes to one position
-    once, and no position's share (a heavy item counts `cost`) is more than one heavy item above another's that has light ones."""
+    once, and no position that has light ones has a larger share (a heavy item counts `cost`) than the level one, all of it over the
+    positions rounded up, or one more heavy item than every position has alone. Dealt evenly, the two kinds apart, 31 of
+    these 70 cases have."""
     src, so = tmp_path / "deal.cpp", tmp_path / "deal.so"
     src.write_text(f'#include "{iu8.PKG}/csrc/kernels/moe_deal.h"\n'
                    'extern "C" int share(int hi, int li, int G, int cost, int w, int *ids) {\n'
@@ -1165,6 +1207,7 @@ def test_routed_items_are_dealt_once_and_level(tmp_path):
     cases = [(0, 1, 256, 2), (24, 1548, 256, 2), (256, 0, 256, 2), (255, 1, 256, 4), (1, 256, 256, 2), (1, 255, 256, 2), (1536, 700, 256, 4),
              (0, 2048, 256, 2), (5, 3, 3, 2), (1, 2, 1, 4)]
     cases += [(int(rng.integers(0, 3000)), int(rng.integers(0, 3000)), int(rng.choice([1, 3, 16, 255, 256])), int(rng.choice([2, 4]))) for _ in range(60)]
+    uneven = 0
     for hi, li, G, cost in cases:
         got, load = [], []
         for w in range(G):
@@ -1172,8 +1215,11 @@ def test_routed_items_are_dealt_once_and_level(tmp_path):
             got += ids[:n]
             load.append((cost * (hi // G + (w < hi % G)) + n, n))
         assert sorted(got) == list(range(li)), (hi, li, G, cost)
-        top = max(x for x, n in load if n) if li else 0
-        assert all(x >= top - 1 - cost for x, _ in load), (hi, li, G, cost)
+        level = max(-(-(cost * hi + li) // G), cost * (hi // G + 1))
+        assert all(x <= level for x, n in load if n), (hi, li, G, cost)
+        even = [(cost * (hi // G + (w < hi % G)) + n, n) for w, n in enumerate(li // G + (G - 1 - w < li % G) for w in range(G))]
+        uneven += any(x > level for x, n in even if n)
+    assert uneven == 31
 
 
 def test_routed_launches_keep_both_cells_on_wide_experts(tmp_path):
