@@ -558,12 +558,8 @@ def test_gemm_streams_in_the_workspaces_of_a_tile_launch(ctx, M, N, K):
     c = torch.zeros((M, N), dtype=torch.int16, device="cuda")
     bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr(), decode_partial=part.data_ptr(), decode_counter=cnt.data_ptr())
     bufs["as"] = s.data_ptr()
-    # a streamed launch on fewer shares than the tile launch has leaves the last shares' slab as it was
-    shares = min(4, 256 // -(-N // 64))
-    slab, streams = shares * M * N * 4, N <= 5440
     for tiles in (False, True, False, False):
         c.zero_()
-        part[:pb] = 0x5A
         if tiles:
             ctx.launch(d, bufs)
         else:
@@ -571,11 +567,35 @@ def test_gemm_streams_in_the_workspaces_of_a_tile_launch(ctx, M, N, K):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(host_u16(c), r["C"])
         assert not cnt[:cb].any() and (cnt[cb:] == 0x5A).all() and (part[pb:] == 0x5A).all()
-        if shares < d.ks:
-            assert (part[slab:pb] == 0x5A).all().item() == (streams and not tiles)
-    assert shares < d.ks or N <= 4096
     with pytest.raises(iu8.IU8Error):
         ctx.gemm(iu8.W4, codes.data_ptr(), s.data_ptr(), wf.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 5120, 16384), (48, 5136, 16384), (45, 5440, 17408), (48, 5456, 16384), (49, 5120, 17408), (64, 5120, 17408)])
+def test_gemm_in_a_tile_launchs_workspaces_is_the_streamed_launch(ctx, M, N, K):
+    """Seen on the card: the streamed launch has fewer shares than the tile launch and leaves the last ones' slab as it was, the tile
+    launch writes it (and so does the call past 5,440 columns, which stays on tiles)."""
+    case = synth.dense_case(M, N, K, seed=M + N)
+    r = ref.linear(case["X"], case["W"], case["ws"], False, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], False)), dev_f32(case["ws"])
+    d = iu8.resolve(iu8.W4, M, N, K)
+    pb, cb = iu8.gemm_workspace(iu8.W4, M, N, K)
+    part, cnt = torch.empty(pb, dtype=torch.uint8, device="cuda"), torch.zeros(cb, dtype=torch.uint8, device="cuda")
+    c = torch.zeros((M, N), dtype=torch.int16, device="cuda")
+    bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr(), decode_partial=part.data_ptr(), decode_counter=cnt.data_ptr())
+    bufs["as"] = s.data_ptr()
+    slab = min(4, 256 // -(-N // 64)) * M * N * 4
+    assert slab < pb
+    for tiles in (False, True):
+        c.zero_()
+        part.fill_(0x5A)
+        if tiles:
+            ctx.launch(d, bufs)
+        else:
+            ctx.gemm(iu8.W4, codes.data_ptr(), s.data_ptr(), wf.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K, part.data_ptr(), cnt.data_ptr())
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host_u16(c), r["C"])
+        assert (part[slab:] == 0x5A).all().item() == (N <= 5440 and not tiles)
 
 
 def test_streamed_split_without_both_workspaces_runs_in_one_piece(ctx):

@@ -1190,7 +1190,34 @@ def test_lines_of_the_calls_that_stream_in_a_tile_launchs_workspaces(tmp_path):
 
 def test_routed_items_are_dealt_once_and_level(tmp_path):
     """The deal of the routed tile launches (csrc/kernels/moe_deal.h, compiled here): every light item goes to one position
-    once, and no position that has light ones has a larger share (a heavy item counts `cost`) than the level one, all of it over the
+    once, and no position's share (a heavy item counts `cost`) is more than one heavy item above another's that has light ones."""
+    src, so = tmp_path / "deal.cpp", tmp_path / "deal.so"
+    src.write_text(f'#include "{iu8.PKG}/csrc/kernels/moe_deal.h"\n'
+                   'extern "C" int share(int hi, int li, int G, int cost, int w, int *ids) {\n'
+                   '  const moe_deal d = moe_deal_of(hi, li, G, cost);\n'
+                   '  int n = 0;\n'
+                   '  for (int r = 0; r < (w < d.more ? d.l_more : d.l_rest); ++r)\n'
+                   '    if (d.light_id(r, w, G) < li) ids[n++] = d.light_id(r, w, G);\n'
+                   '  return n;\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    lib, ids = ctypes.CDLL(str(so)), (ctypes.c_int * 4096)()
+    rng = np.random.default_rng(3)
+    cases = [(0, 1, 256, 2), (24, 1548, 256, 2), (256, 0, 256, 2), (255, 1, 256, 4), (1, 256, 256, 2), (1, 255, 256, 2), (1536, 700, 256, 4),
+             (0, 2048, 256, 2), (5, 3, 3, 2), (1, 2, 1, 4)]
+    cases += [(int(rng.integers(0, 3000)), int(rng.integers(0, 3000)), int(rng.choice([1, 3, 16, 255, 256])), int(rng.choice([2, 4]))) for _ in range(60)]
+    for hi, li, G, cost in cases:
+        got, load = [], []
+        for w in range(G):
+            n = lib.share(hi, li, G, cost, w, ids) if (li // G + cost + 2) < 4096 else 0
+            got += ids[:n]
+            load.append((cost * (hi // G + (w < hi % G)) + n, n))
+        assert sorted(got) == list(range(li)), (hi, li, G, cost)
+        top = max(x for x, n in load if n) if li else 0
+        assert all(x >= top - 1 - cost for x, _ in load), (hi, li, G, cost)
+
+
+def test_routed_items_are_dealt_to_the_level_share(tmp_path):
+    """No position that has light items has a larger share (a heavy item counts `cost`) than the level one, all of it over the
     positions rounded up, or one more heavy item than every position has alone. Dealt evenly, the two kinds apart, 31 of
     these 70 cases have."""
     src, so = tmp_path / "deal.cpp", tmp_path / "deal.so"
