@@ -545,6 +545,7 @@ bool stream_in_tile_workspaces(const saber_iu8_desc &d, saber_iu8_desc *out) {
   static const DecVariant *const TM3 = dec_variant("macaq_iu8_dec_w4_tm3"), *const TM3_N2 = dec_variant("macaq_iu8_dec_w4_tm3_n2"),
                           *const TM4 = dec_variant("macaq_iu8_dec_w4_tm4"), *const TM4_N2 = dec_variant("macaq_iu8_dec_w4_tm4_n2");
   const DecVariant *v = n > 16 * CU_COUNT ? (m <= 48 ? TM3_N2 : TM4_N2) : (m <= 48 ? TM3 : TM4);
+  if (!iu8_stream_shared_words(false, v->tm, (long)k)) return false;  // (its counters would not fit)
   return !describe_dec(*v, (uint32_t)m, (uint32_t)n, (uint32_t)k, z, out);
 }
 

@@ -244,7 +244,7 @@ __device__ __forceinline__ void iu8_stream_body(iu8_u8 *__restrict__ lds, const 
     }
   iu8_stores_done();
   __syncthreads();
-  const iu8_arrival arrival = iu8_arrival_of(B.bx, Z);
+  const iu8_arrival arrival = iu8_arrival_of(B.bx, Z, iu8_stream_shared_words(W8, TM, K));
   int *const word = &cnt[arrival.word];
   if (tid == 0) s_last = arrival.last((unsigned)iu8_arrive(word, (int)arrival.one()), Z);
   __syncthreads();

@@ -33,9 +33,12 @@ constexpr bool iu8_stream_wide(int kw, int own, long m, long n, long k, long ks)
   return !aligned && last > IU8_STREAM_FEW_LAST[0] && last <= IU8_STREAM_FEW_LAST[1];
 }
 
-// Where a block of a launch that shares K counts its arrivals: two blocks in one word, 16 bits each, so that a 64-column launch's
-// counters fit where a 128-column tile launch's would (rules.cpp:stream_in_tile_workspaces); a word a block where the shares pass
-// 16 bits (a K of 8.4 million and more, which a pair's halves and a symbol by name take).
+// Where a block of a launch that shares K counts its arrivals: in a word of its own, or, where `two`, two blocks in one word, 16 bits
+// each, so that a 64-column launch's counters fit where a 128-column tile launch's would (rules.cpp:stream_in_tile_workspaces). A word
+// a block is the faster one, 2-5 % of a launch (us, two / one: 9 rows of 3184 x 10368 7.89 / 7.50, 16 of 5120 x 10240 8.73 / 8.38, 36 10.84 / 10.57,
+// 48 of 5120 x 12288 11.97 / 11.75; int8 and K = 17,408 1-2 % or level), so words are shared only by the launches that may stand in such workspaces; and never where
+// the shares pass 16 bits (a K of 8.4 million and more, which a pair's halves and a symbol by name take).
+constexpr bool iu8_stream_shared_words(bool w8, int tm, long k) { return !w8 && tm >= 3 && k >= 16384; }
 struct iu8_arrival {
   int word;
   unsigned shift, mask;
@@ -43,6 +46,6 @@ struct iu8_arrival {
   constexpr bool last(unsigned before, int shares) const { return ((before >> shift) & mask) == (unsigned)(shares - 1); }
   constexpr unsigned all(int shares) const { return (unsigned)shares << shift; }
 };
-constexpr iu8_arrival iu8_arrival_of(int block, int shares) {
-  return shares <= 0xFFFF ? iu8_arrival{block >> 1, (block & 1) * 16u, 0xFFFFu} : iu8_arrival{block, 0u, ~0u};
+constexpr iu8_arrival iu8_arrival_of(int block, int shares, bool two = true) {
+  return two && shares <= 0xFFFF ? iu8_arrival{block >> 1, (block & 1) * 16u, 0xFFFFu} : iu8_arrival{block, 0u, ~0u};
 }

@@ -598,6 +598,31 @@ def test_gemm_in_a_tile_launchs_workspaces_is_the_streamed_launch(ctx, M, N, K):
         assert (part[slab:] == 0x5A).all().item() == (N <= 5440 and not tiles)
 
 
+@pytest.mark.parametrize("kernel,M,N", [("macaq_iu8_dec_w4_tm3", 33, 208), ("macaq_iu8_dec_w4_tm4_n2", 64, 80), ("macaq_iu8_dec_w8_tm3_n2", 48, 144)])
+@pytest.mark.parametrize("K", [16256, 16384])
+def test_arrivals_either_side_of_shared_words(ctx, kernel, M, N, K):
+    """K shares of three row tiles and more, below and from the K at which an int4 launch counts two blocks in one word: the oracle's
+    bytes twice on the same counters, none of them touched behind the blocks', all left at zero."""
+    w8 = "_w8_" in kernel
+    case = synth.dense_case(M, N, K, w8=w8, seed=M + N + K)
+    r = ref.linear(case["X"], case["W"], case["ws"], w8, threads=8)
+    codes, s, wf, ws = dev_u8(iu8.repack_a(r["q"])), dev_f32(r["a_scale"]), dev_u8(iu8.repack_weights(case["W"], w8)), dev_f32(case["ws"])
+    d = iu8.describe(kernel, M, N, K, ks=3)
+    cb = d.workspace("decode_counter").bytes
+    part = torch.empty(d.workspace("decode_partial").bytes, dtype=torch.uint8, device="cuda")
+    cnt = torch.full((cb + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    cnt[:cb] = 0
+    c = torch.zeros((M, N), dtype=torch.int16, device="cuda")
+    bufs = dict(a=codes.data_ptr(), w=wf.data_ptr(), ws=ws.data_ptr(), c=c.data_ptr(), decode_partial=part.data_ptr(), decode_counter=cnt.data_ptr())
+    bufs["as"] = s.data_ptr()
+    for _ in range(2):
+        c.zero_()
+        ctx.launch(d, bufs)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(host_u16(c), r["C"])
+        assert not cnt[:cb].any() and (cnt[cb:] == 0x5A).all()
+
+
 def test_streamed_split_without_both_workspaces_runs_in_one_piece(ctx):
     """The law's own split with one workspace missing, or bound to NULL, needs neither: `gemm` and `launch` run it in one
     piece, write the oracle's bytes and leave the workspace that is there alone."""

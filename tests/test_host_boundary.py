@@ -1188,6 +1188,33 @@ def test_lines_of_the_calls_that_stream_in_a_tile_launchs_workspaces(tmp_path):
     assert taken > 1000
 
 
+def test_words_are_shared_only_in_a_tile_launchs_workspaces(tmp_path):
+    """Two column blocks count in one word only where a streamed launch may stand in a tile launch's workspaces
+    (csrc/kernels/iu8_stream_law.h, compiled here): every launch that does so shares its words, and the law's own K shares, which
+    list a counter a block, count in a word each (at two in one, 9 to 48 rows lost 2-5 %)."""
+    src, so = tmp_path / "shared.cpp", tmp_path / "shared.so"
+    src.write_text(f'#include "{iu8.ROOT}/include/saber_iu8.h"\n#include "{iu8.PKG}/csrc/host/rules.h"\n#include "{iu8.PKG}/csrc/kernels/iu8_stream_law.h"\n'
+                   'extern "C" int streams(const saber_iu8_desc *d, saber_iu8_desc *out) { return iu8::stream_in_tile_workspaces(*d, out); }\n'
+                   'extern "C" int two(int w8, int tm, long k) { return iu8_stream_shared_words(w8, tm, k); }\n'
+                   'extern "C" int words(int blocks, int shares, int w8, int tm, long k) {\n'
+                   '  return iu8_arrival_of(blocks - 1, shares, iu8_stream_shared_words(w8, tm, k)).word + 1;\n}\n')
+    lib_dir = os.path.dirname(iu8.lib()._name)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(src), "-o", str(so), f"-L{lib_dir}", "-lsaber_iu8", f"-Wl,-rpath,{lib_dir}"], check=True)
+    lib = ctypes.CDLL(str(so))
+    rng, called, split = np.random.default_rng(5), 0, 0
+    for _ in range(6000):
+        m, n, k, kind = int(rng.integers(9, 65)), 16 * int(rng.integers(180, 360)), 128 * int(rng.integers(60, 300)), int(rng.choice([iu8.W4, iu8.W8]))
+        d, out = iu8.resolve(kind, m, n, k), iu8.Desc()
+        tm = -(-m // 16)
+        if kind == iu8.W4 and lib.streams(ctypes.byref(d), ctypes.byref(out)):
+            called += 1
+            assert lib.two(0, tm, k) and 4 * lib.words(out.grid[0], out.ks, 0, tm, k) <= d.workspace("decode_counter").bytes
+        elif d.kernel.startswith(b"macaq_iu8_dec_") and d.ks > 1:
+            split += 1
+            assert not lib.two(kind == iu8.W8, tm, k) and 4 * lib.words(d.grid[0], d.ks, kind == iu8.W8, tm, k) == d.workspace("decode_counter").bytes
+    assert called > 300 and split > 300
+
+
 def test_routed_items_are_dealt_once_and_level(tmp_path):
     """The deal of the routed tile launches (csrc/kernels/moe_deal.h, compiled here): every light item goes to one position
     once, and no position's share (a heavy item counts `cost`) is more than one heavy item above another's that has light ones."""
