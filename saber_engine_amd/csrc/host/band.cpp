@@ -180,7 +180,7 @@ std::string band_toml() {
   o += "# macaq_iu8_pf_{w4,w8}_t*_r, before the other lines but the shares of K of tiles, from K = k_min, over rows_over up to rows_max rows. 16x16 up to few_rows rows of few_n\n";
   o += "# columns (from K = few_deep_k few_deep_n, int8 w8_few_n), and above, from n_64_rows columns up to 64 rows, with cu_count blocks at\n";
   o += "# most. int4 alone: 16x32 over few_rows rows with cu_count blocks; from 65 rows 32x32 with cu_count\n";
-  o += "# (blocks_32 below K = k_min_32) and 32x64 from K = k_min_64 with blocks_64 (up to rows_64 rows cu_count)\n";
+  o += "# (blocks_32 below K = k_min_32, below K = short_32_k up to short_32_n columns or short_32_rows rows, from K = short_32_rows_k short_32_rows_deep) and 32x64 from K = k_min_64 with blocks_64 (up to rows_64 rows cu_count)\n";
   put(o, "rows_over", ROWS_CELL_ROWS_OVER);
   put(o, "rows_max", ROWS_CELL_ROWS_MAX);
   put(o, "k_min", ROWS_CELL_K);
@@ -190,6 +190,11 @@ std::string band_toml() {
   put(o, "few_deep_k", ROWS_CELL_FEW_DEEP_K);
   put(o, "w8_few_n", ROWS_CELL_W8_FEW_N);
   put(o, "n_64_rows", ROWS_CELL_64_ROWS_N);
+  put(o, "short_32_k", ROWS_CELL_32_SHORT_K);
+  put(o, "short_32_n", ROWS_CELL_32_SHORT_N);
+  put(o, "short_32_rows", ROWS_CELL_32_SHORT_ROWS);
+  put(o, "short_32_rows_deep", ROWS_CELL_32_SHORT_ROWS_DEEP);
+  put(o, "short_32_rows_k", ROWS_CELL_32_SHORT_ROWS_K);
   put(o, "k_min_32", ROWS_CELL_32_K);
   put(o, "blocks_32", ROWS_CELL_32_BLOCKS);
   put(o, "k_min_64", ROWS_CELL_64_K);

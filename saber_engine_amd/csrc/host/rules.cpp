@@ -487,7 +487,10 @@ static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint
 // faster, 16 x 32 1.62, 32 x 32 1.45, 32 x 64 1.22, int8 16 x 16 1.32; none slower by more than 3 % but an int8 launch of 52 rows of 64 columns (5).
 // Where the lines lie: up to 48 rows the streamed law has a cell of few columns already: 512 x 2048 at 17 / 45 rows 3.0 / 3.2, here 3.2 /
 // 3.5, but 512 x 5120 4.5 / 5.9 -> 4.4 / 5.0 (int8 1024 x 5120 level, 80 x 2432 at 17 rows 3.4 -> 3.5). A second round loses: 16 x 16 on 1024 x 2048
-// at 200 rows (832 blocks) 1.02, on 1024 x 5120 at 400 0.64. 32 x 32 on more than 200 blocks at K = 1,024 0.95-1.06; 32 x 64 at K = 2,048 0.93-1.11, at
+// at 200 rows (832 blocks) 1.02, on 1024 x 5120 at 400 0.64. 32 x 32 on more than 200 blocks at K = 1,024 0.95-1.06; below K = 1,408 it loses where an
+// XCD reads many rows and many columns: at 193-256 rows of more than 480 columns 0.86-0.97 up to K = 1,024 and 0.94-1.01 to 1,280 (204 rows of
+// 752 x 896 4.5 on 64 x 64, here 5.1), at 161-192 0.93-1.00 and 1.01-1.06, 510 of 368 x 896 0.88, 472 of 352 x 1152 0.91; up to 160 rows 0.98-1.16, up to
+// 256 columns 0.98-1.4, from 1,408 on 0.99-1.57; 32 x 64 at K = 2,048 0.93-1.11, at
 // 5,120 1.06-1.20, at 17,408 1.23-1.50, on more than 208 blocks 0.96 where the 64-row tiles are full (190 rows of 2288 x 5632) and 1.2 where they are
 // not (up to 96 rows). Int8 64 x 64 tiles have nothing to unpack: 16 x 32 on 88-160 blocks 0.91-1.32, 7 % on average, not built. Below K = 768 a
 // launch is mostly its start (96 x 512 at 100 / 777 rows 3.8 -> 2.8, not taken). Three lines are held: 2,048 rows of 96 x 5120 would gain
@@ -512,7 +515,9 @@ static const RowsVariant *rows_cell(bool w8, uint32_t m, uint32_t n, uint32_t k,
   if (w8) return nullptr;
   if (blocks(16, 32) <= CU_COUNT) return W4_16X32;
   if (m <= DECODE_MAX_M) return nullptr;
-  if (blocks(32, 32) <= (k >= ROWS_CELL_32_K ? CU_COUNT : ROWS_CELL_32_BLOCKS)) return W4_32X32;
+  const uint32_t short_rows = k >= ROWS_CELL_32_SHORT_ROWS_K ? ROWS_CELL_32_SHORT_ROWS_DEEP : ROWS_CELL_32_SHORT_ROWS;
+  const bool pays_32 = k >= ROWS_CELL_32_SHORT_K || m <= short_rows || n <= ROWS_CELL_32_SHORT_N;
+  if (pays_32 && blocks(32, 32) <= (k >= ROWS_CELL_32_K ? CU_COUNT : ROWS_CELL_32_BLOCKS)) return W4_32X32;
   return blocks(32, 64) <= (m <= ROWS_CELL_64_ROWS ? CU_COUNT : ROWS_CELL_64_BLOCKS) && k >= ROWS_CELL_64_K ? W4_32X64 : nullptr;
 }
 

@@ -69,6 +69,7 @@ constexpr uint32_t ROWS_CELL_BLOCKS_MAX = 1u << 16;  // blocks a launch of them 
 constexpr uint32_t ROWS_CELL_ROWS_OVER = 16, ROWS_CELL_ROWS_MAX = 2047, ROWS_CELL_K = 768, ROWS_CELL_K_MAX = 1u << 24;
 constexpr uint32_t ROWS_CELL_FEW_ROWS = 48, ROWS_CELL_FEW_N = 256, ROWS_CELL_FEW_DEEP_N = 1024, ROWS_CELL_FEW_DEEP_K = 4096;
 constexpr uint32_t ROWS_CELL_W8_FEW_N = 512, ROWS_CELL_64_ROWS_N = 64;
+constexpr uint32_t ROWS_CELL_32_SHORT_K = 1408, ROWS_CELL_32_SHORT_N = 256, ROWS_CELL_32_SHORT_ROWS = 160, ROWS_CELL_32_SHORT_ROWS_DEEP = 192, ROWS_CELL_32_SHORT_ROWS_K = 1152;
 constexpr uint32_t ROWS_CELL_32_K = 2048, ROWS_CELL_32_BLOCKS = 200, ROWS_CELL_64_K = 4096, ROWS_CELL_64_ROWS = 96, ROWS_CELL_64_BLOCKS = 208;
 constexpr uint32_t HAD_T1024_ROWS = 256, HAD_T1024_WIDTH = 4096;  // the Hadamard-basis producers' 16-wave forms: up to / from
 constexpr uint32_t T1024_WIDTH_OVER = 4096;

@@ -989,6 +989,16 @@ def test_lines_of_the_streamed_cells_on_row_tiles():
         iu8.describe("macaq_iu8_pf_w4_t16x16_r", 1 << 20, 96, 1024)   # more blocks than a launch holds
 
 
+def test_32x32_row_tiles_of_a_short_k():
+    """Below K = 1,408 32 x 32 blocks lose to 64 x 64 tiles on outputs of more than 160 rows (192 from K = 1,152) and more than 256 columns
+    (204 rows of 752 x 896 5.1 us for 4.5): such a launch is on tiles, either side of each line."""
+    for (m, n, k), cell in {(204, 752, 896): "t64x64_s", (510, 368, 896): "t64x64_s", (241, 736, 768): "t64x64_s", (160, 928, 896): "t32x32_r", (161, 928, 896): "t64x64_s",
+                            (161, 928, 1024): "t64x64_s", (192, 928, 1152): "t32x32_r", (193, 864, 1152): "t64x64_s", (193, 864, 1280): "t64x64_s", (193, 864, 1408): "t32x32_r",
+                            (750, 256, 768): "t32x32_r", (700, 272, 768): "t64x64_s", (700, 272, 1408): "t32x32_r",
+                            (1593, 80, 768): "t32x32_r", (66, 2000, 768): "t32x32_r"}.items():
+        assert iu8.resolve(iu8.W4, m, n, k).kernel.decode() == "macaq_iu8_pf_w4_" + cell, (m, n, k)
+
+
 def test_row_tiles_leave_operands_past_4_gib_to_the_other_cells():
     """An operand past 4 GiB, which the tile GEMM refuses by name, is refused for an output of few tiles as for any other, on either
     side of the limit in rows, columns and K; up to 64 rows the streamed form, which has no such limit, has it."""
