@@ -155,6 +155,7 @@ std::string band_toml() {
   o += "# K shares of a streamed decode launch: with b = ceil(n / 64), min(shares_max, cu_count / b) of them where that is shares_min\n";
   o += "# at least and 4 * b at least three quarters of cu_count, from K = k_min (k_min_16_rows up to 16 rows, else k_min_4096_columns\n";
   o += "# up to 4,096 columns). int4 from 33 rows: K >= 16384 is on tiles before this, where the bands say so\n";
+  o += "# (saber_iu8_gemm alone streams there, up to 64 rows, on these shares in the tile launch's workspaces; the descriptor is the tile launch)\n";
   put(o, "rows_over", STREAM_SPLIT_ROWS_OVER);
   put(o, "rows_max", STREAM_SPLIT_ROWS_MAX);
   put(o, "shares_min", STREAM_SPLIT_SHARES_MIN);
@@ -177,7 +178,7 @@ std::string band_toml() {
   put(o, "aligned_rows", IU8_STREAM_ALIGNED_ROWS);
   put(o, "aligned_last_max", IU8_STREAM_ALIGNED_LAST);
   o += "\n[row_tiles]\n";
-  o += "# macaq_iu8_pf_{w4,w8}_t*_r, before the other lines but the shares of K of tiles, from K = k_min, over rows_over up to rows_max rows. 16x16 up to few_rows rows of few_n\n";
+  o += "# macaq_iu8_pf_{w4,w8}_t*_r, before the other lines but the shares of K of tiles, from K = k_min, over rows_over up to rows_max rows, operands up to 4 GiB. 16x16 up to few_rows rows of few_n\n";
   o += "# columns (from K = few_deep_k few_deep_n, int8 w8_few_n), and above, from n_64_rows columns up to 64 rows, with cu_count blocks at\n";
   o += "# most. int4 alone: 16x32 over few_rows rows with cu_count blocks; from 65 rows 32x32 with cu_count\n";
   o += "# (blocks_32 below K = k_min_32, below K = short_32_k up to short_32_n columns or short_32_rows rows, from K = short_32_rows_k short_32_rows_deep) and 32x64 from K = k_min_64 with blocks_64 (up to rows_64 rows cu_count)\n";

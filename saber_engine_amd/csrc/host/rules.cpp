@@ -484,14 +484,14 @@ static const WideVariant *stream_wide_cell(bool w8, uint32_t m, uint32_t n, uint
 // 777 11.8 / 11.9 -> 5.9 / 8.4, 1024 at 45 / 100 / 200 6.4 / 11.9 / 11.8 -> 5.1 / 7.5 / 8.8, 2048 at 100 11.9 -> 7.9, 5120 at 80 / 96 12.4 / 12.4
 // -> 10.2 / 10.4, 512 at 777 12.0 -> 10.4; 96 x 17408 at 400 32.6 -> 11.4, 256 x 1024 at 100 / 777 4.8 / 4.8 -> 3.7 / 3.7.
 // Int8: 96 x 5120 at 64 / 200 8.0 / 9.2 -> 5.8 / 6.8, 512 x 5120 at 100 9.3 -> 7.7. Over 240 shapes drawn over the whole of it 16 x 16 1.83 times
-// faster, 16 x 32 1.62, 32 x 32 1.45, 32 x 64 1.22, int8 16 x 16 1.32; none slower by more than 3 % but an int8 launch of 52 rows of 64 columns (5).
+// faster, 16 x 32 1.62, 32 x 32 1.45, 32 x 64 1.22, int8 16 x 16 1.32.
 // Where the lines lie: up to 48 rows the streamed law has a cell of few columns already: 512 x 2048 at 17 / 45 rows 3.0 / 3.2, here 3.2 /
 // 3.5, but 512 x 5120 4.5 / 5.9 -> 4.4 / 5.0 (int8 1024 x 5120 level, 80 x 2432 at 17 rows 3.4 -> 3.5). A second round loses: 16 x 16 on 1024 x 2048
 // at 200 rows (832 blocks) 1.02, on 1024 x 5120 at 400 0.64. 32 x 32 on more than 200 blocks at K = 1,024 0.95-1.06; below K = 1,408 it loses where an
 // XCD reads many rows and many columns: at 193-256 rows of more than 480 columns 0.86-0.97 up to K = 1,024 and 0.94-1.01 to 1,280 (204 rows of
 // 752 x 896 4.5 on 64 x 64, here 5.1), at 161-192 0.93-1.00 and 1.01-1.06, 510 of 368 x 896 0.88, 472 of 352 x 1152 0.91; up to 160 rows 0.98-1.16, up to
 // 256 columns 0.98-1.4, from 1,408 on 0.99-1.57; 32 x 64 at K = 2,048 0.93-1.11, at
-// 5,120 1.06-1.20, at 17,408 1.23-1.50, on more than 208 blocks 0.96 where the 64-row tiles are full (190 rows of 2288 x 5632) and 1.2 where they are
+// 5,120 1.06-1.20, at 17,408 1.23-1.50 (those against 64 x 64 tiles of one wave a wave tile; against their two k-waves 0.94-1.28 at 4,096-6,144, 7 % on average), on more than 208 blocks 0.96 where the 64-row tiles are full (190 rows of 2288 x 5632) and 1.2 where they are
 // not (up to 96 rows). Int8 64 x 64 tiles have nothing to unpack: 16 x 32 on 88-160 blocks 0.91-1.32, 7 % on average, not built. Below K = 768 a
 // launch is mostly its start (96 x 512 at 100 / 777 rows 3.8 -> 2.8, not taken). Three lines are held: 2,048 rows of 96 x 5120 would gain
 // as 1,500 do, 49-64 rows of fewer than 64 columns as 64 columns do, and the tile launches that share K (96 x 17408 at 45 rows 17.0 -> 9.5).
@@ -679,7 +679,7 @@ int resolve(int wkind, uint32_t m, uint32_t n, uint32_t k, saber_iu8_desc *out) 
   // 16384 x 5120 36.9 / 39.4 -> 29.3 / 32.4, 227 of 16384 x 4096 1.25, 152 of 14336 x 256 1.26 times faster. From K = 2,048 (2,048 level to 1.11, 3,072 1.07-1.27, 5,120
   // and more 1.05-1.38, 1,024 0.95-1.05), from 4,096 on a count that is not whole eighths (854 rows of 1776 x 3072 0.88); with no more 64 x 64 tiles than
   // CUs those stay (160 of 5120 x 3072 0.80). Over 305 shapes of 65 to 4,096 rows that moved, drawn after the lines, 128 x 64 1.20 times faster, 128 x 128 1.26, the
-  // slowest 0.99. 256 rows are held on the 64 x 128 cell (5120 x 5120 21.3 for 18.6).
+  // slowest 0.99. 256 rows are held on the 64 x 128 cell (5120 x 5120 / 6144 / 17408 21.7 / 24.7 / 63.5 for 18.9 / 21.5 / 53.1).
   if (w8 && m > 64) {
     auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)((n + bn - 1) / bn) * ((m + bm - 1) / bm); };
     static const PfVariant *const T128X160 = pf_variant("macaq_iu8_pf_w8_t128x160"), *const T128X64 = pf_variant("macaq_iu8_pf_w8_t128x64_s"),

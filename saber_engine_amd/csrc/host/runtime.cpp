@@ -807,15 +807,15 @@ uint32_t saber_iu8_moe_tiles_cap_shared(uint32_t tokens, uint32_t topk, uint32_t
   return saber_iu8_moe_tiles_cap(tokens, topk, experts, tile_blocks) + ((tokens + 15) / 16 + g - 1) / g;
 }
 // Rows a tile (x16). 16-row tiles on the streaming cell while routes are few (up to 7 routes an
-// expert on average); above, the MFMA cells, whose sparse forms make a thinly filled tile cost about
-// its weight traffic and which stream an expert's weights once instead of once a 16-row tile:
-// 128-row tiles while an expert's routes on average do not fill one (the two-cell kernels, which run
-// the thin tiles on a small cell), 256-row tiles (one tile an expert more often than not, on the
-// dense GEMM's fastest shape) from 128 routes an expert. Speed data of this card, 128 experts, top-8,
-// 4096 x 1536, us a layer at tile_blocks 1 / 8 / 16: T=32 255 / 309 / 328, T=64 296 / 335 / 347,
-// T=80 318 / 340, T=128 363 / 347 / 362, T=256 730 / 293 / 298, T=512 1282 / 315 / 319,
-// T=1024 2349 / 377 / 402, T=1280 - / 425 / 458, T=1536 - / 472 / 528, T=1792 - / 493 / 516,
-// T=1920 - / 526 / 532, T=2048 - / 586 / 544, T=4096 - / 960 / 916.
+// expert on average); above, the MFMA cells, which stream an expert's weights once instead of once a
+// 16-row tile and run the thin tiles on a small cell: 128-row tiles while an expert's routes on average
+// do not fill one, 256-row tiles (one tile an expert more often than not, on the dense GEMM's fastest
+// shape) from 128 routes an expert. Speed data of this card, 128 experts, top-8, 4096 x 1536, logits
+// N(0, 1), us a layer at tile_blocks 1 / 8 / 16: T=16 136 / 166, T=64 229 / 239, T=80 244 / 243, T=112 270 /
+// 247, T=128 283 / 247, T=256 432 / 256 / 255, T=512 - / 280 / 276, T=1024 - / 333 / 358, T=1536 - / 391 / 434,
+// T=1792 - / 427 / 453, T=1920 - / 451 / 465, T=2048 - / 499 / 483, T=2304 - / 579 / 522, T=4096 - / 836 / 793.
+// (The first line is older than the small cell: 81 to 112 tokens would gain up to 8 %. It is held, with
+// the two-launch back half that goes with 16-row tiles.)
 uint32_t saber_iu8_moe_tile_blocks(uint32_t tokens, uint32_t topk, uint32_t experts) {
   const uint64_t routes = (uint64_t)tokens * topk;
   if (routes <= 7ull * experts) return 1u;
